@@ -892,8 +892,8 @@ int lv_nearest_polygon(lv_ctx *ctx, int32_t m, const double *q, int32_t *idx)
     LV_HIP_CHECK(hipMalloc(&dq.p, sizeof(double) * 2 * m));
     LV_HIP_CHECK(hipMalloc(&di.p, sizeof(int) * m));
     LV_HIP_CHECK(hipMemcpyAsync(dq.p, q, sizeof(double) * 2 * m, hipMemcpyHostToDevice, ctx->s));
-    LV_HIP_CHECK(lv_launch_nearest(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->path_i,
-                                   ctx->path_rr, m, (const double *)dq.p, (int *)di.p, ctx->s));
+    LV_HIP_CHECK(lv_launch_nearest(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
+                                   ctx->max_items, ctx->path_i, ctx->path_rr, m, (const double *)dq.p, (int *)di.p, ctx->s));
     LV_HIP_CHECK(hipMemcpyAsync(idx, di.p, sizeof(int) * m, hipMemcpyDeviceToHost, ctx->s));
     LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
     for (int t = 0; t < m; t++)
@@ -915,8 +915,8 @@ int lv_movingls(lv_ctx *ctx, int32_t order, int32_t field, int32_t comp, double 
     const size_t bytes = sizeof(double) * (size_t)N * ctx->n;
     dev_buf d;
     LV_HIP_CHECK(hipMalloc(&d.p, bytes));
-    LV_HIP_CHECK(lv_launch_movingls(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->path_i,
-                                    ctx->path_rr, order, f, h, (double *)d.p, ctx->s));
+    LV_HIP_CHECK(lv_launch_movingls(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
+                                    ctx->max_items, ctx->path_i, ctx->path_rr, order, f, h, (double *)d.p, ctx->s));
     LV_HIP_CHECK(hipMemcpyAsync(coeffs, d.p, bytes, hipMemcpyDeviceToHost, ctx->s));
     LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
     return LV_OK;
@@ -935,8 +935,8 @@ int lv_point_values(lv_ctx *ctx, int32_t m, const double *q, int32_t field, int3
     LV_HIP_CHECK(hipMalloc(&dq.p, sizeof(double) * 2 * m));
     LV_HIP_CHECK(hipMalloc(&dout.p, sizeof(double) * m));
     LV_HIP_CHECK(hipMemcpyAsync(dq.p, q, sizeof(double) * 2 * m, hipMemcpyHostToDevice, ctx->s));
-    LV_HIP_CHECK(lv_launch_point_value(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->path_i,
-                                       ctx->path_rr, m, (const double *)dq.p, f, ctx->g.h, (double *)dout.p, ctx->s));
+    LV_HIP_CHECK(lv_launch_point_value(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
+                                       ctx->max_items, ctx->path_i, ctx->path_rr, m, (const double *)dq.p, f, ctx->g.h, (double *)dout.p, ctx->s));
     LV_HIP_CHECK(hipMemcpyAsync(out, dout.p, sizeof(double) * m, hipMemcpyDeviceToHost, ctx->s));
     LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
     for (int t = 0; t < m; t++)
@@ -963,8 +963,8 @@ int lv_point_values_noalloc(lv_ctx *ctx, int32_t m, const double *q, int32_t fie
     double *dq = ctx->scratch;                       // q1[m], q2[m]
     double *dout = ctx->scratch + 2 * (size_t)m;     // the m values
     LV_HIP_CHECK(hipMemcpyAsync(dq, q, sizeof(double) * 2 * m, hipMemcpyHostToDevice, ctx->s));
-    LV_HIP_CHECK(lv_launch_point_value(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->path_i,
-                                       ctx->path_rr, m, (const double *)dq, f, ctx->g.h, dout, ctx->s));
+    LV_HIP_CHECK(lv_launch_point_value(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
+                                       ctx->max_items, ctx->path_i, ctx->path_rr, m, (const double *)dq, f, ctx->g.h, dout, ctx->s));
     LV_HIP_CHECK(hipMemcpyAsync(out, dout, sizeof(double) * m, hipMemcpyDeviceToHost, ctx->s));
     LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
     for (int t = 0; t < m; t++)

@@ -86,3 +86,38 @@ def test_populate_initialisers(lv, gpu):
     seen = []
     g = lv.populate_rect(lv.VoronoiGrid(lv.UnitRectangle(), dr), ic=lambda grid: seen.append(grid.n))
     assert seen == [361]
+
+
+@pytest.mark.parametrize("K,hf", [(8, 2.0), (15, 2.0), (17, 3.0), (24, 2.0)])
+def test_walks_on_short_and_long_periods_match_oracle(lv, oracle, gpu, K, hf):
+    """the expansion's walk keeps the reference's bound where a period is shorter than r_max + h and two
+    cells (a seed can then be listed within h twice) and stops at h^2 where it is longer; on a plain
+    lattice too, where seeds lie at exactly h"""
+    print("walks K=%d h=%g dr" % (K, hf), flush=True)
+    dr = 1.0 / K
+    rng = np.random.default_rng(K)
+    for jitter in (0.2, 0.0):
+        x = lv.inputs.jittered_lattice(K, K, dr, jitter=jitter, seed=0x5EED0920)
+        grid = lv.VoronoiGrid(lv.UnitRectangle(), dr, xperiodic=True, yperiodic=True, positions=x)
+        lv.remesh(grid)
+        w = mls_ref.Walk(oracle.Grid((0.0, 0.0), (1.0, 1.0), dr, xperiodic=True, yperiodic=True), x)
+        f = np.cos(7 * x[:K * K]) + x[K * K:] ** 2
+        grid.set_soa("P", f)
+        got = lv.movingls(1, grid, "P", h=hf * dr)
+        ref = np.array([mls_ref.movingls(w, 1, f, i, hf * dr) for i in range(grid.n)])
+        assert np.max(np.abs(got - ref) / np.abs(ref).max()) <= 1e-12
+        q = rng.random((40, 2))
+        assert list(lv.nearest_polygon(grid, q)) == [mls_ref.nearest_polygon(w, a, b) for a, b in q]
+
+
+def test_many_queries_equal_few(lv, oracle, gpu):
+    """calls of many queries take fewer lanes a query: the same polygons, and values that differ by the
+    order of at most 90 FP64 additions (1e-13)"""
+    print("many queries", flush=True)
+    grid, op, x, dr = make_pair(lv, oracle, "walls", K=40, seed=0x5EED0921)
+    q = np.random.default_rng(3).random((33001, 2))
+    idx, val = lv.nearest_polygon(grid, q), lv.point_value(grid, q, "P")
+    few = np.r_[0:2000, 31001:33001]
+    assert np.array_equal(idx[few], lv.nearest_polygon(grid, q[few]))
+    assert rel_err(val[few], lv.point_value(grid, q[few], "P")) <= 1e-13
+    assert idx[0] == lv.nearest_polygon(grid, q[0])[0]
