@@ -33,6 +33,7 @@ constexpr float R_FLOOR = 1e-4f;
 constexpr float OCLAMP = 8.0f;
 
 typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 v8bf;
+typedef __attribute__((__vector_size__(8 * sizeof(uint16_t)))) uint16_t v8us;
 typedef __attribute__((__vector_size__(16 * sizeof(float)))) float v16f;
 
 __device__ __forceinline__ __bf16 f2bf(float f) { return (__bf16)f; }
@@ -547,24 +548,32 @@ __global__ __launch_bounds__(B) void k_loss_partials(int n, int P, const float *
 // Relative spread of Mt At over the probes (invariant to the scale of Mt, as CG is):
 //   c = (1/P) sum_q v_q.y_q / |v_q|^2,   S = (1/P) sum_q |y_q - c v_q|^2 / |v_q|^2,   L = S / c^2.
 // out[0] = L, out[1] = c, out[2] = S, out[3+q] = 1/|v_q|^2
-__global__ __launch_bounds__(64) void k_loss_final(int P, int nb, const double *__restrict__ part,
-                                                   double *__restrict__ out)
+// A wavefront sums a probe's partials (they were one thread's 3 P nb dependent loads: 37 us at P = 8).
+__global__ __launch_bounds__(B) void k_loss_final(int P, int nb, const double *__restrict__ part,
+                                                  double *__restrict__ out)
 {
-    if (threadIdx.x != 0) return;
-    double yy[64], vy[64], vv[64];
-    double c = 0.0;
-    for (int q = 0; q < P; q++) {
+    __shared__ double yy[64], vy[64], vv[64];
+    const int lane = threadIdx.x & 63;
+    for (int q = threadIdx.x >> 6; q < P; q += B / 64) {
         double a = 0.0, b = 0.0, d = 0.0;
-        for (int k = 0; k < nb; k++) {
+        for (int k = lane; k < nb; k += 64) {
             a += part[(size_t)(3 * q) * nb + k];
             b += part[(size_t)(3 * q + 1) * nb + k];
             d += part[(size_t)(3 * q + 2) * nb + k];
         }
-        yy[q] = a;
-        vy[q] = b;
-        vv[q] = d;
-        c += (d > 0.0) ? b / d : 0.0;
+        a = lv_wave_sum(a);
+        b = lv_wave_sum(b);
+        d = lv_wave_sum(d);
+        if (lane == 0) {
+            yy[q] = a;
+            vy[q] = b;
+            vv[q] = d;
+        }
     }
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    double c = 0.0;
+    for (int q = 0; q < P; q++) c += (vv[q] > 0.0) ? vy[q] / vv[q] : 0.0;
     c /= P;
     double S = 0.0;
     for (int q = 0; q < P; q++) {
@@ -595,7 +604,8 @@ __global__ __launch_bounds__(B) void k_grad_y(int n, int P, const float *__restr
 __global__ __launch_bounds__(B) void k_grad_w(int n, int P, const int *__restrict__ rp, const int *__restrict__ cols,
                                               const float *__restrict__ w, const float *__restrict__ gy,
                                               const float *__restrict__ u, const float *__restrict__ delta,
-                                              float *__restrict__ G, float *__restrict__ don)
+                                              const float *__restrict__ on, float *__restrict__ G,
+                                              float *__restrict__ don)
 {
     const int i = blockIdx.x * B + threadIdx.x;
     if (i >= n) return;
@@ -608,7 +618,7 @@ __global__ __launch_bounds__(B) void k_grad_w(int n, int P, const int *__restric
         const float sg = (w[p] > 0.0f) ? 1.0f : ((w[p] < 0.0f) ? -1.0f : 0.0f);
         G[p] = g + gd * sg;
     }
-    don[i] = gd * delta[i];
+    don[i] = (fabsf(on[i]) < OCLAMP) ? gd * delta[i] : 0.0f;
 }
 
 __global__ __launch_bounds__(B) void k_grad_o(int E, const int *__restrict__ rev, const float *__restrict__ G,
@@ -623,54 +633,73 @@ __global__ __launch_bounds__(B) void k_grad_o(int E, const int *__restrict__ rev
     doe[p] = (q >= 0) ? 0.5f * (G[p] + G[q]) * w[p] * live : G[p] * w[p] * live;
 }
 
-__global__ __launch_bounds__(B) void k_clamp_mask(int n, const float *__restrict__ on, float *__restrict__ don)
-{
-    const int i = blockIdx.x * B + threadIdx.x;
-    if (i < n && !(fabsf(on[i]) < OCLAMP)) don[i] = 0.0f;
-}
-
 // ---- backward of the decoders -----------------------------------------------------------------
 
-// dX[t][c] = do[t] * v[c] (+= if accumulate); partial sums of do[t]*X[t][c] and do[t] per block
-__global__ __launch_bounds__(B) void k_decode_back(int count, const __bf16 *__restrict__ Xb,
-                                                   const float *__restrict__ Xf, const float *__restrict__ v,
-                                                   const float *__restrict__ dout, float *__restrict__ dX, int accum,
+// The reductions over edges or nodes below (decoders, biases, encoders) give a lane a channel and a
+// wavefront every (4 gridDim.x)-th row: loads and stores of a row are one coalesced run, and the sums stay in
+// FP64 registers until a block stores one partial a channel, summed by k_sum_small.  Adding each product to
+// LDS with atomics instead serialised 64 lanes on one address (k_decode_back 138 us at 48 x 48), and one
+// partial per 256 products left a handful of threads a chain of thousands of dependent loads
+// (k_sum_parts up to 500 us).
+constexpr int RED_BLOCKS = 256;  // blocks of a reduction: 1024 wavefronts, at most 256 partials to sum
+
+// the four wavefronts' sums of this lane's channel, in wavefront order (valid in wavefront 0)
+__device__ __forceinline__ double block_channel_sum(double v, double (*s)[H])
+{
+    const int c = threadIdx.x & 63, w = threadIdx.x >> 6;
+    __syncthreads();
+    s[w][c] = v;
+    __syncthreads();
+    return ((s[0][c] + s[1][c]) + s[2][c]) + s[3][c];
+}
+
+// dX[t][c] = do[t] * v[c]; partial sums of do[t]*X[t][c] and do[t] per block
+template <typename TX>
+__global__ __launch_bounds__(B) void k_decode_back(int count, const TX *__restrict__ X, const float *__restrict__ v,
+                                                   const float *__restrict__ dout, float *__restrict__ dX,
                                                    float *__restrict__ part /* [nb][H+1] */)
 {
-    __shared__ float sp[H + 1];
-    if (threadIdx.x <= H) sp[threadIdx.x] = 0.0f;
-    __syncthreads();
-    const int64_t t = (int64_t)blockIdx.x * B + threadIdx.x;
-    if (t < count) {
+    __shared__ double sp[B / 64][H];
+    const int c = threadIdx.x & 63;
+    const float vc = v[c];
+    double a = 0.0, b = 0.0;
+#pragma unroll 4
+    for (int64_t t = (int64_t)blockIdx.x * (B / 64) + (threadIdx.x >> 6); t < count; t += (int64_t)gridDim.x * (B / 64)) {
         const float g = dout[t];
-        for (int c = 0; c < H; c++) {
-            const float x = Xf ? Xf[t * H + c] : bf2f(Xb[t * H + c]);
-            const float val = g * v[c];
-            if (accum) dX[t * H + c] += val;
-            else dX[t * H + c] = val;
-            atomicAdd(&sp[c], g * x);
-        }
-        atomicAdd(&sp[H], g);
+        a += (double)g * (double)(float)X[t * H + c];
+        b += (double)g;
+        dX[t * H + c] = g * vc;
     }
-    __syncthreads();
-    if (threadIdx.x <= H) part[(size_t)blockIdx.x * (H + 1) + threadIdx.x] = sp[threadIdx.x];
+    a = block_channel_sum(a, sp);
+    b = block_channel_sum(b, sp);
+    if (threadIdx.x < H) part[(size_t)blockIdx.x * (H + 1) + c] = (float)a;
+    if (threadIdx.x == 0) part[(size_t)blockIdx.x * (H + 1) + H] = (float)b;
 }
 
 // ---- backward of a message-passing layer ------------------------------------------------------
 
-// dM[p] += dH[src p] / deg(src);  dZ = dM * (M > 0)  (BF16 copy for the MFMA)
+// dM[p] + dH[src p] / deg(src), times (M > 0): dZ (BF16 for the MFMA), and per block the partial
+// column sums of dZ, the bias gradient.  dM row p starts at dM + p * ld (the e part of the layer
+// above's dX, or the decoder's dE).
 __global__ __launch_bounds__(B) void k_mp_dz(int E, const int *__restrict__ src, const int *__restrict__ rp,
                                              const float *__restrict__ dH, const __bf16 *__restrict__ Mb,
-                                             float *__restrict__ dM, __bf16 *__restrict__ dZb)
+                                             const float *__restrict__ dM, int ld, __bf16 *__restrict__ dZb,
+                                             float *__restrict__ part /* [nb][H] */)
 {
-    const int64_t t = (int64_t)blockIdx.x * B + threadIdx.x;
-    if (t >= (int64_t)E * H) return;
-    const int64_t p = t / H;
-    const int c = (int)(t % H);
-    const int i = src[p];
-    const float deg = (float)(rp[i + 1] - rp[i]);
-    const float g = dM[t] + dH[(size_t)i * H + c] / deg;
-    dZb[t] = f2bf((bf2f(Mb[t]) > 0.0f) ? g : 0.0f);
+    __shared__ double sp[B / 64][H];
+    const int c = threadIdx.x & 63;
+    double a = 0.0;
+#pragma unroll 4
+    for (int64_t p = (int64_t)blockIdx.x * (B / 64) + (threadIdx.x >> 6); p < E; p += (int64_t)gridDim.x * (B / 64)) {
+        const int i = src[p];
+        const float deg = (float)(rp[i + 1] - rp[i]);
+        const float g = dM[(size_t)p * ld + c] + dH[(size_t)i * H + c] / deg;
+        const __bf16 z = f2bf((bf2f(Mb[p * H + c]) > 0.0f) ? g : 0.0f);
+        dZb[p * H + c] = z;
+        a += (double)bf2f(z);
+    }
+    a = block_channel_sum(a, sp);
+    if (threadIdx.x < H) part[(size_t)blockIdx.x * H + c] = (float)a;
 }
 
 // dX = dZ W^T: a wavefront computes 32 edges x 192 features; Wk is W row-major (Wk[k*64 + c])
@@ -713,37 +742,58 @@ __global__ __launch_bounds__(256) void k_mp_dx(int E, const __bf16 *__restrict__
         }
 }
 
-// dW partial over a chunk of 64 edges per wavefront: dW[f][c] = sum_p X[p][f] dZ[p][c].
-// Each wavefront owns one 32x32 (f, c) tile for its chunk; 12 tiles cover 192 x 64.
+// dW partial over a chunk of edges: dW[f][c] = sum_p X[p][f] dZ[p][c].  Each wavefront owns one 32x32
+// (f, c) tile for its chunk; 12 tiles cover 192 x 64, and block row y's four take the h_src (0), h_dst (1)
+// or e (2) features.  The MFMA's k runs over edges, so a lane's operand is a column of X or dZ: the rows
+// come into LDS with 16-byte loads, DW_ROWS edges at a time, and the columns are read from there (a row
+// stride of 72 puts the two half-wavefronts' rows, 8 apart, on different banks).  2-byte gathers from
+// memory, one edge index and one branch each, took 43 us a layer at 48 x 48 (13,800 edges), with the
+// indices in LDS and several steps' loads in flight 35 us, this 8.6 us.
 // Partials land in part[chunk][192*64].
+constexpr int DW_CHUNK = 256, DW_ROWS = 128, DW_LD = 72;
+
 __global__ __launch_bounds__(256) void k_mp_dw(int E, const int *__restrict__ src, const int *__restrict__ dst,
                                                const __bf16 *__restrict__ Hb, const __bf16 *__restrict__ Ein,
-                                               const __bf16 *__restrict__ dZb, int chunk, float *__restrict__ part)
+                                               const __bf16 *__restrict__ dZb, float *__restrict__ part)
 {
+    __shared__ __attribute__((aligned(16))) uint16_t sx[DW_ROWS * DW_LD], sz[DW_ROWS * DW_LD];
     const int lane = threadIdx.x & 63;
     const int wave = blockIdx.y * 4 + (threadIdx.x >> 6);   // 0..11 (3 blocks of 4 waves)
     const int ft = wave / 2, ct = wave % 2;                  // f tile 0..5, c tile 0..1
-    const int64_t c0 = (int64_t)blockIdx.x * chunk;
     const int r = lane & 31, half = lane >> 5;
+    const int *idx = blockIdx.y == 0 ? src : dst;
+    const __bf16 *Xg = blockIdx.y == 2 ? Ein : Hb;
+    const uint16_t *X = sx + 32 * (ft & 1) + r, *Z = sz + 32 * ct + r;
+    const int row0 = threadIdx.x >> 3, col = (threadIdx.x & 7) * 8;  // 8 lanes load a row
     v16f acc = {0};
-    const int f = 32 * ft + r;  // this lane's A row (feature)
-    for (int64_t s = 0; s < chunk; s += 16) {
-        const int64_t e = c0 + s + 8 * half;  // this lane's 8 edges (k)
-        v8bf av, bv;
+    for (int h = 0; h < DW_CHUNK; h += DW_ROWS) {
+        const int64_t c0 = (int64_t)blockIdx.x * DW_CHUNK + h;
+        __syncthreads();
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int64_t p = e + j;
-            float x = 0.0f, g = 0.0f;
-            if (p < E) {
-                if (f < H) x = bf2f(Hb[(size_t)src[p] * H + f]);
-                else if (f < 2 * H) x = bf2f(Hb[(size_t)dst[p] * H + (f - H)]);
-                else x = bf2f(Ein[(size_t)p * H + (f - 2 * H)]);
-                g = bf2f(dZb[(size_t)p * H + 32 * ct + r]);
-            }
-            av[j] = f2bf(x);
-            bv[j] = f2bf(g);
+        for (int q = 0; q < DW_ROWS / 32; q++) {
+            // past the last edge the loads take that edge again and dZ is zero: the product adds nothing
+            const int e = row0 + 32 * q;
+            const int p = (int)min(c0 + e, (int64_t)E - 1);
+            const int node = idx[p];
+            v8us x = *(const v8us *)(Xg + (size_t)(blockIdx.y == 2 ? p : node) * H + col);
+            v8us z = *(const v8us *)(dZb + (size_t)p * H + col);
+            if (c0 + e >= E) z = (v8us){0};
+            *(v8us *)(sx + e * DW_LD + col) = x;
+            *(v8us *)(sz + e * DW_LD + col) = z;
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av, bv, acc, 0, 0, 0);
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < DW_ROWS; s += 16) {
+            v8us xb, gb;
+#pragma unroll
+            for (int j = 0; j < 8; j++) {
+                const int e = s + 8 * half + j;  // this lane's 8 edges (k)
+                xb[j] = X[e * DW_LD];
+                gb[j] = Z[e * DW_LD];
+            }
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8bf, xb), __builtin_bit_cast(v8bf, gb),
+                                                          acc, 0, 0, 0);
+        }
     }
     float *o = part + (size_t)blockIdx.x * (KX * H);
 #pragma unroll
@@ -753,18 +803,8 @@ __global__ __launch_bounds__(256) void k_mp_dw(int E, const int *__restrict__ sr
     }
 }
 
-// db partial: column sums of dZ per block of edges
-__global__ __launch_bounds__(H) void k_mp_db(int E, const __bf16 *__restrict__ dZb, int chunk, float *__restrict__ part)
-{
-    const int c = threadIdx.x;
-    const int64_t c0 = (int64_t)blockIdx.x * chunk;
-    float s = 0.0f;
-    for (int64_t p = c0; p < c0 + chunk && p < E; p++) s += bf2f(dZb[(size_t)p * H + c]);
-    part[(size_t)blockIdx.x * H + c] = s;
-}
-
-// dH_l[i] = dH_{l+1}[i] + sum_{p in row i} dX[p][0:64] + sum_{p in row i} dX[rev p][64:128];
-// dE_l[p] = dX[p][128:192]
+// dH_l[i] = dH_{l+1}[i] + sum_{p in row i} dX[p][0:64] + sum_{p in row i} dX[rev p][64:128]
+// (dE_l[p] is dX[p][128:192], read from there)
 __global__ __launch_bounds__(B) void k_mp_dh(int n, const int *__restrict__ rp, const int *__restrict__ rev,
                                              const float *__restrict__ dX, float *__restrict__ dH)
 {
@@ -780,55 +820,103 @@ __global__ __launch_bounds__(B) void k_mp_dh(int n, const int *__restrict__ rp, 
     dH[t] = s;
 }
 
-__global__ __launch_bounds__(B) void k_mp_de(int E, const float *__restrict__ dX, float *__restrict__ dE)
-{
-    const int64_t t = (int64_t)blockIdx.x * B + threadIdx.x;
-    if (t >= (int64_t)E * H) return;
-    const int64_t p = t / H;
-    const int c = (int)(t % H);
-    dE[t] = dX[p * KX + 2 * H + c];
-}
-
-// encoder backward partials: dW[k][c] = sum_t in[t][k] dZ[t][c], db[c] = sum_t dZ[t][c], dZ = dOut*(Out>0)
+// encoder backward partials: dW[k][c] = sum_t in[t][k] dZ[t][c], db[c] = sum_t dZ[t][c], dZ = dOut*(Out>0);
+// row t of dOut starts at dout + t * ld
 __global__ __launch_bounds__(B) void k_encode_back(int count, const float *__restrict__ in,
                                                    const __bf16 *__restrict__ outb, const float *__restrict__ dout,
-                                                   float *__restrict__ part /* [nb][5*H] */)
+                                                   int ld, float *__restrict__ part /* [nb][5*H] */)
 {
-    __shared__ float sp[5 * H];
-    for (int k = threadIdx.x; k < 5 * H; k += B) sp[k] = 0.0f;
-    __syncthreads();
-    const int64_t t = (int64_t)blockIdx.x * B + threadIdx.x;
-    if (t < (int64_t)count * H) {
-        const int64_t r = t / H;
-        const int c = (int)(t % H);
-        const float g = (bf2f(outb[t]) > 0.0f) ? dout[t] : 0.0f;
-        if (g != 0.0f) {
-#pragma unroll
-            for (int k = 0; k < 4; k++) atomicAdd(&sp[k * H + c], in[4 * r + k] * g);
-            atomicAdd(&sp[4 * H + c], g);
+    __shared__ double sp[B / 64][H];
+    const int c = threadIdx.x & 63;
+    double a[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4
+    for (int64_t t = (int64_t)blockIdx.x * (B / 64) + (threadIdx.x >> 6); t < count; t += (int64_t)gridDim.x * (B / 64)) {
+        const float4 x = *(const float4 *)(in + 4 * t);
+        const float d = dout[(size_t)t * ld + c];
+        const double g = (bf2f(outb[t * H + c]) > 0.0f) ? (double)d : 0.0;
+        if (g != 0.0) {
+            a[0] += (double)x.x * g;
+            a[1] += (double)x.y * g;
+            a[2] += (double)x.z * g;
+            a[3] += (double)x.w * g;
+            a[4] += g;
         }
     }
-    __syncthreads();
-    for (int k = threadIdx.x; k < 5 * H; k += B) part[(size_t)blockIdx.x * 5 * H + k] = sp[k];
+#pragma unroll
+    for (int k = 0; k < 5; k++) {
+        const double v = block_channel_sum(a[k], sp);
+        if (threadIdx.x < H) part[(size_t)blockIdx.x * 5 * H + k * H + c] = (float)v;
+    }
 }
 
-// out[k] (+)= sum_b part[b][k]  (fixed order: deterministic)
-__global__ __launch_bounds__(B) void k_sum_parts(int nb, int width, const float *__restrict__ part,
-                                                 float *__restrict__ out, int accum)
+// out[k] = sum_b part[b][k], in FP64: 16 wavefronts take every 16th partial of 64 columns
+__device__ __forceinline__ void sum_parts(int nb, int width, const float *__restrict__ part, float *__restrict__ out,
+                                          int block)
 {
-    const int k = blockIdx.x * B + threadIdx.x;
-    if (k >= width) return;
-    double s = 0.0;
-    for (int b = 0; b < nb; b++) s += part[(size_t)b * width + k];
-    out[k] = accum ? out[k] + (float)s : (float)s;
+    __shared__ double sp[16][64];
+    const int c = threadIdx.x & 63, w = threadIdx.x >> 6, k = block * 64 + c;
+    double a = 0.0;
+    if (k < width) {
+#pragma unroll 4
+        for (int b = w; b < nb; b += 16) a += (double)part[(size_t)b * width + k];
+    }
+    sp[w][c] = a;
+    __syncthreads();
+    if (w == 0 && k < width) {
+        double s = 0.0;
+#pragma unroll
+        for (int q = 0; q < 16; q++) s += sp[q][c];
+        out[k] = (float)s;
+    }
+}
+
+__global__ __launch_bounds__(1024) void k_sum_parts(int nb, int width, const float *__restrict__ part,
+                                                    float *__restrict__ out)
+{
+    sum_parts(nb, width, part, out, blockIdx.x);
+}
+
+// the partials of the small gradients (two decoders, three biases, two encoders) in one launch: segment y
+struct sum_segments {
+    int nb[7], width[7];
+    const float *part[7];
+    float *out[7];
+};
+
+__global__ __launch_bounds__(1024) void k_sum_small(sum_segments S)
+{
+    const int y = blockIdx.y;
+    if ((int)blockIdx.x * 64 < S.width[y]) sum_parts(S.nb[y], S.width[y], S.part[y], S.out[y], blockIdx.x);
 }
 
 // ---- parameters ------------------------------------------------------------------------------
 
-// Adam (Kingma & Ba 2015) with bias correction; FP32 master parameters
+// BF16 copies of the layer weights: Wt[l][c][k] (forward B operand) and Wk[l][k][c] (backward), of
+// parameter t if it is a layer weight
+__device__ __forceinline__ void pack_weight(int t, float v, __bf16 *__restrict__ Wt, __bf16 *__restrict__ Wk)
+{
+#pragma unroll
+    for (int l = 0; l < 3; l++) {
+        const int o = t - LV_SPAI_OFF_W(l);
+        if (o < 0 || o >= KX * H) continue;
+        const __bf16 b = f2bf(v);
+        Wk[l * KX * H + o] = b;
+        Wt[l * KX * H + (o % H) * KX + o / H] = b;
+    }
+}
+
+__global__ __launch_bounds__(B) void k_pack_w(int count, const float *__restrict__ theta, __bf16 *__restrict__ Wt,
+                                              __bf16 *__restrict__ Wk)
+{
+    const int t = blockIdx.x * B + threadIdx.x;
+    if (t < count) pack_weight(t, theta[t], Wt, Wk);
+}
+
+// Adam (Kingma & Ba 2015) with bias correction; FP32 master parameters, and the weights' BF16 copies
 __global__ __launch_bounds__(B) void k_adam(int count, float *__restrict__ theta, const float *__restrict__ g,
                                             float *__restrict__ m, float *__restrict__ v, float lr, float b1, float b2,
-                                            float c1, float c2, float eps)
+                                            float c1, float c2, float eps, __bf16 *__restrict__ Wt,
+                                            __bf16 *__restrict__ Wk)
 {
     const int k = blockIdx.x * B + threadIdx.x;
     if (k >= count) return;
@@ -837,19 +925,9 @@ __global__ __launch_bounds__(B) void k_adam(int count, float *__restrict__ theta
     const float vk = b2 * v[k] + (1.0f - b2) * gk * gk;
     m[k] = mk;
     v[k] = vk;
-    theta[k] -= lr * (mk / c1) / (sqrtf(vk / c2) + eps);
-}
-
-// BF16 copies of the layer weights: Wt[c][k] (forward B operand) and Wk[k][c] (backward)
-__global__ __launch_bounds__(B) void k_pack_w(const float *__restrict__ W, __bf16 *__restrict__ Wt,
-                                              __bf16 *__restrict__ Wk)
-{
-    const int t = blockIdx.x * B + threadIdx.x;
-    if (t >= KX * H) return;
-    const int k = t / H, c = t % H;
-    const __bf16 b = f2bf(W[t]);
-    Wk[t] = b;
-    Wt[(size_t)c * KX + k] = b;
+    const float th = theta[k] - lr * (mk / c1) / (sqrtf(vk / c2) + eps);
+    theta[k] = th;
+    pack_weight(k, th, Wt, Wk);
 }
 
 inline dim3 g1(int64_t count) { return dim3((unsigned)std::max<int64_t>(1, (count + B - 1) / B)); }
@@ -896,7 +974,7 @@ hipError_t lv_spai_init(lv_spai *S)
     SP_CHECK(hipMalloc(&S->adam_v, sizeof(float) * LV_SPAI_NPARAM));
     SP_CHECK(hipMalloc(&S->Wt, sizeof(__bf16) * 3 * KX * H));
     SP_CHECK(hipMalloc(&S->Wk, sizeof(__bf16) * 3 * KX * H));
-    SP_CHECK(hipMalloc(&S->scal, sizeof(double) * 64));
+    SP_CHECK(hipMalloc(&S->scal, sizeof(double) * (3 + 64)));  // k_loss_final: 3 + P, P <= 64
     SP_CHECK(hipMemset(S->adam_m, 0, sizeof(float) * LV_SPAI_NPARAM));
     SP_CHECK(hipMemset(S->adam_v, 0, sizeof(float) * LV_SPAI_NPARAM));
     S->has_params = 0;
@@ -916,9 +994,8 @@ void lv_spai_free(lv_spai *S)
 hipError_t lv_spai_set_params(lv_spai *S, const float *host, hipStream_t s)
 {
     SP_CHECK(hipMemcpyAsync(S->theta, host, sizeof(float) * LV_SPAI_NPARAM, hipMemcpyHostToDevice, s));
-    for (int l = 0; l < 3; l++)
-        hipLaunchKernelGGL(k_pack_w, g1(KX * H), dim3(B), 0, s, S->theta + LV_SPAI_OFF_W(l), S->Wt + l * KX * H,
-                           S->Wk + l * KX * H);
+    hipLaunchKernelGGL(k_pack_w, g1(LV_SPAI_NPARAM), dim3(B), 0, s, (int)LV_SPAI_NPARAM, (const float *)S->theta, S->Wt,
+                       S->Wk);
     SP_CHECK(hipMemsetAsync(S->adam_m, 0, sizeof(float) * LV_SPAI_NPARAM, s));
     SP_CHECK(hipMemsetAsync(S->adam_v, 0, sizeof(float) * LV_SPAI_NPARAM, s));
     S->adam_t = 0;
@@ -1073,12 +1150,15 @@ hipError_t lv_spai_loss_grad(lv_spai *S, const lv_pressure_system &A, int n, con
                        (const int *)A.cols, (const float *)S->w, (const float *)S->mdiag, (const float *)S->u, S->y);
     hipLaunchKernelGGL(k_loss_partials, dim3(nbl, P), dim3(B), 0, s, n, P, (const float *)S->y, (const float *)S->v,
                        S->lpart, nbl);
-    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(64), 0, s, P, nbl, (const double *)S->lpart, S->scal);
-    if (loss_host) {
+    hipLaunchKernelGGL(k_loss_final, dim3(1), dim3(B), 0, s, P, nbl, (const double *)S->lpart, S->scal);
+    // the loss is read once everything is enqueued (nothing below writes it)
+    auto read_loss = [&]() -> hipError_t {
+        SP_CHECK(hipGetLastError());
+        if (!loss_host) return hipSuccess;
         SP_CHECK(hipMemcpyAsync(loss_host, S->scal, sizeof(double), hipMemcpyDeviceToHost, s));
-        SP_CHECK(hipStreamSynchronize(s));
-    }
-    if (!want_grad) return hipGetLastError();
+        return hipStreamSynchronize(s);
+    };
+    if (!want_grad) return read_loss();
 
     // ---- backward ----
     SP_CHECK(grow(&S->G, &S->cap_G, (size_t)E));
@@ -1088,63 +1168,67 @@ hipError_t lv_spai_loss_grad(lv_spai *S, const lv_pressure_system &A, int n, con
     SP_CHECK(grow(&S->dH, &S->cap_dH, nh));
     SP_CHECK(grow(&S->dX, &S->cap_dX, (size_t)E * KX));
     SP_CHECK(grow(&S->dZb, &S->cap_dZb, eh));
-    const int chunk = 256;
-    const int nchunks = (E + chunk - 1) / chunk;
-    const int nbE = (int)((E + B - 1) / B), nbN = (int)((n + B - 1) / B);
-    const size_t part_want = std::max(std::max((size_t)nchunks * KX * H, (size_t)nbE * (H + 1)),
-                                      std::max((size_t)g1((int64_t)E * H).x * 5 * H, (size_t)nbN * (H + 1)));
+    const int nchunks = (E + DW_CHUNK - 1) / DW_CHUNK;
+    // partials: the layer weights' [nchunks][KX][H], then the small gradients' segments
+    const int nbE = std::max(1, std::min(RED_BLOCKS, (E + 3) / 4)), nbN = std::max(1, std::min(RED_BLOCKS, (n + 3) / 4));
+    const size_t small[7] = {(size_t)nbE * (H + 1), (size_t)nbN * (H + 1), (size_t)nbE * H, (size_t)nbE * H,
+                             (size_t)nbE * H, (size_t)nbE * 5 * H, (size_t)nbN * 5 * H};
+    size_t part_want = (size_t)nchunks * KX * H;
+    for (size_t w : small) part_want += w;
     SP_CHECK(grow(&S->part, &S->cap_part, part_want));
     float *gr = S->grad;
     const float *th = S->theta;
-    SP_CHECK(hipMemsetAsync(gr, 0, sizeof(float) * LV_SPAI_NPARAM, s));
+    sum_segments seg;
+    {
+        const int widths[7] = {H + 1, H + 1, H, H, H, 5 * H, 5 * H};
+        float *outs[7] = {gr + LV_SPAI_OFF_VE, gr + LV_SPAI_OFF_UN, gr + LV_SPAI_OFF_B(0), gr + LV_SPAI_OFF_B(1),
+                          gr + LV_SPAI_OFF_B(2), gr + LV_SPAI_OFF_WE, gr + LV_SPAI_OFF_WN};
+        float *at = S->part + (size_t)nchunks * KX * H;
+        for (int k = 0; k < 7; k++) {
+            seg.nb[k] = (int)(small[k] / widths[k]);
+            seg.width[k] = widths[k];
+            seg.part[k] = at;
+            seg.out[k] = outs[k];
+            at += small[k];
+        }
+    }
+    auto part_of = [&](int k) { return const_cast<float *>(seg.part[k]); };
     hipLaunchKernelGGL(k_grad_y, g1((int64_t)np), dim3(B), 0, s, n, P, (const float *)S->y, (const float *)S->v,
                        (const double *)S->scal, S->gy);
     hipLaunchKernelGGL(k_grad_w, g1(n), dim3(B), 0, s, n, P, (const int *)A.row_ptr, (const int *)A.cols,
-                       (const float *)S->w, (const float *)S->gy, (const float *)S->u, (const float *)S->delta, S->G,
-                       S->don);
+                       (const float *)S->w, (const float *)S->gy, (const float *)S->u, (const float *)S->delta,
+                       (const float *)S->on, S->G, S->don);
     hipLaunchKernelGGL(k_grad_o, g1(E), dim3(B), 0, s, E, (const int *)S->rev, (const float *)S->G,
                        (const float *)S->w, (const float *)S->oe, S->doe);
-    hipLaunchKernelGGL(k_clamp_mask, g1(n), dim3(B), 0, s, n, (const float *)S->on, S->don);
     // decoders: dE3 = doe ve, dH3 = don un; parameter partials
-    hipLaunchKernelGGL(k_decode_back, dim3(nbE), dim3(B), 0, s, E, (const __bf16 *)(S->Eb + 3 * eh),
-                       (const float *)nullptr, th + LV_SPAI_OFF_VE, (const float *)S->doe, S->dE, 0, S->part);
-    hipLaunchKernelGGL(k_sum_parts, g1(H + 1), dim3(B), 0, s, nbE, H + 1, (const float *)S->part,
-                       gr + LV_SPAI_OFF_VE, 0);
-    hipLaunchKernelGGL(k_decode_back, dim3(nbN), dim3(B), 0, s, n, (const __bf16 *)nullptr,
-                       (const float *)(S->Hf + 3 * nh), th + LV_SPAI_OFF_UN, (const float *)S->don, S->dH, 0, S->part);
-    hipLaunchKernelGGL(k_sum_parts, g1(H + 1), dim3(B), 0, s, nbN, H + 1, (const float *)S->part,
-                       gr + LV_SPAI_OFF_UN, 0);
+    hipLaunchKernelGGL(k_decode_back<__bf16>, dim3(nbE), dim3(B), 0, s, E, (const __bf16 *)(S->Eb + 3 * eh),
+                       th + LV_SPAI_OFF_VE, (const float *)S->doe, S->dE, part_of(0));
+    hipLaunchKernelGGL(k_decode_back<float>, dim3(nbN), dim3(B), 0, s, n, (const float *)(S->Hf + 3 * nh),
+                       th + LV_SPAI_OFF_UN, (const float *)S->don, S->dH, part_of(1));
     // message-passing layers, last to first.  Incoming: dH (of h_{l+1}) and dE (of m_l = e_{l+1}).
     const unsigned tiles = (unsigned)((E + 31) / 32);
     for (int l = 2; l >= 0; l--) {
-        hipLaunchKernelGGL(k_mp_dz, g1((int64_t)E * H), dim3(B), 0, s, E, (const int *)S->src,
-                           (const int *)A.row_ptr, (const float *)S->dH, (const __bf16 *)(S->Eb + (l + 1) * eh), S->dE,
-                           S->dZb);
+        const float *dM = (l == 2) ? S->dE : S->dX + 2 * H;
+        hipLaunchKernelGGL(k_mp_dz, dim3(nbE), dim3(B), 0, s, E, (const int *)S->src, (const int *)A.row_ptr,
+                           (const float *)S->dH, (const __bf16 *)(S->Eb + (l + 1) * eh), dM, (l == 2) ? H : KX, S->dZb,
+                           part_of(2 + l));
         hipLaunchKernelGGL(k_mp_dx, dim3((tiles + 3) / 4), dim3(256), 0, s, E, (const __bf16 *)S->dZb,
                            (const __bf16 *)(S->Wk + l * KX * H), S->dX);
         hipLaunchKernelGGL(k_mp_dw, dim3(nchunks, 3), dim3(256), 0, s, E, (const int *)S->src, (const int *)A.cols,
                            (const __bf16 *)(S->Hb + l * nh), (const __bf16 *)(S->Eb + l * eh), (const __bf16 *)S->dZb,
-                           chunk, S->part);
-        hipLaunchKernelGGL(k_sum_parts, g1(KX * H), dim3(B), 0, s, nchunks, KX * H, (const float *)S->part,
-                           gr + LV_SPAI_OFF_W(l), 0);
-        hipLaunchKernelGGL(k_mp_db, dim3(nchunks), dim3(H), 0, s, E, (const __bf16 *)S->dZb, chunk, S->part);
-        hipLaunchKernelGGL(k_sum_parts, g1(H), dim3(B), 0, s, nchunks, H, (const float *)S->part,
-                           gr + LV_SPAI_OFF_B(l), 0);
+                           S->part);
+        hipLaunchKernelGGL(k_sum_parts, dim3(KX * H / 64), dim3(1024), 0, s, nchunks, KX * H, (const float *)S->part,
+                           gr + LV_SPAI_OFF_W(l));
         hipLaunchKernelGGL(k_mp_dh, g1((int64_t)n * H), dim3(B), 0, s, n, (const int *)A.row_ptr,
                            (const int *)S->rev, (const float *)S->dX, S->dH);
-        hipLaunchKernelGGL(k_mp_de, g1((int64_t)E * H), dim3(B), 0, s, E, (const float *)S->dX, S->dE);
     }
-    // encoders
-    const unsigned nbEH = g1((int64_t)E * H).x, nbNH = g1((int64_t)n * H).x;
-    hipLaunchKernelGGL(k_encode_back, dim3(nbEH), dim3(B), 0, s, E, (const float *)S->ff, (const __bf16 *)S->Eb,
-                       (const float *)S->dE, S->part);
-    hipLaunchKernelGGL(k_sum_parts, g1(5 * H), dim3(B), 0, s, (int)nbEH, 5 * H, (const float *)S->part,
-                       gr + LV_SPAI_OFF_WE, 0);
-    hipLaunchKernelGGL(k_encode_back, dim3(nbNH), dim3(B), 0, s, n, (const float *)S->xf, (const __bf16 *)S->Hb,
-                       (const float *)S->dH, S->part);
-    hipLaunchKernelGGL(k_sum_parts, g1(5 * H), dim3(B), 0, s, (int)nbNH, 5 * H, (const float *)S->part,
-                       gr + LV_SPAI_OFF_WN, 0);
-    return hipGetLastError();
+    // encoders (dE_0 is the e part of layer 0's dX), then every small gradient's partials
+    hipLaunchKernelGGL(k_encode_back, dim3(nbE), dim3(B), 0, s, E, (const float *)S->ff, (const __bf16 *)S->Eb,
+                       (const float *)(S->dX + 2 * H), KX, part_of(5));
+    hipLaunchKernelGGL(k_encode_back, dim3(nbN), dim3(B), 0, s, n, (const float *)S->xf, (const __bf16 *)S->Hb,
+                       (const float *)S->dH, H, part_of(6));
+    hipLaunchKernelGGL(k_sum_small, dim3(5, 7), dim3(1024), 0, s, seg);
+    return read_loss();
 }
 
 hipError_t lv_spai_adam(lv_spai *S, double lr, hipStream_t s)
@@ -1153,9 +1237,7 @@ hipError_t lv_spai_adam(lv_spai *S, double lr, hipStream_t s)
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - powf(b1, (float)S->adam_t), c2 = 1.0f - powf(b2, (float)S->adam_t);
     hipLaunchKernelGGL(k_adam, g1(LV_SPAI_NPARAM), dim3(B), 0, s, (int)LV_SPAI_NPARAM, S->theta,
-                       (const float *)S->grad, S->adam_m, S->adam_v, (float)lr, b1, b2, c1, c2, 1e-8f);
-    for (int l = 0; l < 3; l++)
-        hipLaunchKernelGGL(k_pack_w, g1(KX * H), dim3(B), 0, s, S->theta + LV_SPAI_OFF_W(l), S->Wt + l * KX * H,
-                           S->Wk + l * KX * H);
+                       (const float *)S->grad, S->adam_m, S->adam_v, (float)lr, b1, b2, c1, c2, 1e-8f, S->Wt,
+                       S->Wk);
     return hipGetLastError();
 }

@@ -190,3 +190,83 @@ def test_trained_network_gains_over_jacobi(lv, oracle, gpu):
     print("inner iterations: jacobi %d, untrained %d, trained %d" % (it_jac, its["untrained"], its["trained"]))
     assert its["trained"] <= 0.6 * it_jac, (its, it_jac)
     assert its["trained"] <= its["untrained"], its
+
+
+def _bf16_forward(torch, acc):
+    """spai_ref.forward with operands rounded to BF16 where the kernels round them, forward and backward, the
+    layers' products and the node features accumulated in the type acc"""
+    R = lambda t: t.to(torch.bfloat16).to(torch.float64)
+    mul = lambda a, b: (a.to(acc) @ b.to(acc)).to(torch.float64)
+    keep = lambda t: t + (t.to(acc).to(torch.float64) - t).detach()
+
+    class Store(torch.autograd.Function):  # an activation kept in BF16: the gradient passes unrounded
+        @staticmethod
+        def forward(ctx, t):
+            return R(t)
+
+        @staticmethod
+        def backward(ctx, g):
+            return g
+
+    class Layer(torch.autograd.Function):  # X W + b with BF16 operands; dZ rounded before it is used
+        @staticmethod
+        def forward(ctx, X, W, b):
+            ctx.save_for_backward(X, W)
+            return (mul(X, R(W)) + b).to(acc).to(torch.float64)
+
+        @staticmethod
+        def backward(ctx, g):
+            X, W = ctx.saved_tensors
+            z = R(g)
+            return mul(z, R(W).T), mul(X.T, z), z.to(acc).sum(0).to(torch.float64)
+
+    def forward(th, g):
+        r, H, t = spai_ref, spai_ref.H, spai_ref._t
+        src, dst, deg = torch.as_tensor(g.src), torch.as_tensor(g.cols), t(g.deg)
+        h = keep(torch.relu(t(g.x) @ th[r.OFF_WN:r.OFF_BN].reshape(4, H) + th[r.OFF_BN:r.OFF_WE]))
+        e = Store.apply(torch.relu(t(g.f) @ th[r.OFF_WE:r.OFF_BE].reshape(4, H) + th[r.OFF_BE:r.OFF_W(0)]))
+        for l in range(3):
+            hb = Store.apply(h)
+            z = Layer.apply(torch.cat([hb[src], hb[dst], e], dim=1), th[r.OFF_W(l):r.OFF_B(l)].reshape(192, H),
+                            th[r.OFF_B(l):r.OFF_B(l) + H])
+            e = Store.apply(torch.relu(z))
+            h = keep(h + torch.zeros_like(h).index_add_(0, src, e) / torch.clamp(deg, min=1.0)[:, None])
+        oe = e @ th[r.OFF_VE:r.OFF_CE] + th[r.OFF_CE]
+        on = h @ th[r.OFF_UN:r.OFF_CN] + th[r.OFF_CN]
+        rev = torch.as_tensor(np.where(g.rev >= 0, g.rev, np.arange(g.rev.size)))
+        w = t(g.a) * torch.exp(torch.clamp(0.5 * (oe + oe[rev]), -r.OCLAMP, r.OCLAMP))
+        delta = t(g.rfl) * torch.exp(torch.clamp(on, -r.OCLAMP, r.OCLAMP))
+        md = torch.zeros(g.n, dtype=torch.float64).index_add_(0, src, torch.abs(w)) + delta
+        return oe, on, w, md, delta
+
+    return forward
+
+
+@pytest.mark.parametrize("K,P", [(6, 1), (23, 64), (37, 8)])
+def test_spai_gradient_at_partial_chunks_matches_bf16_oracle(lv, oracle, gpu, monkeypatch, K, P):
+    """the backward pass's reductions where rows, MFMA chunks (256 edges) and wavefronts are partly empty,
+    from one probe to the most there can be, against the FP64 oracle with operands rounded to BF16 where the
+    kernels round them.  What is left is FP32 accumulation, which turns the BF16 rounding (and the ReLU mask) of
+    a few values: the oracle itself moves by as much between FP64 and FP32 accumulation, so each block of
+    parameters may be off by eight times that (and 1e-4)."""
+    import torch
+
+    grid, solver, g = _system(lv, oracle, K=K)
+    assert g.cols.size % 256 != 0
+    th = _theta(5)
+    lv.spai.set_params(grid, th)
+    L_gpu, G_gpu = lv.spai.loss_grad(grid, nprobe=P, seed=31, use_data=True)
+    assert lv.spai.loss_grad(grid, nprobe=P, seed=31, use_data=True, want_grad=False)[0] == L_gpu
+    ref = []
+    for acc in (torch.float64, torch.float32):
+        monkeypatch.setattr(spai_ref, "forward", _bf16_forward(torch, acc))
+        ref.append(spai_ref.loss_and_grad(th.astype(np.float64), g, spai_ref.probes(g, P, 31, x=grid.get("P"))))
+    (L_ref, G_ref), (L_32, G_32) = ref
+    assert abs(L_gpu - L_ref) <= 8 * abs(L_32 - L_ref) + 1e-4 * abs(L_ref)
+    for a, b in [(spai_ref.OFF_WN, spai_ref.OFF_WE), (spai_ref.OFF_WE, spai_ref.OFF_W(0)),
+                 *[(spai_ref.OFF_W(l), spai_ref.OFF_B(l)) for l in range(3)],
+                 *[(spai_ref.OFF_B(l), spai_ref.OFF_B(l) + 64) for l in range(3)],
+                 (spai_ref.OFF_VE, spai_ref.OFF_UN), (spai_ref.OFF_UN, spai_ref.NPARAM)]:
+        gr = G_ref[a:b]
+        far, own = (np.linalg.norm(G[a:b] - gr) for G in (G_gpu.astype(np.float64), G_32))
+        assert far <= 8 * own + 1e-4 * np.linalg.norm(gr), (a, b, far, own)
