@@ -30,6 +30,10 @@ struct lv_amg {
     lv_amg_level lev[LV_AMG_MAXLEV + 1];
     float *dense_inv;    // nc * nc, column-major
     float *tail_img;     // the tail levels' constant arrays in their LDS layout (packed per set-up)
+    float *tail_mat, *ext_mat;  // a singular system's W-visit of the tail as a matrix on its first level, and of
+    size_t cap_tail_mat, cap_ext_mat;  // the level above it when that is small enough
+    const float *mat;    // the one the cycle multiplies by, on level lmat, leading dimension mat_ld (0: none, the
+    int lmat, mat_ld;    // visit runs its program on level lmat = ltail)
     double *pw;          // power-iteration partials and norms
     float *pv, *pu;      // power-iteration vectors (n0)
     size_t cap_pv, cap_pu;

@@ -1192,6 +1192,10 @@ __global__ __launch_bounds__(B) void k_st_up2(st_pair Q, const float *__restrict
 // workgroup).  Reads the right-hand side of level first, writes its final correction.
 constexpr int TB = 1024;
 constexpr int TAIL_MAX = 1024;  // levels of at most this many cells run in the tail
+// A singular system's cycle multiplies by the matrix of its first level of at most MAT_MAX cells: 26 MB, what
+// the eight L2s hold, so that a small system's cycles find it there (above that the two stencil launches
+// that the level saves cost less than the bytes).
+constexpr int MAT_MAX = 2560;
 enum tail_op { OP_DOWN = 0, OP_DENSE = 1, OP_UP = 2, OP_WSAVE = 3, OP_WADD = 4 };
 constexpr int OP_SHIFT = 5;  // an operation is op << OP_SHIFT | level
 static_assert(LV_AMG_MAXLEV < (1 << OP_SHIFT), "levels fit the operation code");
@@ -1299,8 +1303,20 @@ __global__ __launch_bounds__(TB) void k_tail(tail_levels T, const int *__restric
 // The constant arrays come from img (k_tail_pack's image of them in this layout) by one flat copy
 // whose loads are all issued before the done flag is tested and the first LDS store is made; a copy
 // loop per array would wait for a global round trip per iteration.
+//
+// The W-visited tail as a matrix (COLS).  A visit is a linear, symmetric operator on the right-hand side of the
+// tail's first level: for a singular system set-up applies the program to every unit vector, one workgroup a
+// column (the right-hand side is that of cell blockIdx.x, and the correction becomes row blockIdx.x of mat, of
+// leading dimension ld: the operator is symmetric), and each cycle multiplies by the matrix (k_mat_mv).  The
+// W-visit is a serial chain of about 30 operations on one CU, 25-29 us a cycle whatever the rest of the device
+// does; the product reads at most 4 MB spread over the device in one round trip, 2.7-4.7 us, and the columns
+// take 72 us once per set-up (25 x 25 cells, 3 turns of the device).  A nonsingular system keeps the program: its V-visit takes 10.4 us, and its
+// solves keep their iterates bit for bit (velocities near rest are small differences of pressures, and
+// would show another rounding of the cycle magnified).
+template <bool COLS>
 __global__ __launch_bounds__(TB) void k_tail_lds(tail_levels T, tail_layout Y, const int *__restrict__ prog,
-                                                 int nprog, const float *__restrict__ img, const lv_cg_scalars *S)
+                                                 int nprog, const float *__restrict__ img, const lv_cg_scalars *S,
+                                                 float *__restrict__ mat, int ld)
 {
     __shared__ __align__(16) float lds[TAIL_LDS];
     __shared__ int lprog[LV_AMG_MAXPROG];
@@ -1315,7 +1331,9 @@ __global__ __launch_bounds__(TB) void k_tail_lds(tail_levels T, tail_layout Y, c
         if (q * TB + (int)threadIdx.x < n4) v[q] = img4[q * TB + threadIdx.x];
     const int n0 = T.Kx[first] * T.Ky[first];
     const int f0 = threadIdx.x;  // n0 <= TAIL_MAX == TB: one right-hand side entry per lane
-    const float r0 = (f0 < n0) ? T.r[first][f0] : 0.0f;
+    float r0 = 0.0f;
+    if (COLS) r0 = f0 == (int)blockIdx.x ? 1.0f : 0.0f;
+    else if (f0 < n0) r0 = T.r[first][f0];
     const int pr = (int)threadIdx.x < nprog ? prog[threadIdx.x] : 0;  // nprog <= LV_AMG_MAXPROG <= TB
     if (S && S->done) return;  // tested after the loads above are issued (they read valid arrays)
     f4 *lds4 = reinterpret_cast<f4 *>(lds);
@@ -1327,7 +1345,95 @@ __global__ __launch_bounds__(TB) void k_tail_lds(tail_levels T, tail_layout Y, c
     if ((int)threadIdx.x < nprog) lprog[threadIdx.x] = pr;
     __syncthreads();
     run_tail(T, tail_in_lds{lds, Y}, lprog, nprog);
-    for (int f = threadIdx.x; f < n0; f += TB) T.t[first][f] = lds[Y.t[first] + f];
+    if (COLS) {
+        float *row = mat + (size_t)blockIdx.x * ld;
+        for (int f = threadIdx.x; f < ld; f += TB) row[f] = f < n0 ? lds[Y.t[first] + f] : 0.0f;
+    } else {
+        for (int f = threadIdx.x; f < n0; f += TB) T.t[first][f] = lds[Y.t[first] + f];
+    }
+}
+
+// The matrix of level L from that of the next level (nc cells, leading dimension ldc): row j is the
+// V-visit of the unit vector of cell j = blockIdx.x, one workgroup each.  The right-hand side it leaves the
+// next level has a handful of entries, so that level's correction is a sum of as many rows of its matrix.
+// At 50 x 50 cells (level 1 of 100^2 particles) it takes 99 us once per set-up and the product 5.1 us, against
+// the 11 us of the two stencil launches, the product and the prolongation that it replaces in each cycle.
+__global__ __launch_bounds__(B) void k_mat_extend(st_level L, int Kyc, int nc, const float *__restrict__ matc, int ldc,
+                                                  float *__restrict__ mat, int ld)
+{
+    __shared__ float r[MAT_MAX], z[MAT_MAX], rc[TAIL_MAX], ec[TAIL_MAX];
+    __shared__ int nz[TAIL_MAX], cnt;
+    const int n = L.Kx * L.Ky;
+    for (int f = threadIdx.x; f < n; f += B) r[f] = f == (int)blockIdx.x ? 1.0f : 0.0f;
+    __syncthreads();
+    for (int base = 0; base < nc * CF2; base += B) {  // uniform trip count: every lane shuffles
+        const int tid = base + threadIdx.x;
+        const int P = tid / CF2, q = tid % CF2;
+        const float t = sum_children(st_down_lane(L, Kyc, nc, P, q, r, z));
+        if (q == 0 && P < nc) rc[P] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {  // its nonzero entries in order
+        int m = 0;
+        for (int base = 0; base < nc; base += 64) {
+            const int P = base + threadIdx.x;
+            const bool on = P < nc && rc[P] != 0.0f;
+            const unsigned long long b = __ballot(on);
+            if (on) nz[m + __popcll(b & ((1ull << threadIdx.x) - 1ull))] = P;
+            m += __popcll(b);
+        }
+        if (threadIdx.x == 0) cnt = m;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < nc; i += B) {
+        float a = 0.0f;
+        for (int q = 0; q < cnt; q++) a += rc[nz[q]] * matc[(size_t)nz[q] * ldc + i];
+        ec[i] = a;
+    }
+    __syncthreads();
+    float *row = mat + (size_t)blockIdx.x * ld;
+    for (int f = threadIdx.x; f < ld; f += B) {
+        if (f < n) st_up_cell(L, Kyc, f, r, z, ec, row);
+        else row[f] = 0.0f;
+    }
+}
+
+// t = mat r for the matrix level (n cells, at most 256 PER): a wavefront a row, every load of the row and
+// of r issued before the done flag is tested.  r is allocated to a multiple of 4; the entries past n are
+// dropped.  PROLONG (level 1 in the aggregate order): also the prolongation of each cell's correction into
+// its rows of z0, as k_prolong1 forms it.
+template <int PER, bool PROLONG>
+__global__ __launch_bounds__(B) void k_mat_mv(int n, int ld, const float *__restrict__ mat, const float *__restrict__ r,
+                                              float *__restrict__ t, const lv_cg_scalars *S,
+                                              const int *__restrict__ start, float alpha0, float *__restrict__ z0)
+{
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63, row = blockIdx.x * (B / 64) + (threadIdx.x >> 6);
+    const int rw = row < n ? row : n - 1;
+    const f4 *m4 = reinterpret_cast<const f4 *>(mat + (size_t)rw * ld);
+    const f4 *r4 = reinterpret_cast<const f4 *>(r);
+    f4 m[PER], x[PER];
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int k = q * 64 + lane, kk = 4 * k < ld ? k : 0;
+        m[q] = m4[kk];
+        x[q] = r4[kk];
+    }
+    const int b0 = PROLONG ? start[rw] : 0, e = PROLONG ? start[rw + 1] : 0;
+    if (S && S->done) return;
+    float a = 0.0f;
+#pragma unroll
+    for (int q = 0; q < PER; q++) {
+        const int k = 4 * (q * 64 + lane);
+#pragma unroll
+        for (int c = 0; c < 4; c++) a += k + c < n ? m[q][c] * x[q][c] : 0.0f;
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
+    if (row >= n) return;
+    if (lane == 0) t[row] = a;
+    if (PROLONG)
+        for (int i = b0 + lane; i < e; i += 64) z0[i] += alpha0 * a;
 }
 static_assert(B == 256 && FUSE_ROWS + 64 <= FUSE_CAP, "fused blocks fit their LDS rows");
 static_assert(LV_AMG_DENSE_MAX * 16 == TB, "the dense solve of the tail maps 16 lanes to a row");
@@ -1525,7 +1631,7 @@ hipError_t lv_amg_init(lv_amg *G)
 
 void lv_amg_free(lv_amg *G)
 {
-    void *ptrs[] = {G->agg, G->cnt, G->start, G->cursor, G->list, G->scan_tmp, G->t0, G->z0, G->dense_inv, G->tail_img,
+    void *ptrs[] = {G->agg, G->cnt, G->start, G->cursor, G->list, G->scan_tmp, G->t0, G->z0, G->dense_inv, G->tail_img, G->tail_mat, G->ext_mat,
                     G->pw, G->pv, G->pu, G->prog, G->iperm, G->aggp, G->pdeg, G->poff, G->pev32, G->pev16,
                     G->pdiag32, G->pdinv32, G->pmval, G->pmdg, G->pflag, G->bfirst, G->ooff, G->oev32};
     for (void *p : ptrs)
@@ -1552,7 +1658,7 @@ static hipError_t level_alloc(lv_amg_level &L, int Kx, int Ky)
         AMG_CHECK(hipMalloc(&L.d, sizeof(float) * m));
         AMG_CHECK(hipMalloc(&L.c, sizeof(float) * 8 * m));
         AMG_CHECK(hipMalloc(&L.dinv, sizeof(float) * m));
-        AMG_CHECK(hipMalloc(&L.r, sizeof(float) * m));
+        AMG_CHECK(hipMalloc(&L.r, sizeof(float) * ((m + 3) & ~(size_t)3)));  // read as float4 by k_tail_mv
         AMG_CHECK(hipMalloc(&L.z, sizeof(float) * m));
         AMG_CHECK(hipMalloc(&L.t, sizeof(float) * m));
         AMG_CHECK(hipMalloc(&L.acc, sizeof(float) * m));
@@ -1769,27 +1875,44 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
     int lt = G->nlev;
     while (lt > 1 && G->lev[lt - 1].n <= TAIL_MAX) lt--;
     G->ltail = lt;
+    G->wcycle = A.singular ? 1 : 0;
+    G->nprog = tail_program(lt, G->nlev, G->wcycle != 0, G->hprog);
+    // a singular system's tail as a matrix (k_tail_lds<true>), and the level above it when it is small
+    const tail_layout Y = tail_layout_of(G);
+    const bool fits = tail_fits_lds(G, Y), mat = fits && G->wcycle;
+    G->lmat = mat && lt > 1 && G->lev[lt - 1].n <= MAT_MAX ? lt - 1 : lt;
+    G->mat_ld = mat ? (G->lev[G->lmat].n + 3) & ~3 : 0;
     // pairs of levels above the tail that run as one kernel each way, from the tail upwards (the
     // smallest levels gain most): level l at least PAIR_MIN_K wide, a multiple of 4 on a periodic axis
     memset(G->pair, 0, sizeof(G->pair));
-    for (int k = lt - 2; k >= 2;) {
+    for (int k = G->lmat - 2; k >= 2;) {
         const lv_amg_level &L = G->lev[k];
         const bool ok = L.Kx >= PAIR_MIN_K && L.Ky >= PAIR_MIN_K && (!G->xper || L.Kx % 4 == 0) &&
                         (!G->yper || L.Ky % 4 == 0);
         G->pair[k] = ok ? 1 : 0;
         k -= ok ? 2 : 1;
     }
-    G->wcycle = A.singular ? 1 : 0;
-    G->nprog = tail_program(lt, G->nlev, G->wcycle != 0, G->hprog);
     AMG_CHECK(hipMemcpyAsync(G->prog, G->hprog, sizeof(int) * G->nprog, hipMemcpyHostToDevice, s));
     const lv_amg_level &D = G->lev[l];
     hipLaunchKernelGGL(k_dense_inverse, dim3(1), dim3(DTB), 0, s, D.Kx, D.Ky, G->xper, G->yper, (const float *)D.d,
                        (const float *)D.c, A.singular, G->dense_inv);
-    {
-        const tail_layout Y = tail_layout_of(G);
-        if (tail_fits_lds(G, Y))
-            hipLaunchKernelGGL(k_tail_pack, dim3(64), dim3(B), 0, s, tail_levels_of(G), Y,
-                               (const float *)G->dense_inv, G->tail_img);
+    const tail_levels T = tail_levels_of(G);
+    if (fits)
+        hipLaunchKernelGGL(k_tail_pack, dim3(64), dim3(B), 0, s, T, Y, (const float *)G->dense_inv, G->tail_img);
+    if (mat) {
+        const int nt = G->lev[lt].n, ldt = (nt + 3) & ~3;
+        AMG_CHECK(grow(&G->tail_mat, &G->cap_tail_mat, (size_t)nt * ldt));
+        hipLaunchKernelGGL(k_tail_lds<true>, dim3(nt), dim3(TB), 0, s, T, Y, (const int *)G->prog, G->nprog,
+                           (const float *)G->tail_img, (const lv_cg_scalars *)nullptr, G->tail_mat, ldt);
+        G->mat = G->tail_mat;
+        if (G->lmat < lt) {
+            const lv_amg_level &L = G->lev[G->lmat];
+            AMG_CHECK(grow(&G->ext_mat, &G->cap_ext_mat, (size_t)L.n * G->mat_ld));
+            hipLaunchKernelGGL(k_mat_extend, dim3(L.n), dim3(B), 0, s,
+                               st_level{L.Kx, L.Ky, G->xper, G->yper, L.d, L.c, L.dinv, L.alpha}, G->lev[lt].Ky, nt,
+                               (const float *)G->tail_mat, ldt, G->ext_mat, G->mat_ld);
+            G->mat = G->ext_mat;
+        }
     }
     // fine smoother
     G->fine_learned = (mval && mdg) ? 1 : 0;
@@ -1883,7 +2006,7 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
                            (const float *)G->t0, L1.r, S);
     } else if (!list && G->nbfuse > 0) {
         // level 1 above the tail: its pre-smoothed z stored here, gathered by its down pass
-        z1_given = G->ltail > 1;
+        z1_given = G->lmat > 1;
         float *z1 = z1_given ? L1.z : nullptr;
         const int *done = S ? &S->done : G->bfirst + 2 * (G->nbfuse + 1);
         if (z0_ready && G->z0_in)
@@ -1901,7 +2024,7 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
     }
     // coarse levels above the tail, down: each level's pre-smoothed z and the next level's
     // right-hand side
-    const int lt = G->ltail;
+    const int lt = G->lmat;
     const bool pairs = !G->level_kernels;
     for (int l = 1; l < lt; l++) {
         const lv_amg_level &L = G->lev[l], &C = G->lev[l + 1];
@@ -1921,18 +2044,25 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
             hipLaunchKernelGGL(k_st_down<false>, g1((int64_t)C.n * CF2), dim3(B), 0, s, sl, C.Ky, C.n,
                                (const float *)L.r, L.z, C.r, S);
     }
-    // the tail: levels lt..nlev down, dense, and up; the final correction of level lt in its t
-    const tail_levels T = tail_levels_of(G);
+    // the tail: levels lt..nlev down, dense, and up, or the matrix of that; the final correction of level
+    // lt in its t.  Then the coarse levels above it, up: each level's final correction in t; level 1 in the
+    // aggregate order with the Jacobi smoother also prolongates into z0.
+    const lv_amg_level &LT = G->lev[lt];
     const tail_layout Y = tail_layout_of(G);
-    if (tail_fits_lds(G, Y))
-        hipLaunchKernelGGL(k_tail_lds, dim3(1), dim3(TB), 0, s, T, Y, (const int *)G->prog, G->nprog,
-                           (const float *)G->tail_img, S);
+    const bool prolong_in_up = (lt > 1 || G->mat_ld) && !G->fine_learned && list == nullptr;
+    if (G->mat_ld) {
+        const bool pr = lt == 1 && prolong_in_up;
+        auto kern = LT.n <= TAIL_MAX ? (pr ? k_mat_mv<TAIL_MAX / 256, true> : k_mat_mv<TAIL_MAX / 256, false>)
+                                     : (pr ? k_mat_mv<MAT_MAX / 256, true> : k_mat_mv<MAT_MAX / 256, false>);
+        hipLaunchKernelGGL(kern, dim3((LT.n + B / 64 - 1) / (B / 64)), dim3(B), 0, s, LT.n, G->mat_ld,
+                           (const float *)G->mat, (const float *)LT.r, LT.t, S,
+                           pr ? (const int *)G->start : (const int *)nullptr, G->fine_alpha, G->z0);
+    } else if (tail_fits_lds(G, Y))
+        hipLaunchKernelGGL(k_tail_lds<false>, dim3(1), dim3(TB), 0, s, tail_levels_of(G), Y, (const int *)G->prog,
+                           G->nprog, (const float *)G->tail_img, S, (float *)nullptr, 0);
     else
-        hipLaunchKernelGGL(k_tail, dim3(1), dim3(TB), 0, s, T, (const int *)G->prog, G->nprog,
+        hipLaunchKernelGGL(k_tail, dim3(1), dim3(TB), 0, s, tail_levels_of(G), (const int *)G->prog, G->nprog,
                            (const float *)G->dense_inv, S);
-    // coarse levels above the tail, up: each level's final correction in t; level 1 in the aggregate
-    // order with the Jacobi smoother also prolongates into z0
-    const bool prolong_in_up = lt > 1 && !G->fine_learned && list == nullptr;
     for (int l = lt - 1; l >= 1; l--) {
         if (pairs && l >= 3 && G->pair[l - 1]) {
             const lv_amg_level &L = G->lev[l - 1], &C = G->lev[l], &C2 = G->lev[l + 1];

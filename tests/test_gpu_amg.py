@@ -405,3 +405,23 @@ def test_solve_from_converged_guess_skips_the_sweep(lv, oracle, gpu):
         assert st2["relres"][0] <= 1e-8 and st2["relres0"][0] == st2["relres"][0], (method, st2)
         assert st2["solve_ms"][0] < 15.0, (method, st2["solve_ms"])
         assert np.array_equal(P2, P1), method
+
+
+@pytest.mark.parametrize("kind,K", [("walls", 24), ("walls", 64), ("walls", 72), ("walls", 100), ("walls", 140),
+                                    ("periodic", 67), ("tall", 50), ("xperiodic", 143)])
+def test_matrix_of_the_coarse_levels_matches_oracle(lv, oracle, gpu, kind, K):
+    """a singular system's cycle multiplies by the matrix of its small levels: the tail alone as level 1 (24,
+    64) and below stencil levels, the level above it with the prolongation in the product (72, 100: 2500
+    cells; 67: odd and periodic; a tall domain) and as level 2 (140, 143).  The product adds the same terms
+    in FP32 in another order, so the cycle's own tolerance holds, with both layouts."""
+    _flush("matrix level %s %d" % (kind, K))
+    grid, op, solver, x, dr, d, rp, cols, coef = _system(lv, oracle, kind, K, "cavity", 1e-3)
+    r = np.random.default_rng(12).standard_normal(grid.n)
+    zr = _hier(kind, x, dr, d, rp, cols, coef).apply(r)
+    z = solver.apply_preconditioner(r, "amg")
+    assert np.linalg.norm(z - zr) <= 1e-4 * np.linalg.norm(zr), (np.linalg.norm(z - zr) / np.linalg.norm(zr))
+    b = r - r.mean()
+    solver.solve(b, np.zeros(grid.n), method="amg", tol=1e-8, amg_layout=1)  # leaves its layout to the next apply
+    zr = _hier(kind, x, dr, d, rp, cols, coef, fine_bf16=False).apply(r)
+    z = solver.apply_preconditioner(r, "amg")
+    assert np.linalg.norm(z - zr) <= 1e-4 * np.linalg.norm(zr), (np.linalg.norm(z - zr) / np.linalg.norm(zr))
