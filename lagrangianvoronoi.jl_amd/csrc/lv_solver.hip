@@ -953,6 +953,342 @@ __global__ __launch_bounds__(B) void k_correct(int n, double *__restrict__ x, co
     if (Pxs) block_partials<1>(v, Pxs, gridDim.x);
 }
 
+// ---- FP64 Jacobi-PCG of a small system in one launch ---------------------------------------------
+//
+// Below PS_MAX_ROWS rows the two launches of an iteration are all latency (5.0 + 3.6 us at 10,000 rows, and
+// the host's turn between them: 11.8 us an iteration), so one launch runs the whole solve: a thread owns a
+// row and keeps its couplings, x, r, p and q in registers, and what an iteration exchanges, z and two
+// reductions, goes through memory between workgroups that are all resident: 5.0 us an iteration.
+//
+// The exchange: each workgroup publishes its partial sums with agent-scope stores, which are written
+// through to where every XCD sees them, into slots that hold a sentinel until then, and each of its threads
+// polls one workgroup's slots (ps_sum): the reduction is its own barrier.  Four sets of slots rotate; at
+// sync j a workgroup puts the sentinel back into what it published at sync j - 2, which every workgroup has
+// read by then (it had to, to publish j - 1, which this one has seen); that store is complete when ps_sum
+// returns (s_waitcnt after the poll), so before this workgroup publishes j + 1, and so before anyone polls that
+// set again at j + 2.
+// z goes the same way: three vectors rotate, a row polls its neighbours' entries, and each owner puts the
+// sentinel into the vector after next when it stores z_k: what that holds, z_{k-2}, was read by
+// every workgroup before it published the p.q of iteration k - 2, and the sentinel is in place when this
+// one returns from the reduction of r.z, before it publishes the p.q of iteration k, and nobody polls for
+// z_{k+1} before that.  So z's way to the
+// neighbours runs beside the reduction of r.z, not before it (with z complete before its partials were
+// published, and gathered after they had been seen, an iteration took 5.8 us).
+//
+// A wait ends after 20 ms at the latest: a workgroup that has not been scheduled by then (other work
+// fills the device) makes the launch give up, x untouched or at a valid iterate, and the host runs
+// the solve launch by launch.  256 workgroups of 256 threads at 4 wavefronts per SIMD and more leave room
+// for the four hardware queues of a process to run one each.
+//
+// Rows, partial sums and their order are those of k_means, k_cg64_init, k_cg_s, k_cg_u, k_sum1, k_shift and
+// k_resid64 with one workgroup per 256 rows, so the iterates are the same bit for bit.
+constexpr int PS_MAX_ROWS = 256 * B;
+constexpr int PS_SLOTS = 4 * 3 * 256;                       // sets, values, workgroups
+constexpr unsigned long long PS_EMPTY = 0x7FF8A5C3DEADBEEFull;  // a NaN no arithmetic produces by itself
+constexpr unsigned long long PS_WAIT = 2000000;             // 20 ms of the 100 MHz clock
+enum { PS_OK = 0, PS_GAVE_UP = 2 };
+
+__device__ __forceinline__ void ps_store(double *p, double v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double ps_load(const double *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// entry at byte offset o (a 32-bit offset from a uniform base costs one register an address, not two)
+__device__ __forceinline__ double ps_load(const double *p, unsigned o)
+{
+    return ps_load(reinterpret_cast<const double *>(reinterpret_cast<const char *>(p) + o));
+}
+
+__device__ __forceinline__ bool ps_empty(double v) { return (unsigned long long)__double_as_longlong(v) == PS_EMPTY; }
+
+// a NaN that is the sentinel by its bits becomes another
+__device__ __forceinline__ double ps_value(double v) { return ps_empty(v) ? __builtin_nan("") : v; }
+
+struct ps_state {
+    double *slots;
+    int nb, sync;    // workgroups; syncs so far
+    int at1, at2;    // the slots this workgroup published in at the last two syncs
+};
+
+// the sums over all workgroups of their threads' v (at: this workgroup's place in the order of
+// summation), the same in every thread; false when the wait was given up
+// HARD: every earlier store of the workgroup is complete before it publishes (for what others load unpolled)
+template <int NV, bool HARD = true>
+__device__ __forceinline__ bool ps_sum(ps_state &Q, const double (&v)[NV], int at, double (&out)[NV], bool mine = true)
+{
+    __shared__ double sm[NV][B / 64], so[NV][B / 64];
+    __shared__ int late[2];  // by parity of the sync: reset while the last sync's may still be read
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        const double s = lv_wave_sum(v[q]);
+        if (lane == 0) sm[q][w] = s;
+    }
+    const int lp = Q.sync & 1;
+    if (t == 0) late[lp] = 0;
+    if (HARD) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    double *set = Q.slots + (size_t)(Q.sync & 3) * 3 * 256;
+    if (t == 0) {
+        double *old = Q.slots + (size_t)((Q.sync + 2) & 3) * 3 * 256;
+        if (Q.sync >= 2)
+            for (int q = 0; q < 3; q++) ps_store(old + q * 256 + Q.at2, __longlong_as_double((long long)PS_EMPTY));
+#pragma unroll
+        for (int q = 0; q < NV; q++) {
+            double s = 0.0;
+            for (int k = 0; k < B / 64; k++) s += sm[q][k];
+            ps_store(set + q * 256 + at, ps_value(s));
+        }
+    }
+    Q.at2 = Q.at1;
+    Q.at1 = at;
+    Q.sync++;
+    if (!mine) late[lp] = 1;  // (this thread has already given up)
+    double p[NV];
+    if (t < Q.nb) {
+        unsigned long long t0 = 0;
+        bool expired = false;  // one more look after the time has run out, so that a wavefront that was
+                               // itself held up does not give up on what has long been published
+        for (int spin = 0;; spin++) {
+            bool got = true;
+#pragma unroll
+            for (int q = 0; q < NV; q++) p[q] = ps_load(set + q * 256 + t);
+#pragma unroll
+            for (int q = 0; q < NV; q++) got = got && !ps_empty(p[q]);
+            if (got) break;
+            if (expired) {
+                late[lp] = 1;
+                break;
+            }
+            if ((spin & 63) == 0) {
+                const unsigned long long now = wall_clock64();
+                if (spin == 0) t0 = now;
+                else expired = now - t0 > PS_WAIT;
+            }
+        }
+    }
+    // this wavefront's stores are complete, and what follows is loaded after the partials were seen
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        const double s = lv_wave_sum(t < Q.nb ? 0.0 + p[q] : 0.0);
+        if (lane == 0) so[q][w] = s;
+    }
+    __syncthreads();
+    const bool ok = late[lp] == 0;
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        double s = 0.0;
+        for (int k = 0; k < B / 64; k++) s += so[q][k];
+        out[q] = s;
+    }
+    return ok;
+}
+
+// (A y)_i of the owned row from its registers (slots past the eighth from memory), y gathered with
+// agent-scope loads; POLL: until none of the entries is empty any more (ok is cleared when that takes too
+// long)
+template <bool POLL>
+__device__ __forceinline__ double ps_row(const lv_ell_own<double> &A, int i, int n, int deg, const unsigned (&c)[8],
+                                         const double (&v)[8], double di, double yi, const double *y, bool &ok)
+{
+    unsigned long long t0 = 0;
+    auto wait = [&](int spin) {  // false: too long, and looked once more since
+        if (spin & 63) return true;
+        const unsigned long long now = wall_clock64();
+        if (spin == 0) t0 = now;
+        else if (t0 == 0) return false;
+        else if (now - t0 > PS_WAIT) t0 = 0;
+        return true;
+    };
+    double yj[8];
+    for (int spin = 0;; spin++) {
+        bool got = true;
+#pragma unroll
+        for (int k = 0; k < 8; k++) yj[k] = ps_load(y, c[k]);
+#pragma unroll
+        for (int k = 0; k < 8; k++) got = got && !ps_empty(yj[k]);
+        if (!POLL || got) break;
+        if (!wait(spin)) {
+            ok = false;
+            break;
+        }
+    }
+    double acc = di * yi;
+#pragma unroll
+    for (int k = 0; k < 8; k++) acc += v[k] * (yi - yj[k]);
+    for (int k = 8; k < deg; k++) {
+        const size_t e = (size_t)k * n + i;
+        const double *yk = y + A.column(e, i, n);
+        double t;
+        for (int spin = 0;; spin++) {
+            t = ps_load(yk);
+            if (!POLL || !ps_empty(t)) break;
+            if (!wait(spin)) {
+                ok = false;
+                break;
+            }
+        }
+        acc += A.value(e) * (yi - t);
+    }
+    return acc;
+}
+
+struct ps_ring {
+    double *z[3];
+};
+
+__global__ __launch_bounds__(B) void k_ps_init(lv_cg_scalars *S, double tol2, int itmax, int singular,
+                                               double *__restrict__ slots, int n, ps_ring Z)
+{
+    const double empty = __longlong_as_double((long long)PS_EMPTY);
+    const int t = blockIdx.x * B + threadIdx.x;
+    for (int k = t; k < PS_SLOTS; k += gridDim.x * B) slots[k] = empty;
+    if (t < n)
+        for (int q = 0; q < 3; q++) Z.z[q][t] = empty;
+    if (t != 0) return;
+    lv_cg_scalars z = {};
+    z.tol2 = tol2;
+    z.itmax = itmax;
+    z.singular = singular;
+    *S = z;
+}
+
+// x (in/out), r (out: the FP64 residual of the returned x), Z (work); the scalars the host reads in S and
+// published in pub under seq
+__global__ __launch_bounds__(B, 4) void k_pcg_small(int n, lv_ell_own<double> A, const double *__restrict__ diag,
+                                                    const double *__restrict__ dinv, const double *__restrict__ b,
+                                                    double *x, double *__restrict__ r_out, ps_ring Z, double tol2,
+                                                    int itmax, int singular, double *slots, lv_cg_scalars *S,
+                                                    lv_progress *pub, int seq)
+{
+    const int blk = lv_xcd_block(blockIdx.x, gridDim.x);  // the 256 rows this workgroup owns
+    const int i = blk * B + threadIdx.x;
+    const bool on = i < n;
+    const int row = on ? i : n - 1;
+    ps_state Q{slots, (int)gridDim.x, 0, 0, 0};
+    unsigned c[8];  // byte offsets
+    double v[8];
+    int deg;
+    {
+        int col[8];
+        deg = lv_ell_head<8>(A, row, n, col, v);
+#pragma unroll
+        for (int k = 0; k < 8; k++) c[k] = (unsigned)col[k] * sizeof(double);
+    }
+    const double di = diag[row], dv = dinv[row];
+    double xi = x[row];
+    int status = PS_OK, k = 0, done = 0;
+    double bmean = 0.0, xmean0 = 0.0, rr64 = 0.0, bb = 0.0, rr0 = 0.0, rr = 0.0, rz = 0.0, thr2 = 0.0, xshift = 0.0;
+    double ri = 0.0, zi = 0.0, pi = 0.0, qi = 0.0;
+    double *za = Z.z[0], *zb = Z.z[1], *zc = Z.z[2];  // z_k, z_{k+1}, z_{k+2}
+    bool ok = true;
+    do {
+        const double b0 = b[row];
+        if (singular) {
+            const double m[2] = {on ? b0 : 0.0, on ? xi : 0.0};
+            double o[2];
+            if (!ps_sum<2>(Q, m, blk, o)) { status = PS_GAVE_UP; break; }
+            bmean = o[0] / n;
+            xmean0 = o[1] / n;
+        }
+        {
+            const double bi = b0 - bmean;
+            ri = bi - ps_row<false>(A, row, n, deg, c, v, di, xi, x, ok);
+            zi = dv * ri;
+            if (on) ps_store(za + i, ps_value(zi));
+            const double m[3] = {on ? ri * zi : 0.0, on ? ri * ri : 0.0, on ? bi * bi : 0.0};
+            double o[3];
+            if (!ps_sum<3>(Q, m, blk, o)) { status = PS_GAVE_UP; break; }
+            rz = o[0];
+            rr = o[1];
+            thr2 = tol2 * o[2];
+        }
+        double rzp = 0.0;
+        for (;; k++) {  // (every workgroup sees the same sums and leaves the loop at the same k)
+            if (k == 0) rr0 = rr;
+            const bool conv = rr <= thr2;
+            if (conv || k >= itmax || !(rr == rr)) {
+                done = conv ? 1 : 2;
+                break;
+            }
+            const double beta = k == 0 ? 0.0 : rz / rzp;
+            const double w = ps_row<true>(A, row, n, deg, c, v, di, zi, za, ok);
+            qi = k == 0 ? w : w + beta * qi;
+            pi = k == 0 ? zi : zi + beta * pi;
+            const double m1[1] = {on ? pi * qi : 0.0};
+            double pq[1];
+            if (!ps_sum<1, false>(Q, m1, (int)blockIdx.x, pq, ok)) { status = PS_GAVE_UP; break; }
+            const double a = rz / pq[0];
+            xi += a * pi;
+            ri = ri - a * qi;
+            zi = dv * ri;
+            double *t = za;  // holds z_k, read by everyone: z_{k+3} next
+            za = zb;
+            zb = zc;
+            zc = t;
+            if (on) {
+                ps_store(za + i, ps_value(zi));
+                if (k > 0) ps_store(zb + i, __longlong_as_double((long long)PS_EMPTY));
+            }
+            const double m2[2] = {on ? ri * zi : 0.0, on ? ri * ri : 0.0};
+            double o[2];
+            if (!ps_sum<2, false>(Q, m2, blk, o)) { status = PS_GAVE_UP; break; }
+            rzp = rz;
+            rz = o[0];
+            rr = o[1];
+        }
+        if (status != PS_OK) break;
+        if (singular) {
+            const double m[1] = {on ? xi : 0.0};
+            double o[1];
+            if (!ps_sum<1>(Q, m, blk, o)) { status = PS_GAVE_UP; break; }
+            xshift = o[0] / n - xmean0;
+            xi -= xshift;
+        }
+        // the FP64 residual of the returned x
+        if (on) ps_store(x + i, xi);
+        const double none[1] = {0.0};
+        double o1[1];
+        if (!ps_sum<1>(Q, none, blk, o1)) { status = PS_GAVE_UP; break; }
+        const double bi = b0 - bmean;
+        const double rf = bi - ps_row<false>(A, row, n, deg, c, v, di, xi, x, ok);
+        if (on) r_out[i] = rf;
+        const double m[2] = {on ? rf * rf : 0.0, on ? bi * bi : 0.0};
+        double o[2];
+        if (!ps_sum<2>(Q, m, blk, o)) { status = PS_GAVE_UP; break; }
+        rr64 = o[0];
+        bb = o[1];
+    } while (false);
+    // on success workgroup 0 reports; a workgroup that gave up reports that (any of them, the same)
+    if (threadIdx.x != 0 || (status == PS_OK && blockIdx.x != 0)) return;
+    if (status == PS_OK) {
+        S->bmean = bmean;
+        S->xmean0 = xmean0;
+        S->xshift = 0.0;
+        S->bb = bb;
+        S->thr2 = tol2 * bb;
+        S->rr64 = rr64;
+        S->rr64_0 = rr0;
+        S->rr0 = rr0;
+        S->rr = rr;
+        S->iters = k;
+        S->done = done;
+        pub->rr64 = rr64;
+        pub->rr64_0 = rr0;
+        pub->bb = bb;
+        pub->thr2 = tol2 * bb;
+        pub->iters = k;
+    }
+    S->skip = status;
+    pub->skip = status;
+    __threadfence_system();
+    __hip_atomic_store(&pub->fseq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // ---- small FP64 vector algebra for the Picard extrapolation -----------------------------------
 
 // operands of the multi-dot and combination kernels; the a's and x's may be FP32 (the Picard
@@ -1091,7 +1427,7 @@ hipError_t lv_launch_write_P(lv_fields F, int n, const double *P, hipStream_t s)
 size_t lv_partials_bytes(int n)
 {
     (void)n;
-    return (size_t)8 * NBMAX * sizeof(double);
+    return ((size_t)8 * NBMAX + PS_SLOTS) * sizeof(double);  // block partials, then k_pcg_small's slots
 }
 
 namespace {
@@ -1335,6 +1671,33 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
     const parts P = parts_of(W.partials);
     lv_cg_scalars h;
     memset(&h, 0, sizeof(h));
+    // a small FP64 solve in one launch (not while its launches are being timed)
+    if (opt.method == LV_SOLVER_PCG64 && n <= PS_MAX_ROWS && !(t64 && t64->on)) {
+        double *slots = W.partials + (size_t)8 * NBMAX;
+        const double tol2 = opt.tol * opt.tol;
+        const int itmax = opt.itmax > 0 ? opt.itmax : 1000, seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
+        const ps_ring Z{{W.z, W.p, W.q}};
+        hipLaunchKernelGGL(k_ps_init, G, dim3(B), 0, s, W.S, tol2, itmax, (int)A.singular, slots, n, Z);
+        hipLaunchKernelGGL(k_pcg_small, G, dim3(B), 0, s, n, own64(A, n), (const double *)A.diag64,
+                           (const double *)A.dinv64, b, x, W.r, Z, tol2, itmax, (int)A.singular, slots, W.S, W.dprog,
+                           seq);
+        hipError_t e1 = hipGetLastError();
+        if (e1 != hipSuccess) return e1;
+        e1 = await_published(W.hprog, seq, W.S, W.hS, &h, s);
+        if (e1 != hipSuccess) return e1;
+        if (h.skip == PS_OK) {
+            *iters = h.iters;
+            *sweeps = 0;
+            *relres0 = (h.bb > 0.0) ? sqrt(h.rr64_0 / h.bb) : sqrt(h.rr64_0);
+            *relres = (h.bb > 0.0) ? sqrt(h.rr64 / h.bb) : sqrt(h.rr64);
+            *converged = (h.rr64 <= h.thr2);
+            return hipSuccess;
+        }
+        // some workgroup was not scheduled in time: launch by launch, after the last of them has ended
+        e1 = hipStreamSynchronize(s);
+        if (e1 != hipSuccess) return e1;
+        memset(&h, 0, sizeof(h));
+    }
     hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, opt.tol * opt.tol,
                        opt.itmax > 0 ? opt.itmax : 1000, (int)A.singular);
     hipError_t e = hipSuccess;
