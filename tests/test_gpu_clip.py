@@ -1,0 +1,52 @@
+"""The two ways clipping runs (a group of lanes per seed up to 49152 seeds and for polygons that outgrow eight
+slots, a thread per seed above): mesh bit for bit the oracle's on either side of the line, on regular,
+strongly jittered and random seeds."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+
+def _same_mesh(lv, oracle, x, dr, periodic, r_max=None):
+    grid = lv.VoronoiGrid(lv.UnitRectangle(), dr, r_max=r_max, xperiodic=periodic, yperiodic=periodic, positions=x)
+    lv.remesh(grid)
+    op = oracle.Particles(oracle.Grid((0.0, 0.0), (1.0, 1.0), dr, r_max=r_max, xperiodic=periodic,
+                                      yperiodic=periodic), x)
+    op.remesh()
+    for a, b in zip(grid.mesh(), op.mesh()):
+        assert np.array_equal(a, b)
+    assert np.array_equal(grid.get("area"), op.area())
+    return grid
+
+
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("K,jitter", [(12, 0.1), (17, 0.45), (40, 0.0), (221, 0.45), (222, 0.45)])
+def test_mesh_of_lattices_bit_exact(lv, oracle, gpu, K, jitter, periodic):
+    print("clip lattice %d %g" % (K, jitter), flush=True)
+    x = lv.inputs.jittered_lattice(K, K, 1.0 / K, jitter=jitter, seed=0x5EED0B00 + K)
+    grid = _same_mesh(lv, oracle, x, 1.0 / K, periodic)
+    assert (grid.n <= 49152) == (K < 222)
+    if jitter > 0.4:  # some polygons need more than eight slots
+        assert np.max(np.diff(grid.mesh()[0])) > 8
+
+
+@pytest.mark.parametrize("n", [1, 2, 900, 49152, 49153])
+def test_mesh_of_random_seeds_bit_exact(lv, oracle, gpu, n):
+    print("clip random %d" % n, flush=True)
+    x = np.random.default_rng(n).random(2 * n)
+    _same_mesh(lv, oracle, x, 0.2 if n < 900 else 1.0 / np.sqrt(n), False, r_max=3.0 if n < 900 else None)
+
+
+@pytest.mark.parametrize("around,ok", [(12, True), (40, False)])
+def test_polygons_of_too_many_edges_raise(lv, oracle, gpu, around, ok):
+    """a seed inside a ring of seeds: as many edges, at most LV_MAX_EDGES = 16"""
+    print("clip ring %d" % around, flush=True)
+    t = 2 * np.pi * (np.arange(around) + 0.1) / around
+    ring = 0.5 + 0.2 * np.stack([np.cos(t), np.sin(t)])
+    x = np.concatenate([[0.5], ring[0], [0.5], ring[1]])
+    if ok:
+        _same_mesh(lv, oracle, x, 0.1, False, r_max=2.0)
+    else:
+        grid = lv.VoronoiGrid(lv.UnitRectangle(), 0.1, r_max=2.0, positions=x)
+        with pytest.raises(lv.LVError, match="LV_MAX_EDGES"):
+            lv.remesh(grid)
