@@ -87,6 +87,7 @@ struct lv_ctx {
     int amg_layout = -1;   // the fine-level layout it was asked for (lv_solve_opts.amg_layout)
     int spmv32_agg = 0;    // the last FP32 inner solve ran in the aggregate order
     int A_kind = 0;        // what A holds: 0 the pressure operator, 1 the implicit viscous operator
+    double *mesh_stage = nullptr;  // staging of the mesh's rows on their way to the host (first use)
     // multiphase projection work space (allocated on first use)
     lv_mph_work *mph = nullptr;
     // solve timing: event pairs recorded around each solve and read when the API call returns its
@@ -476,6 +477,7 @@ int lv_destroy(lv_ctx *ctx)
         dfree(ctx->pw_P[k]);
         dfree(ctx->pw_AP[k]);
     }
+    dfree(ctx->mesh_stage);
     dfree(ctx->pw_t1);
     dfree(ctx->pw_t2);
     dfree(ctx->pw_dots);
@@ -677,39 +679,101 @@ int lv_remesh(lv_ctx *ctx)
     return LV_OK;
 }
 
+// ---- the mesh in CSR on the host --------------------------------------------------------------------
+
+}  // extern "C"
+
+namespace {
+
+// Edges of particles [i0, i1) from the slot-major mesh into rows: labels (int), and per edge the first PV
+// planes of its vertices (4: v1x, v1y, v2x, v2y; 2: v1 and a zero, as VTK's points).  ptr: the particles'
+// edge offsets; the chunk's rows start at ptr[i0].  A particle's slots are read as coalesced planes and its
+// rows are one run, so that what crosses to the host is the edges that exist, in their order there (the planes
+// hold 16 slots a particle, and gathering them on the host took ten times the copy).
+constexpr int MB = 256;
+template <int PV>
+__global__ __launch_bounds__(MB) void k_mesh_rows(lv_mesh_view M, const int *__restrict__ ptr, int i0, int i1,
+                                                  int *__restrict__ labels, double *__restrict__ verts)
+{
+    const int i = i0 + blockIdx.x * MB + threadIdx.x;
+    if (i >= i1) return;
+    const int o0 = ptr[i] - ptr[i0], ne = M.ne[i];
+    for (int k = 0; k < ne; k++) {
+        const size_t o = (size_t)(o0 + k);
+        if (labels) labels[o] = LV_EL(M, k, i);
+        const double a = LV_EV(M, 0, k, i), b = LV_EV(M, 1, k, i);
+        if (PV == 4) {
+            double4 *v = reinterpret_cast<double4 *>(verts) + o;
+            *v = make_double4(a, b, LV_EV(M, 2, k, i), LV_EV(M, 3, k, i));
+        } else {
+            verts[3 * o] = a;
+            verts[3 * o + 1] = b;
+            verts[3 * o + 2] = 0.0;
+        }
+    }
+}
+
+// particles a chunk of rows holds: its staging (at most LV_MAXE edges of 4 + 32 bytes each) is 18 MiB
+constexpr int MESH_CHUNK = 32768;
+
+// the edge offsets of every particle into ctx->clip_retry (work space of the next remesh, n + 1 ints) and
+// the number of edges
+int mesh_offsets(lv_ctx *ctx, int64_t *nedges)
+{
+    const int n = ctx->n;
+    int *ptr = ctx->clip_retry;
+    LV_HIP_CHECK(lv_exclusive_scan_i32(ctx->ne, ptr, n, ptr + n, ctx->scan_temp, ctx->s));
+    int total = 0;
+    LV_HIP_CHECK(hipMemcpyAsync(&total, ptr + n, sizeof(int), hipMemcpyDeviceToHost, ctx->s));
+    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+    *nedges = total;
+    return LV_OK;
+}
+
+// the rows of the whole mesh on the host, chunk by chunk (labels may be null); ptr: the offsets already there
+template <int PV>
+int mesh_rows(lv_ctx *ctx, const int *hptr, int32_t *labels, double *verts)
+{
+    const int n = ctx->n;
+    constexpr size_t W = PV == 4 ? 4 : 3;
+    if (!ctx->mesh_stage) LV_HIP_CHECK(dalloc(&ctx->mesh_stage, (size_t)MESH_CHUNK * LV_MAXE * 4 + MESH_CHUNK * LV_MAXE / 2));
+    double *dv = ctx->mesh_stage;
+    int *dl = reinterpret_cast<int *>(dv + (size_t)MESH_CHUNK * LV_MAXE * 4);
+    for (int i0 = 0; i0 < n; i0 += MESH_CHUNK) {
+        const int i1 = std::min(n, i0 + MESH_CHUNK);
+        const size_t o = (size_t)hptr[i0], m = (size_t)hptr[i1] - o;
+        if (m == 0) continue;
+        hipLaunchKernelGGL(k_mesh_rows<PV>, dim3((i1 - i0 + MB - 1) / MB), dim3(MB), 0, ctx->s, mesh_view(ctx),
+                           (const int *)ctx->clip_retry, i0, i1, labels ? dl : (int *)nullptr, dv);
+        LV_HIP_CHECK(hipGetLastError());
+        if (labels) LV_HIP_CHECK(hipMemcpyAsync(labels + o, dl, sizeof(int) * m, hipMemcpyDeviceToHost, ctx->s));
+        LV_HIP_CHECK(hipMemcpyAsync(verts + W * o, dv, sizeof(double) * W * m, hipMemcpyDeviceToHost, ctx->s));
+    }
+    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+    return LV_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int lv_mesh_size(lv_ctx *ctx, int64_t *nedges)
 {
     int rc = check_ctx(ctx, true);
     if (rc) return rc;
-    std::vector<int> ne(ctx->n);
-    LV_HIP_CHECK(hipMemcpy(ne.data(), ctx->ne, sizeof(int) * ctx->n, hipMemcpyDeviceToHost));
-    int64_t t = 0;
-    for (int v : ne) t += v;
-    *nedges = t;
-    return LV_OK;
+    return mesh_offsets(ctx, nedges);
 }
 
 int lv_get_mesh(lv_ctx *ctx, int32_t *edge_ptr, int32_t *labels, double *verts)
 {
+    int64_t total;
     int rc = check_ctx(ctx, true);
     if (rc) return rc;
-    const int n = ctx->n;
-    std::vector<int> ne(n), el((size_t)LV_MAXE * n);
-    std::vector<double> ev((size_t)4 * LV_MAXE * n);
-    LV_HIP_CHECK(hipMemcpy(ne.data(), ctx->ne, sizeof(int) * n, hipMemcpyDeviceToHost));
-    LV_HIP_CHECK(hipMemcpy(el.data(), ctx->el, sizeof(int) * LV_MAXE * n, hipMemcpyDeviceToHost));
-    LV_HIP_CHECK(hipMemcpy(ev.data(), ctx->ev, sizeof(double) * 4 * LV_MAXE * n, hipMemcpyDeviceToHost));
-    int64_t o = 0;
-    for (int i = 0; i < n; i++) {
-        edge_ptr[i] = (int32_t)o;
-        for (int k = 0; k < ne[i]; k++) {
-            labels[o] = el[(size_t)k * n + i];
-            for (int p = 0; p < 4; p++) verts[4 * o + p] = ev[(size_t)(p * LV_MAXE + k) * n + i];
-            o++;
-        }
-    }
-    edge_ptr[n] = (int32_t)o;
-    return LV_OK;
+    if ((rc = mesh_offsets(ctx, &total))) return rc;
+    LV_HIP_CHECK(hipMemcpyAsync(edge_ptr, ctx->clip_retry, sizeof(int) * ((size_t)ctx->n + 1), hipMemcpyDeviceToHost,
+                                ctx->s));
+    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+    return mesh_rows<4>(ctx, edge_ptr, labels, verts);
 }
 
 // ---- VTK export (src/IO.jl:9-71) ------------------------------------------------------------------
@@ -790,26 +854,15 @@ int lv_export_grid(lv_ctx *ctx, const char *filename, const int32_t *fields, int
     if (rc) return rc;
     if (!filename || nfields < 0 || (nfields > 0 && !fields)) return lv_fail(ctx, LV_E_INVALID, "lv_export_grid");
     const int n = ctx->n;
-    std::vector<int> ne(n), dummy;
-    std::vector<double> ev((size_t)2 * LV_MAXE * n);
-    if (n) {
-        LV_HIP_CHECK(hipMemcpy(ne.data(), ctx->ne, sizeof(int) * n, hipMemcpyDeviceToHost));
-        // the v1 planes of the edge slots
-        LV_HIP_CHECK(hipMemcpy(ev.data(), ctx->ev, sizeof(double) * 2 * LV_MAXE * n, hipMemcpyDeviceToHost));
-    }
     // every polygon's edges in their (chained) order: its vertices are the edges' v1 (src/IO.jl:17-27)
-    std::vector<double> pts;
-    std::vector<int64_t> conn, offs(n);
     int64_t o = 0;
-    for (int i = 0; i < n; i++) {
-        for (int k = 0; k < ne[i]; k++) {
-            pts.push_back(ev[(size_t)k * n + i]);
-            pts.push_back(ev[(size_t)(LV_MAXE + k) * n + i]);
-            pts.push_back(0.0);
-            conn.push_back(o++);
-        }
-        offs[i] = o;
-    }
+    if ((rc = mesh_offsets(ctx, &o))) return rc;
+    std::vector<int> ptr((size_t)n + 1);
+    LV_HIP_CHECK(hipMemcpy(ptr.data(), ctx->clip_retry, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToHost));
+    std::vector<double> pts((size_t)3 * o);
+    if ((rc = mesh_rows<2>(ctx, ptr.data(), nullptr, pts.data()))) return rc;
+    std::vector<int64_t> conn(o), offs(ptr.begin() + 1, ptr.end());
+    for (int64_t k = 0; k < o; k++) conn[k] = k;
     std::vector<std::vector<double>> cols;
     std::vector<lv_vtk_array> arr;
     rc = export_columns(ctx, fields, nfields, cols, arr);
