@@ -33,14 +33,18 @@ struct lv_amg {
     float *tail_mat, *ext_mat;  // a singular system's W-visit of the tail as a matrix on its first level, and of
     size_t cap_tail_mat, cap_ext_mat;  // the level above it when that is small enough
     const float *mat;    // the one the cycle multiplies by, on level lmat, leading dimension mat_ld (0: none, the
-    int lmat, mat_ld;    // visit runs its program on level lmat = ltail)
+    int lmat, mat_ld;    // visit runs its program)
     double *pw;          // power-iteration partials and norms
     float *pv, *pu;      // power-iteration vectors (n0)
     size_t cap_pv, cap_pu;
-    int ltail;           // first level of the single-workgroup kernel (levels ltail..nlev)
-    int pair[LV_AMG_MAXLEV + 1];  // pair[l]: levels l and l+1 (both above ltail) run as one down and
+    int lk;              // first level of the single-workgroup kernel's program (levels lk..nlev)
+    int lds_ok;          // 1: their arrays fit its LDS
+    int *desc;           // their descriptors (device) and the host copy
+    int hdesc[(LV_AMG_MAXLEV + 1) * 16];
+    int tail_coef, tail_inv, tail_total;  // the LDS image's size, its dense inverse, and the LDS in use
+    int pair[LV_AMG_MAXLEV + 1];  // pair[l]: levels l and l+1 (both above that kernel's) run as one down and
                                   // one up kernel
-    int level_kernels;   // 1: every level above ltail runs as its own kernels (pairs not used)
+    int level_kernels;   // 1: every level above lk runs as its own kernels (pairs not used)
     int wcycle;          // 1: the levels of that kernel are visited by a W-cycle
     int *prog;           // its operations (device), nprog of them; hprog: the host copy
     int nprog;

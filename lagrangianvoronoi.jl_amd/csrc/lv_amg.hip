@@ -1196,6 +1196,12 @@ constexpr int TAIL_MAX = 1024;  // levels of at most this many cells run in the 
 // the eight L2s hold, so that a small system's cycles find it there (above that the two stencil launches
 // that the level saves cost less than the bytes).
 constexpr int MAT_MAX = 2560;
+// A nonsingular system, whose tail is visited once a cycle, starts it at its first level of at most LDS_MAX
+// cells (33 x 33 cells: 11.0 us with them, 9.0 and two launches of 3.3 without; the level above, 65 x 65 cells with
+// its couplings in registers, cost it 17 us more, so that level keeps its launches)
+constexpr int LDS_MAX = 1280;
+constexpr int LV_DESC = 16;  // ints of a level's descriptor (tail_descriptors)
+constexpr int LV_CELL = 12;  // floats of a cell's constants in the LDS image: c[8], d, 1 / (d + sum c), two unused
 enum tail_op { OP_DOWN = 0, OP_DENSE = 1, OP_UP = 2, OP_WSAVE = 3, OP_WADD = 4 };
 constexpr int OP_SHIFT = 5;  // an operation is op << OP_SHIFT | level
 static_assert(LV_AMG_MAXLEV < (1 << OP_SHIFT), "levels fit the operation code");
@@ -1207,94 +1213,206 @@ struct tail_levels {
     float *r[LV_AMG_MAXLEV + 1], *z[LV_AMG_MAXLEV + 1], *t[LV_AMG_MAXLEV + 1], *acc[LV_AMG_MAXLEV + 1];
 };
 
-// where the tail keeps its levels: global memory (the levels' own arrays) or LDS (offsets into
-// one workgroup array); both give the same values, operation by operation
-struct tail_in_global {
-    const tail_levels &T;
-    const float *inv_;
-    __device__ const float *d(int l) const { return T.d[l]; }
-    __device__ const float *c(int l) const { return T.c[l]; }
-    __device__ const float *dinv(int l) const { return T.dinv[l]; }
-    __device__ float *r(int l) const { return T.r[l]; }
-    __device__ float *z(int l) const { return T.z[l]; }
-    __device__ float *t(int l) const { return T.t[l]; }
-    __device__ float *acc(int l) const { return T.acc[l]; }
-    __device__ const float *inv() const { return inv_; }
-};
-
-// offsets (in floats) of every array of the tail levels in the LDS copy; total <= TAIL_LDS
+// The tail levels in LDS, offsets in floats: a level's constants (LV_CELL floats a cell), then the dense
+// inverse; then, zeroed and filled by the program, z and t with a halo of one cell around the level (its periodic
+// neighbours, or zeros outside it), and r and the W-cycle's accumulator.  With the constants of a cell in three
+// 16-byte reads and the neighbours at fixed offsets, an operation has next to no index arithmetic, which is what
+// a single workgroup has to spend its instructions on otherwise (the same program with slot-major
+// couplings, neighbour indices and the neighbours' z recomputed from r and D^-1: 10.1 us at 16 x 32 cells and
+// 11.9 at 32 x 32, against 7.0 and 9.7).
 constexpr int TAIL_LDS = 35 * 1024;
 struct tail_layout {
-    int d[LV_AMG_MAXLEV + 1], c[LV_AMG_MAXLEV + 1], dinv[LV_AMG_MAXLEV + 1];
-    int r[LV_AMG_MAXLEV + 1], z[LV_AMG_MAXLEV + 1], t[LV_AMG_MAXLEV + 1], acc[LV_AMG_MAXLEV + 1];
-    int inv, coef, total;  // [0, coef): the constant arrays, then the work vectors
+    int k[LV_AMG_MAXLEV + 1], r[LV_AMG_MAXLEV + 1], z[LV_AMG_MAXLEV + 1], t[LV_AMG_MAXLEV + 1],
+        acc[LV_AMG_MAXLEV + 1];
+    int inv, coef, total;  // [0, coef): the constants, then the work vectors
 };
 
-struct tail_in_lds {
-    float *lds;
-    const tail_layout &Y;
-    __device__ const float *d(int l) const { return lds + Y.d[l]; }
-    __device__ const float *c(int l) const { return lds + Y.c[l]; }
-    __device__ const float *dinv(int l) const { return lds + Y.dinv[l]; }
-    __device__ float *r(int l) const { return lds + Y.r[l]; }
-    __device__ float *z(int l) const { return lds + Y.z[l]; }
-    __device__ float *t(int l) const { return lds + Y.t[l]; }
-    __device__ float *acc(int l) const { return lds + Y.acc[l]; }
-    __device__ const float *inv() const { return lds + Y.inv; }
-};
-
-// the program's operations, each followed by a barrier that makes its writes visible to the
-// workgroup
-template <class M>
-__device__ __forceinline__ void run_tail(const tail_levels &T, const M &m, const int *prog, int nprog)
+// the program on the levels' own arrays in global memory, each operation followed by a barrier that makes its
+// writes visible to the workgroup
+__global__ __launch_bounds__(TB) void k_tail(tail_levels T, const int *__restrict__ prog, int nprog,
+                                             const float *__restrict__ inv, const lv_cg_scalars *S)
 {
+    if (S && S->done) return;
     for (int pc = 0; pc < nprog; pc++) {
         const int code = prog[pc];
         const int op = code >> OP_SHIFT, l = code & ((1 << OP_SHIFT) - 1);
-        const st_level L{T.Kx[l], T.Ky[l], T.xper, T.yper, m.d(l), m.c(l), m.dinv(l), T.alpha[l]};
+        const st_level L{T.Kx[l], T.Ky[l], T.xper, T.yper, T.d[l], T.c[l], T.dinv[l], T.alpha[l]};
         const int n = T.Kx[l] * T.Ky[l];
         if (op == OP_DOWN) {
             const int Kyc = T.Ky[l + 1], nc = T.Kx[l + 1] * T.Ky[l + 1];
-            float *rl = m.r(l), *zl = m.z(l), *rc = m.r(l + 1);
             for (int base = 0; base < nc * CF2; base += TB) {  // uniform trip count: every lane shuffles
                 const int tid = base + threadIdx.x;
                 const int P = tid / CF2, q = tid % CF2;
-                const float t = sum_children(st_down_lane(L, Kyc, nc, P, q, rl, zl));
-                if (q == 0 && P < nc) rc[P] = t;
+                const float t = sum_children(st_down_lane(L, Kyc, nc, P, q, T.r[l], T.z[l]));
+                if (q == 0 && P < nc) T.r[l + 1][P] = t;
             }
         } else if (op == OP_DENSE) {
             // t = inv r: 16 lanes per row (LV_AMG_DENSE_MAX * 16 == TB)
             const int i = threadIdx.x >> 4, q = threadIdx.x & 15;
-            const float *rd = m.r(l), *iv = m.inv();
             float acc = 0.0f;
             if (i < n)
-                for (int j = q; j < n; j += 16) acc += iv[j * n + i] * rd[j];
+                for (int j = q; j < n; j += 16) acc += inv[j * n + i] * T.r[l][j];
             acc += __shfl_xor(acc, 1);
             acc += __shfl_xor(acc, 2);
             acc += __shfl_xor(acc, 4);
             acc += __shfl_xor(acc, 8);
-            if (q == 0 && i < n) m.t(l)[i] = acc;
+            if (q == 0 && i < n) T.t[l][i] = acc;
         } else if (op == OP_UP) {
-            const float *rl = m.r(l), *zl = m.z(l), *ec = m.t(l + 1);
-            float *out = m.t(l);
-            for (int f = threadIdx.x; f < n; f += TB) st_up_cell(L, T.Ky[l + 1], f, rl, zl, ec, out);
+            for (int f = threadIdx.x; f < n; f += TB) st_up_cell(L, T.Ky[l + 1], f, T.r[l], T.z[l], T.t[l + 1], T.t[l]);
         } else if (op == OP_WSAVE) {
-            float *rl = m.r(l), *tl = m.t(l), *al = m.acc(l);
-            for (int f = threadIdx.x; f < n; f += TB) st_wsave_cell(L, f, rl, tl, al);
+            for (int f = threadIdx.x; f < n; f += TB) st_wsave_cell(L, f, T.r[l], T.t[l], T.acc[l]);
         } else {  // OP_WADD
-            float *tl = m.t(l);
-            const float *al = m.acc(l);
-            for (int f = threadIdx.x; f < n; f += TB) tl[f] += al[f];
+            for (int f = threadIdx.x; f < n; f += TB) T.t[l][f] += T.acc[l][f];
         }
         __syncthreads();
     }
 }
 
-__global__ __launch_bounds__(TB) void k_tail(tail_levels T, const int *__restrict__ prog, int nprog,
-                                             const float *__restrict__ inv, const lv_cg_scalars *S)
+// a / K with rK = 1 / K in FP32, for 0 <= a < 8192: (a + 1/2) / K is at least 1 / (2 K) from an integer, a
+// relative 6e-5, and the product is off by 2e-7 at most
+__device__ __forceinline__ int div_small(int a, float rK) { return (int)(((float)a + 0.5f) * rK); }
+
+// a level in LDS
+struct tail_lev {
+    int Kx, Ky, n, ld;
+    float rKy, alpha;
+    const float *k;          // constants
+    float *r, *z, *t, *acc;  // z and t with halo, leading dimension ld = Ky + 2
+};
+__device__ __forceinline__ tail_lev tail_level(float *lds, const int *D)
 {
-    if (S && S->done) return;
-    run_tail(T, tail_in_global{T, inv}, prog, nprog);
+    return tail_lev{D[0], D[1], D[2], D[1] + 2, __int_as_float(D[4]), __int_as_float(D[3]), lds + D[5], lds + D[6],
+                    lds + D[7], lds + D[8], lds + D[9]};
+}
+struct tail_cell {
+    float c[8], d, dinv;
+};
+__device__ __forceinline__ tail_cell tail_consts(const tail_lev &L, int f)
+{
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    const f4 *k = reinterpret_cast<const f4 *>(L.k + f * LV_CELL);
+    const f4 a = k[0], b = k[1], e = k[2];
+    return tail_cell{{a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w}, e.x, e.y};
+}
+// v into cell (cx, cy) of the haloed array a, and into the halo cells that stand for it on periodic axes
+__device__ __forceinline__ void tail_put(float *a, const tail_lev &L, int xper, int yper, int cx, int cy, float v)
+{
+    const int ld = L.ld;
+    a[(cx + 1) * ld + cy + 1] = v;
+    const bool x0 = xper && cx == 0, x1 = xper && cx == L.Kx - 1, y0 = yper && cy == 0, y1 = yper && cy == L.Ky - 1;
+    if (!(x0 || x1 || y0 || y1)) return;
+    auto column = [&](int px) {
+        if (y0) a[px * ld + L.Ky + 1] = v;
+        if (y1) a[px * ld] = v;
+    };
+    column(cx + 1);
+    if (x0) {
+        a[(L.Kx + 1) * ld + cy + 1] = v;
+        column(L.Kx + 1);
+    }
+    if (x1) {
+        a[cy + 1] = v;
+        column(0);
+    }
+}
+// the neighbours of the haloed array's entry at p, in slot order
+__device__ __forceinline__ void tail_nbrs(const float *a, int p, int ld, float (&v)[8])
+{
+    v[0] = a[p - ld - 1];
+    v[1] = a[p - ld];
+    v[2] = a[p - ld + 1];
+    v[3] = a[p - 1];
+    v[4] = a[p + 1];
+    v[5] = a[p + ld - 1];
+    v[6] = a[p + ld];
+    v[7] = a[p + ld + 1];
+}
+
+// One operation in LDS, the arithmetic of st_down_lane, st_up_cell and st_wsave_cell (L: its level, C: the next).  A
+// right-hand side is stored with its level's pre-smoothed z = w D^-1 r.  (A neighbour outside a level has
+// coupling 0 there, by construction, and a zero in the halo.)
+__device__ __forceinline__ void tail_step(int op, const tail_lev &L, const tail_lev &C, bool dense_next, const float *inv,
+                                          int xper, int yper)
+{
+    if (op == OP_DOWN) {
+        for (int base = 0; base < C.n * CF2; base += TB) {  // uniform trip count: every lane shuffles
+            const int tid = base + threadIdx.x;
+            const int P = tid / CF2, q = tid % CF2, Px = div_small(P, C.rKy), Py = P - Px * C.Ky;
+            const int cx = CF * Px + q / CF, cy = CF * Py + q % CF;
+            float t = 0.0f;
+            if (P < C.n && cx < L.Kx && cy < L.Ky) {
+                const int f = cx * L.Ky + cy, p = (cx + 1) * L.ld + cy + 1;
+                const tail_cell k = tail_consts(L, f);
+                float zj[8];
+                tail_nbrs(L.z, p, L.ld, zj);
+                const float zf = L.z[p];
+                float acc = k.d * zf;
+#pragma unroll
+                for (int e = 0; e < 8; e++) acc += k.c[e] * (zf - zj[e]);
+                t = L.r[f] - acc;
+            }
+            t = sum_children(t);
+            if (q == 0 && P < C.n) {
+                C.r[P] = t;
+                if (!dense_next) tail_put(C.z, C, xper, yper, Px, Py, OMEGA * C.k[P * LV_CELL + 9] * t);
+            }
+        }
+    } else if (op == OP_DENSE) {
+        // t = inv r: 16 lanes per row (LV_AMG_DENSE_MAX * 16 == TB)
+        const int n = L.n, i = threadIdx.x >> 4, q = threadIdx.x & 15;
+        float acc = 0.0f;
+        if (i < n)
+            for (int j = q; j < n; j += 16) acc += inv[j * n + i] * L.r[j];
+        acc += __shfl_xor(acc, 1);
+        acc += __shfl_xor(acc, 2);
+        acc += __shfl_xor(acc, 4);
+        acc += __shfl_xor(acc, 8);
+        if (q == 0 && i < n) {
+            const int cx = div_small(i, L.rKy);
+            tail_put(L.t, L, xper, yper, cx, i - cx * L.Ky, acc);
+        }
+    } else if (op == OP_UP) {
+        for (int f = threadIdx.x; f < L.n; f += TB) {
+            const int cx = div_small(f, L.rKy), cy = f - cx * L.Ky, p = (cx + 1) * L.ld + cy + 1;
+            const tail_cell k = tail_consts(L, f);
+            float zj[8];
+            tail_nbrs(L.z, p, L.ld, zj);
+            // the parents of the neighbours on each side: the cell's own, or the next one (with the halo, at
+            // the ends of the level too; a last cell without a sibling has the next parent on its right)
+            const int Px = cx / CF + 1, Py = cy / CF + 1;
+            const int xl = (cx % CF ? Px : Px - 1) * C.ld, xr = (cx % CF || cx + 1 == L.Kx ? Px + 1 : Px) * C.ld;
+            const int yl = cy % CF ? Py : Py - 1, yr = cy % CF || cy + 1 == L.Ky ? Py + 1 : Py;
+            const int xo = Px * C.ld;
+            const float a = L.alpha;
+            const float ej[8] = {a * C.t[xl + yl], a * C.t[xl + Py], a * C.t[xl + yr], a * C.t[xo + yl],
+                                 a * C.t[xo + yr], a * C.t[xr + yl], a * C.t[xr + Py], a * C.t[xr + yr]};
+            const float z1 = L.z[p] + a * C.t[xo + Py];
+            float acc = k.d * z1;
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc += k.c[e] * (z1 - (zj[e] + ej[e]));
+            tail_put(L.t, L, xper, yper, cx, cy, z1 + OMEGA * k.dinv * (L.r[f] - acc));
+        }
+    } else if (op == OP_WSAVE) {
+        for (int f = threadIdx.x; f < L.n; f += TB) {
+            const int cx = div_small(f, L.rKy), cy = f - cx * L.Ky, p = (cx + 1) * L.ld + cy + 1;
+            const tail_cell k = tail_consts(L, f);
+            float tj[8];
+            tail_nbrs(L.t, p, L.ld, tj);
+            const float tf = L.t[p];
+            float acc = k.d * tf;
+#pragma unroll
+            for (int e = 0; e < 8; e++) acc += k.c[e] * (tf - tj[e]);
+            L.acc[f] = tf;
+            const float r = L.r[f] - acc;
+            L.r[f] = r;
+            tail_put(L.z, L, xper, yper, cx, cy, OMEGA * k.dinv * r);
+        }
+    } else {  // OP_WADD
+        for (int f = threadIdx.x; f < L.n; f += TB) {
+            const int cx = div_small(f, L.rKy), cy = f - cx * L.Ky;
+            tail_put(L.t, L, xper, yper, cx, cy, L.t[(cx + 1) * L.ld + cy + 1] + L.acc[f]);
+        }
+    }
 }
 
 // The same program with the tail levels in LDS: the couplings, the dense inverse, the program
@@ -1310,46 +1428,71 @@ __global__ __launch_bounds__(TB) void k_tail(tail_levels T, const int *__restric
 // leading dimension ld: the operator is symmetric), and each cycle multiplies by the matrix (k_mat_mv).  The
 // W-visit is a serial chain of about 30 operations on one CU, 25-29 us a cycle whatever the rest of the device
 // does; the product reads at most 4 MB spread over the device in one round trip, 2.7-4.7 us, and the columns
-// take 72 us once per set-up (25 x 25 cells, 3 turns of the device).  A nonsingular system keeps the program: its V-visit takes 10.4 us, and its
+// take 60 us once per set-up (25 x 25 cells, 3 turns of the device).  A nonsingular system keeps the program: its V-visit takes 7-11 us, and its
 // solves keep their iterates bit for bit (velocities near rest are small differences of pressures, and
 // would show another rounding of the cycle magnified).
+struct tail_lds_args {
+    const int *desc, *prog;  // the levels' descriptors (LV_DESC ints each), the operations
+    int nprog;
+    const float *img;
+    int coef, total, first, last, n0, xper, yper, inv;
+    const float *r, *dinv;  // right-hand side, 1 / (d + sum c) and correction of level `first`
+    float *t;
+};
+
 template <bool COLS>
-__global__ __launch_bounds__(TB) void k_tail_lds(tail_levels T, tail_layout Y, const int *__restrict__ prog,
-                                                 int nprog, const float *__restrict__ img, const lv_cg_scalars *S,
-                                                 float *__restrict__ mat, int ld)
+__global__ __launch_bounds__(TB) void k_tail_lds(tail_lds_args T, const lv_cg_scalars *S, float *__restrict__ mat, int ld)
 {
     __shared__ __align__(16) float lds[TAIL_LDS];
-    __shared__ int lprog[LV_AMG_MAXPROG];
-    const int first = T.first;
+    __shared__ int lprog[LV_AMG_MAXPROG], desc[(LV_AMG_MAXLEV + 1) * LV_DESC];
     constexpr int PER4 = (TAIL_LDS / 4 + TB - 1) / TB;  // float4s per lane
-    const int n4 = Y.coef / 4;
+    const int n4 = T.coef / 4, t = threadIdx.x;
     typedef float f4 __attribute__((ext_vector_type(4)));
-    const f4 *img4 = reinterpret_cast<const f4 *>(img);
+    const f4 *img4 = reinterpret_cast<const f4 *>(T.img);
     f4 v[PER4];
 #pragma unroll
     for (int q = 0; q < PER4; q++)
-        if (q * TB + (int)threadIdx.x < n4) v[q] = img4[q * TB + threadIdx.x];
-    const int n0 = T.Kx[first] * T.Ky[first];
-    const int f0 = threadIdx.x;  // n0 <= TAIL_MAX == TB: one right-hand side entry per lane
-    float r0 = 0.0f;
-    if (COLS) r0 = f0 == (int)blockIdx.x ? 1.0f : 0.0f;
-    else if (f0 < n0) r0 = T.r[first][f0];
-    const int pr = (int)threadIdx.x < nprog ? prog[threadIdx.x] : 0;  // nprog <= LV_AMG_MAXPROG <= TB
+        if (q * TB + t < n4) v[q] = img4[q * TB + t];
+    const int pr = t < T.nprog ? T.prog[t] : 0;  // nprog <= LV_AMG_MAXPROG <= TB
+    const int de = t < (LV_AMG_MAXLEV + 1) * LV_DESC ? T.desc[t] : 0;
+    float r0[2], v0[2];  // n0 <= LDS_MAX <= 2 TB
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int f = h * TB + t;
+        r0[h] = f < T.n0 ? (COLS ? (f == (int)blockIdx.x ? 1.0f : 0.0f) : T.r[f]) : 0.0f;
+        v0[h] = f < T.n0 ? T.dinv[f] : 0.0f;
+    }
     if (S && S->done) return;  // tested after the loads above are issued (they read valid arrays)
     f4 *lds4 = reinterpret_cast<f4 *>(lds);
 #pragma unroll
     for (int q = 0; q < PER4; q++)
-        if (q * TB + (int)threadIdx.x < n4) lds4[q * TB + threadIdx.x] = v[q];
-    for (int f = 4 * n4 + threadIdx.x; f < Y.coef; f += TB) lds[f] = img[f];
-    if (f0 < n0) lds[Y.r[first] + f0] = r0;
-    if ((int)threadIdx.x < nprog) lprog[threadIdx.x] = pr;
+        if (q * TB + t < n4) lds4[q * TB + t] = v[q];
+    for (int f = T.coef + t; f < T.total; f += TB) lds[f] = 0.0f;
+    if (t < T.nprog) lprog[t] = pr;
+    if (t < (LV_AMG_MAXLEV + 1) * LV_DESC) desc[t] = de;
     __syncthreads();
-    run_tail(T, tail_in_lds{lds, Y}, lprog, nprog);
-    if (COLS) {
-        float *row = mat + (size_t)blockIdx.x * ld;
-        for (int f = threadIdx.x; f < ld; f += TB) row[f] = f < n0 ? lds[Y.t[first] + f] : 0.0f;
-    } else {
-        for (int f = threadIdx.x; f < n0; f += TB) T.t[first][f] = lds[Y.t[first] + f];
+    const tail_lev L0 = tail_level(lds, desc + T.first * LV_DESC);
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int f = h * TB + t;
+        if (f >= T.n0) continue;
+        L0.r[f] = r0[h];
+        const int cx = div_small(f, L0.rKy);
+        if (T.first < T.last) tail_put(L0.z, L0, T.xper, T.yper, cx, f - cx * L0.Ky, OMEGA * v0[h] * r0[h]);
+    }
+    __syncthreads();
+    for (int pc = 0; pc < T.nprog; pc++) {
+        const int code = lprog[pc];
+        const int op = code >> OP_SHIFT, l = code & ((1 << OP_SHIFT) - 1);
+        const int *D = desc + l * LV_DESC;
+        tail_step(op, tail_level(lds, D), tail_level(lds, D + (l < T.last ? LV_DESC : 0)), l + 1 == T.last, lds + T.inv,
+                  T.xper, T.yper);
+        __syncthreads();
+    }
+    float *row = COLS ? mat + (size_t)blockIdx.x * ld : T.t;
+    for (int f = t; f < (COLS ? ld : T.n0); f += TB) {
+        const int cx = div_small(f, L0.rKy);
+        row[f] = f < T.n0 ? L0.t[(cx + 1) * L0.ld + (f - cx * L0.Ky) + 1] : 0.0f;
     }
 }
 
@@ -1437,24 +1580,26 @@ __global__ __launch_bounds__(B) void k_mat_mv(int n, int ld, const float *__rest
 }
 static_assert(B == 256 && FUSE_ROWS + 64 <= FUSE_CAP, "fused blocks fit their LDS rows");
 static_assert(LV_AMG_DENSE_MAX * 16 == TB, "the dense solve of the tail maps 16 lanes to a row");
-static_assert(TAIL_MAX <= TB && LV_AMG_MAXPROG <= TB, "one right-hand side entry and one operation per lane");
+static_assert(TAIL_MAX <= LDS_MAX && LDS_MAX <= 2 * TB && LV_AMG_MAXPROG <= TB && LDS_MAX * CF2 <= 8192 &&
+                  (LV_AMG_MAXLEV + 1) * LV_DESC <= TB,
+              "right-hand side entries, operations and descriptors per lane, and indices that div_small divides");
 static_assert(TAIL_LDS % 4 == 0, "the LDS image is copied as float4");
 
-// the tail levels' constant arrays (diagonals, couplings, dense inverse) into img in the LDS layout
+// the tail levels' constants and the dense inverse into img in the LDS layout
 __global__ __launch_bounds__(B) void k_tail_pack(tail_levels T, tail_layout Y, const float *__restrict__ inv,
                                                  float *__restrict__ img)
 {
     const int stride = gridDim.x * B;
     for (int l = T.first; l < T.last; l++) {
         const int n = T.Kx[l] * T.Ky[l];
-        for (int f = blockIdx.x * B + threadIdx.x; f < n; f += stride) {
-            img[Y.d[l] + f] = T.d[l][f];
-            img[Y.dinv[l] + f] = T.dinv[l][f];
+        for (int f = blockIdx.x * B + threadIdx.x; f < LV_CELL * n; f += stride) {
+            const int i = f / LV_CELL, k = f - i * LV_CELL;
+            img[Y.k[l] + f] = k < 8 ? T.c[l][(size_t)k * n + i] : k == 8 ? T.d[l][i] : k == 9 ? T.dinv[l][i] : 0.0f;
         }
-        for (int f = blockIdx.x * B + threadIdx.x; f < 8 * n; f += stride) img[Y.c[l] + f] = T.c[l][f];
     }
     const int nd = T.Kx[T.last] * T.Ky[T.last];
-    for (int f = blockIdx.x * B + threadIdx.x; f < nd * nd; f += stride) img[Y.inv + f] = inv[f];
+    for (int f = blockIdx.x * B + threadIdx.x; f < ((nd * nd + 3) & ~3); f += stride)
+        img[Y.inv + f] = f < nd * nd ? inv[f] : 0.0f;
 }
 
 // ---- power iteration for the scale of the learned fine smoother ----------------------------------
@@ -1625,6 +1770,8 @@ hipError_t lv_amg_init(lv_amg *G)
     AMG_CHECK(hipMalloc(&G->tail_img, sizeof(float) * TAIL_LDS));
     AMG_CHECK(hipMalloc(&G->pw, sizeof(double) * (2 * LV_NBMAX + 2)));
     AMG_CHECK(hipMalloc(&G->prog, sizeof(int) * LV_AMG_MAXPROG));
+    AMG_CHECK(hipMalloc(&G->desc, sizeof(G->hdesc)));
+    static_assert(sizeof(G->hdesc) == sizeof(int) * (LV_AMG_MAXLEV + 1) * LV_DESC, "a descriptor per level");
     AMG_CHECK(hipMalloc(&G->pflag, 2 * sizeof(int)));
     return hipSuccess;
 }
@@ -1632,7 +1779,7 @@ hipError_t lv_amg_init(lv_amg *G)
 void lv_amg_free(lv_amg *G)
 {
     void *ptrs[] = {G->agg, G->cnt, G->start, G->cursor, G->list, G->scan_tmp, G->t0, G->z0, G->dense_inv, G->tail_img, G->tail_mat, G->ext_mat,
-                    G->pw, G->pv, G->pu, G->prog, G->iperm, G->aggp, G->pdeg, G->poff, G->pev32, G->pev16,
+                    G->pw, G->pv, G->pu, G->prog, G->desc, G->iperm, G->aggp, G->pdeg, G->poff, G->pev32, G->pev16,
                     G->pdiag32, G->pdinv32, G->pmval, G->pmdg, G->pflag, G->bfirst, G->ooff, G->oev32};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -1760,16 +1907,16 @@ static int tail_program(int first, int last, bool W, int *prog)
     return np;
 }
 
-// the levels ltail..nlev of the single-workgroup kernel
+// the levels lk..nlev of the single-workgroup kernel
 static tail_levels tail_levels_of(const lv_amg *G)
 {
     tail_levels T;
     memset(&T, 0, sizeof(T));
-    T.first = G->ltail;
+    T.first = G->lk;
     T.last = G->nlev;
     T.xper = G->xper;
     T.yper = G->yper;
-    for (int l = G->ltail; l <= G->nlev; l++) {
+    for (int l = G->lk; l <= G->nlev; l++) {
         const lv_amg_level &L = G->lev[l];
         T.Kx[l] = L.Kx;
         T.Ky[l] = L.Ky;
@@ -1785,9 +1932,7 @@ static tail_levels tail_levels_of(const lv_amg *G)
     return T;
 }
 
-// their LDS layout: the constant arrays first (diagonals, couplings, dense inverse), then the work
-// vectors; about 14 floats per cell of the levels above the dense one, whose total stays below
-// twice TAIL_MAX
+// their LDS layout
 static tail_layout tail_layout_of(const lv_amg *G)
 {
     tail_layout Y;
@@ -1795,34 +1940,46 @@ static tail_layout tail_layout_of(const lv_amg *G)
     int off = 0;
     auto put = [&off](int count) {
         const int o = off;
-        off += count;
+        off += (count + 3) & ~3;
         return o;
     };
-    for (int l = G->ltail; l < G->nlev; l++) {
-        const int nl = G->lev[l].n;
-        Y.d[l] = put(nl);
-        Y.dinv[l] = put(nl);
-        Y.c[l] = put(8 * nl);
-    }
+    for (int l = G->lk; l < G->nlev; l++) Y.k[l] = put(LV_CELL * G->lev[l].n);
     Y.inv = put(G->lev[G->nlev].n * G->lev[G->nlev].n);
     Y.coef = off;
-    for (int l = G->ltail; l <= G->nlev; l++) {
-        const int nl = G->lev[l].n;
-        if (l < G->nlev) {
-            Y.z[l] = put(nl);
-            Y.acc[l] = put(nl);
-        }
-        Y.r[l] = put(nl);
-        Y.t[l] = put(nl);
+    for (int l = G->lk; l <= G->nlev; l++) {
+        const lv_amg_level &L = G->lev[l];
+        const int halo = (L.Kx + 2) * (L.Ky + 2);
+        Y.r[l] = put(L.n);
+        Y.t[l] = put(halo);
+        if (l < G->nlev) Y.z[l] = put(halo);
+        if (l < G->nlev && G->wcycle) Y.acc[l] = put(L.n);
     }
     Y.total = off;
     return Y;
 }
 
-// the tail runs in LDS when its levels fit (the usual case), else in global memory
-static bool tail_fits_lds(const lv_amg *G, const tail_layout &Y)
+// the levels' descriptors for the LDS kernel
+static void tail_descriptors(const lv_amg *G, const tail_layout &Y, int *D)
 {
-    return Y.total <= TAIL_LDS && G->nprog <= LV_AMG_MAXPROG;
+    auto bits = [](float f) {
+        int i;
+        memcpy(&i, &f, sizeof(i));
+        return i;
+    };
+    memset(D, 0, sizeof(int) * (LV_AMG_MAXLEV + 1) * LV_DESC);
+    for (int l = G->lk; l <= G->nlev; l++) {
+        const lv_amg_level &L = G->lev[l];
+        const int v[10] = {L.Kx,    L.Ky,   L.n,    bits(L.alpha), bits(1.0f / (float)L.Ky), Y.k[l], Y.r[l],
+                           Y.z[l], Y.t[l], Y.acc[l]};
+        memcpy(D + l * LV_DESC, v, sizeof(v));
+    }
+}
+
+static tail_lds_args tail_args_of(const lv_amg *G)
+{
+    const lv_amg_level &L = G->lev[G->lk];
+    return tail_lds_args{G->desc,  G->prog, G->nprog, G->tail_img, G->tail_coef, G->tail_total, G->lk, G->nlev,
+                         L.n, G->xper, G->yper, G->tail_inv, L.r, L.dinv, L.t};
 }
 
 hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, const lv_pressure_system &A, int n,
@@ -1874,13 +2031,22 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
         G->lev[k].alpha = (k < G->nlev && G->lev[k + 1].n > TAIL_MAX) ? ALPHA_COARSE : 1.0f;
     int lt = G->nlev;
     while (lt > 1 && G->lev[lt - 1].n <= TAIL_MAX) lt--;
-    G->ltail = lt;
     G->wcycle = A.singular ? 1 : 0;
-    G->nprog = tail_program(lt, G->nlev, G->wcycle != 0, G->hprog);
-    // a singular system's tail as a matrix (k_tail_lds<true>), and the level above it when it is small
+    // the first level of the single-workgroup kernel: a singular system W-visits the levels of at most TAIL_MAX
+    // cells, a nonsingular one may start a level earlier
+    G->lk = lt;
+    if (!G->wcycle)
+        while (G->lk > 1 && G->lev[G->lk - 1].n <= LDS_MAX) G->lk--;
+    const int lk = G->lk;
+    G->nprog = tail_program(lk, G->nlev, G->wcycle != 0, G->hprog);
     const tail_layout Y = tail_layout_of(G);
-    const bool fits = tail_fits_lds(G, Y), mat = fits && G->wcycle;
-    G->lmat = mat && lt > 1 && G->lev[lt - 1].n <= MAT_MAX ? lt - 1 : lt;
+    G->lds_ok = Y.total <= TAIL_LDS && G->nprog <= LV_AMG_MAXPROG ? 1 : 0;  // else its arrays stay in global memory
+    G->tail_coef = Y.coef;
+    G->tail_inv = Y.inv;
+    G->tail_total = Y.total;
+    // a singular system's tail as a matrix (k_tail_lds<true>), and the level above it when it is small
+    const bool mat = G->lds_ok && G->wcycle;
+    G->lmat = mat && lk > 1 && G->lev[lk - 1].n <= MAT_MAX ? lk - 1 : lk;
     G->mat_ld = mat ? (G->lev[G->lmat].n + 3) & ~3 : 0;
     // pairs of levels above the tail that run as one kernel each way, from the tail upwards (the
     // smallest levels gain most): level l at least PAIR_MIN_K wide, a multiple of 4 on a periodic axis
@@ -1896,20 +2062,23 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
     const lv_amg_level &D = G->lev[l];
     hipLaunchKernelGGL(k_dense_inverse, dim3(1), dim3(DTB), 0, s, D.Kx, D.Ky, G->xper, G->yper, (const float *)D.d,
                        (const float *)D.c, A.singular, G->dense_inv);
-    const tail_levels T = tail_levels_of(G);
-    if (fits)
-        hipLaunchKernelGGL(k_tail_pack, dim3(64), dim3(B), 0, s, T, Y, (const float *)G->dense_inv, G->tail_img);
+    if (G->lds_ok) {
+        hipLaunchKernelGGL(k_tail_pack, dim3(64), dim3(B), 0, s, tail_levels_of(G), Y, (const float *)G->dense_inv,
+                           G->tail_img);
+        tail_descriptors(G, Y, G->hdesc);
+        AMG_CHECK(hipMemcpyAsync(G->desc, G->hdesc, sizeof(G->hdesc), hipMemcpyHostToDevice, s));
+    }
     if (mat) {
-        const int nt = G->lev[lt].n, ldt = (nt + 3) & ~3;
+        const int nt = G->lev[lk].n, ldt = (nt + 3) & ~3;
         AMG_CHECK(grow(&G->tail_mat, &G->cap_tail_mat, (size_t)nt * ldt));
-        hipLaunchKernelGGL(k_tail_lds<true>, dim3(nt), dim3(TB), 0, s, T, Y, (const int *)G->prog, G->nprog,
-                           (const float *)G->tail_img, (const lv_cg_scalars *)nullptr, G->tail_mat, ldt);
+        hipLaunchKernelGGL(k_tail_lds<true>, dim3(nt), dim3(TB), 0, s, tail_args_of(G), (const lv_cg_scalars *)nullptr,
+                           G->tail_mat, ldt);
         G->mat = G->tail_mat;
-        if (G->lmat < lt) {
+        if (G->lmat < lk) {
             const lv_amg_level &L = G->lev[G->lmat];
             AMG_CHECK(grow(&G->ext_mat, &G->cap_ext_mat, (size_t)L.n * G->mat_ld));
             hipLaunchKernelGGL(k_mat_extend, dim3(L.n), dim3(B), 0, s,
-                               st_level{L.Kx, L.Ky, G->xper, G->yper, L.d, L.c, L.dinv, L.alpha}, G->lev[lt].Ky, nt,
+                               st_level{L.Kx, L.Ky, G->xper, G->yper, L.d, L.c, L.dinv, L.alpha}, G->lev[lk].Ky, nt,
                                (const float *)G->tail_mat, ldt, G->ext_mat, G->mat_ld);
             G->mat = G->ext_mat;
         }
@@ -1997,6 +2166,8 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
 {
     const int n = G->n0;
     const lv_amg_level &L1 = G->lev[1];
+    const bool pairs = !G->level_kernels;
+    const int lt = G->lmat;  // the levels below it have kernels of their own
     bool z1_given = false;  // the fused down pass stored level 1's pre-smoothed z
     // level 0, down: z0 (in G->z0) and its residual t (in G->t0), restricted to level 1
     if (G->fine_learned) {
@@ -2006,7 +2177,7 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
                            (const float *)G->t0, L1.r, S);
     } else if (!list && G->nbfuse > 0) {
         // level 1 above the tail: its pre-smoothed z stored here, gathered by its down pass
-        z1_given = G->lmat > 1;
+        z1_given = lt > 1;
         float *z1 = z1_given ? L1.z : nullptr;
         const int *done = S ? &S->done : G->bfirst + 2 * (G->nbfuse + 1);
         if (z0_ready && G->z0_in)
@@ -2024,8 +2195,6 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
     }
     // coarse levels above the tail, down: each level's pre-smoothed z and the next level's
     // right-hand side
-    const int lt = G->lmat;
-    const bool pairs = !G->level_kernels;
     for (int l = 1; l < lt; l++) {
         const lv_amg_level &L = G->lev[l], &C = G->lev[l + 1];
         const st_level sl{L.Kx, L.Ky, G->xper, G->yper, L.d, L.c, L.dinv, L.alpha};
@@ -2048,7 +2217,6 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
     // lt in its t.  Then the coarse levels above it, up: each level's final correction in t; level 1 in the
     // aggregate order with the Jacobi smoother also prolongates into z0.
     const lv_amg_level &LT = G->lev[lt];
-    const tail_layout Y = tail_layout_of(G);
     const bool prolong_in_up = (lt > 1 || G->mat_ld) && !G->fine_learned && list == nullptr;
     if (G->mat_ld) {
         const bool pr = lt == 1 && prolong_in_up;
@@ -2057,9 +2225,8 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
         hipLaunchKernelGGL(kern, dim3((LT.n + B / 64 - 1) / (B / 64)), dim3(B), 0, s, LT.n, G->mat_ld,
                            (const float *)G->mat, (const float *)LT.r, LT.t, S,
                            pr ? (const int *)G->start : (const int *)nullptr, G->fine_alpha, G->z0);
-    } else if (tail_fits_lds(G, Y))
-        hipLaunchKernelGGL(k_tail_lds<false>, dim3(1), dim3(TB), 0, s, tail_levels_of(G), Y, (const int *)G->prog,
-                           G->nprog, (const float *)G->tail_img, S, (float *)nullptr, 0);
+    } else if (G->lds_ok)
+        hipLaunchKernelGGL(k_tail_lds<false>, dim3(1), dim3(TB), 0, s, tail_args_of(G), S, (float *)nullptr, 0);
     else
         hipLaunchKernelGGL(k_tail, dim3(1), dim3(TB), 0, s, tail_levels_of(G), (const int *)G->prog, G->nprog,
                            (const float *)G->dense_inv, S);

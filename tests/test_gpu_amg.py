@@ -425,3 +425,17 @@ def test_matrix_of_the_coarse_levels_matches_oracle(lv, oracle, gpu, kind, K):
     zr = _hier(kind, x, dr, d, rp, cols, coef, fine_bf16=False).apply(r)
     z = solver.apply_preconditioner(r, "amg")
     assert np.linalg.norm(z - zr) <= 1e-4 * np.linalg.norm(zr), (np.linalg.norm(z - zr) / np.linalg.norm(zr))
+
+
+@pytest.mark.parametrize("kind,K", [("periodic", 14), ("periodic", 66), ("periodic", 131), ("walls", 71),
+                                    ("xperiodic", 134), ("tall", 46)])
+def test_single_workgroup_levels_match_oracle(lv, oracle, gpu, kind, K):
+    """the V-visit of the small levels in one workgroup, in LDS with a halo: only the dense level (14), level 1
+    in it (66: 33 x 33 cells, odd and periodic; 46), odd levels that pair a last cell with none on periodic
+    axes (131: 65, 33, 17, 9, 5), walls, and one periodic axis"""
+    _flush("single workgroup levels %s %d" % (kind, K))
+    grid, op, solver, x, dr, d, rp, cols, coef = _system(lv, oracle, kind, K, "tg", 8e-3 * 64 / K)
+    r = np.random.default_rng(14).standard_normal(grid.n)
+    z = solver.apply_preconditioner(r, "amg")
+    zr = _hier(kind, x, dr, d, rp, cols, coef).apply(r)
+    assert np.linalg.norm(z - zr) <= 1e-4 * np.linalg.norm(zr), (np.linalg.norm(z - zr) / np.linalg.norm(zr))
