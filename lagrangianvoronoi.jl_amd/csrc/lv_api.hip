@@ -46,7 +46,6 @@ struct lv_ctx {
     int64_t max_items = 0;
     int nitems = 0;
     void *cl_temp = nullptr;
-    int *d_nitems = nullptr;
     // magic path prefix
     int *path_i = nullptr;
     double *path_rr = nullptr;
@@ -60,7 +59,8 @@ struct lv_ctx {
     bool rg_alloc = false;
     int *deg = nullptr;
     void *scan_temp = nullptr;
-    int *d_flags = nullptr;   // [0] error word, [1] nonsingular flag, [2] a column offset wider than 16 bits
+    int *d_flags = nullptr;   // [0] error word, [1] nonsingular flag, [2] a column offset wider than 16 bits,
+                              // [3] items of the cell list
     lv_timer *timers[LV_NKTIMERS] = {nullptr, nullptr, nullptr, nullptr};
     // Picard extrapolation: orthonormal A-images q_k of past Picard corrections and their
     // preimages z_k (A z_k = q_k), the last two Picard iterates and their A-images
@@ -378,8 +378,7 @@ int lv_create(const lv_grid_desc *d, lv_ctx **out)
     ALLOC(ctx->el, LV_MAXE * cap);
     ALLOC(ctx->clip_retry, cap + 1);
     ALLOC(ctx->cell_start, ncells + 1);
-    ALLOC(ctx->d_nitems, 1);
-    ALLOC(ctx->d_flags, 3);
+    ALLOC(ctx->d_flags, 4);
     ALLOC(ctx->path_i, 2 * (size_t)std::max(1, g.npath));
     ALLOC(ctx->path_rr, (size_t)std::max(1, g.npath));
     // pressure system and solver work
@@ -426,7 +425,7 @@ int lv_create(const lv_grid_desc *d, lv_ctx **out)
         if (e == hipSuccess)
             e = hipMemcpy(ctx->path_rr, ctx->h_path_rr.data(), sizeof(double) * g.npath, hipMemcpyHostToDevice);
     }
-    if (e == hipSuccess) e = hipMemset(ctx->d_flags, 0, 3 * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(ctx->d_flags, 0, 4 * sizeof(int));
     if (e == hipSuccess) {
         e = lv_spai_init(&ctx->spai);
         ctx->spai_ok = (e == hipSuccess);
@@ -457,7 +456,7 @@ int lv_destroy(lv_ctx *ctx)
                     ctx->F.mass, ctx->F.energy, ctx->F.quality, ctx->F.mu, ctx->F.D, ctx->F.area, ctx->F.cent,
                     ctx->F.phase, ctx->ne, ctx->ev, ctx->el, ctx->clip_retry, ctx->cell_start, ctx->cell_labels,
                     ctx->cell_x,
-                    ctx->cl_temp, ctx->d_nitems, ctx->d_flags, ctx->path_i, ctx->path_rr, ctx->A.row_ptr,
+                    ctx->cl_temp, ctx->d_flags, ctx->path_i, ctx->path_rr, ctx->A.row_ptr,
                     ctx->A.cols, ctx->A.val64, ctx->A.val32, ctx->A.diag64, ctx->A.dinv64, ctx->A.diag32,
                     ctx->A.dinv32, ctx->deg, ctx->A.ecol, ctx->A.ev64, ctx->A.ev32, ctx->A.ocol, ctx->A.oev64,
                     ctx->A.oev32, ctx->A.deg8, ctx->A.ecol16, ctx->A.ocol16, ctx->b, ctx->P0, ctx->GP, ctx->W.r, ctx->W.z, ctx->W.p,
@@ -613,68 +612,74 @@ int lv_field_device_ptr(lv_ctx *ctx, int32_t field, void **dptr)
 
 // ---- remesh ----------------------------------------------------------------------------------------
 
+}  // extern "C"
+
+namespace {
+
+// room for `want` items in the cell list (whatever the lists held is dropped)
+int grow_cell_list(lv_ctx *ctx, int64_t want)
+{
+    const int64_t ncells = (int64_t)ctx->g.n1 * ctx->g.n2;
+    dfree(ctx->cell_labels);
+    dfree(ctx->cell_x);
+    dfree(ctx->cl_temp);
+    ctx->cell_labels = nullptr;
+    ctx->cell_x = nullptr;
+    ctx->cl_temp = nullptr;
+    ctx->max_items = 0;
+    LV_HIP_CHECK(dalloc(&ctx->cell_labels, want));
+    LV_HIP_CHECK(dalloc(&ctx->cell_x, 2 * want));
+    LV_HIP_CHECK(hipMalloc(&ctx->cl_temp, lv_celllist_temp_bytes(want, ncells)));
+    LV_HIP_CHECK(lv_celllist_temp_init(ctx->cl_temp, ncells, ctx->s));
+    ctx->max_items = want;
+    return LV_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int lv_remesh(lv_ctx *ctx)
 {
     int rc = check_ctx(ctx, false);
     if (rc) return rc;
     const int n = ctx->n;
-    const int64_t ncells = (int64_t)ctx->g.n1 * ctx->g.n2;
     if (ctx->max_items == 0) {
         int64_t want = (int64_t)n + n / 4 + 4096;
         if (!ctx->g.xperiodic && !ctx->g.yperiodic) want = n + 1;
-        want = std::min<int64_t>(want, 9LL * n);
-        ctx->max_items = want;
-        LV_HIP_CHECK(dalloc(&ctx->cell_labels, want));
-        LV_HIP_CHECK(dalloc(&ctx->cell_x, 2 * want));
-        LV_HIP_CHECK(hipMalloc(&ctx->cl_temp, lv_celllist_temp_bytes(std::max<int64_t>(want, n + 1), ncells)));
+        rc = grow_cell_list(ctx, std::min<int64_t>(want, 9LL * n));
+        if (rc) return rc;
     }
-    rc = clear_flags(ctx);
-    if (rc) return rc;
-    lv_timer *tc = timer_if_on(ctx, 3);
-    if (tc && tc->used == LV_TPOOL) lv_timer_flush(tc);
+    lv_timer *tc = timer_if_on(ctx, 3), *tk = timer_if_on(ctx, 2);
+    int flags[4];
     for (int attempt = 0; attempt < 2; attempt++) {
-        hipError_t e = lv_build_cell_list(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
-                                          ctx->max_items, ctx->d_nitems, ctx->cl_temp, ctx->s,
-                                          tc ? tc->ev[2 * tc->used] : nullptr, tc ? tc->ev[2 * tc->used + 1] : nullptr,
-                                          tc != nullptr, &ctx->nitems);
-        if (e == hipErrorInvalidValue && attempt == 0) {
-            // more periodic images than buffered: grow to the count the scan produced and rebuild
-            int m = 0;
-            LV_HIP_CHECK(hipMemcpy(&m, ctx->d_nitems, sizeof(int), hipMemcpyDeviceToHost));
-            if (m <= 0) return lv_fail(ctx, LV_E_INVALID, "cell list: no items");
-            dfree(ctx->cell_labels);
-            dfree(ctx->cell_x);
-            dfree(ctx->cl_temp);
-            ctx->cell_labels = nullptr;
-            ctx->cell_x = nullptr;
-            ctx->cl_temp = nullptr;
-            int64_t want = (int64_t)m + m / 8 + 4096;
-            ctx->max_items = want;
-            LV_HIP_CHECK(dalloc(&ctx->cell_labels, want));
-            LV_HIP_CHECK(dalloc(&ctx->cell_x, 2 * want));
-            LV_HIP_CHECK(hipMalloc(&ctx->cl_temp, lv_celllist_temp_bytes(std::max<int64_t>(want, n + 1), ncells)));
-            continue;
-        }
-        LV_HIP_CHECK(e);
+        rc = clear_flags(ctx);
+        if (rc) return rc;
+        if (tc && tc->used == LV_TPOOL) lv_timer_flush(tc);
+        LV_HIP_CHECK(lv_build_cell_list(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
+                                        ctx->max_items, ctx->d_flags + 3, ctx->cl_temp, ctx->s,
+                                        tc ? tc->ev[2 * tc->used] : nullptr, tc ? tc->ev[2 * tc->used + 1] : nullptr,
+                                        tc != nullptr));
         if (tc) tc->used++;
-        break;
+        if (tk) lv_timer_begin(tk, ctx->s);
+        LV_HIP_CHECK(lv_launch_clip(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x, ctx->path_i,
+                                    ctx->path_rr, ctx->ne, ctx->ev, ctx->el, n, ctx->F.area, ctx->F.cent, ctx->d_flags,
+                                    ctx->clip_retry, ctx->s, (int)ctx->max_items));
+        if (tk) lv_timer_end(tk, ctx->s);
+        ctx->mesh_valid = false;
+        ctx->A.valid = 0;
+        LV_HIP_CHECK(hipMemcpyAsync(flags, ctx->d_flags, 4 * sizeof(int), hipMemcpyDeviceToHost, ctx->s));
+        LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+        ctx->nitems = flags[3];
+        if (ctx->nitems <= ctx->max_items) break;
+        // more periodic images than buffered: the mesh is of a list cut off; room for the count, and again
+        rc = grow_cell_list(ctx, (int64_t)ctx->nitems + ctx->nitems / 8 + 4096);
+        if (rc) return rc;
     }
-    lv_timer *tk = timer_if_on(ctx, 2);
-    if (tk) lv_timer_begin(tk, ctx->s);
-    LV_HIP_CHECK(lv_launch_clip(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x, ctx->path_i,
-                                ctx->path_rr, ctx->ne, ctx->ev, ctx->el, n, ctx->F.area, ctx->F.cent, ctx->d_flags,
-                                ctx->clip_retry, ctx->s, (int)ctx->max_items));
-    if (tk) lv_timer_end(tk, ctx->s);
-    int flags[2];
-    rc = read_flags(ctx, flags);
-    if (rc) return rc;
     if (tk) lv_timer_flush(tk);
     if (tc) lv_timer_flush(tc);
-    ctx->A.valid = 0;
-    if (flags[0] != 0) {
-        ctx->mesh_valid = false;
-        return lv_fail(ctx, flags[0], error_text(flags[0]));
-    }
+    if (n > 0 && ctx->nitems <= 0) return lv_fail(ctx, LV_E_INVALID, "cell list: no items");
+    if (flags[0] != 0) return lv_fail(ctx, flags[0], error_text(flags[0]));
     ctx->mesh_valid = true;
     return LV_OK;
 }
@@ -1934,7 +1939,7 @@ int lv_timing_read(lv_ctx *ctx, int32_t kernel_id, double *total_ms, int64_t *la
         if (kernel_id == 0) b = ctx->spmv32_agg ? 1.0 * n + 4.0 * n * 6 + 6.0 * nnz : 4.0 * n + 4.0 * n * 6 + 8.0 * nnz;
         else if (kernel_id == 1) b = 4.0 * n + 8.0 * n * 6 + 12.0 * nnz;
         else if (kernel_id == 2) b = 16.0 * n + 20.0 * m + 4.0 * (nc + 1) + 4.0 * n + 36.0 * 6.0 * n + 24.0 * n;
-        else if (kernel_id == 3) b = 3.0 * (8.0 + 8.0 + 4.0) * m;              // 3 radix passes over (key, label)
+        else if (kernel_id == 3) b = 16.0 * n + 20.0 * m + 4.0 * (nc + 1);  // positions in; labels, their positions and offsets out
         *bytes_per_launch = b;
     }
     return LV_OK;

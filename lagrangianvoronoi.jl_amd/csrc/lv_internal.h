@@ -129,6 +129,28 @@ __device__ __forceinline__ double lv_wave_sum(double v)
     return v;
 }
 
+// ctr[key] += SIGN (1 or -1) for every active lane, by runs: consecutive active lanes with equal keys
+// form a run, whose first lane adds the run's length in one atomic.  Each lane gets a slot of its own
+// among the key's: counting up, the slots from the old value on; counting down, those from the new
+// value on.  Every lane of the wavefront calls it.
+template <int SIGN>
+__device__ __forceinline__ int lv_run_atomic_add(int *ctr, int key, bool active)
+{
+    const int lane = threadIdx.x & 63;
+    const int prev = __shfl_up(key, 1);
+    const unsigned long long am = __ballot(active);
+    const bool pact = lane > 0 && ((am >> (lane - 1)) & 1ull);
+    const bool head = active && (!pact || prev != key);
+    const unsigned long long heads = __ballot(head);
+    const unsigned long long upto = (2ull << lane) - 1ull;  // lanes 0..lane (every lane at lane 63)
+    const int h = active ? 63 - __clzll((long long)(heads & upto)) : lane;
+    const unsigned long long above = (heads | ~am) & ~upto;  // the run ends at the next one or at a gap
+    const int runlen = (above ? __ffsll((long long)above) - 1 : 64) - lane;
+    int old = 0;
+    if (head) old = atomicAdd(&ctr[key], SIGN * runlen) - (SIGN < 0 ? runlen : 0);
+    return __shfl(old, h) + (lane - h);
+}
+
 template <int BLOCK>
 __device__ __forceinline__ double lv_block_sum(double v, double *smem)
 {
@@ -155,13 +177,15 @@ int lv_fail(lv_ctx *ctx, int code, const char *msg);
 
 // lv_scan.hip
 size_t lv_scan_temp_bytes(int64_t n);
-hipError_t lv_exclusive_scan_i32(const int *in, int *out, int64_t n, int *d_total, void *temp, hipStream_t s);
+hipError_t lv_exclusive_scan_i32(const int *in, int *out, int64_t n, int *d_total, void *temp, hipStream_t s,
+                                 int cap = 0x7fffffff);
 
 // lv_celllist.hip
 size_t lv_celllist_temp_bytes(int64_t max_items, int64_t ncells);
 hipError_t lv_build_cell_list(const lv_grid_params &g, int n, const double *x, int *cell_start, int *cell_labels,
                               double *cell_x, int64_t max_items, int *d_nitems, void *temp, hipStream_t s,
-                              hipEvent_t ev0, hipEvent_t ev1, bool timed, int *h_nitems = nullptr);
+                              hipEvent_t ev0, hipEvent_t ev1, bool timed);
+hipError_t lv_celllist_temp_init(void *temp, int64_t ncells, hipStream_t s);
 
 // lv_clip.hip.  retry: n + 1 ints of work space (the seeds whose polygon needs the full capacity).
 hipError_t lv_launch_clip(const lv_grid_params &g, int n, const double *x, const int *cell_start,
