@@ -628,7 +628,7 @@ int grow_cell_list(lv_ctx *ctx, int64_t want)
     ctx->cl_temp = nullptr;
     ctx->max_items = 0;
     LV_HIP_CHECK(dalloc(&ctx->cell_labels, want));
-    LV_HIP_CHECK(dalloc(&ctx->cell_x, 2 * want));
+    LV_HIP_CHECK(dalloc(&ctx->cell_x, 2 * want + 1));
     LV_HIP_CHECK(hipMalloc(&ctx->cl_temp, lv_celllist_temp_bytes(want, ncells)));
     LV_HIP_CHECK(lv_celllist_temp_init(ctx->cl_temp, ncells, ctx->s));
     ctx->max_items = want;

@@ -352,34 +352,61 @@ struct lds_poly {
     int lab[CAP_SMALL][CB];
 };
 
-__device__ __forceinline__ double influence_rr(const lds_poly &P, int t, int len, double x1, double x2)
+// the slots in registers, read again whenever a cut changed them
+struct reg_poly {
+    double v1x[CAP_SMALL], v1y[CAP_SMALL], v2x[CAP_SMALL], v2y[CAP_SMALL];
+};
+
+__device__ __forceinline__ double load_slots(reg_poly &R, const lds_poly &P, int t, int len, double x1, double x2)
 {
-    double rr = 0.0;
-    for (int k = 0; k < len; k++) {
-        double a = P.v1x[k][t] - x1, b = P.v1y[k][t] - x2;
-        double r = 4.0 * (a * a + b * b);
-        if (r > rr) rr = r;
+    double rr = 0.0;  // influence_rr
+#pragma unroll
+    for (int k = 0; k < CAP_SMALL; k++) {
+        R.v1x[k] = P.v1x[k][t];
+        R.v1y[k] = P.v1y[k][t];
+        R.v2x[k] = P.v2x[k][t];
+        R.v2y[k] = P.v2y[k][t];
+        const double a = R.v1x[k] - x1, b = R.v1y[k] - x2;
+        const double r = 4.0 * (a * a + b * b);
+        if (k < len && r > rr) rr = r;
     }
     return rr;
 }
 
-// voronoicut!(p, y, label): 1 if an edge was added, 0 if not, -1 on overflow
-__device__ __forceinline__ int cut(lds_poly &P, int t, int &len, double x1, double x2, double y1, double y2,
-                                   int label)
+// voronoicut!(p, y, label): 1 if an edge was added, 0 if not, -1 on overflow.  First the ends of all edges
+// against the bisector, from registers and side by side.  Then only the edges that it crosses or removes
+// are taken up, in the order and with the moves of a walk over the slots (a removed edge's slot takes the
+// last edge, which is looked at there).  Bound by instruction issue: some lane of a wavefront cuts at nearly
+// every candidate, so a pre-test of the corners alone costs more than it spares (1.86 ms against 1.76 at
+// 4,194,304 seeds of 0.1 dr of jitter), and lanes that each run ahead to their next cut take 3.4 to 5.6:
+// they no longer go through the path together.  A walk over the slots from LDS, edge by edge, took 2.35.
+__device__ __forceinline__ int cut(lds_poly &P, const reg_poly &R, int t, int &len, double x1, double x2, double y1,
+                                   double y2, int label, bool &changed)
 {
     const double d1 = y1 - x1, d2 = y2 - x2;
     const double m1 = 0.5 * (y1 + x1), m2 = 0.5 * (y2 + x2);
     const double c = d1 * m1 + d2 * m2;
+    unsigned cross = 0, rem = 0;
+#pragma unroll
+    for (int k = 0; k < CAP_SMALL; k++) {
+        const double f1 = (d1 * R.v1x[k] + d2 * R.v1y[k]) - c;
+        const double f2 = (d1 * R.v2x[k] + d2 * R.v2y[k]) - c;
+        const bool p1 = f1 > SIGNUM_EPS, p2 = f2 > SIGNUM_EPS;
+        if (p1 != p2) cross |= 1u << k;
+        if ((p1 || p2) && !(f1 < -SIGNUM_EPS) && !(f2 < -SIGNUM_EPS)) rem |= 1u << k;
+    }
+    unsigned act = (cross | rem) & ((1u << len) - 1u);
+    changed = act != 0;
+    if (!changed) return 0;
     const double qnan = __builtin_nan("");
     double X1 = qnan, X2 = qnan, Y1 = qnan, Y2 = qnan;
-    int i = 0;
-    while (i < len) {
-        const double e1x = P.v1x[i][t], e1y = P.v1y[i][t], e2x = P.v2x[i][t], e2y = P.v2y[i][t];
-        const double f1 = (d1 * e1x + d2 * e1y) - c;
-        const double f2 = (d1 * e2x + d2 * e2y) - c;
-        const int s1 = signum(f1), s2 = signum(f2);
-        const int s12 = s1 + s2;
-        if ((0 <= s12 && s12 <= 1) && ((s1 | s2) != 0)) {
+    do {
+        const int i = __ffs((int)act) - 1;
+        if ((cross >> i) & 1u) {
+            const double e1x = P.v1x[i][t], e1y = P.v1y[i][t], e2x = P.v2x[i][t], e2y = P.v2y[i][t];
+            const double f1 = (d1 * e1x + d2 * e1y) - c;
+            const double f2 = (d1 * e2x + d2 * e2y) - c;
+            const int s1 = signum(f1), s2 = signum(f2);
             Y1 = X1;
             Y2 = X2;
             const double tt = 1.0 / (f1 - f2);
@@ -390,8 +417,8 @@ __device__ __forceinline__ int cut(lds_poly &P, int t, int &len, double x1, doub
             if (s1 == 1) { P.v1x[i][t] = X1; P.v1y[i][t] = X2; }
             else { P.v2x[i][t] = X1; P.v2y[i][t] = X2; }
         }
-        if (1 <= s12) {
-            const int last = len - 1;
+        if ((rem >> i) & 1u) {
+            const int last = --len;
             if (last > i) {
                 P.v1x[i][t] = P.v1x[last][t];
                 P.v1y[i][t] = P.v1y[last][t];
@@ -399,11 +426,13 @@ __device__ __forceinline__ int cut(lds_poly &P, int t, int &len, double x1, doub
                 P.v2y[i][t] = P.v2y[last][t];
                 P.lab[i][t] = P.lab[last][t];
             }
-            len--;
+            cross = (cross & ~(1u << i)) | (((cross >> last) & 1u) << i);
+            rem = (rem & ~(1u << i)) | (((rem >> last) & 1u) << i);
+            act = (cross | rem) & ((1u << len) - 1u) & (~0u << i);
         } else {
-            i++;
+            act &= act - 1u;
         }
-    }
+    } while (act != 0);
     if (!(isnan(Y1) && isnan(Y2)) && (X1 != Y1 || X2 != Y2)) {
         if (len >= CAP_SMALL) return -1;
         const double cr = (Y1 - X1) * (x2 - X2) - (Y2 - X2) * (x1 - X1);  // cross2(Y - X, x - X)
@@ -429,6 +458,19 @@ __device__ __forceinline__ void swap_slots(lds_poly &P, int t, int a, int b)
     int tl = P.lab[a][t]; P.lab[a][t] = P.lab[b][t]; P.lab[b][t] = tl;
 }
 
+// the candidates of the walk's node k (none, and a valid index, beyond the grid and the path's end)
+__device__ __forceinline__ void path_node(const lv_grid_params &g, const int *__restrict__ path_i, int k, int k1,
+                                          int k2, const int *__restrict__ cell_start, int &s0, int &s1)
+{
+    s0 = s1 = 0;
+    if (k >= g.npath) return;
+    const int c1 = k1 + path_i[2 * k], c2 = k2 + path_i[2 * k + 1];
+    if (c1 < 1 || c1 > g.n1 || c2 < 1 || c2 > g.n2) return;
+    const int c = (c1 - 1) + (c2 - 1) * g.n1;
+    s0 = cell_start[c];
+    s1 = cell_start[c + 1];
+}
+
 // one seed's polygon, clipped in P's LDS slots; false when it outgrew them
 __device__ bool clip_seed(const lv_grid_params &g, int n, int i, const double *__restrict__ x,
                           const int *__restrict__ cell_start, const int *__restrict__ cell_labels,
@@ -449,35 +491,51 @@ __device__ bool clip_seed(const lv_grid_params &g, int n, int i, const double *_
         P.v1x[3][t] = Cx; P.v1y[3][t] = Cy; P.v2x[3][t] = Bx; P.v2y[3][t] = By; P.lab[3][t] = -2;
     }
     int len = 4;
-    double prr = influence_rr(P, t, len, x1, x2);
+    reg_poly R;
+    double prr = load_slots(R, P, t, len, x1, x2);
     int k1, k2;
     lv_findkey(g, x1, x2, k1, k2);
     int status = LV_OK;
+    // node k's candidates: cell_start two nodes ahead of their use, a position one candidate ahead (the
+    // first of the next node; a position beyond the items, at most one, is in cell_x's room)
+    int s0, s1, n0, n1, f0, f1;
+    path_node(g, path_i, 0, k1, k2, cell_start, s0, s1);
+    path_node(g, path_i, 1, k1, k2, cell_start, n0, n1);
+    double c1 = cell_x[s0], c2 = cell_x[m + s0];
     for (int k = 0;; k++) {
         if (k == g.npath) {
             if (g.has_next && !(g.next_rr > prr)) status = LV_E_MESH_DESTROYED;  // src/voronoigrid.jl:63-65
             break;
         }
-        const double rr = path_rr[k];
-        if (rr > prr) break;
-        const int c1 = k1 + path_i[2 * k], c2 = k2 + path_i[2 * k + 1];
-        if (c1 < 1 || c1 > g.n1 || c2 < 1 || c2 > g.n2) continue;
-        const int c = (c1 - 1) + (c2 - 1) * g.n1;
-        const int s0 = cell_start[c], s1 = cell_start[c + 1];
+        if (path_rr[k] > prr) break;
+        path_node(g, path_i, k + 2, k1, k2, cell_start, f0, f1);
         for (int s = s0; s < s1; s++) {
-            const int j = cell_labels[s];
+            const int sn = s + 1 < s1 ? s + 1 : n0;
+            const double y1c = c1, y2c = c2;
+            c1 = cell_x[sn];
+            c2 = cell_x[m + sn];
             double y1, y2;
-            lv_arrow_target(g, cell_x[s], cell_x[m + s], x1, x2, y1, y2);
+            lv_arrow_target(g, y1c, y2c, x1, x2, y1, y2);
             const double a = x1 - y1, b = x2 - y2;
             if ((x1 == y1 && x2 == y2) || (a * a + b * b > prr)) continue;
-            const int r = cut(P, t, len, x1, x2, y1, y2, j);
+            bool changed;
+            const int r = cut(P, R, t, len, x1, x2, y1, y2, cell_labels[s], changed);
             if (r < 0) {
                 status = LV_E_POLY_OVERFLOW;
                 break;
             }
-            if (r) prr = influence_rr(P, t, len, x1, x2);
+            if (changed) {
+                const double rr = load_slots(R, P, t, len, x1, x2);
+                if (r) prr = rr;
+            }
         }
         if (status != LV_OK) break;
+        if (s0 >= s1) {
+            c1 = cell_x[n0];
+            c2 = cell_x[m + n0];
+        }
+        s0 = n0; s1 = n1;
+        n0 = f0; n1 = f1;
     }
     if (status == LV_E_POLY_OVERFLOW) return false;
     if (status != LV_OK) {
@@ -521,20 +579,57 @@ __device__ bool clip_seed(const lv_grid_params &g, int n, int i, const double *_
     return true;
 }
 
-// The seed block a workgroup clips.  Workgroups are dispatched round-robin over the 8 XCDs, so
-// workgroup b runs on XCD b mod 8; mapping it to block b would give each XCD every 8th block, and on a
-// lattice whose rows span a multiple of 8 blocks that is the same few column strips of the domain in
-// every row.  The clipping work per seed varies across the domain (it depends on where the seeds sit
-// in their cell-list cells), so XCDs with the costly strips ran up to 28% longer while the others
-// idled for the last third of the launch.  Rotating each group of 8 workgroups by a hash of its group
-// index (the top 3 bits of a multiplicative hash, so that no period of the domain lines up with it)
-// gives every XCD an even share of every column; the last, partial group keeps the identity.
-__device__ __forceinline__ int clip_block(int b, int nb)
+constexpr int CHUNK = 4 * CB;
+
+// The seed of this lane.  Some lane of a wavefront cuts at nearly every candidate unless its seeds see
+// alike candidates in alike order, and that depends on where in its cell a seed sits: on a lattice of two
+// seeds to a cell side neighbours take turns.  So the four wavefronts of a chunk of consecutive seeds share
+// them by NB x NB parts of the cell.  Each of the four orders the chunk for itself (only an order: the
+// mesh does not depend on it).  At 4,194,304 seeds 2.03 -> 1.76 ms on a lattice of 0.1 dr of jitter and 3.26 ->
+// 2.98 with 0.45 dr; 4 x 4 parts 1.83 and 3.02.
+template <int NB>
+__device__ __forceinline__ int clip_seed_of(const lv_grid_params &g, int n, int chunk, int part,
+                                            const double *__restrict__ x, unsigned char *ord)
 {
-    const unsigned q = (unsigned)b >> 3;
-    if (8 * ((int)q + 1) > nb) return b;
+    const int t = threadIdx.x;
+    int key[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const int i = chunk * CHUNK + r * CB + t;
+        key[r] = NB * NB;
+        if (i < n) {
+            const double fx = (x[i] - g.origin0) / g.h, fy = (x[n + i] - g.origin1) / g.h;
+            const int bx = (int)(NB * (fx - floor(fx))), by = (int)(NB * (fy - floor(fy)));
+            key[r] = (bx & (NB - 1)) * NB + ((by ^ (bx & 1 ? NB - 1 : 0)) & (NB - 1));
+        }
+    }
+    const unsigned long long lt = (1ull << t) - 1ull;
+    int off = 0;
+    for (int b = 0; b <= NB * NB; b++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const unsigned long long M = __ballot(key[r] == b);
+            if (key[r] == b) ord[off + __popcll(M & lt)] = (unsigned char)(r * CB + t);
+            off += __popcll(M);
+        }
+    lds_visible();
+    return chunk * CHUNK + ord[part * CB + t];
+}
+
+// The chunk a workgroup works on and its part of it.  Workgroups are dispatched round-robin over the 8
+// XCDs, so workgroup b runs on XCD b mod 8: 32 workgroups take 8 chunks, the four parts of a chunk on one XCD,
+// whose L2 joins their stores.  The clipping work per seed varies across the domain, and mapped straight each XCD would get
+// every 8th chunk, on a lattice whose rows span a multiple of 8 chunks the same few column strips of
+// the domain in every row: XCDs with the costly strips ran up to 28% longer while the others idled for
+// the last third of the launch.  Rotating each group by a hash of its index (the top 3 bits of a
+// multiplicative hash, so that no period of the domain lines up with it) gives every XCD an even share
+// of every column.
+__device__ __forceinline__ void clip_chunk(int b, int &chunk, int &part)
+{
+    const unsigned q = (unsigned)b >> 5;
     const unsigned rot = (q * 2654435761u) >> 29;
-    return (int)((q << 3) | ((b + rot) & 7));
+    chunk = (int)((q << 3) | ((b + rot) & 7));
+    part = (b >> 3) & 3;
 }
 
 // every seed with CAP_SMALL slots; the ones that outgrow them go to the queue retry[1..retry[0]]
@@ -547,8 +642,12 @@ __global__ __launch_bounds__(CB) void k_clip(lv_grid_params g, int n, const doub
                                              int *__restrict__ err, int *__restrict__ retry)
 {
     __shared__ lds_poly P;
+    __shared__ unsigned char ord[CHUNK];
     const int t = threadIdx.x;
-    const int i = clip_block(blockIdx.x, gridDim.x) * CB + t;
+    int chunk, part;
+    clip_chunk(blockIdx.x, chunk, part);
+    if (chunk * CHUNK >= n) return;
+    const int i = clip_seed_of<2>(g, n, chunk, part, x, ord);
     if (i >= n) return;  // no block-wide barriers below
     if (!clip_seed(g, n, i, x, cell_start, cell_labels, cell_x, m, path_i, path_rr, ne, ev, el, ld, area, cent, err, P, t))
         retry[1 + atomicAdd(&retry[0], 1)] = i;
@@ -573,11 +672,11 @@ __global__ __launch_bounds__(GB) void k_clip_group(lv_grid_params g, int n, cons
                         ev, el, ld, area, cent, err, S);
 }
 
-// Up to this many seeds, a group of lanes each.  On jittered lattices (0.1 dr) clipping takes 35 us with groups
-// and 112 us with a thread per seed (and the queue's launch) at 1,024 seeds, 44 and 119 at 10,000, 110 and
-// 128 at 40,000, 131 and 128 at 50,176, 169 and 122 at 65,536, 552 and 217 at 262,144 (with 0.45 dr of jitter
-// the lines cross at 60,000).  The queue worked off by groups instead of threads takes 40 us less: with the
-// thread's chain for each of its seeds these were 137 us at 1,024, 160 at 10,000 and 260 at 262,144.
+// Up to this many seeds, a group of lanes each.  On lattices of 0.1 dr of jitter clipping takes 35 us with
+// groups and 83 us with a thread per seed (and the queue's launch) at 1,024 seeds, 45 and 100 at 10,000,
+// 109 and 105 at 40,000, 125 and 106 at 48,400; with 0.45 dr of jitter 55 and 141, 125 and 153, 145 and
+// 154: the line lies between where the two cross.  A thread per seed takes 97 us at 65,536 (169 with groups)
+// and 168 at 262,144 (552).
 constexpr int GROUP_MAX = 49152;
 
 }  // namespace
@@ -593,7 +692,7 @@ hipError_t lv_launch_clip(const lv_grid_params &g, int n, const double *x, const
     if (!all) {
         hipError_t e = hipMemsetAsync(retry, 0, sizeof(int), s);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_clip, dim3((n + CB - 1) / CB), dim3(CB), 0, s, g, n, x, cell_start, cell_labels, cell_x, m,
+        hipLaunchKernelGGL(k_clip, dim3((n + 8 * CHUNK - 1) / (8 * CHUNK) * 32), dim3(CB), 0, s, g, n, x, cell_start, cell_labels, cell_x, m,
                            path_i, path_rr, ne, ev, el, ld, area, cent, err, retry);
     }
     hipLaunchKernelGGL(k_clip_group, dim3(all ? groups : std::min(RETRY_BLOCKS, groups)), dim3(GB), 0, s, g, n, x,

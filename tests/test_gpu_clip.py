@@ -50,3 +50,11 @@ def test_polygons_of_too_many_edges_raise(lv, oracle, gpu, around, ok):
         grid = lv.VoronoiGrid(lv.UnitRectangle(), 0.1, r_max=2.0, positions=x)
         with pytest.raises(lv.LVError, match="LV_MAX_EDGES"):
             lv.remesh(grid)
+
+
+@pytest.mark.parametrize("n,seed", [(50001, 1), (65536, 2), (57344 + 255, 3)])
+def test_mesh_of_uneven_chunks_bit_exact(lv, oracle, gpu, n, seed):
+    """a thread per seed, the last chunk of 256 seeds and the last group of chunks not full; half of the cells empty"""
+    print("clip chunks %d" % n, flush=True)
+    x = np.random.default_rng(seed).random(2 * n)
+    _same_mesh(lv, oracle, x, 0.5 / np.sqrt(n), True, r_max=9.0 / np.sqrt(n))
