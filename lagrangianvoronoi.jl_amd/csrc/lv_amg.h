@@ -85,9 +85,24 @@ void lv_amg_free(lv_amg *G);
 // (perm_ok), else the operator's own; 1: the operator's own order.
 hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, const lv_pressure_system &A, int n,
                         const float *mval, const float *mdg, int layout, hipStream_t s);
+// What the caller leaves to the start of a cycle instead of a launch of its own (lv_amg_takes_head): in a
+// CG iteration (k >= 0) the convergence test on the residual's partials (|r|^2); before the first
+// (k < 0) the inner solve's threshold from its init's partials (r.z, r.r).
+struct lv_cycle_head {
+    const double *part;
+    int nb;
+    lv_cg_scalars *S;
+    lv_progress *prog;
+    int k;
+    double inner_tol2;
+    int dev;  // k < 0: the first sweep, whose tolerance and skip flag are in S
+};
+// Every workgroup of the down pass sums the partials (nb) for itself, while that costs less than a launch.
+bool lv_amg_takes_head(const lv_amg *G, int nb);
 // z = B r for the symmetric V(1,1) cycle B; writes the (r.z, r.r) partials of lv_nblocks(n) blocks
 // that the next CG kernel reduces.  Every kernel is a no-op once S->done is set.  With perm_ok, r
 // and z are in the aggregate order.  z0_ready (only when G->z0_in): G->z0 already holds
 // fine_scale D^-1 r, bit for bit as the cycle would compute it.
 hipError_t lv_amg_vcycle(const lv_amg *G, const lv_pressure_system &A, const float *r, float *z, double *Prr,
-                         const lv_cg_scalars *S, hipStream_t s, bool z0_ready = false);
+                         const lv_cg_scalars *S, hipStream_t s, bool z0_ready = false,
+                         const lv_cycle_head *head = nullptr);

@@ -496,20 +496,59 @@ __device__ __forceinline__ float down_row_z0(const fine_ops<V> &F, int i, const 
 // barrier: a block's life is a chain of dependent round trips, and the blocks on a CU take several
 // turns.  A lane past the block's cells loads cell na - 1's and drops them; dinv1 (level 1's
 // diagonal) is read whether or not z1 is stored.
-template <class V, bool Z0>
+// HEAD: first what the caller left to the cycle (lv_cycle_head), with the done flag; the workgroups all come
+// to the same verdict, and block 0 records it.
+template <class V, bool Z0, bool HEAD>
 __global__ __launch_bounds__(B) void k_fine_down_jr(fine_ops<V> F, const float *__restrict__ r,
                                                     float *__restrict__ z0, const int *__restrict__ start,
                                                     const int2 *__restrict__ blk, int na, float *__restrict__ rc,
                                                     const float *__restrict__ dinv1, float *__restrict__ z1,
-                                                    const int *__restrict__ done)
+                                                    const int *__restrict__ done, lv_cycle_head H)
 {
     __shared__ float tl[FUSE_CAP];
     const int b = lv_xcd_block(blockIdx.x, gridDim.x);
     const int2 p0 = blk[b], p1 = blk[b + 1];
-    const int dn = *done;
-    // the bounds and the flag in one round trip: without this the bounds' loads sink below the test
-    asm volatile("" ::"s"(p0.x), "s"(p0.y), "s"(p1.x), "s"(p1.y), "s"(dn));
-    if (dn) return;
+    if constexpr (HEAD) {
+        if (H.k < 0) {
+            const int skip = H.dev && H.S->skip;
+            if (blockIdx.x == 0) {
+                double o[2];
+                reduce_all<2>(H.part, H.nb, o);
+                if (threadIdx.x == 0) {
+                    H.S->thr2 = (H.dev ? H.S->itol2 : H.inner_tol2) * o[1];
+                    H.S->iters = 0;
+                    H.S->done = skip ? 1 : 0;
+                }
+            }
+            if (skip) return;
+        } else {
+            // the bounds, the partials, the flag and the threshold in one round trip
+            double pp[1][LV_RED_PER], o[1];
+            reduce_all_load<1>(H.part, H.nb, pp);
+            const int dn = *done;
+            const double thr2 = H.S->thr2;
+            reduce_all_pin<1>(pp);
+            asm volatile("" ::"s"(p0.x), "s"(p0.y), "s"(p1.x), "s"(p1.y), "s"(dn), "s"(thr2));
+            if (dn) return;
+            reduce_all_sum<1>(H.part, H.nb, pp, o);
+            const bool conv = o[0] <= thr2;
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+                if (conv) {
+                    H.S->rr = o[0];
+                    H.S->iters = H.k + 1;
+                    H.S->done = 1;
+                    if (H.prog) __hip_atomic_store(&H.prog->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                }
+                if (H.prog) __hip_atomic_store(&H.prog->seen, H.k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+            }
+            if (conv) return;
+        }
+    } else {
+        const int dn = *done;
+        // the bounds and the flag in one round trip: without this the bounds' loads sink below the test
+        asm volatile("" ::"s"(p0.x), "s"(p0.y), "s"(p1.x), "s"(p1.y), "s"(dn));
+        if (dn) return;
+    }
     const int c0 = p0.x, c1 = p1.x, R0 = p0.y, R1 = p1.y;
     int sa[FUSE_RPT], sb[FUSE_RPT];
     float dv[FUSE_RPT];
@@ -2137,7 +2176,8 @@ static st_pair st_pair_of(const lv_amg *G, int l)
 // (null when they are consecutive)
 template <class V>
 static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, const int *list, const float *r,
-                         float *z, double *Prr, const lv_cg_scalars *S, hipStream_t s, bool z0_ready)
+                         float *z, double *Prr, const lv_cg_scalars *S, hipStream_t s, bool z0_ready,
+                         const lv_cycle_head *head)
 {
     const int n = G->n0;
     const lv_amg_level &L1 = G->lev[1];
@@ -2155,14 +2195,16 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
         z1_given = lt > 1;
         float *z1 = z1_given ? L1.z : nullptr;
         const int *done = S ? &S->done : G->bfirst + 2 * (G->nbfuse + 1);
-        if (z0_ready && G->z0_in)
-            hipLaunchKernelGGL((k_fine_down_jr<V, true>), dim3(G->nbfuse), dim3(B), 0, s, F, r, G->z0,
-                               (const int *)G->start, reinterpret_cast<const int2 *>(G->bfirst), G->na, L1.r,
-                               (const float *)L1.dinv, z1, done);
-        else
-            hipLaunchKernelGGL((k_fine_down_jr<V, false>), dim3(G->nbfuse), dim3(B), 0, s, F, r, G->z0,
-                               (const int *)G->start, reinterpret_cast<const int2 *>(G->bfirst), G->na, L1.r,
-                               (const float *)L1.dinv, z1, done);
+#define LV_DOWN_JR(Z0, HEAD)                                                                                     \
+    hipLaunchKernelGGL((k_fine_down_jr<V, Z0, HEAD>), dim3(G->nbfuse), dim3(B), 0, s, F, r, G->z0,                 \
+                       (const int *)G->start, reinterpret_cast<const int2 *>(G->bfirst), G->na, L1.r,              \
+                       (const float *)L1.dinv, z1, done, head ? *head : lv_cycle_head{})
+        const bool z0_in = z0_ready && G->z0_in;
+        if (z0_in && head) LV_DOWN_JR(true, true);
+        else if (z0_in) LV_DOWN_JR(true, false);
+        else if (head) LV_DOWN_JR(false, true);
+        else LV_DOWN_JR(false, false);
+#undef LV_DOWN_JR
     } else {
         hipLaunchKernelGGL(k_fine_down_j<V>, g1(n), dim3(B), 0, s, F, r, G->z0, G->t0, S);
         hipLaunchKernelGGL(k_restrict1, g1((int64_t)G->na * RL), dim3(B), 0, s, G->na, (const int *)G->start, list,
@@ -2240,10 +2282,19 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
 }
 
 hipError_t lv_amg_vcycle(const lv_amg *G, const lv_pressure_system &A, const float *r, float *z, double *Prr,
-                         const lv_cg_scalars *S, hipStream_t s, bool z0_ready)
+                         const lv_cg_scalars *S, hipStream_t s, bool z0_ready, const lv_cycle_head *head)
 {
     if (G->perm_ok)
         return vcycle(G, fine_agg<lv_ell_agg16>(G, (const uint16_t *)G->pev16), (const int *)G->aggp,
-                      (const int *)nullptr, r, z, Prr, S, s, z0_ready);
-    return vcycle(G, fine_own(G, A), (const int *)G->agg, (const int *)G->list, r, z, Prr, S, s, false);
+                      (const int *)nullptr, r, z, Prr, S, s, z0_ready, head);
+    return vcycle(G, fine_own(G, A), (const int *)G->agg, (const int *)G->list, r, z, Prr, S, s, false, nullptr);
+}
+
+// The test in the down pass adds 0.5 us to it at 65,536 and 265,225 rows and 1.0 at 1,000,000, for a launch of 2.6 us
+// and its gap; at 4,194,304 rows 8.2 for a launch of 4.8.  The line (2 M rows) lies between, in what the workgroups
+// read together.
+static constexpr int64_t HEAD_MAX = 1ll << 21;
+bool lv_amg_takes_head(const lv_amg *G, int nb)
+{
+    return G->perm_ok && !G->fine_learned && G->nbfuse > 0 && (int64_t)G->nbfuse * nb <= HEAD_MAX;
 }

@@ -412,12 +412,21 @@ __global__ __launch_bounds__(B) void k_write_P(lv_fields F, int n, const double 
     if (i < n) F.P[i] = P[i];
 }
 
+// S as a solve starts from it
+__device__ __forceinline__ void init_scalars(lv_cg_scalars *S, double tol2, int itmax, int singular)
+{
+    lv_cg_scalars z = {};
+    z.tol2 = tol2;
+    z.itmax = itmax;
+    z.singular = singular;
+    *S = z;
+}
+
 // single-block finalisers of the one-off reductions
-enum { FIN_MEANS = 0, FIN_INIT64 = 1, FIN_RESID = 2, FIN_SUM1 = 3, FIN_INIT32 = 4, FIN_RESID0 = 5 };
+enum { FIN_MEANS = 0, FIN_INIT64 = 1, FIN_RESID = 2, FIN_SUM1 = 3 };
 
 __global__ __launch_bounds__(B) void k_finalize(const double *__restrict__ partials, int nb, int mode, int n,
-                                                double inner_tol2, lv_cg_scalars *S, lv_progress *pub = nullptr,
-                                                int seq = 0)
+                                                lv_cg_scalars *S, lv_progress *pub = nullptr, int seq = 0)
 {
     double o[3];
     {
@@ -454,34 +463,15 @@ __global__ __launch_bounds__(B) void k_finalize(const double *__restrict__ parti
             __hip_atomic_store(&pub->fseq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
         }
         break;
-    case FIN_RESID0: {  // the initial residual: the host's tests before the first sweep, made here
-        // (inner_tol2 carries the per-sweep floor of the inner tolerance, not squared)
-        const double rr = o[0], thr2 = S->tol2 * o[1];
-        S->rr64 = rr;
-        S->rr64_0 = rr;
-        S->bb = o[1];
-        S->thr2 = thr2;
-        S->skip = (rr <= thr2 || !(rr == rr)) ? 1 : 0;
-        const double need = 0.8 * sqrt(thr2 / rr);
-        double itol = need > inner_tol2 ? need : inner_tol2;
-        if (itol > 0.8) itol = 0.8;
-        S->itol2 = itol * itol;
-        break;
-    }
     case FIN_SUM1:
         S->xmean = o[0] / n;
         S->xshift = S->xmean - S->xmean0;
-        break;
-    case FIN_INIT32:  // reads the (r.z, r.r) partials of the inner init: |r32|^2 = 1 up to rounding
-        S->thr2 = inner_tol2 * o[1];
-        S->iters = 0;
-        S->done = 0;
         break;
     }
 }
 
 // thr2 of an inner FP32 solve from the (r.z, r.r) partials of its init.  dev: the first sweep, whose
-// inner tolerance and skip flag k_finalize (FIN_RESID0) left in S; a skipped sweep starts done, and
+// inner tolerance and skip flag k_cg32_init left in S; a skipped sweep starts done, and
 // its first k_cg_s reports that to the host.
 __global__ __launch_bounds__(B) void k_finalize2(const double *__restrict__ Prr, int nb, double inner_tol2,
                                                  lv_cg_scalars *S, int dev)
@@ -852,14 +842,15 @@ __device__ __forceinline__ double spmv_row_shifted(int i, int n, const lv_ell_ow
 
 // true residual r = (b - bmean) - A x; partials |r|^2, |b'|^2 (FP64).  With Pxs (the partial sums
 // of x written by k_correct, singular systems) the residual is that of x - d, d = mean(x) - xmean0,
-// the x that k_shift stores at the end of the solve; block 0 records d.
+// the x that k_shift stores at the end of the solve; block 0 records d.  Of S, bmean is read in
+// singular systems only.
 template <bool COMPACT, class V = lv_ell_own<double>>
 __global__ __launch_bounds__(B) void k_resid64(int n, V A, const double *__restrict__ diag,
                                                const double *__restrict__ b, const double *__restrict__ x,
                                                double *__restrict__ r, double *__restrict__ partials,
-                                               const double *__restrict__ Pxs, lv_cg_scalars *S)
+                                               const double *__restrict__ Pxs, lv_cg_scalars *S, int singular)
 {
-    const double bmean = S->bmean;
+    const double bmean = singular ? S->bmean : 0.0;
     double d = 0.0;
     if (Pxs) {
         double t[1];
@@ -905,22 +896,51 @@ __global__ __launch_bounds__(B) void k_shift(int n, double *__restrict__ x, cons
 
 // ---- FP32 inner PCG of the refinement --------------------------------------------------------
 
-// A first sweep that k_finalize (FIN_RESID0) flagged skip (initial residual within tol, zero, or
-// NaN) must leave x as it is: its FP32 vectors are zeros and its correction scale is 0, so neither
+// A first sweep that k_cg32_init flagged skip (initial residual within tol, zero, or NaN) must leave x as it is: its FP32 vectors are zeros and its correction scale is 0, so neither
 // 1/sqrt(0) nor a NaN residual reaches x.
 __device__ inline bool sweep_skipped(const lv_cg_scalars *S, int first) { return first && S->skip; }
 
 // r32 = r64 / |r64|, e = 0, z = dinv r, p = z; partials r.z, r.r.  With perm, the FP32 vectors
 // are in the aggregate order: r32[i] comes from r64[perm[i]].  With z0 also z0 = sc dinv r (the
-// multilevel cycle's pre-smoothed correction).  first: this is the solve's first sweep.
+// multilevel cycle's pre-smoothed correction).  F.first: this is the solve's first sweep.  Then the tests
+// on the initial residual that the host makes between sweeps are made here, by every block for itself
+// from the partials of the FP64 residual (F.part), and block 0 records them with what the
+// solve starts from (in a singular system FIN_MEANS did, with the means).
+struct first_sweep {
+    const double *part;
+    double tol2, floor_tol;  // floor_tol: the per-sweep floor of the inner tolerance
+    int itmax, singular, first;
+};
 __global__ __launch_bounds__(B) void k_cg32_init(int n, const double *__restrict__ r64, const int *__restrict__ perm,
                                                  const float *__restrict__ dinv, float *__restrict__ e,
                                                  float *__restrict__ r, float *__restrict__ z,
-                                                 double *__restrict__ Prr, const lv_cg_scalars *S,
-                                                 float *__restrict__ z0, float sc, int first)
+                                                 double *__restrict__ Prr, lv_cg_scalars *S,
+                                                 float *__restrict__ z0, float sc, first_sweep F)
 {
-    const bool skip = sweep_skipped(S, first);
-    const double inv = skip ? 0.0 : 1.0 / sqrt(S->rr64);
+    double rr;
+    bool skip = false;
+    if (F.first) {
+        double o[2];
+        reduce_all<2>(F.part, gridDim.x, o);
+        rr = o[0];
+        const double thr2 = F.tol2 * o[1];
+        skip = rr <= thr2 || !(rr == rr);
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            if (!F.singular) init_scalars(S, F.tol2, F.itmax, 0);
+            S->rr64 = rr;
+            S->rr64_0 = rr;
+            S->bb = o[1];
+            S->thr2 = thr2;
+            S->skip = skip ? 1 : 0;
+            const double need = 0.8 * sqrt(thr2 / rr);
+            double itol = need > F.floor_tol ? need : F.floor_tol;
+            if (itol > 0.8) itol = 0.8;
+            S->itol2 = itol * itol;
+        }
+    } else {
+        rr = S->rr64;
+    }
+    const double inv = skip ? 0.0 : 1.0 / sqrt(rr);
     double v[2] = {0.0, 0.0};
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
         const float ri = skip ? 0.0f : (float)(r64[perm ? perm[i] : i] * inv);
@@ -1309,20 +1329,21 @@ struct lv_comb8 {
 template <typename TA, int M>
 __global__ __launch_bounds__(B) void k_multidot(int n, lv_vec8<TA> V, double *__restrict__ partials)
 {
-    double v[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    double v[M] = {};
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
 #pragma unroll
         for (int q = 0; q < M; q++) v[q] += (double)V.a[q][i] * V.b[q][i];
     }
-    block_partials<8>(v, partials, gridDim.x);
+    block_partials<M>(v, partials, gridDim.x);
 }
 
+// a block per dot product (one block for all eight took 4.7 us)
 __global__ __launch_bounds__(B) void k_multidot_fin(const double *__restrict__ partials, int nb,
                                                     double *__restrict__ out)
 {
-    double o[8];
-    reduce_all<8>(partials, nb, o);
-    if (threadIdx.x < 8) out[threadIdx.x] = o[threadIdx.x];
+    double o[1];
+    reduce_all<1>(partials + (size_t)blockIdx.x * nb, nb, o);
+    if (threadIdx.x == 0) out[blockIdx.x] = o[0];
 }
 
 // y = alpha*y + sum_q c_q x_q  (y may be one of the x_q only if its c is applied via alpha).  The
@@ -1480,12 +1501,7 @@ hipError_t await_published(lv_progress *hprog, int seq, lv_cg_scalars *dS, lv_cg
 
 __global__ void k_init_scalars(lv_cg_scalars *S, double tol2, int itmax, int singular)
 {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    lv_cg_scalars z = {};
-    z.tol2 = tol2;
-    z.itmax = itmax;
-    z.singular = singular;
-    *S = z;
+    if (threadIdx.x == 0 && blockIdx.x == 0) init_scalars(S, tol2, itmax, singular);
 }
 
 // the operator's own ELL as the kernels read it, with its compact overflow when it has one
@@ -1538,20 +1554,20 @@ static lv_ell_own<float> own32(const lv_pressure_system &A, int n, int layout = 
 // columns when every offset fits (2 bytes a slot and 1 a row instead of 4 and 4)
 template <class V>
 static void launch_resid64_v(const V &Av, dim3 G, hipStream_t s, int n, const double *diag, const double *b,
-                             const double *x, double *r, double *p3, const double *Pxs, lv_cg_scalars *S)
+                             const double *x, double *r, double *p3, const double *Pxs, lv_cg_scalars *S, int singular)
 {
     if (Av.ocap > 0)
-        hipLaunchKernelGGL((k_resid64<true, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, S);
+        hipLaunchKernelGGL((k_resid64<true, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, S, singular);
     else
-        hipLaunchKernelGGL((k_resid64<false, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, S);
+        hipLaunchKernelGGL((k_resid64<false, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, S, singular);
 }
 static void launch_resid64(const lv_pressure_system &A, int layout, dim3 G, hipStream_t s, int n, const double *b,
                            const double *x, double *r, double *p3, const double *Pxs, lv_cg_scalars *S)
 {
     if (A.narrow)
-        launch_resid64_v(own64s(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, S);
+        launch_resid64_v(own64s(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, S, (int)A.singular);
     else
-        launch_resid64_v(own64(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, S);
+        launch_resid64_v(own64(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, S, (int)A.singular);
 }
 template <class V>
 static void launch_spmv64_v(const V &Av, dim3 G, hipStream_t s, int n, const double *diag, const double *x, double *y)
@@ -1572,8 +1588,8 @@ inline parts parts_of(double *base) { return parts{base, base + 3 * NBMAX, base 
 // application) until the device flags completion; *dflag is the done flag (1 converged, 2 stopped).
 // It returns without synchronising: S (iterations, residuals) is read by the caller's next read.
 // The host launches iteration k once the device has marked iteration k - 1 seen in prog (pinned
-// host memory): k_cg_s marks it when it starts, or, with a preconditioner, k_conv_check once its
-// test has run, so the host launches the next iteration while the device applies the
+// host memory): k_cg_s marks it when it starts, or, with a preconditioner, k_conv_check (or the down pass that
+// makes its test) once the test has run, so the host launches the next iteration while the device applies the
 // preconditioner.  It stops launching as soon as prog->done is set: at most one iteration (with a
 // preconditioner, one application of it) runs as no-ops after convergence.  If the record does not
 // advance for 20 ms the host synchronises and reads the scalars instead, so the loop ends whatever
@@ -1633,10 +1649,13 @@ hipError_t cg_iterate(int n, V A, const T *diag, const T *dinv, T *x, T *r, T *z
                 }
             hipLaunchKernelGGL((k_cg_u<T, false>), dim3(nb), dim3(B), 0, s, n, x, r, z, (const T *)p,
                                (const T *)q, dinv, (const double *)P.pq, P.rr, P.ur, dS, par, z0, sc);
-            hipLaunchKernelGGL(k_conv_check, dim3(1), dim3(B), 0, s, (const double *)P.ur, nb, dS, dprog, k);
+            const bool head = M->amg && lv_amg_takes_head(M->amg, nb);
+            if (!head)
+                hipLaunchKernelGGL(k_conv_check, dim3(1), dim3(B), 0, s, (const double *)P.ur, nb, dS, dprog, k);
             if (M->amg) {
+                const lv_cycle_head H{P.ur, nb, dS, dprog, k, 0.0, 0};
                 hipError_t e = lv_amg_vcycle(M->amg, *M->A, (const float *)r, (float *)z, P.rr,
-                                             (const lv_cg_scalars *)dS, s, z0 != nullptr);
+                                             (const lv_cg_scalars *)dS, s, z0 != nullptr, head ? &H : nullptr);
                 if (e != hipSuccess) return e;
             } else if constexpr (std::is_same<V, lv_ell_own<float>>::value) {
                 hipLaunchKernelGGL(k_apply_m32, dim3(nb), dim3(B), 0, s, n, A.deg, A.col, M->mval, M->mdg,
@@ -1698,22 +1717,22 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
         if (e1 != hipSuccess) return e1;
         memset(&h, 0, sizeof(h));
     }
-    hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, opt.tol * opt.tol,
-                       opt.itmax > 0 ? opt.itmax : 1000, (int)A.singular);
+    const double tol2 = opt.tol * opt.tol;
+    const int itmax = opt.itmax > 0 ? opt.itmax : 1000;
+    if (A.singular || opt.method == LV_SOLVER_PCG64)
+        hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, tol2, itmax, (int)A.singular);
     hipError_t e = hipSuccess;
-    // the means of b and x serve singular systems only (bmean stays the 0 k_init_scalars set, and xmean0
+    // the means of b and x serve singular systems only (elsewhere bmean stays the 0 that S starts from, and xmean0
     // is read only where x's mean is restored)
     if (A.singular) {
         hipLaunchKernelGGL(k_means, G, dim3(B), 0, s, n, b, (const double *)x, P.p3);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_MEANS, n, 0.0,
-                           W.S);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_MEANS, n, W.S);
     }
     int total = 0, nsweep = 0, skipped = 0;
     if (opt.method == LV_SOLVER_PCG64) {
         LV_LAUNCH_BY_OCAP(k_cg64_init, own64(A, n, opt.amg_layout), G, dim3(B), 0, s, n, own64(A, n, opt.amg_layout), (const double *)A.diag64, (const double *)A.dinv64, b,
                            (const double *)x, W.r, W.z, P.rr, P.p3, (const lv_cg_scalars *)W.S);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_INIT64, n, 0.0,
-                           W.S);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_INIT64, n, W.S);
         int done = 0;
         e = cg_iterate<double>(n, own64(A, n, opt.amg_layout), (const double *)A.diag64,
                                (const double *)A.dinv64, x, W.r, W.z, W.p, W.q, P, W.S, W.hprog,
@@ -1732,21 +1751,17 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
         double *Pxs = A.singular ? P.ur : nullptr;
         // the iterations of a sweep are still in S at the next sweep's read of the FP64 residual
         // (k_resid64 and k_finalize leave them), so a sweep ends without a synchronising read.
-        // Nor does the first sweep wait for one: k_finalize (FIN_RESID0) makes the tests below on
-        // the device, and a first sweep with nothing to solve starts done and changes nothing
+        // Nor does the first sweep wait for one: k_cg32_init makes the tests below on the device, and a first sweep with nothing to solve starts done and changes nothing
         // (its correction is zero).
         bool pending = false;
         double itol = 0.0;
         for (;;) {
             launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3,
                            nsweep > 0 ? (const double *)Pxs : (const double *)nullptr, W.S);
-            if (nsweep == 0) {
-                hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID0,
-                                   n, floor_tol, W.S);
-            } else {
+            if (nsweep > 0) {
                 const int seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
                 hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n,
-                                   0.0, W.S, W.dprog, seq);
+                                   W.S, W.dprog, seq);
                 e = await_published(W.hprog, seq, W.S, W.hS, &h, s);
                 if (e != hipSuccess) return e;
                 if (pending) total += h.iters;
@@ -1760,7 +1775,7 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
                 // the FP32 residual's drift from the FP64 one (a few per cent at these reductions: at
                 // margins up to 0.9 no 2048^2 benchmark solve needed an extra sweep), but not below
                 // what FP32 arithmetic can deliver in one sweep (the first sweep's is the same rule,
-                // evaluated by k_finalize)
+                // evaluated by k_cg32_init)
                 const double need = 0.8 * sqrt(h.thr2 / h.rr64);
                 itol = need > floor_tol ? need : floor_tol;
                 if (itol > 0.8) itol = 0.8;
@@ -1774,15 +1789,18 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
                 float *z0 = (Mi && Mi->amg && Mi->amg->z0_in) ? Mi->amg->z0 : nullptr;
                 hipLaunchKernelGGL(k_cg32_init, G, dim3(B), 0, s, n, (const double *)W.r,
                                    Gp ? (const int *)Gp->list : (const int *)nullptr, dinv32, W.e32, W.r32, W.z32,
-                                   P.rr, (const lv_cg_scalars *)W.S, z0, z0 ? Mi->amg->fine_scale : 0.0f,
-                                   nsweep == 0 ? 1 : 0);
-                // k_finalize2 clears the done flag of the previous sweep, so it precedes the first
-                // application of the learned preconditioner (which is skipped while done is set)
-                hipLaunchKernelGGL(k_finalize2, dim3(1), dim3(B), 0, s, (const double *)P.rr, nb, itol * itol, W.S,
-                                   nsweep == 0 ? 1 : 0);
+                                   P.rr, W.S, z0, z0 ? Mi->amg->fine_scale : 0.0f,
+                                   first_sweep{P.p3, tol2, floor_tol, itmax, (int)A.singular, nsweep == 0 ? 1 : 0});
+                // the threshold, and the done flag of the previous sweep cleared: before the first
+                // application of the preconditioner (which is skipped while done is set), or at its start
+                const bool head = Mi && Mi->amg && lv_amg_takes_head(Mi->amg, nb);
+                if (!head)
+                    hipLaunchKernelGGL(k_finalize2, dim3(1), dim3(B), 0, s, (const double *)P.rr, nb, itol * itol,
+                                       W.S, nsweep == 0 ? 1 : 0);
                 if (Mi && Mi->amg) {
+                    const lv_cycle_head H{P.rr, nb, W.S, W.dprog, -1, itol * itol, nsweep == 0 ? 1 : 0};
                     e = lv_amg_vcycle(Mi->amg, A, (const float *)W.r32, W.z32, P.rr, (const lv_cg_scalars *)W.S, s,
-                                      z0 != nullptr);
+                                      z0 != nullptr, head ? &H : nullptr);
                     if (e != hipSuccess) return e;
                 } else if (Mi) {
                     hipLaunchKernelGGL(k_apply_m32, G, dim3(B), 0, s, n, (const int *)A.deg, (const int *)A.ecol,
@@ -1821,13 +1839,11 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
         // final FP64 residual of the returned x
         if (A.singular) {
             hipLaunchKernelGGL(k_sum1, G, dim3(B), 0, s, n, (const double *)x, P.p3);
-            hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_SUM1, n, 0.0,
-                               W.S);
+            hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_SUM1, n, W.S);
             hipLaunchKernelGGL(k_shift, G, dim3(B), 0, s, n, x, (const lv_cg_scalars *)W.S);
         }
         launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3, (const double *)nullptr, W.S);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n, 0.0,
-                           W.S);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n, W.S);
         e = read_scalars(W.S, W.hS, &h, s);
         if (e != hipSuccess) return e;
     }
@@ -1914,9 +1930,9 @@ hipError_t dots_device(int n, const TA *const *a, const double *const *b, int m,
         LV_MD(1) LV_MD(2) LV_MD(3) LV_MD(4) LV_MD(5) LV_MD(6) LV_MD(7) LV_MD(8)
 #undef LV_MD
     default:
-        hipLaunchKernelGGL((k_multidot<TA, 0>), dim3(nb), dim3(B), 0, s, n, V, partials);
+        return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(k_multidot_fin, dim3(1), dim3(B), 0, s, (const double *)partials, nb, dout);
+    hipLaunchKernelGGL(k_multidot_fin, dim3(m), dim3(B), 0, s, (const double *)partials, nb, dout);
     return hipGetLastError();
 }
 

@@ -439,3 +439,26 @@ def test_single_workgroup_levels_match_oracle(lv, oracle, gpu, kind, K):
     z = solver.apply_preconditioner(r, "amg")
     zr = _hier(kind, x, dr, d, rp, cols, coef).apply(r)
     assert np.linalg.norm(z - zr) <= 1e-4 * np.linalg.norm(zr), (np.linalg.norm(z - zr) / np.linalg.norm(zr))
+
+
+@pytest.mark.parametrize("kind", ["periodic", "walls"])
+@pytest.mark.parametrize("K", [5, 16, 17, 40])
+def test_solves_that_start_and_end_in_the_cycle(lv, oracle, gpu, kind, K):
+    """the convergence test and the first threshold at the start of the down pass (layout 0: one workgroup up to
+    several) and as launches of their own (layout 1): a solve, the same from its result and one of nothing"""
+    _flush("cycle head %s %d" % (kind, K))
+    grid, op, solver, x, dr, d, rp, cols, coef = _system(lv, oracle, kind, K, "tg" if kind == "periodic" else "cavity", 1e-3)
+    b = np.random.default_rng(K).standard_normal(grid.n)
+    if not np.any(d > 0):
+        b -= b.mean()
+    P = []
+    for layout in (0, 1):
+        p = solver.solve(b, np.zeros(grid.n), method="amg", tol=1e-8, amg_layout=layout)
+        st = solver.last_stats
+        assert st["relres"][0] <= 1e-8 and st["iters"][0] > 0 and st["fallbacks"] == 0
+        again = solver.solve(b, p, method="amg", tol=1e-8, amg_layout=layout)
+        assert solver.last_stats["iters"][0] == 0 and np.array_equal(again, p)
+        none = solver.solve(np.zeros(grid.n), np.zeros(grid.n), method="amg", tol=1e-8, amg_layout=layout)
+        assert solver.last_stats["iters"][0] == 0 and not np.any(none)
+        P.append((p, st["iters"][0]))
+    assert abs(P[0][1] - P[1][1]) <= max(2, 0.2 * P[1][1])
