@@ -1211,7 +1211,8 @@ int lv_pressure_rhs(lv_ctx *ctx, double dt, int32_t gp_step, const double vbc[8]
     const int n = ctx->n;
     const lv_mesh_view M = mesh_view(ctx);
     LV_HIP_CHECK(lv_launch_rhs_geom(ctx->g, ctx->F, M, n, dt, v, ctx->rg, ctx->s));
-    LV_HIP_CHECK(lv_launch_gp(M, n, ctx->rg, ctx->F.P, ctx->F.mass, ctx->GP, nullptr, nullptr, ctx->s));
+    LV_HIP_CHECK(lv_launch_gp(M, n, ctx->rg, ctx->F.P, ctx->F.mass, ctx->GP, nullptr, nullptr, nullptr, ctx->b, ctx->W,
+                              ctx->s));
     LV_HIP_CHECK(lv_launch_rhs_b(M, n, gp_step, ctx->rg, ctx->GP, ctx->F.area, ctx->F.P, ctx->b, ctx->P0, ctx->s));
     if (b) LV_HIP_CHECK(hipMemcpyAsync(b, ctx->b, sizeof(double) * ctx->n, hipMemcpyDeviceToHost, ctx->s));
     if (GP) LV_HIP_CHECK(hipMemcpyAsync(GP, ctx->GP, sizeof(double) * 2 * ctx->n, hipMemcpyDeviceToHost, ctx->s));
@@ -1407,37 +1408,20 @@ static int ensure_picard_window(lv_ctx *ctx, int w)
     return LV_OK;
 }
 
-// Adds the Picard correction (P_cur - P_prev, AP_cur - AP_prev) to the window: one round of
+// The Picard correction (P_cur - P_prev, AP_cur - AP_prev) enters the window with one round of
 // classical Gram-Schmidt against the stored q's (applied identically to the z's), then
 // normalisation; the oldest direction makes room when the window is full.  (A second round left
 // the iterations of the 2048^2 benchmark steps unchanged and cost 0.8 ms per step.)  The dots stay on the
-// device (the combinations read them there), so the host never waits; a correction with no
+// device (the next kernel reads them there), so the host never waits; a correction with no
 // component left enters as a zero direction, which adds nothing to later projections.
-// the direction in pw_t1 with its image A pw_t1 in pw_t2 (both overwritten) into the set (Q, Z) of
-// at most w
-static int picard_add_pair(lv_ctx *ctx, float **Q, float **Z, int w, int *cnt)
+
+// The direction in pw_t1 with its image A pw_t1 in pw_t2 made orthogonal to the set (Q, Z) of at most w, and
+// a place for it made at the set's end: it is still to be scaled into it.  pw_dots holds <q_k, pw_t2>,
+// or |pw_t2|^2 of an empty set, and is left with |pw_t2|^2.
+static int picard_orthogonalise(lv_ctx *ctx, float **Q, float **Z, int w, int *cnt)
 {
-    const int n = ctx->n;
-    hipStream_t s = ctx->s;
-    const double *xp[8];
-    const float *xf[8];
-    double c[8];
-    if (*cnt > 0) {
-        const double *b[8];
-        for (int k = 0; k < *cnt; k++) {
-            xf[k] = Q[k];
-            b[k] = ctx->pw_t2;
-        }
-        LV_HIP_CHECK(lv_dots_device(n, xf, b, *cnt, ctx->W.partials, ctx->pw_dots, s));
-        for (int k = 0; k < *cnt; k++) c[k] = -1.0;  // -<q_k, t2>
-        LV_HIP_CHECK(lv_combine(n, ctx->pw_t2, 1.0, xf, c, *cnt, s, ctx->pw_dots, 1));
-        for (int k = 0; k < *cnt; k++) xf[k] = Z[k];
-        LV_HIP_CHECK(lv_combine(n, ctx->pw_t1, 1.0, xf, c, *cnt, s, ctx->pw_dots, 1));
-    }
-    {
-        const double *a[1] = {ctx->pw_t2}, *b[1] = {ctx->pw_t2};
-        LV_HIP_CHECK(lv_dots_device(n, a, b, 1, ctx->W.partials, ctx->pw_dots, s));
-    }
+    if (*cnt > 0)
+        LV_HIP_CHECK(lv_pw_out(ctx->n, ctx->pw_t1, ctx->pw_t2, Q, Z, *cnt, ctx->W.partials, ctx->pw_dots, ctx->s));
     if (*cnt == w) {  // drop the oldest direction
         float *q0 = Q[0], *z0 = Z[0];
         for (int k = 1; k < w; k++) {
@@ -1448,64 +1432,23 @@ static int picard_add_pair(lv_ctx *ctx, float **Q, float **Z, int w, int *cnt)
         Z[w - 1] = z0;
         (*cnt)--;
     }
-    xp[0] = ctx->pw_t2;
-    c[0] = 1.0;  // 1 / |t2|
-    LV_HIP_CHECK(lv_combine(n, Q[*cnt], 0.0, xp, c, 1, s, ctx->pw_dots, 2));
-    xp[0] = ctx->pw_t1;
-    LV_HIP_CHECK(lv_combine(n, Z[*cnt], 0.0, xp, c, 1, s, ctx->pw_dots, 2));
     (*cnt)++;
     return LV_OK;
 }
 
-static int picard_add_direction(lv_ctx *ctx, int w, int *cnt, const double *Pcur, const double *Pprev,
-                                const double *APcur, const double *APprev)
-{
-    const double *xp[2] = {Pcur, Pprev};
-    const double c[2] = {1.0, -1.0};
-    LV_HIP_CHECK(lv_combine(ctx->n, ctx->pw_t1, 0.0, xp, c, 2, ctx->s));
-    xp[0] = APcur;
-    xp[1] = APprev;
-    LV_HIP_CHECK(lv_combine(ctx->n, ctx->pw_t2, 0.0, xp, c, 2, ctx->s));
-    return picard_add_pair(ctx, ctx->pw_q, ctx->pw_z, w, cnt);
-}
-
-// P_cur - P_prev into y
-static int picard_record(lv_ctx *ctx, double *y, const double *Pcur, const double *Pprev)
-{
-    const double *xp[2] = {Pcur, Pprev};
-    const double c[2] = {1.0, -1.0};
-    LV_HIP_CHECK(lv_combine(ctx->n, y, 0.0, xp, c, 2, ctx->s));
-    return LV_OK;
-}
-
-// P0 += sum_k <q_k, r> z_k over the set (Q, Z): the guess whose residual is r minus its projection
-// on the q's.  r is b - AP_cur (APcur given), or pw_t2 as a previous projection left it (APcur null);
-// with keep, pw_t2 is left holding the projected residual.
-static int picard_project(lv_ctx *ctx, float *const *Q, float *const *Z, int cnt, const double *APcur, bool keep)
+// the direction z of an earlier call, with its image under this call's operator, into the set (Q, Z) of at most two
+static int picard_add_carried(lv_ctx *ctx, const double *z, float **Q, float **Z, int *cnt)
 {
     const int n = ctx->n;
     hipStream_t s = ctx->s;
-    const double *xp[8] = {ctx->b, APcur};
-    double c[8] = {1.0, -1.0};
-    if (APcur) LV_HIP_CHECK(lv_combine(n, ctx->pw_t2, 0.0, xp, c, 2, s));
-    const float *xf[8];
-    const double *b[8];
-    for (int k = 0; k < cnt; k++) {
-        xf[k] = Q[k];
-        b[k] = ctx->pw_t2;
-        c[k] = 1.0;  // <q_k, r>
-    }
-    if (cnt == 0) return LV_OK;
-    LV_HIP_CHECK(lv_dots_device(n, xf, b, cnt, ctx->W.partials, ctx->pw_dots, s));
-    for (int k = 0; k < cnt; k++) xf[k] = Z[k];
-    LV_HIP_CHECK(lv_combine(n, ctx->P0, 1.0, xf, c, cnt, s, ctx->pw_dots, 1));
-    if (keep) {
-        for (int k = 0; k < cnt; k++) {
-            xf[k] = Q[k];
-            c[k] = -1.0;
-        }
-        LV_HIP_CHECK(lv_combine(n, ctx->pw_t2, 1.0, xf, c, cnt, s, ctx->pw_dots, 1));
-    }
+    LV_HIP_CHECK(hipMemcpyAsync(ctx->pw_t1, z, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
+    LV_HIP_CHECK(lv_spmv64(ctx->A, n, z, ctx->pw_t2, s));
+    if (*cnt > 0) LV_HIP_CHECK(lv_dot_device(n, Q[0], ctx->pw_t2, ctx->W.partials, ctx->pw_dots, s));
+    else LV_HIP_CHECK(lv_dot_device(n, ctx->pw_t2, ctx->pw_t2, ctx->W.partials, ctx->pw_dots, s));
+    int rc = picard_orthogonalise(ctx, Q, Z, 2, cnt);
+    if (rc) return rc;
+    LV_HIP_CHECK(lv_normalise(n, Q[*cnt - 1], ctx->pw_t2, ctx->pw_dots, s));
+    LV_HIP_CHECK(lv_normalise(n, Z[*cnt - 1], ctx->pw_t1, ctx->pw_dots, s));
     return LV_OK;
 }
 
@@ -1551,11 +1494,7 @@ int lv_find_pressure(lv_ctx *ctx, double dt, int32_t niter, const lv_solve_opts 
         }
         if (ctx->pc_n == ctx->n) {
             for (int k = 0; k < ctx->pc_cnt; k++) {
-                const double *xp[1] = {ctx->pc_z[k]};
-                const double c1[1] = {1.0};
-                LV_HIP_CHECK(lv_combine(ctx->n, ctx->pw_t1, 0.0, xp, c1, 1, ctx->s));
-                LV_HIP_CHECK(lv_spmv64(ctx->A, ctx->n, ctx->pc_z[k], ctx->pw_t2, ctx->s));
-                rc = picard_add_pair(ctx, ctx->pc_q, ctx->pc_o, 2, &ccnt);
+                rc = picard_add_carried(ctx, ctx->pc_z[k], ctx->pc_q, ctx->pc_o, &ccnt);
                 if (rc) return rc;
             }
         }
@@ -1571,39 +1510,44 @@ int lv_find_pressure(lv_ctx *ctx, double dt, int32_t niter, const lv_solve_opts 
             LV_HIP_CHECK(lv_launch_rhs_b(mesh_view(ctx), ctx->n, 0, ctx->rg, ctx->GP, ctx->F.area, ctx->F.P, ctx->b,
                                          ctx->P0, ctx->s));
         } else {
-            // (with the Picard window, also its record of the last iterate, pw_P[0])
+            // (with the Picard window, also its record of the last iterate, pw_P[0], and A times it)
             LV_HIP_CHECK(lv_launch_gp(mesh_view(ctx), ctx->n, ctx->rg, ctx->P0, ctx->F.mass, ctx->GP, ctx->F.P,
-                                      (w > 0 && have >= 1) ? ctx->pw_P[0] : nullptr, ctx->s));
+                                      (w > 0 && have >= 1) ? ctx->pw_P[0] : nullptr, ctx->pw_AP[0], ctx->b, ctx->W,
+                                      ctx->s));
             LV_HIP_CHECK(lv_launch_rhs_b(mesh_view(ctx), ctx->n, 1, ctx->rg, ctx->GP, ctx->F.area, ctx->P0, ctx->b,
                                          nullptr, ctx->s));
         }
+        // The guess P0 += sum_k <q_k, r> z_k, whose residual is r = b - A P0 minus its projection on the
+        // window's q's; then the same with the carried directions and what is left of r
         if (w > 0 && have >= 1) {
+            const int n = ctx->n;
+            double *part = ctx->W.partials, *dots = ctx->pw_dots, *t1 = ctx->pw_t1, *t2 = ctx->pw_t2;
+            float *const *none = nullptr;
+            const bool use_carried = ccnt > 0 && it <= 4;
             if (have >= 2) {
                 // the corrections P_2 - P_1 and P_3 - P_2, recorded for the next call
-                if (carry && (it == 3 || it == 4)) {
-                    rc = picard_record(ctx, ctx->pc_new[it - 3], ctx->pw_P[0], ctx->pw_P[1]);
-                    if (rc) return rc;
-                }
-                rc = picard_add_direction(ctx, w, &cnt, ctx->pw_P[0], ctx->pw_P[1], ctx->pw_AP[0], ctx->pw_AP[1]);
+                double *rec = carry && (it == 3 || it == 4) ? ctx->pc_new[it - 3] : nullptr;
+                LV_HIP_CHECK(lv_pw_enter(n, ctx->pw_P[0], ctx->pw_P[1], ctx->pw_AP[0], ctx->pw_AP[1], t1, rec, t2,
+                                         ctx->pw_q, cnt, part, dots, ctx->s));
+                rc = picard_orthogonalise(ctx, ctx->pw_q, ctx->pw_z, w, &cnt);
                 if (rc) return rc;
+                LV_HIP_CHECK(lv_pw_resid(n, t1, t2, ctx->pw_q, ctx->pw_z[cnt - 1], cnt, ctx->b, ctx->pw_AP[0], part,
+                                         dots, ctx->s));
+                LV_HIP_CHECK(lv_pw_guess(n, ctx->P0, t2, ctx->pw_q, ctx->pw_z, cnt, ctx->pc_q, use_carried ? ccnt : 0,
+                                         part, dots, ctx->s));
+            } else if (use_carried) {
+                LV_HIP_CHECK(lv_pw_resid(n, t1, t2, ctx->pc_q, nullptr, ccnt, ctx->b, ctx->pw_AP[0], part, dots,
+                                         ctx->s));
             }
-            const bool use_carried = ccnt > 0 && it <= 4;
-            if (cnt > 0) {
-                rc = picard_project(ctx, ctx->pw_q, ctx->pw_z, cnt, ctx->pw_AP[0], use_carried);
-                if (rc) return rc;
-            }
-            if (use_carried) {
-                rc = picard_project(ctx, ctx->pc_q, ctx->pc_o, ccnt, cnt > 0 ? nullptr : ctx->pw_AP[0], false);
-                if (rc) return rc;
-            }
+            if (use_carried)
+                LV_HIP_CHECK(lv_pw_guess(n, ctx->P0, t2, ctx->pc_q, ctx->pc_o, ccnt, none, 0, part, dots, ctx->s));
         }
         rc = solve_on_device(ctx, ctx->b, ctx->P0, o, stats);
         if (rc == LV_E_NOT_CONVERGED) status = rc;
         else if (rc) return rc;
-        if (w > 0 && it < niter) {  // remember P_it (copied by the next iteration's k_gp) and A P_it = b' - r
+        if (w > 0 && it < niter) {  // remember P_it and A P_it = b' - r (copied by the next iteration's k_gp)
             std::swap(ctx->pw_P[0], ctx->pw_P[1]);
             std::swap(ctx->pw_AP[0], ctx->pw_AP[1]);
-            LV_HIP_CHECK(lv_apply_from_residual(ctx->n, ctx->b, ctx->W.r, ctx->pw_AP[0], ctx->W, ctx->s));
             have = std::min(have + 1, 2);
         }
     }

@@ -111,10 +111,12 @@ struct lv_rhs_geom {
 };
 hipError_t lv_launch_rhs_geom(const lv_grid_params &g, lv_fields F, lv_mesh_view M, int n, double dt, lv_vbc vbc,
                               const lv_rhs_geom &R, hipStream_t s);
-// GP of P (Pout, Pout2: also P written there, either may be null); b of P with (gp_step) or without the
+// GP of P (Pout: also P written there; Prec, APrec: also P and A P = b' - r of the solve that ended with
+// W.r; either may be null); b of P with (gp_step) or without the
 // GP term (P0: also P0 = P)
 hipError_t lv_launch_gp(lv_mesh_view M, int n, const lv_rhs_geom &R, const double *P, const double *mass, double *GP,
-                        double *Pout, double *Pout2, hipStream_t s);
+                        double *Pout, double *Prec, double *APrec, const double *b, const lv_solver_work &W,
+                        hipStream_t s);
 hipError_t lv_launch_rhs_b(lv_mesh_view M, int n, int gp_step, const lv_rhs_geom &R, const double *GP,
                            const double *area, const double *P, double *b, double *P0, hipStream_t s);
 hipError_t lv_launch_visc_rhs(int n, const double *mass, const double *vc, double dt, double *b, double *x,
@@ -127,20 +129,23 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
 
 // Picard extrapolation helpers (vectors of length n on stream s; the window's stored directions
 // are FP32, everything else FP64; sums in FP64)
-// the dots into the device array dout[0..m) without a host copy
-hipError_t lv_dots_device(int n, const double *const *a, const double *const *b, int m, double *partials,
-                          double *dout, hipStream_t s);
-hipError_t lv_dots_device(int n, const float *const *a, const double *const *b, int m, double *partials,
-                          double *dout, hipStream_t s);
-// y = alpha y + sum_q c_q x_q, the c_q scaled by device values: dmode 0 none, 1 c_q dc[q],
-// 2 c_q / sqrt(dc[0]) (0 unless dc[0] is positive and finite)
-hipError_t lv_combine(int n, double *y, double alpha, const double *const *x, const double *c, int m, hipStream_t s,
-                      const double *dc = nullptr, int dmode = 0);
-hipError_t lv_combine(int n, double *y, double alpha, const float *const *x, const double *c, int m, hipStream_t s,
-                      const double *dc = nullptr, int dmode = 0);
-hipError_t lv_combine(int n, float *y, double alpha, const double *const *x, const double *c, int m, hipStream_t s,
-                      const double *dc = nullptr, int dmode = 0);
-hipError_t lv_apply_from_residual(int n, const double *b, const double *r, double *Ax, const lv_solver_work &W,
-                                  hipStream_t s);
+// dots[0] = a . b, on the device
+hipError_t lv_dot_device(int n, const float *a, const double *b, double *partials, double *dots, hipStream_t s);
+hipError_t lv_dot_device(int n, const double *a, const double *b, double *partials, double *dots, hipStream_t s);
+// y = x / sqrt(*h) (0 unless *h is positive and finite)
+hipError_t lv_normalise(int n, float *y, const double *x, const double *h, hipStream_t s);
+// The Picard window (lv_find_pressure), m directions Q (images) and Z; dots: 8 device doubles.
+// t1 = Pc - Pp (rec, if given, a copy), t2 = APc - APp; dots[q] = Q_q . t2, or with m = 0 dots[0] = t2 . t2
+hipError_t lv_pw_enter(int n, const double *Pc, const double *Pp, const double *APc, const double *APp, double *t1,
+                       double *rec, double *t2, float *const *Q, int m, double *partials, double *dots, hipStream_t s);
+// (t2, t1) -= sum_q dots[q] (Q_q, Z_q); dots[0] = t2 . t2
+hipError_t lv_pw_out(int n, double *t1, double *t2, float *const *Q, float *const *Z, int m, double *partials,
+                     double *dots, hipStream_t s);
+// with znew first (Q_{m-1}, znew) = (t2, t1) / sqrt(dots[0]); t2 = b - AP, dots[q] = Q_q . t2
+hipError_t lv_pw_resid(int n, const double *t1, double *t2, float *const *Q, float *znew, int m, const double *b,
+                       const double *AP, double *partials, double *dots, hipStream_t s);
+// P0 += sum_q dots[q] Z_q; with no > 0 (at most 2) also t2 -= sum_q dots[q] Q_q, dots[q] = O_q . t2, q < no
+hipError_t lv_pw_guess(int n, double *P0, double *t2, float *const *Q, float *const *Z, int m, float *const *O, int no,
+                       double *partials, double *dots, hipStream_t s);
 // y = A x in FP64
 hipError_t lv_spmv64(const lv_pressure_system &A, int n, const double *x, double *y, hipStream_t s);

@@ -328,10 +328,16 @@ __device__ __forceinline__ void rhs_head(const rhs_slots &S, const int *oel, con
 }
 
 // GP from P; with Pout also the write-back of P into the particles (find_pressure!'s p.P = P), with
-// Pout2 a second copy of P (the Picard window's record of the last iterate)
+// rec.P the Picard window's record of the last iterate: P and A P = b' - r of the finished solve
+// (b' = b - bmean, r its final residual)
+struct pw_record {
+    double *P, *AP;
+    const double *b, *r;
+    const lv_cg_scalars *S;
+};
 __global__ __launch_bounds__(B) void k_gp(lv_mesh_view M, int n, lv_rhs_geom R, const double *__restrict__ P,
                                           const double *__restrict__ mass, double *__restrict__ GP,
-                                          double *__restrict__ Pout, double *__restrict__ Pout2)
+                                          double *__restrict__ Pout, pw_record rec)
 {
     const int i = blockIdx.x * B + threadIdx.x;
     const int ne = i < n ? M.ne[i] : 0;
@@ -364,7 +370,10 @@ __global__ __launch_bounds__(B) void k_gp(lv_mesh_view M, int n, lv_rhs_geom R, 
     GP[i] = gx / mi;
     GP[n + i] = gy / mi;
     if (Pout) Pout[i] = Pi;
-    if (Pout2) Pout2[i] = Pi;
+    if (rec.P) {
+        rec.P[i] = Pi;
+        rec.AP[i] = (rec.b[i] - rec.S->bmean) - rec.r[i];
+    }
 }
 
 // b = A P/(rho c2 dt^2) + bdiv (+ corr(GP) when gp); with P0 also the initial guess P0 = P
@@ -1311,30 +1320,16 @@ __global__ __launch_bounds__(B, 4) void k_pcg_small(int n, lv_ell_own<double> A,
 
 // ---- small FP64 vector algebra for the Picard extrapolation -----------------------------------
 
-// operands of the multi-dot and combination kernels; the a's and x's may be FP32 (the Picard
-// window's stored directions), everything is accumulated in FP64
-template <typename TA>
-struct lv_vec8 {
-    const TA *a[8];
-    const double *b[8];
-};
-template <typename TX>
-struct lv_comb8 {
-    const TX *x[8];
-    double c[8];
-};
+// ---- Picard extrapolation: the stored directions are FP32, everything is accumulated in FP64 ----------
 
-// M <= 8 dot products a_q . b_q in one pass (M a template parameter, so that a row's loads are
-// issued together rather than each behind a branch on the count)
-template <typename TA, int M>
-__global__ __launch_bounds__(B) void k_multidot(int n, lv_vec8<TA> V, double *__restrict__ partials)
+// partials of a . b
+template <typename TA>
+__global__ __launch_bounds__(B) void k_dot(int n, const TA *__restrict__ a, const double *__restrict__ b,
+                                           double *__restrict__ partials)
 {
-    double v[M] = {};
-    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
-#pragma unroll
-        for (int q = 0; q < M; q++) v[q] += (double)V.a[q][i] * V.b[q][i];
-    }
-    block_partials<M>(v, partials, gridDim.x);
+    double v[1] = {0.0};
+    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) v[0] += (double)a[i] * b[i];
+    block_partials<1>(v, partials, gridDim.x);
 }
 
 // a block per dot product (one block for all eight took 4.7 us)
@@ -1346,42 +1341,129 @@ __global__ __launch_bounds__(B) void k_multidot_fin(const double *__restrict__ p
     if (threadIdx.x == 0) out[blockIdx.x] = o[0];
 }
 
-// y = alpha*y + sum_q c_q x_q  (y may be one of the x_q only if its c is applied via alpha).  The
-// coefficients are C.c scaled by device values dc (the output of k_multidot_fin): dmode 0 none,
-// 1 c_q dc[q], 2 c_q / sqrt(dc[0]) (0 when dc[0] is not positive and finite).  Accumulated in FP64
-// and rounded once to y's type.
-// (M, the number of x's, a template parameter as in k_multidot)
-template <typename TX, typename TY, int M>
-__global__ __launch_bounds__(B) void k_combine(int n, TY *__restrict__ y, double alpha, lv_comb8<TX> C,
-                                               const double *__restrict__ dc, int dmode)
+// 1 / sqrt(h), or 0 when h is not positive and finite
+__device__ __forceinline__ double inv_norm(double h)
 {
-    double c[8];
-#pragma unroll
-    for (int q = 0; q < 8; q++) c[q] = C.c[q];
-    if (dmode == 1) {
-#pragma unroll
-        for (int q = 0; q < M; q++) c[q] = C.c[q] * dc[q];
-    } else if (dmode == 2) {
-        const double h = dc[0];
-        const double f = (h > 0.0 && h <= 1.7976931348623157e308) ? 1.0 / sqrt(h) : 0.0;
-#pragma unroll
-        for (int q = 0; q < 8; q++) c[q] = C.c[q] * f;
-    }
-    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
-        double acc = (alpha != 0.0) ? alpha * (double)y[i] : 0.0;  // alpha = 0 never reads y (may be uninitialised)
-#pragma unroll
-        for (int q = 0; q < M; q++) acc += c[q] * (double)C.x[q][i];
-        y[i] = (TY)acc;
-    }
+    return (h > 0.0 && h <= 1.7976931348623157e308) ? 1.0 / sqrt(h) : 0.0;
 }
 
-// A x = b' - r: recovers A P of a finished solve from its final residual (b' = b - bmean)
-__global__ __launch_bounds__(B) void k_apply_from_residual(int n, const double *__restrict__ b,
-                                                          const double *__restrict__ r, double *__restrict__ Ax,
-                                                          const lv_cg_scalars *S)
+// y = x / sqrt(*h), rounded once
+__global__ __launch_bounds__(B) void k_normalise(int n, float *__restrict__ y, const double *__restrict__ x,
+                                                 const double *__restrict__ h)
 {
-    const double bmean = S->bmean;
-    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) Ax[i] = (b[i] - bmean) - r[i];
+    const double f = inv_norm(*h);
+    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) y[i] = (float)(0.0 + f * x[i]);
+}
+
+// The Picard window's vector work (lv_find_pressure), each kernel one pass over what it reads: bound by
+// bytes at millions of rows, by launches below some 10^5.  A kernel for each combination and for each set of dots
+// took twice the launches (14 a Picard iteration, now 7) and read the temporaries again for each (a step of 65,536
+// particles 4.62 -> 4.40 ms, of 4,194,304 53.0 -> 52.8).
+// Q, Z: the window's directions, unused ones any valid pointer.  Sums are left as partials, k_multidot_fin's.
+struct lv_dirs8 {
+    float *v[8];
+};
+
+// t1 = Pc - Pp (rec: a second copy), t2 = APc - APp; the sums of Q_q . t2, q < M, or with M = 0 of t2 . t2
+template <int M>
+__global__ __launch_bounds__(B) void k_pw_enter(int n, const double *__restrict__ Pc, const double *__restrict__ Pp,
+                                                const double *__restrict__ APc, const double *__restrict__ APp,
+                                                double *__restrict__ t1, double *__restrict__ rec,
+                                                double *__restrict__ t2, lv_dirs8 Q, double *__restrict__ partials)
+{
+    constexpr int NV = M > 0 ? M : 1;
+    double v[NV] = {};
+    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
+        const double a = (0.0 + Pc[i]) - Pp[i], y = (0.0 + APc[i]) - APp[i];
+        t1[i] = a;
+        if (rec) rec[i] = a;
+        t2[i] = y;
+        if constexpr (M == 0) {
+            v[0] += y * y;
+        } else {
+#pragma unroll
+            for (int q = 0; q < M; q++) v[q] += (double)Q.v[q][i] * y;
+        }
+    }
+    block_partials<NV>(v, partials, gridDim.x);
+}
+
+// t2 -= sum_q dots[q] Q_q, t1 -= sum_q dots[q] Z_q; the sum of t2 . t2
+template <int M>
+__global__ __launch_bounds__(B) void k_pw_out(int n, double *__restrict__ t1, double *__restrict__ t2, lv_dirs8 Q,
+                                              lv_dirs8 Z, const double *__restrict__ dots,
+                                              double *__restrict__ partials)
+{
+    double c[M];
+#pragma unroll
+    for (int q = 0; q < M; q++) c[q] = -dots[q];
+    double v[1] = {0.0};
+    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
+        double y = t2[i], a = t1[i];
+#pragma unroll
+        for (int q = 0; q < M; q++) {
+            y += c[q] * (double)Q.v[q][i];
+            a += c[q] * (double)Z.v[q][i];
+        }
+        t2[i] = y;
+        t1[i] = a;
+        v[0] += y * y;
+    }
+    block_partials<1>(v, partials, gridDim.x);
+}
+
+// STORE: the newest direction Q_{M-1} = t2 / |t2|, Z_{M-1} = t1 / |t2| (|t2|^2 = dots[0]; zero when that is
+// not positive and finite).  Then t2 = b - AP and the sums of Q_q . t2, q < M.
+template <int M, bool STORE>
+__global__ __launch_bounds__(B) void k_pw_resid(int n, const double *__restrict__ t1, double *__restrict__ t2,
+                                                lv_dirs8 Q, float *__restrict__ znew, const double *__restrict__ dots,
+                                                const double *__restrict__ b, const double *__restrict__ AP,
+                                                double *__restrict__ partials)
+{
+    double f = 0.0;
+    if (STORE) f = inv_norm(dots[0]);
+    double v[M] = {};
+    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
+        float qn = 0.0f;
+        if (STORE) {
+            qn = (float)(0.0 + f * t2[i]);
+            Q.v[M - 1][i] = qn;
+            znew[i] = (float)(0.0 + f * t1[i]);
+        }
+        const double y = (0.0 + b[i]) - AP[i];
+        t2[i] = y;
+#pragma unroll
+        for (int q = 0; q < M; q++) v[q] += (double)(STORE && q == M - 1 ? qn : Q.v[q][i]) * y;
+    }
+    block_partials<M>(v, partials, gridDim.x);
+}
+
+// P0 += sum_q dots[q] Z_q; KEEP: also t2 -= sum_q dots[q] Q_q and the sums of O_q . t2, q < NO <= 2
+template <int M, bool KEEP>
+__global__ __launch_bounds__(B) void k_pw_guess(int n, double *__restrict__ P0, double *__restrict__ t2, lv_dirs8 Q,
+                                                lv_dirs8 Z, const float *__restrict__ O0,
+                                                const float *__restrict__ O1, const double *__restrict__ dots,
+                                                double *__restrict__ partials)
+{
+    double c[M];
+#pragma unroll
+    for (int q = 0; q < M; q++) c[q] = dots[q];
+    double v[2] = {0.0, 0.0};
+    for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
+        double p = P0[i];
+#pragma unroll
+        for (int q = 0; q < M; q++) p += c[q] * (double)Z.v[q][i];
+        P0[i] = p;
+        if (KEEP) {
+            double y = t2[i];
+#pragma unroll
+            for (int q = 0; q < M; q++) y += -c[q] * (double)Q.v[q][i];
+            t2[i] = y;
+            v[0] += (double)O0[i] * y;
+            v[1] += (double)O1[i] * y;
+        }
+    }
+    if (KEEP) block_partials<2>(v, partials, gridDim.x);
 }
 
 inline dim3 grid_of(int n) { return dim3((n + B - 1) / B); }
@@ -1419,9 +1501,11 @@ hipError_t lv_launch_rhs_geom(const lv_grid_params &g, lv_fields F, lv_mesh_view
 }
 
 hipError_t lv_launch_gp(lv_mesh_view M, int n, const lv_rhs_geom &R, const double *P, const double *mass, double *GP,
-                        double *Pout, double *Pout2, hipStream_t s)
+                        double *Pout, double *Prec, double *APrec, const double *b, const lv_solver_work &W,
+                        hipStream_t s)
 {
-    hipLaunchKernelGGL(k_gp, grid_of(n), dim3(B), 0, s, M, n, R, P, mass, GP, Pout, Pout2);
+    hipLaunchKernelGGL(k_gp, grid_of(n), dim3(B), 0, s, M, n, R, P, mass, GP, Pout,
+                       pw_record{Prec, APrec, b, W.r, W.S});
     return hipGetLastError();
 }
 
@@ -1911,82 +1995,6 @@ hipError_t lv_apply_precond(const lv_pressure_system &A, lv_solver_work &W, int 
 
 // ---- host helpers for the Picard extrapolation ------------------------------------------------
 
-namespace {
-template <typename TA>
-hipError_t dots_device(int n, const TA *const *a, const double *const *b, int m, double *partials, double *dout,
-                       hipStream_t s)
-{
-    lv_vec8<TA> V;
-    for (int q = 0; q < 8; q++) {
-        V.a[q] = (q < m) ? a[q] : a[0];
-        V.b[q] = (q < m) ? b[q] : b[0];
-    }
-    const int nb = nblocks_of(n);
-    switch (m) {
-#define LV_MD(M)                                                                                         \
-    case M:                                                                                              \
-        hipLaunchKernelGGL((k_multidot<TA, M>), dim3(nb), dim3(B), 0, s, n, V, partials);             \
-        break;
-        LV_MD(1) LV_MD(2) LV_MD(3) LV_MD(4) LV_MD(5) LV_MD(6) LV_MD(7) LV_MD(8)
-#undef LV_MD
-    default:
-        return hipErrorInvalidValue;
-    }
-    hipLaunchKernelGGL(k_multidot_fin, dim3(m), dim3(B), 0, s, (const double *)partials, nb, dout);
-    return hipGetLastError();
-}
-
-template <typename TX, typename TY>
-hipError_t combine(int n, TY *y, double alpha, const TX *const *x, const double *c, int m, hipStream_t s,
-                   const double *dc, int dmode)
-{
-    lv_comb8<TX> C;
-    for (int q = 0; q < 8; q++) {  // unused slots (q >= m, never read) hold a valid device pointer
-        C.x[q] = (q < m) ? x[q] : (m > 0 ? x[0] : reinterpret_cast<const TX *>(y));
-        C.c[q] = (q < m) ? c[q] : 0.0;
-    }
-    const dim3 G(nblocks_of(n));
-    switch (m) {
-#define LV_CB(M)                                                                                         \
-    case M:                                                                                              \
-        hipLaunchKernelGGL((k_combine<TX, TY, M>), G, dim3(B), 0, s, n, y, alpha, C, dc, dmode);      \
-        break;
-        LV_CB(1) LV_CB(2) LV_CB(3) LV_CB(4) LV_CB(5) LV_CB(6) LV_CB(7) LV_CB(8)
-#undef LV_CB
-    default:
-        hipLaunchKernelGGL((k_combine<TX, TY, 0>), G, dim3(B), 0, s, n, y, alpha, C, dc, dmode);
-    }
-    return hipGetLastError();
-}
-}  // namespace
-
-hipError_t lv_dots_device(int n, const double *const *a, const double *const *b, int m, double *partials,
-                          double *dout, hipStream_t s)
-{
-    return dots_device(n, a, b, m, partials, dout, s);
-}
-hipError_t lv_dots_device(int n, const float *const *a, const double *const *b, int m, double *partials,
-                          double *dout, hipStream_t s)
-{
-    return dots_device(n, a, b, m, partials, dout, s);
-}
-
-hipError_t lv_combine(int n, double *y, double alpha, const double *const *x, const double *c, int m, hipStream_t s,
-                      const double *dc, int dmode)
-{
-    return combine(n, y, alpha, x, c, m, s, dc, dmode);
-}
-hipError_t lv_combine(int n, double *y, double alpha, const float *const *x, const double *c, int m, hipStream_t s,
-                      const double *dc, int dmode)
-{
-    return combine(n, y, alpha, x, c, m, s, dc, dmode);
-}
-hipError_t lv_combine(int n, float *y, double alpha, const double *const *x, const double *c, int m, hipStream_t s,
-                      const double *dc, int dmode)
-{
-    return combine(n, y, alpha, x, c, m, s, dc, dmode);
-}
-
 hipError_t lv_spmv64(const lv_pressure_system &A, int n, const double *x, double *y, hipStream_t s)
 {
     if (A.narrow)
@@ -1996,10 +2004,102 @@ hipError_t lv_spmv64(const lv_pressure_system &A, int n, const double *x, double
     return hipGetLastError();
 }
 
-hipError_t lv_apply_from_residual(int n, const double *b, const double *r, double *Ax, const lv_solver_work &W,
-                                  hipStream_t s)
+#define LV_PW_BY(m, ...)                                                                                              \
+    switch (m) {                                                                                                      \
+    case 1: { constexpr int M = 1; __VA_ARGS__; } break;                                                              \
+    case 2: { constexpr int M = 2; __VA_ARGS__; } break;                                                              \
+    case 3: { constexpr int M = 3; __VA_ARGS__; } break;                                                              \
+    case 4: { constexpr int M = 4; __VA_ARGS__; } break;                                                              \
+    case 5: { constexpr int M = 5; __VA_ARGS__; } break;                                                              \
+    case 6: { constexpr int M = 6; __VA_ARGS__; } break;                                                              \
+    case 7: { constexpr int M = 7; __VA_ARGS__; } break;                                                              \
+    case 8: { constexpr int M = 8; __VA_ARGS__; } break;                                                              \
+    default: return hipErrorInvalidValue;                                                                             \
+    }
+
+static lv_dirs8 dirs_of(float *const *v, int m)
 {
-    hipLaunchKernelGGL(k_apply_from_residual, dim3(nblocks_of(n)), dim3(B), 0, s, n, b, r, Ax,
-                       (const lv_cg_scalars *)W.S);
+    lv_dirs8 D;
+    for (int q = 0; q < 8; q++) D.v[q] = v[q < m ? q : 0];
+    return D;
+}
+static hipError_t pw_fin(int m, int nb, const double *partials, double *dots, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_multidot_fin, dim3(m), dim3(B), 0, s, partials, nb, dots);
+    return hipGetLastError();
+}
+
+hipError_t lv_dot_device(int n, const float *a, const double *b, double *partials, double *dots, hipStream_t s)
+{
+    const int nb = nblocks_of(n);
+    hipLaunchKernelGGL(k_dot<float>, dim3(nb), dim3(B), 0, s, n, a, b, partials);
+    return pw_fin(1, nb, partials, dots, s);
+}
+hipError_t lv_dot_device(int n, const double *a, const double *b, double *partials, double *dots, hipStream_t s)
+{
+    const int nb = nblocks_of(n);
+    hipLaunchKernelGGL(k_dot<double>, dim3(nb), dim3(B), 0, s, n, a, b, partials);
+    return pw_fin(1, nb, partials, dots, s);
+}
+
+hipError_t lv_normalise(int n, float *y, const double *x, const double *h, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_normalise, dim3(nblocks_of(n)), dim3(B), 0, s, n, y, x, h);
+    return hipGetLastError();
+}
+
+hipError_t lv_pw_enter(int n, const double *Pc, const double *Pp, const double *APc, const double *APp, double *t1,
+                       double *rec, double *t2, float *const *Q, int m, double *partials, double *dots, hipStream_t s)
+{
+    const int nb = nblocks_of(n);
+    if (m == 0) {
+        hipLaunchKernelGGL(k_pw_enter<0>, dim3(nb), dim3(B), 0, s, n, Pc, Pp, APc, APp, t1, rec, t2, lv_dirs8{},
+                           partials);
+        return pw_fin(1, nb, partials, dots, s);
+    }
+    const lv_dirs8 D = dirs_of(Q, m);
+    LV_PW_BY(m, hipLaunchKernelGGL(k_pw_enter<M>, dim3(nb), dim3(B), 0, s, n, Pc, Pp, APc, APp, t1, rec, t2, D,
+                                   partials))
+    return pw_fin(m, nb, partials, dots, s);
+}
+
+hipError_t lv_pw_out(int n, double *t1, double *t2, float *const *Q, float *const *Z, int m, double *partials,
+                     double *dots, hipStream_t s)
+{
+    const int nb = nblocks_of(n);
+    const lv_dirs8 D = dirs_of(Q, m), E = dirs_of(Z, m);
+    LV_PW_BY(m, hipLaunchKernelGGL(k_pw_out<M>, dim3(nb), dim3(B), 0, s, n, t1, t2, D, E, (const double *)dots,
+                                   partials))
+    return pw_fin(1, nb, partials, dots, s);
+}
+
+hipError_t lv_pw_resid(int n, const double *t1, double *t2, float *const *Q, float *znew, int m, const double *b,
+                       const double *AP, double *partials, double *dots, hipStream_t s)
+{
+    const int nb = nblocks_of(n);
+    const lv_dirs8 D = dirs_of(Q, m);
+    if (znew) {
+        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_resid<M, true>), dim3(nb), dim3(B), 0, s, n, t1, t2, D, znew,
+                                       (const double *)dots, b, AP, partials))
+    } else {
+        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_resid<M, false>), dim3(nb), dim3(B), 0, s, n, t1, t2, D, znew,
+                                       (const double *)dots, b, AP, partials))
+    }
+    return pw_fin(m, nb, partials, dots, s);
+}
+
+hipError_t lv_pw_guess(int n, double *P0, double *t2, float *const *Q, float *const *Z, int m, float *const *O, int no,
+                       double *partials, double *dots, hipStream_t s)
+{
+    const int nb = nblocks_of(n);
+    const lv_dirs8 D = dirs_of(Q, m), E = dirs_of(Z, m);
+    if (no > 0) {
+        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_guess<M, true>), dim3(nb), dim3(B), 0, s, n, P0, t2, D, E,
+                                       (const float *)O[0], (const float *)O[no > 1 ? 1 : 0], (const double *)dots,
+                                       partials))
+        return pw_fin(no, nb, partials, dots, s);
+    }
+    LV_PW_BY(m, hipLaunchKernelGGL((k_pw_guess<M, false>), dim3(nb), dim3(B), 0, s, n, P0, t2, D, E,
+                                   (const float *)nullptr, (const float *)nullptr, (const double *)dots, partials))
     return hipGetLastError();
 }

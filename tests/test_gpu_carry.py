@@ -70,3 +70,23 @@ def test_carry_dropped_for_a_new_particle_set(lv, oracle, gpu):
     lv.stiffened_eos(grid, 1.4, 2500.0 / 1.4)
     st_b = lv.find_pressure(solver, 1e-3, 10)
     assert st_b["iters"] == st_a["iters"] and max(st_b["relres"]) <= 1e-10
+
+
+@pytest.mark.parametrize("K", [9, 40])
+@pytest.mark.parametrize("w", [1, 2, 3, 4, 5, 6, 7, 8])
+def test_windows_of_every_width(lv, oracle, gpu, w, K):
+    """a window of w directions, filled and past it (12 Picard solves): the pressure of plain warm starts to the
+    solves' tolerance, and every guess projected on w directions at least as good as the plain one"""
+    _flush("picard window %d, %d" % (w, K))
+    res = {}
+    for width in (0, w):
+        grid, op, x, dr = make_pair(lv, oracle, "periodic", K=K, seed=0x5EED0063, ic="tg")
+        lv.stiffened_eos(grid, 1.4, 2500.0 / 1.4)
+        solver = lv.PressureSolver(grid, method="pcg64", tol=1e-11, itmax=4000, picard_window=width)
+        st = lv.find_pressure(solver, 1e-3, 12)
+        assert max(st["relres"]) <= 1e-11
+        res[width] = (grid.get("P"), st)
+    assert rel_err(res[w][0], res[0][0]) <= 1e-7
+    # (two solves of 1e-11 each stand between the two residuals)
+    for a, b in zip(res[w][1]["relres0"][2:], res[0][1]["relres0"][2:]):
+        assert a <= 1.05 * b + 1e-10, (res[w][1]["relres0"], res[0][1]["relres0"])
