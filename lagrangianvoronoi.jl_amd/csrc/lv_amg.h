@@ -43,7 +43,7 @@ struct lv_amg {
     int hdesc[(LV_AMG_MAXLEV + 1) * 16];
     int tail_coef, tail_inv, tail_total;  // the LDS image's size, its dense inverse, and the LDS in use
     int pair[LV_AMG_MAXLEV + 1];  // pair[l]: levels l and l+1 (both above that kernel's) run as one down and
-                                  // one up kernel
+                                  // one up kernel (2: the kernels for odd periodic axes)
     int level_kernels;   // 1: every level above lk runs as its own kernels (pairs not used)
     int wcycle;          // 1: the levels of that kernel are visited by a W-cycle
     int *prog;           // its operations (device), nprog of them; hprog: the host copy

@@ -924,9 +924,10 @@ __global__ __launch_bounds__(B) void k_st_up(st_level L, int Kyc, const float *_
 // A block owns a tile of cells and recomputes in LDS what its stencils read from the cells around the
 // tile (a halo), with the expressions and the order of st_down_lane, sum_children and st_up_cell, so
 // every value is bit for bit the one the one-level kernels give.  Cells are addressed by unwrapped
-// coordinates; on a periodic axis the width of level l is a multiple of 4, so that the parent map
-// x -> x >> 1 commutes with the wrap on levels l and l+1.  Level l is at least PAIR_MIN_K cells wide
-// on both axes, so the unwrapped coordinates of every region stay within one width of the level and
+// coordinates; the last cell of an odd periodic axis is its parent's only child, so that beyond the
+// wrap children and parents lie one cell nearer than twice and half (child_near, parent_near; ODD: a
+// periodic axis of level l or l+1 is odd.  The arithmetic costs a pair 1 us, so even ones go without).  Level
+// l is at least PAIR_MIN_K cells wide on both axes, so the unwrapped coordinates of every region stay within one width of the level and
 // one conditional add or subtract wraps them.  The down tile is small (PD = 4: 4 lanes of work per
 // cell of level l+2) so that the small levels spread over many workgroups; 8 x 8 tiles left one
 // wavefront per SIMD working through six halo cells a lane, no faster than two one-level kernels.
@@ -950,6 +951,28 @@ __device__ __forceinline__ int cell_of(int x, int y, int Kx, int Ky, int xper, i
     y = wrap_near(y, Ky, yper, oky);
     ok = okx && oky;
     return ok ? x * Ky + y : 0;
+}
+
+// on an axis of K cells whose parents are Kc: the parent of cell x and the first child of parent X, all
+// unwrapped within one width (outside a non-periodic axis: any nearby coordinate); and whether X has two children
+template <bool ODD>
+__device__ __forceinline__ int parent_near(int x, int K, int Kc, int per)
+{
+    if (!ODD) return x >> 1;
+    const int d = per ? 2 * Kc - K : 0;
+    return (x < 0 ? x - d : (x >= K ? x + d : x)) >> 1;
+}
+template <bool ODD>
+__device__ __forceinline__ int child_near(int X, int K, int Kc, int per)
+{
+    if (!ODD) return 2 * X;
+    const int d = per ? 2 * Kc - K : 0;
+    return X < 0 ? 2 * X + d : (X >= Kc ? 2 * X - d : 2 * X);
+}
+template <bool ODD>
+__device__ __forceinline__ bool two_children(int X, int K, int Kc, int per)
+{
+    return !ODD || !(per && (K & 1)) || !(X == Kc - 1 || X == -1);
 }
 
 // the couplings of cell f = (x, y) (unwrapped) of level L and the mask of its neighbours inside the
@@ -992,6 +1015,7 @@ __device__ __forceinline__ float st_resid_lds(float rf, float d, const float ck[
 // of level l+2, as k_st_down<false> on level l and then on level l+1.  Regions of a block (level,
 // first cell relative to its tile's first cell, side): A (l, -3, 4PD+6) z and r, B (l, -2, 4PD+4)
 // the residual, C (l+1, -1, 2PD+2) r and z, D (l+1, 0, 2PD) the residual.
+template <bool ODD>
 __global__ __launch_bounds__(B) void k_st_down2(st_pair Q, const float *__restrict__ r0, float *__restrict__ z0,
                                                 float *__restrict__ r1, float *__restrict__ z1,
                                                 float *__restrict__ r2, const lv_cg_scalars *S)
@@ -1041,7 +1065,7 @@ __global__ __launch_bounds__(B) void k_st_down2(st_pair Q, const float *__restri
     int fD = cell_of(Xd, Yd, L1.Kx, L1.Ky, L1.xper, L1.yper, okd);
     const float dD = L1.d[fD];
     const unsigned okD = st_coefs(L1, Xd, Yd, fD, cD);
-    fD = (okd && tid < SD * SD) ? fD : -1;
+    fD = (okd && tid < SD * SD && Xd < L1.Kx && Yd < L1.Ky) ? fD : -1;  // (none beyond the wrap)
     // A: z = w D^-1 r of level l
 #pragma unroll
     for (int i = 0; i < IA; i++) {
@@ -1079,11 +1103,14 @@ __global__ __launch_bounds__(B) void k_st_down2(st_pair Q, const float *__restri
             zC[s] = 0.0f;
             continue;
         }
-        const int b = 2 * sx * SB + 2 * sy;
-        const float r = (tB[b] + tB[b + 1]) + (tB[b + SB] + tB[b + SB + 1]);
+        const int X = cx + sx, Y = cy + sy;
+        const int b = (child_near<ODD>(X, L0.Kx, L1.Kx, L0.xper) - (ax + 1)) * SB +
+                      (child_near<ODD>(Y, L0.Ky, L1.Ky, L0.yper) - (ay + 1));
+        const bool x2 = two_children<ODD>(X, L0.Kx, L1.Kx, L0.xper), y2 = two_children<ODD>(Y, L0.Ky, L1.Ky, L0.yper);
+        const float r = (tB[b] + (y2 ? tB[b + 1] : 0.0f)) +
+                        ((x2 ? tB[b + SB] : 0.0f) + (x2 && y2 ? tB[b + SB + 1] : 0.0f));
         rC[s] = r;
         zC[s] = OMEGA * dvC[i] * r;
-        const int X = cx + sx, Y = cy + sy;
         if (sx >= 1 && sx < 2 * PD + 1 && sy >= 1 && sy < 2 * PD + 1 && X < L1.Kx && Y < L1.Ky) r1[fC[i]] = r;
     }
     __syncthreads();
@@ -1091,7 +1118,7 @@ __global__ __launch_bounds__(B) void k_st_down2(st_pair Q, const float *__restri
     if (tid < SD * SD) {
         const int c = (dxs + 1) * SC + dys + 1;
         tD[tid] = fD >= 0 ? st_resid_lds<SC>(rC[c], dD, cD, okD, zC + c) : 0.0f;
-        if (fD >= 0 && Xd < L1.Kx && Yd < L1.Ky) z1[fD] = zC[c];
+        if (fD >= 0) z1[fD] = zC[c];
     }
     __syncthreads();
     // E: r of level l+2
@@ -1107,20 +1134,22 @@ __global__ __launch_bounds__(B) void k_st_down2(st_pair Q, const float *__restri
 // up on levels l+1 and l: the final correction t0 of level l from the final correction t2 of level
 // l+2, as k_st_up<false> on level l+1 and then on level l (level l+1's own correction stays in LDS).
 // Regions of a block (level, first cell relative to the tile's, side): Z0 (l, -1, PU+2) z, V (l+1,
-// -1, PU/2+2) the correction, Z1 (l+1, -2, PU/2+4) z, E (l+2, -1, PU/4+2) t2.
+// -1, PU/2+2) the correction, Z1 (l+1, -2, PU/2+4) z, E t2 of level l+2 (-1, PU/4+2; odd: -2, PU/4+4).
+template <bool ODD>
 __global__ __launch_bounds__(B) void k_st_up2(st_pair Q, const float *__restrict__ r0, const float *__restrict__ z0,
                                               const float *__restrict__ r1, const float *__restrict__ z1,
                                               const float *__restrict__ t2, float *__restrict__ t0,
                                               const lv_cg_scalars *S)
 {
-    constexpr int SZ0 = PU + 2, SV = PU / 2 + 2, SZ1 = PU / 2 + 4, SE = PU / 4 + 2;
+    constexpr int SZ0 = PU + 2, SV = PU / 2 + 2, SZ1 = PU / 2 + 4, EH = ODD ? 2 : 1,
+                  SE = PU / 4 + 2 * EH;
     constexpr int NZ0 = SZ0 * SZ0, IZ0 = (NZ0 + B - 1) / B;
     static_assert(PU * PU == B && SZ1 * SZ1 <= B && SV * SV <= B, "one cell of each region a lane");
     __shared__ float zl[NZ0], vm[SV * SV], zm[SZ1 * SZ1], e2[SE * SE];
     if (S && S->done) return;
     const st_level &L0 = Q.L0, &L1 = Q.L1;
     const int x0 = blockIdx.x * PU, y0 = blockIdx.y * PU;  // the tile's first cell on level l
-    const int vx = x0 / 2 - 1, vy = y0 / 2 - 1, ex = x0 / 4 - 1, ey = y0 / 4 - 1;
+    const int vx = x0 / 2 - 1, vy = y0 / 2 - 1, ex = x0 / 4 - EH, ey = y0 / 4 - EH;
     const int tid = threadIdx.x;
     // every global load first, unconditionally (from cell 0 outside a level or a region)
     float zv[IZ0];
@@ -1163,7 +1192,10 @@ __global__ __launch_bounds__(B) void k_st_up2(st_pair Q, const float *__restrict
         if (fV >= 0) {
             const float a = L1.alpha;
             const int zc = (vxs + 1) * SZ1 + vys + 1;
-            const float pe = e2[((Xv >> 1) - ex) * SE + ((Yv >> 1) - ey)];
+            auto pe_of = [&](int X, int Y) {
+                return e2[(parent_near<ODD>(X, L1.Kx, Q.Kx2, L1.xper) - ex) * SE + parent_near<ODD>(Y, L1.Ky, Q.Ky2, L1.yper) - ey];
+            };
+            const float pe = pe_of(Xv, Yv);
             const float z1c = zm[zc] + a * pe;
             float acc = dV * z1c;
 #pragma unroll
@@ -1172,7 +1204,7 @@ __global__ __launch_bounds__(B) void k_st_up2(st_pair Q, const float *__restrict
                 offset_of(k, ox, oy);
                 const bool in = (okV >> k) & 1;
                 const float zj = in ? zm[zc + ox * SZ1 + oy] : zm[zc];
-                const float ej = a * (in ? e2[(((Xv + ox) >> 1) - ex) * SE + (((Yv + oy) >> 1) - ey)] : pe);
+                const float ej = a * (in ? pe_of(Xv + ox, Yv + oy) : pe);
                 acc += cV[k] * (z1c - (zj + ej));
             }
             v = z1c + OMEGA * dvV * (rV - acc);
@@ -1184,7 +1216,10 @@ __global__ __launch_bounds__(B) void k_st_up2(st_pair Q, const float *__restrict
     if (own) {
         const float a = L0.alpha;
         const int zc = (txs + 1) * SZ0 + tys + 1;
-        const float pv = vm[((x >> 1) - vx) * SV + ((y >> 1) - vy)];
+        auto pv_of = [&](int X, int Y) {
+            return vm[(parent_near<ODD>(X, L0.Kx, L1.Kx, L0.xper) - vx) * SV + parent_near<ODD>(Y, L0.Ky, L1.Ky, L0.yper) - vy];
+        };
+        const float pv = pv_of(x, y);
         const float z1c = zl[zc] + a * pv;
         float acc = dT * z1c;
 #pragma unroll
@@ -1193,7 +1228,7 @@ __global__ __launch_bounds__(B) void k_st_up2(st_pair Q, const float *__restrict
             offset_of(k, ox, oy);
             const bool in = (okT >> k) & 1;
             const float zj = in ? zl[zc + ox * SZ0 + oy] : zl[zc];
-            const float ej = a * (in ? vm[(((x + ox) >> 1) - vx) * SV + (((y + oy) >> 1) - vy)] : pv);
+            const float ej = a * (in ? pv_of(x + ox, y + oy) : pv);
             acc += cT[k] * (z1c - (zj + ej));
         }
         t0[f] = z1c + OMEGA * dvT * (rT - acc);
@@ -2063,13 +2098,13 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
     G->lmat = mat && lk > 1 && G->lev[lk - 1].n <= MAT_MAX ? lk - 1 : lk;
     G->mat_ld = mat ? (G->lev[G->lmat].n + 3) & ~3 : 0;
     // pairs of levels above the tail that run as one kernel each way, from the tail upwards (the
-    // smallest levels gain most): level l at least PAIR_MIN_K wide, a multiple of 4 on a periodic axis
+    // smallest levels gain most): level l at least PAIR_MIN_K wide
     memset(G->pair, 0, sizeof(G->pair));
     for (int k = G->lmat - 2; k >= 2;) {
         const lv_amg_level &L = G->lev[k];
-        const bool ok = L.Kx >= PAIR_MIN_K && L.Ky >= PAIR_MIN_K && (!G->xper || L.Kx % 4 == 0) &&
-                        (!G->yper || L.Ky % 4 == 0);
-        G->pair[k] = ok ? 1 : 0;
+        const bool ok = L.Kx >= PAIR_MIN_K && L.Ky >= PAIR_MIN_K;
+        const bool odd = (G->xper && L.Kx % 4 != 0) || (G->yper && L.Ky % 4 != 0);
+        G->pair[k] = ok ? (odd ? 2 : 1) : 0;
         k -= ok ? 2 : 1;
     }
     AMG_CHECK(hipMemcpyAsync(G->prog, G->hprog, sizeof(int) * G->nprog, hipMemcpyHostToDevice, s));
@@ -2218,7 +2253,7 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
         if (pairs && G->pair[l]) {
             const lv_amg_level &C2 = G->lev[l + 2];
             const st_pair q = st_pair_of(G, l);
-            hipLaunchKernelGGL(k_st_down2, dim3((C2.Kx + PD - 1) / PD, (C2.Ky + PD - 1) / PD), dim3(B), 0, s, q,
+            hipLaunchKernelGGL(G->pair[l] == 2 ? k_st_down2<true> : k_st_down2<false>, dim3((C2.Kx + PD - 1) / PD, (C2.Ky + PD - 1) / PD), dim3(B), 0, s, q,
                                (const float *)L.r, L.z, C.r, C.z, C2.r, S);
             l++;
             continue;
@@ -2250,7 +2285,7 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
     for (int l = lt - 1; l >= 1; l--) {
         if (pairs && l >= 3 && G->pair[l - 1]) {
             const lv_amg_level &L = G->lev[l - 1], &C = G->lev[l], &C2 = G->lev[l + 1];
-            hipLaunchKernelGGL(k_st_up2, dim3((L.Kx + PU - 1) / PU, (L.Ky + PU - 1) / PU), dim3(B), 0, s,
+            hipLaunchKernelGGL(G->pair[l - 1] == 2 ? k_st_up2<true> : k_st_up2<false>, dim3((L.Kx + PU - 1) / PU, (L.Ky + PU - 1) / PU), dim3(B), 0, s,
                                st_pair_of(G, l - 1), (const float *)L.r, (const float *)L.z, (const float *)C.r,
                                (const float *)C.z, (const float *)C2.t, L.t, S);
             l--;

@@ -462,3 +462,22 @@ def test_solves_that_start_and_end_in_the_cycle(lv, oracle, gpu, kind, K):
         assert solver.last_stats["iters"][0] == 0 and not np.any(none)
         P.append((p, st["iters"][0]))
     assert abs(P[0][1] - P[1][1]) <= max(2, 0.2 * P[1][1])
+
+
+@pytest.mark.parametrize("kind,ic,K", [("periodic", "tg", 515), ("periodic", "tg", 394), ("periodic", "tg", 389),
+                                       ("xperiodic", "cavity", 411), ("periodic", "cavity", 270)])
+def test_paired_levels_of_odd_periodic_widths_are_bit_identical(lv, oracle, gpu, kind, ic, K):
+    """periodic axes whose paired levels are odd or twice odd: 129 over 65 cells at 515^2, 99 over 50 at 394^2, 98 over
+    49 at 389^2, an odd periodic axis beside a walled one, and a singular system"""
+    _flush("amg odd pairs %s %d" % (kind, K))
+    grid, op, solver, x, dr, d, rp, cols, coef = _system(lv, oracle, kind, K, ic, 1e-3)
+    r = np.random.default_rng(14).standard_normal(grid.n)
+    b = r - r.mean() if not np.any(d > 0) else r
+    out = {}
+    for lk in (1, 0):
+        P = solver.solve(b, np.zeros(grid.n), method="amg", amg_level_kernels=lk)
+        out[lk] = (P, solver.apply_preconditioner(r, "amg"), list(solver.last_stats["iters"][:1]))
+    assert np.all(np.isfinite(out[0][1])) and np.linalg.norm(out[0][1]) > 0
+    assert np.array_equal(out[0][1], out[1][1])
+    assert np.array_equal(out[0][0], out[1][0])
+    assert out[0][2] == out[1][2]
