@@ -23,9 +23,9 @@ struct lv_amg {
     int nlev;       // coarse levels; level nlev is the dense one
     int n0, na;     // fine rows, level-1 cells
     int xper, yper;
-    int *agg, *cnt, *start, *cursor, *list;
+    int *agg, *cnt, *start, *list;
     void *scan_tmp;
-    size_t cap_agg, cap_list, cap_t0, cap_z0, cap_cnt, cap_start, cap_cursor, cap_scan;
+    size_t cap_agg, cap_list, cap_t0, cap_z0, cap_cnt, cap_start, cap_scan;
     float *t0, *z0; // fine residual and pre-smoothed correction
     lv_amg_level lev[LV_AMG_MAXLEV + 1];
     float *dense_inv;    // nc * nc, column-major
@@ -40,7 +40,6 @@ struct lv_amg {
     int lk;              // first level of the single-workgroup kernel's program (levels lk..nlev)
     int lds_ok;          // 1: their arrays fit its LDS
     int *desc;           // their descriptors (device) and the host copy
-    int hdesc[(LV_AMG_MAXLEV + 1) * 16];
     int tail_coef, tail_inv, tail_total;  // the LDS image's size, its dense inverse, and the LDS in use
     int pair[LV_AMG_MAXLEV + 1];  // pair[l]: levels l and l+1 (both above that kernel's) run as one down and
                                   // one up kernel (2: the kernels for odd periodic axes)
@@ -62,6 +61,7 @@ struct lv_amg {
     float *oev32;        // read by the Krylov operator: offsets and FP32 couplings, LV_OVF_CAP per group
     int ovf_cap;         // groups with at most this many overflow slots use it (0: none)
     size_t cap_ooff, cap_oev32;
+    lv_mailbox mail;     // by which the host reads pflag
     int *pflag;          // [0] set when a column offset does not fit 16 bits, [1] when a level-1 cell
                          // is too large for the fused down pass
     int *bfirst;         // fused down pass: (first level-1 cell, first row) of each block (nbfuse + 1 pairs), then (0, 0)

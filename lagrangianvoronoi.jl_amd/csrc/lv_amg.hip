@@ -123,14 +123,14 @@ __global__ __launch_bounds__(B) void k_agg_key(int n, const double *__restrict__
     (void)lv_run_atomic_add<1>(cnt, a, act);  // half the atomics, which bound this kernel and the next
 }
 
-// (the order of a cell's rows in list is then fixed by k_agg_sort)
+// (the order of a cell's rows in list is then fixed by k_agg_sort; cnt is back at zero for the next set-up)
 __global__ __launch_bounds__(B) void k_agg_fill(int n, const int *__restrict__ agg, const int *__restrict__ start,
-                                                int *__restrict__ cursor, int *__restrict__ list)
+                                                int *__restrict__ cnt, int *__restrict__ list)
 {
     const int i = blockIdx.x * B + threadIdx.x;
     const bool act = i < n;
     const int a = act ? agg[i] : 0;
-    const int p = lv_run_atomic_add<1>(cursor, a, act);
+    const int p = lv_run_atomic_add<-1>(cnt, a, act);
     if (act) list[start[a] + p] = i;
 }
 
@@ -1634,6 +1634,20 @@ static_assert(TAIL_MAX <= LDS_MAX && LDS_MAX <= 2 * TB && LV_AMG_MAXPROG <= TB &
               "right-hand side entries, operations and descriptors per lane, and indices that div_small divides");
 static_assert(TAIL_LDS % 4 == 0, "the LDS image is copied as float4");
 
+// the program and the levels' descriptors, by value in the launch: two copies from pageable memory would
+// each hold the host up
+struct tail_tables {
+    uint8_t prog[LV_AMG_MAXPROG];
+    int desc[(LV_AMG_MAXLEV + 1) * LV_DESC];
+};
+static_assert((OP_WADD << OP_SHIFT | LV_AMG_MAXLEV) < 256, "an operation fits a byte");
+__global__ __launch_bounds__(TB) void k_tail_put(tail_tables H, int nprog, int *__restrict__ prog, int *__restrict__ desc)
+{
+    const int t = threadIdx.x;
+    if (t < nprog) prog[t] = H.prog[t];
+    if (t < (LV_AMG_MAXLEV + 1) * LV_DESC) desc[t] = H.desc[t];
+}
+
 // the tail levels' constants and the dense inverse into img in the LDS layout
 __global__ __launch_bounds__(B) void k_tail_pack(tail_levels T, tail_layout Y, const float *__restrict__ inv,
                                                  float *__restrict__ img)
@@ -1819,19 +1833,21 @@ hipError_t lv_amg_init(lv_amg *G)
     AMG_CHECK(hipMalloc(&G->tail_img, sizeof(float) * TAIL_LDS));
     AMG_CHECK(hipMalloc(&G->pw, sizeof(double) * (2 * LV_NBMAX + 2)));
     AMG_CHECK(hipMalloc(&G->prog, sizeof(int) * LV_AMG_MAXPROG));
-    AMG_CHECK(hipMalloc(&G->desc, sizeof(G->hdesc)));
-    static_assert(sizeof(G->hdesc) == sizeof(int) * (LV_AMG_MAXLEV + 1) * LV_DESC, "a descriptor per level");
+    AMG_CHECK(hipMalloc(&G->desc, sizeof(int) * (LV_AMG_MAXLEV + 1) * LV_DESC));
     AMG_CHECK(hipMalloc(&G->pflag, 2 * sizeof(int)));
+    AMG_CHECK(hipMemset(G->pflag, 0, 2 * sizeof(int)));
+    AMG_CHECK(lv_mail_init(&G->mail));
     return hipSuccess;
 }
 
 void lv_amg_free(lv_amg *G)
 {
-    void *ptrs[] = {G->agg, G->cnt, G->start, G->cursor, G->list, G->scan_tmp, G->t0, G->z0, G->dense_inv, G->tail_img, G->tail_mat, G->ext_mat,
+    void *ptrs[] = {G->agg, G->cnt, G->start, G->list, G->scan_tmp, G->t0, G->z0, G->dense_inv, G->tail_img, G->tail_mat, G->ext_mat,
                     G->pw, G->pv, G->pu, G->prog, G->desc, G->iperm, G->aggp, G->pdeg, G->poff, G->pev32, G->pev16,
                     G->pdiag32, G->pdinv32, G->pmval, G->pmdg, G->pflag, G->bfirst, G->ooff, G->oev32};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    lv_mail_free(&G->mail);
     for (int l = 0; l <= LV_AMG_MAXLEV; l++) {
         lv_amg_level &L = G->lev[l];
         void *q[] = {L.d, L.c, L.dinv, L.r, L.z, L.t, L.acc};
@@ -2045,19 +2061,61 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
     AMG_CHECK(grow(&G->list, &G->cap_list, (size_t)n));
     AMG_CHECK(grow(&G->t0, &G->cap_t0, (size_t)n));
     AMG_CHECK(grow(&G->z0, &G->cap_z0, (size_t)n));
+    const size_t cap_cnt = G->cap_cnt;
     AMG_CHECK(grow(&G->cnt, &G->cap_cnt, (size_t)na + 1));
+    if (G->cap_cnt != cap_cnt) AMG_CHECK(hipMemsetAsync(G->cnt, 0, sizeof(int) * (na + 1), s));
     AMG_CHECK(grow(&G->start, &G->cap_start, (size_t)na + 1));
-    AMG_CHECK(grow(&G->cursor, &G->cap_cursor, (size_t)na + 1));
     AMG_CHECK(grow((char **)&G->scan_tmp, &G->cap_scan, lv_scan_temp_bytes((int64_t)na + 1)));
-    AMG_CHECK(hipMemsetAsync(G->cnt, 0, sizeof(int) * (na + 1), s));
-    AMG_CHECK(hipMemsetAsync(G->cursor, 0, sizeof(int) * (na + 1), s));
     hipLaunchKernelGGL(k_agg_key, g1(n), dim3(B), 0, s, n, x, g.bxmin0, g.bxmin1, Lx / Kx, Ly / Ky, Kx, Ky, G->agg,
                        G->cnt);
     AMG_CHECK(lv_exclusive_scan_i32(G->cnt, G->start, (int64_t)na + 1, nullptr, G->scan_tmp, s));
-    hipLaunchKernelGGL(k_agg_fill, g1(n), dim3(B), 0, s, n, (const int *)G->agg, (const int *)G->start, G->cursor,
+    hipLaunchKernelGGL(k_agg_fill, g1(n), dim3(B), 0, s, n, (const int *)G->agg, (const int *)G->start, G->cnt,
                        G->list);
     AMG_CHECK(level_alloc(G->lev[1], Kx, Ky));
     hipLaunchKernelGGL(k_agg_sort, g1(na), dim3(B), 0, s, na, (const int *)G->start, G->list);
+    // fine smoother
+    G->fine_learned = (mval && mdg) ? 1 : 0;
+    G->mval = mval;
+    G->mdg = mdg;
+    G->fine_scale = OMEGA;
+    // the aggregate order: the rows of each level-1 cell consecutive (list, sorted within a cell)
+    G->perm_ok = 0;
+    G->nbfuse = 0;
+    G->z0_in = 0;
+    const bool aggregate = layout == 0 || layout >= 2;
+    const int nbf = n / FUSE_ROWS + 1;
+    if (aggregate) {
+        const size_t m = (size_t)LV_MAXE * n;
+        AMG_CHECK(grow(&G->iperm, &G->cap_iperm, (size_t)n));
+        AMG_CHECK(grow(&G->aggp, &G->cap_aggp, (size_t)n));
+        AMG_CHECK(grow(&G->pdeg, &G->cap_pdeg, (size_t)n));
+        AMG_CHECK(grow(&G->poff, &G->cap_poff, m));
+        AMG_CHECK(grow(&G->pev32, &G->cap_pev32, m));
+        AMG_CHECK(grow(&G->pev16, &G->cap_pev16, m));
+        const size_t mo = ((size_t)n / 64 + 1) * LV_OVF_CAP;
+        AMG_CHECK(grow(&G->ooff, &G->cap_ooff, mo));
+        AMG_CHECK(grow(&G->oev32, &G->cap_oev32, mo));
+        // (below 65536 rows launches, not the padding, set the kernels' time: no compact copy)
+        G->ovf_cap = (layout == 0 && n >= 65536) ? LV_OVF_CAP : layout == 3 ? 16 : 0;
+        AMG_CHECK(grow(&G->pdiag32, &G->cap_pdiag32, (size_t)n));
+        AMG_CHECK(grow(&G->pdinv32, &G->cap_pdinv32, (size_t)n));
+        if (G->fine_learned) {
+            AMG_CHECK(grow(&G->pmval, &G->cap_pmval, m));
+            AMG_CHECK(grow(&G->pmdg, &G->cap_pmdg, (size_t)n));
+        }
+        hipLaunchKernelGGL(k_perm_index, g1(n), dim3(B), 0, s, n, (const int *)G->list, (const int *)G->agg, G->iperm,
+                           G->aggp);
+        hipLaunchKernelGGL(k_perm_ell, g1(n), dim3(B), 0, s, n, (const int *)G->list, (const int *)G->iperm,
+                           (const int *)A.deg, (const int *)A.ecol, (const float *)A.ev32, (const float *)A.diag32,
+                           (const float *)A.dinv32, G->fine_learned ? mval : nullptr,
+                           G->fine_learned ? mdg : nullptr, G->pdeg, G->poff, G->pev32, G->pev16, G->pdiag32,
+                           G->pdinv32, G->pmval, G->pmdg, G->pflag, G->ooff, G->oev32, G->ovf_cap);
+        // the blocks of the fused down pass (Jacobi smoother)
+        AMG_CHECK(grow(&G->bfirst, &G->cap_bfirst, 2 * ((size_t)nbf + 2)));
+        hipLaunchKernelGGL(k_fuse_blocks, g1((int64_t)na + 1), dim3(B), 0, s, na, nbf, (const int *)G->start,
+                           reinterpret_cast<int2 *>(G->bfirst), G->pflag);
+        AMG_CHECK(lv_mail_post(&G->mail, G->pflag, 2, 2, s));  // read when the coarse levels are launched
+    }
     hipLaunchKernelGGL(k_coarse1, g1((int64_t)na * RL), dim3(B), 0, s, na, Kx, Ky, G->xper, G->yper,
                        (const int *)G->start, (const int *)G->list,
                        (const int *)G->agg, n, (const int *)A.deg, (const int *)A.ecol, (const double *)A.ev64,
@@ -2107,15 +2165,16 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
         G->pair[k] = ok ? (odd ? 2 : 1) : 0;
         k -= ok ? 2 : 1;
     }
-    AMG_CHECK(hipMemcpyAsync(G->prog, G->hprog, sizeof(int) * G->nprog, hipMemcpyHostToDevice, s));
+    tail_tables H;
+    for (int k = 0; k < G->nprog; k++) H.prog[k] = (uint8_t)G->hprog[k];
+    tail_descriptors(G, Y, H.desc);
+    hipLaunchKernelGGL(k_tail_put, dim3(1), dim3(TB), 0, s, H, G->nprog, G->prog, G->desc);
     const lv_amg_level &D = G->lev[l];
     hipLaunchKernelGGL(k_dense_inverse, dim3(1), dim3(DTB), 0, s, D.Kx, D.Ky, G->xper, G->yper, (const float *)D.d,
                        (const float *)D.c, A.singular, G->dense_inv);
     if (G->lds_ok) {
         hipLaunchKernelGGL(k_tail_pack, dim3(64), dim3(B), 0, s, tail_levels_of(G), Y, (const float *)G->dense_inv,
                            G->tail_img);
-        tail_descriptors(G, Y, G->hdesc);
-        AMG_CHECK(hipMemcpyAsync(G->desc, G->hdesc, sizeof(G->hdesc), hipMemcpyHostToDevice, s));
     }
     if (mat) {
         const int nt = G->lev[lk].n, ldt = (nt + 3) & ~3;
@@ -2132,50 +2191,9 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
             G->mat = G->ext_mat;
         }
     }
-    // fine smoother
-    G->fine_learned = (mval && mdg) ? 1 : 0;
-    G->mval = mval;
-    G->mdg = mdg;
-    G->fine_scale = OMEGA;
-    // the aggregate order: the rows of each level-1 cell consecutive (list, sorted within a cell)
-    G->perm_ok = 0;
-    G->nbfuse = 0;
-    G->z0_in = 0;
-    if (layout == 0 || layout >= 2) {
-        const size_t m = (size_t)LV_MAXE * n;
-        AMG_CHECK(grow(&G->iperm, &G->cap_iperm, (size_t)n));
-        AMG_CHECK(grow(&G->aggp, &G->cap_aggp, (size_t)n));
-        AMG_CHECK(grow(&G->pdeg, &G->cap_pdeg, (size_t)n));
-        AMG_CHECK(grow(&G->poff, &G->cap_poff, m));
-        AMG_CHECK(grow(&G->pev32, &G->cap_pev32, m));
-        AMG_CHECK(grow(&G->pev16, &G->cap_pev16, m));
-        const size_t mo = ((size_t)n / 64 + 1) * LV_OVF_CAP;
-        AMG_CHECK(grow(&G->ooff, &G->cap_ooff, mo));
-        AMG_CHECK(grow(&G->oev32, &G->cap_oev32, mo));
-        // (below 65536 rows launches, not the padding, set the kernels' time: no compact copy)
-        G->ovf_cap = (layout == 0 && n >= 65536) ? LV_OVF_CAP : layout == 3 ? 16 : 0;
-        AMG_CHECK(grow(&G->pdiag32, &G->cap_pdiag32, (size_t)n));
-        AMG_CHECK(grow(&G->pdinv32, &G->cap_pdinv32, (size_t)n));
-        if (G->fine_learned) {
-            AMG_CHECK(grow(&G->pmval, &G->cap_pmval, m));
-            AMG_CHECK(grow(&G->pmdg, &G->cap_pmdg, (size_t)n));
-        }
-        AMG_CHECK(hipMemsetAsync(G->pflag, 0, 2 * sizeof(int), s));
-        hipLaunchKernelGGL(k_perm_index, g1(n), dim3(B), 0, s, n, (const int *)G->list, (const int *)G->agg, G->iperm,
-                           G->aggp);
-        hipLaunchKernelGGL(k_perm_ell, g1(n), dim3(B), 0, s, n, (const int *)G->list, (const int *)G->iperm,
-                           (const int *)A.deg, (const int *)A.ecol, (const float *)A.ev32, (const float *)A.diag32,
-                           (const float *)A.dinv32, G->fine_learned ? mval : nullptr,
-                           G->fine_learned ? mdg : nullptr, G->pdeg, G->poff, G->pev32, G->pev16, G->pdiag32,
-                           G->pdinv32, G->pmval, G->pmdg, G->pflag, G->ooff, G->oev32, G->ovf_cap);
-        // the blocks of the fused down pass (Jacobi smoother)
-        const int nbf = n / FUSE_ROWS + 1;
-        AMG_CHECK(grow(&G->bfirst, &G->cap_bfirst, 2 * ((size_t)nbf + 2)));
-        hipLaunchKernelGGL(k_fuse_blocks, g1((int64_t)na + 1), dim3(B), 0, s, na, nbf, (const int *)G->start,
-                           reinterpret_cast<int2 *>(G->bfirst), G->pflag);
-        int flags[2] = {1, 1};
-        AMG_CHECK(hipMemcpyAsync(flags, G->pflag, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
-        AMG_CHECK(hipStreamSynchronize(s));
+    if (aggregate) {
+        int flags[2];
+        AMG_CHECK(lv_mail_await(&G->mail, flags, 2, s));
         G->perm_ok = flags[0] ? 0 : 1;
         G->nbfuse = (G->perm_ok && !flags[1]) ? nbf : 0;
         G->z0_in = (G->nbfuse > 0 && !G->fine_learned) ? 1 : 0;

@@ -59,8 +59,9 @@ struct lv_ctx {
     bool rg_alloc = false;
     int *deg = nullptr;
     void *scan_temp = nullptr;
-    int *d_flags = nullptr;   // [0] error word, [1] nonsingular flag, [2] a column offset wider than 16 bits,
-                              // [3] items of the cell list
+    int *d_flags = nullptr;   // [0] error word, [1] nonsingular flag, [2] a column offset wider than 16 bits (these
+                              // three zero between their uses), [3] items of the cell list, [4] couplings
+    lv_mailbox mail = {};     // by which the host reads them
     lv_timer *timers[LV_NKTIMERS] = {nullptr, nullptr, nullptr, nullptr};
     // Picard extrapolation: orthonormal A-images q_k of past Picard corrections and their
     // preimages z_k (A z_k = q_k), the last two Picard iterates and their A-images
@@ -241,18 +242,9 @@ double *field_ptr(lv_ctx *c, int f, size_t *count, size_t *elem, bool *readonly)
 
 lv_mesh_view mesh_view(lv_ctx *c) { return lv_mesh_view{c->ne, c->ev, c->el, c->n}; }
 
-int read_flags(lv_ctx *ctx, int *flags2)
-{
-    LV_HIP_CHECK(hipMemcpyAsync(flags2, ctx->d_flags, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->s));
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
-    return LV_OK;
-}
-
-int clear_flags(lv_ctx *ctx)
-{
-    LV_HIP_CHECK(hipMemsetAsync(ctx->d_flags, 0, 3 * sizeof(int), ctx->s));
-    return LV_OK;
-}
+constexpr int NFLAGS = 5;
+hipError_t post_flags(lv_ctx *ctx) { return lv_mail_post(&ctx->mail, ctx->d_flags, NFLAGS, 3, ctx->s); }
+hipError_t await_flags(lv_ctx *ctx, int *flags) { return lv_mail_await(&ctx->mail, flags, NFLAGS, ctx->s); }
 
 int check_ctx(lv_ctx *ctx, bool need_mesh)
 {
@@ -378,7 +370,7 @@ int lv_create(const lv_grid_desc *d, lv_ctx **out)
     ALLOC(ctx->el, LV_MAXE * cap);
     ALLOC(ctx->clip_retry, cap + 1);
     ALLOC(ctx->cell_start, ncells + 1);
-    ALLOC(ctx->d_flags, 4);
+    ALLOC(ctx->d_flags, NFLAGS);
     ALLOC(ctx->path_i, 2 * (size_t)std::max(1, g.npath));
     ALLOC(ctx->path_rr, (size_t)std::max(1, g.npath));
     // pressure system and solver work
@@ -416,6 +408,7 @@ int lv_create(const lv_grid_desc *d, lv_ctx **out)
         memset(ctx->W.hprog, 0, sizeof(lv_progress));
         e = hipHostGetDevicePointer((void **)&ctx->W.dprog, ctx->W.hprog, 0);
     }
+    if (e == hipSuccess) e = lv_mail_init(&ctx->mail);
     if (e == hipSuccess) e = hipHostMalloc((void **)&ctx->W.hS, sizeof(lv_cg_scalars), hipHostMallocDefault);
     if (e == hipSuccess) e = hipMalloc(&ctx->W.partials, lv_partials_bytes((int)cap));
     if (e == hipSuccess) e = hipMalloc(&ctx->scan_temp, lv_scan_temp_bytes((int64_t)cap + 1) + 256);
@@ -425,7 +418,7 @@ int lv_create(const lv_grid_desc *d, lv_ctx **out)
         if (e == hipSuccess)
             e = hipMemcpy(ctx->path_rr, ctx->h_path_rr.data(), sizeof(double) * g.npath, hipMemcpyHostToDevice);
     }
-    if (e == hipSuccess) e = hipMemset(ctx->d_flags, 0, 4 * sizeof(int));
+    if (e == hipSuccess) e = hipMemset(ctx->d_flags, 0, NFLAGS * sizeof(int));
     if (e == hipSuccess) {
         e = lv_spai_init(&ctx->spai);
         ctx->spai_ok = (e == hipSuccess);
@@ -463,6 +456,7 @@ int lv_destroy(lv_ctx *ctx)
                     ctx->W.q, ctx->W.e32, ctx->W.r32, ctx->W.z32, ctx->W.p32, ctx->W.q32, ctx->W.S,
                     ctx->W.partials, ctx->scan_temp};
     for (void *p : ptrs) dfree(p);
+    lv_mail_free(&ctx->mail);
     if (ctx->W.hprog) (void)hipHostFree(ctx->W.hprog);
     if (ctx->W.hS) (void)hipHostFree(ctx->W.hS);
     if (ctx->spai_ok) lv_spai_free(&ctx->spai);
@@ -639,10 +633,12 @@ int grow_cell_list(lv_ctx *ctx, int64_t want)
 
 extern "C" {
 
-int lv_remesh(lv_ctx *ctx)
+}  // extern "C"
+
+// remesh!; after a move whose error, if any, is in the flags
+static int remesh(lv_ctx *ctx)
 {
-    int rc = check_ctx(ctx, false);
-    if (rc) return rc;
+    int rc = LV_OK;
     const int n = ctx->n;
     if (ctx->max_items == 0) {
         int64_t want = (int64_t)n + n / 4 + 4096;
@@ -651,10 +647,8 @@ int lv_remesh(lv_ctx *ctx)
         if (rc) return rc;
     }
     lv_timer *tc = timer_if_on(ctx, 3), *tk = timer_if_on(ctx, 2);
-    int flags[4];
+    int flags[NFLAGS];
     for (int attempt = 0; attempt < 2; attempt++) {
-        rc = clear_flags(ctx);
-        if (rc) return rc;
         if (tc && tc->used == LV_TPOOL) lv_timer_flush(tc);
         LV_HIP_CHECK(lv_build_cell_list(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
                                         ctx->max_items, ctx->d_flags + 3, ctx->cl_temp, ctx->s,
@@ -667,9 +661,10 @@ int lv_remesh(lv_ctx *ctx)
                                     ctx->clip_retry, ctx->s, (int)ctx->max_items));
         if (tk) lv_timer_end(tk, ctx->s);
         ctx->mesh_valid = false;
+        LV_HIP_CHECK(post_flags(ctx));
+        LV_HIP_CHECK(await_flags(ctx, flags));
+        if (flags[0] == LV_E_NAN_VELOCITY) break;  // the move's
         ctx->A.valid = 0;
-        LV_HIP_CHECK(hipMemcpyAsync(flags, ctx->d_flags, 4 * sizeof(int), hipMemcpyDeviceToHost, ctx->s));
-        LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
         ctx->nitems = flags[3];
         if (ctx->nitems <= ctx->max_items) break;
         // more periodic images than buffered: the mesh is of a list cut off; room for the count, and again
@@ -678,10 +673,19 @@ int lv_remesh(lv_ctx *ctx)
     }
     if (tk) lv_timer_flush(tk);
     if (tc) lv_timer_flush(tc);
-    if (n > 0 && ctx->nitems <= 0) return lv_fail(ctx, LV_E_INVALID, "cell list: no items");
+    if (n > 0 && ctx->nitems <= 0 && flags[0] != LV_E_NAN_VELOCITY)
+        return lv_fail(ctx, LV_E_INVALID, "cell list: no items");
     if (flags[0] != 0) return lv_fail(ctx, flags[0], error_text(flags[0]));
     ctx->mesh_valid = true;
     return LV_OK;
+}
+
+extern "C" {
+
+int lv_remesh(lv_ctx *ctx)
+{
+    int rc = check_ctx(ctx, false);
+    return rc ? rc : remesh(ctx);
 }
 
 // ---- the mesh in CSR on the host --------------------------------------------------------------------
@@ -1069,15 +1073,9 @@ int lv_move(lv_ctx *ctx, double dt)
 {
     int rc = check_ctx(ctx, false);
     if (rc) return rc;
-    rc = clear_flags(ctx);
-    if (rc) return rc;
     LV_HIP_CHECK(lv_launch_move(ctx->g, ctx->F, mesh_view(ctx), ctx->n, dt, ctx->d_flags, ctx->s));
-    int flags[2];
-    rc = read_flags(ctx, flags);
-    if (rc) return rc;
     ctx->mesh_valid = false;
-    if (flags[0]) return lv_fail(ctx, flags[0], error_text(flags[0]));
-    return lv_remesh(ctx);
+    return remesh(ctx);
 }
 
 int lv_gravity_step(lv_ctx *ctx, const double g[2], double dt)
@@ -1120,14 +1118,20 @@ static int assemble_system(lv_ctx *ctx, double dt, int mode, int64_t *nnz, const
     if (rc) return rc;
     const int n = ctx->n;
     lv_mesh_view M = mesh_view(ctx);
-    LV_HIP_CHECK(lv_launch_degree(M, n, ctx->deg, ctx->s));
+    // the degrees, with what the host has to know of the operator; it reads that while the operator is formed
+    LV_HIP_CHECK(lv_launch_degree(ctx->F, M, n, dt, mode, ctx->deg, ctx->d_flags + 1, ctx->d_flags + 2, ctx->s));
     // row_ptr[0..n] = exclusive scan of the n degrees followed by one extra slot: deg[n] is 0
-    LV_HIP_CHECK(hipMemsetAsync(ctx->deg + n, 0, sizeof(int), ctx->s));
-    LV_HIP_CHECK(lv_exclusive_scan_i32(ctx->deg, ctx->A.row_ptr, n + 1, nullptr, ctx->scan_temp, ctx->s));
-    int total = 0;
-    LV_HIP_CHECK(hipMemcpyAsync(&total, ctx->A.row_ptr + n, sizeof(int), hipMemcpyDeviceToHost, ctx->s));
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
-    if (total > ctx->A.nnz_cap) {
+    LV_HIP_CHECK(lv_exclusive_scan_i32(ctx->deg, ctx->A.row_ptr, n + 1, ctx->d_flags + 4, ctx->scan_temp, ctx->s));
+    LV_HIP_CHECK(post_flags(ctx));
+    auto assemble = [&]() {  // (does nothing where the couplings have no room)
+        return lv_launch_assemble(ctx->g, ctx->F, M, n, dt, mode, ctx->A, ctx->s, rhs_vbc, rhs_vbc ? &ctx->rg : nullptr);
+    };
+    if (ctx->A.nnz_cap > 0) LV_HIP_CHECK(assemble());
+    int flags[NFLAGS];
+    LV_HIP_CHECK(await_flags(ctx, flags));
+    const int total = flags[4];
+    if (total > ctx->A.nnz_cap || ctx->A.nnz_cap == 0) {
+        LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
         dfree(ctx->A.cols);
         dfree(ctx->A.val64);
         dfree(ctx->A.val32);
@@ -1136,16 +1140,10 @@ static int assemble_system(lv_ctx *ctx, double dt, int mode, int64_t *nnz, const
         LV_HIP_CHECK(dalloc(&ctx->A.val64, want));
         LV_HIP_CHECK(dalloc(&ctx->A.val32, want));
         ctx->A.nnz_cap = want;
+        LV_HIP_CHECK(assemble());
     }
     ctx->A.nnz = total;
     ctx->A.deg = ctx->deg;
-    rc = clear_flags(ctx);
-    if (rc) return rc;
-    LV_HIP_CHECK(lv_launch_assemble(ctx->g, ctx->F, M, n, dt, mode, ctx->A, ctx->d_flags + 1, ctx->d_flags + 2,
-                                    ctx->s, rhs_vbc, rhs_vbc ? &ctx->rg : nullptr));
-    int flags[3];
-    LV_HIP_CHECK(hipMemcpyAsync(flags, ctx->d_flags, 3 * sizeof(int), hipMemcpyDeviceToHost, ctx->s));
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
     ctx->A.singular = (flags[1] == 0);
     ctx->A.narrow = (flags[2] == 0);
     ctx->assembly_id++;
@@ -1155,7 +1153,13 @@ static int assemble_system(lv_ctx *ctx, double dt, int mode, int64_t *nnz, const
     return LV_OK;
 }
 
-int lv_assemble_pressure(lv_ctx *ctx, double dt, int64_t *nnz) { return assemble_system(ctx, dt, 0, nnz); }
+int lv_assemble_pressure(lv_ctx *ctx, double dt, int64_t *nnz)
+{
+    int rc = assemble_system(ctx, dt, 0, nnz);
+    if (rc) return rc;
+    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+    return LV_OK;
+}
 
 static int need_pressure_operator(lv_ctx *ctx)
 {

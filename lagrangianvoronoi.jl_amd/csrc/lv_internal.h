@@ -175,6 +175,19 @@ struct lv_ctx;
 int lv_fail_hip(lv_ctx *ctx, hipError_t e, const char *what, const char *file, int line);
 int lv_fail(lv_ctx *ctx, int code, const char *msg);
 
+// lv_mail.hip: cnt <= LV_MAIL_MAX device integers to the host (the first nclear of them are zeroed once read).
+// One request at a time: posted, then awaited on the same stream.  If it has not come after 20 ms (a
+// kernel failed, or a long one runs) the host synchronises.
+constexpr int LV_MAIL_MAX = 32;
+struct lv_mailbox {
+    int *host, *dev;  // pinned: the request's number, then the integers
+    int seq;
+};
+hipError_t lv_mail_init(lv_mailbox *mb);
+void lv_mail_free(lv_mailbox *mb);
+hipError_t lv_mail_post(lv_mailbox *mb, int *src, int cnt, int nclear, hipStream_t s);
+hipError_t lv_mail_await(lv_mailbox *mb, int *out, int cnt, hipStream_t s);
+
 // lv_scan.hip
 size_t lv_scan_temp_bytes(int64_t n);
 hipError_t lv_exclusive_scan_i32(const int *in, int *out, int64_t n, int *d_total, void *temp, hipStream_t s,

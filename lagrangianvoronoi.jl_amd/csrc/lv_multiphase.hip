@@ -12,6 +12,8 @@
 #include "lv_internal.h"
 #include "lv_reduce.h"
 
+#include <cstring>
+
 namespace {
 
 constexpr int B = 256;
@@ -25,11 +27,14 @@ struct mph_scalars {
     double rr[2], rr0, pq, thr2;
     int iters, itmax, done;
 };
+constexpr int MPH_INTS = sizeof(mph_scalars) / sizeof(int);
+static_assert(MPH_INTS <= LV_MAIL_MAX && sizeof(mph_scalars) % sizeof(int) == 0, "the scalars fit one request");
 
-// 1 if particle i has a neighbour of another phase
+// 1 if particle i has a neighbour of another phase; flag[n] = 0
 __global__ __launch_bounds__(B) void k_mph_flag(lv_fields F, lv_mesh_view M, int n, int *__restrict__ flag)
 {
     const int i = blockIdx.x * B + threadIdx.x;
+    if (i == n) flag[n] = 0;
     if (i >= n) return;
     const int ph = F.phase[i];
     int f = 0;
@@ -282,6 +287,7 @@ struct lv_mph_work {
     void *scan_tmp;
     double *b, *x, *r, *p, *q, *T, *part;
     mph_scalars *S;
+    lv_mailbox mail;
     int cap;
 };
 
@@ -300,6 +306,7 @@ hipError_t lv_mph_alloc(lv_mph_work **out, int cap)
     MPH_CHECK(hipMalloc(&w->T, sizeof(double) * 2 * c));
     MPH_CHECK(hipMalloc(&w->part, sizeof(double) * 2 * LV_NBMAX));
     MPH_CHECK(hipMalloc(&w->S, sizeof(mph_scalars)));
+    MPH_CHECK(lv_mail_init(&w->mail));
     *out = w;
     return hipSuccess;
 }
@@ -310,19 +317,19 @@ void lv_mph_free(lv_mph_work *w)
     void *ptrs[] = {w->flag, w->pos, w->list, w->inv, w->scan_tmp, w->b, w->x, w->r, w->p, w->q, w->T, w->part, w->S};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    lv_mail_free(&w->mail);
     delete w;
 }
 
 // the interface set; returns its size m (host)
 static hipError_t mph_compact(lv_mph_work *w, lv_fields F, lv_mesh_view M, int n, int *m, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_mph_flag, g1(n), dim3(B), 0, s, F, M, n, w->flag);
-    MPH_CHECK(hipMemsetAsync(w->flag + n, 0, sizeof(int), s));
+    hipLaunchKernelGGL(k_mph_flag, g1((int64_t)n + 1), dim3(B), 0, s, F, M, n, w->flag);
     MPH_CHECK(lv_exclusive_scan_i32(w->flag, w->pos, (int64_t)n + 1, nullptr, w->scan_tmp, s));
     hipLaunchKernelGGL(k_mph_compact, g1(n), dim3(B), 0, s, n, (const int *)w->flag, (const int *)w->pos, w->list,
                        w->inv);
-    MPH_CHECK(hipMemcpyAsync(m, w->pos + n, sizeof(int), hipMemcpyDeviceToHost, s));
-    return hipStreamSynchronize(s);
+    MPH_CHECK(lv_mail_post(&w->mail, w->pos + n, 1, 0, s));
+    return lv_mail_await(&w->mail, m, 1, s);
 }
 
 // multiphase_projection!: the right-hand side, CG to |r| <= atol + rtol |b|, the dv update.
@@ -355,8 +362,10 @@ hipError_t lv_mph_projection(lv_mph_work *w, const lv_grid_params &g, lv_fields 
             hipLaunchKernelGGL(k_mph_dir, dim3(nb), dim3(B), 0, s, m, (const double *)w->r, w->p,
                                (const double *)Prr, nb, k, k & 1, w->S);
         }
-        MPH_CHECK(hipMemcpyAsync(&h, w->S, sizeof(h), hipMemcpyDeviceToHost, s));
-        MPH_CHECK(hipStreamSynchronize(s));
+        MPH_CHECK(lv_mail_post(&w->mail, reinterpret_cast<int *>(w->S), MPH_INTS, 0, s));
+        int hs[MPH_INTS];
+        MPH_CHECK(lv_mail_await(&w->mail, hs, MPH_INTS, s));
+        memcpy(&h, hs, sizeof(h));
         if (h.done) break;
     }
     hipLaunchKernelGGL(k_mph_apply_dv, g1(m), dim3(B), 0, s, g, F, M, n, m, (const int *)w->list, (const int *)w->inv,

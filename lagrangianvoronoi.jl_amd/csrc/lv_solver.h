@@ -89,13 +89,15 @@ struct lv_precond {
 size_t lv_partials_bytes(int n);
 hipError_t lv_apply_precond(const lv_pressure_system &A, lv_solver_work &W, int n, const lv_precond *M,
                             const double *r, double *z, hipStream_t s);
-hipError_t lv_launch_degree(lv_mesh_view M, int n, int *deg, hipStream_t s);
+// deg[0..n] (deg[n] = 0); *nonsingular set when some d_i != 0, *wide when some column offset needs more than 16 bits
+hipError_t lv_launch_degree(lv_fields F, lv_mesh_view M, int n, double dt, int mode, int *deg, int *nonsingular,
+                            int *wide, hipStream_t s);
 struct lv_rhs_geom;
 // refresh!(A) into A (mode 0 the pressure operator, 1 ViscousSolver's); with R (mode 0) the same pass
 // also stores the P-independent parts of refresh!(solver) for boundary velocity vbc
 // (wide: set when a column offset does not fit the 16-bit copy)
 hipError_t lv_launch_assemble(const lv_grid_params &g, lv_fields F, lv_mesh_view M, int n, double dt, int mode,
-                              lv_pressure_system &A, int *nonsingular, int *wide, hipStream_t s,
+                              lv_pressure_system &A, hipStream_t s,
                               const lv_vbc *vbc = nullptr, const lv_rhs_geom *R = nullptr);
 // The P-independent parts of refresh!(solver) for one find_pressure!: per mesh edge slot
 // w = lrr (m - x_i) and u = lrr (m - z) (each two planes of LV_MAXE x ld doubles, interior edges only),

@@ -30,14 +30,46 @@ constexpr int B = 256;
 
 // ---- assembly ----------------------------------------------------------------------------------
 
-__global__ __launch_bounds__(B) void k_degree(lv_mesh_view M, int n, int *__restrict__ deg)
+// the compressibility term d_i of refresh!(A), or ViscousSolver's m_i / dt (mode 1)
+__device__ __forceinline__ double row_diag(const lv_fields &F, int i, double dt, int mode)
+{
+    const double rho = F.rho[i];
+    return (mode == 0) ? F.mass[i] / (((rho * rho) * F.c2[i]) * (dt * dt)) : F.mass[i] / dt;
+}
+
+// the offset j - i of a column, taken into [-(n/2), n/2] modulo n (lv_ell_col undoes it)
+__device__ __forceinline__ int col_offset(int i, int j, int n)
+{
+    int off = j - i;
+    if (off > n / 2) off -= n;
+    if (off < -(n / 2)) off += n;
+    return off;
+}
+
+// deg[0..n), deg[n] = 0, and the two flags the host has to know before it can go on: the system is singular
+// iff every d_i == 0 (c2 = Inf), and its columns are narrow iff every offset fits 16 bits
+__global__ __launch_bounds__(B) void k_degree(lv_fields F, lv_mesh_view M, int n, double dt, int mode,
+                                              int *__restrict__ deg, int *__restrict__ nonsingular,
+                                              int *__restrict__ wide)
 {
     const int i = blockIdx.x * B + threadIdx.x;
+    if (i == n) deg[n] = 0;
     if (i >= n) return;
     int d = 0;
+    bool w16 = false;
     const int ne = M.ne[i];
-    for (int k = 0; k < ne; k++) d += (LV_EL(M, k, i) >= 0);
+    for (int k = 0; k < ne; k++) {
+        const int j = LV_EL(M, k, i);
+        if (j < 0) continue;
+        d++;
+        const int off = col_offset(i, j, n);
+        w16 |= (off < -32768 || off > 32767);
+    }
     deg[i] = d;
+    const double dd = row_diag(F, i, dt, mode);
+    // one flag write per wavefront at most
+    if (__any(w16) && (threadIdx.x & 63) == 0) atomicOr(wide, 1);
+    if (__any(dd != 0.0) && (threadIdx.x & 63) == 0 && *nonsingular == 0) atomicOr(nonsingular, 1);
 }
 
 // refresh!(A, grid, dt), src/pressure.jl:104-117 (mode 0), or the operator of ViscousSolver's
@@ -97,15 +129,14 @@ __device__ __forceinline__ void assemble_row(const lv_grid_params &g, const lv_f
                                              float *__restrict__ diag32, double *__restrict__ dinv64,
                                              float *__restrict__ dinv32, int *__restrict__ ecol,
                                              double *__restrict__ ev64, float *__restrict__ ev32,
-                                             int *__restrict__ nonsingular, const lv_vbc &vbc, const lv_rhs_geom &R,
+                                             const lv_vbc &vbc, const lv_rhs_geom &R,
                                              int *__restrict__ ocol, double *__restrict__ oev64,
                                              float *__restrict__ oev32, uint8_t *__restrict__ deg8,
-                                             int16_t *__restrict__ ecol16, int16_t *__restrict__ ocol16,
-                                             int *__restrict__ wide)
+                                             int16_t *__restrict__ ecol16, int16_t *__restrict__ ocol16)
 {
     const double x1 = F.x[i], x2 = F.x[n + i];
     const double rho = F.rho[i];
-    const double d = (mode == 0) ? F.mass[i] / (((rho * rho) * F.c2[i]) * (dt * dt)) : F.mass[i] / dt;
+    const double d = row_diag(F, i, dt, mode);
     const double mui = F.mu[i];
     const bool geom = R.w1 != nullptr;
     const double pv1 = F.v[i], pv2 = F.v[n + i];
@@ -153,22 +184,12 @@ __device__ __forceinline__ void assemble_row(const lv_grid_params &g, const lv_f
         sc[q] = j;
         sv[q] = c;
     }
-    // the 16-bit copy's offsets j - i, taken into [-(n/2), n/2] modulo n (lv_ell_col undoes it)
-    auto off16 = [&](int j) {
-        int off = j - i;
-        if (off > n / 2) off -= n;
-        if (off < -(n / 2)) off += n;
-        return off;
-    };
-    bool w16 = false;
     for (int k = 0; k < m; k++) {
         const size_t es = (size_t)k * n + i;
         ecol[es] = sc[k];
         ev64[es] = sv[k];
         ev32[es] = (float)sv[k];
-        const int off = off16(sc[k]);
-        w16 |= (off < -32768 || off > 32767);
-        ecol16[es] = (int16_t)off;
+        ecol16[es] = (int16_t)col_offset(i, sc[k], n);
     }
     deg8[i] = (uint8_t)m;
     // slots LV_OVF_BASE.. also into the compact copy of the row's 64-row group (a block's
@@ -181,17 +202,14 @@ __device__ __forceinline__ void assemble_row(const lv_grid_params &g, const lv_f
             ocol[eo] = sc[k];
             oev64[eo] = sv[k];
             oev32[eo] = (float)sv[k];
-            ocol16[eo] = (int16_t)off16(sc[k]);
+            ocol16[eo] = (int16_t)col_offset(i, sc[k], n);
         }
     }
-    if (__any(w16) && (threadIdx.x & 63) == 0) atomicOr(wide, 1);
     if (geom) {
         R.bdiv[i] = bd;
         R.den[i] = (rho * F.c2[i]) * (dt * dt);
         if (R.ocap > 0) rhs_geom_compact(M, R, i, n, ne);
     }
-    // the system is singular iff every d_i == 0 (c2 = Inf): one flag write per wavefront at most
-    if (__any(d != 0.0) && (threadIdx.x & 63) == 0 && *nonsingular == 0) atomicOr(nonsingular, 1);
     diag64[i] = d;
     diag32[i] = (float)d;
     dinv64[i] = 1.0 / dd;
@@ -207,12 +225,13 @@ __global__ __launch_bounds__(B) void k_assemble(lv_grid_params g, lv_fields F, l
                                                 double *__restrict__ diag64, float *__restrict__ diag32,
                                                 double *__restrict__ dinv64, float *__restrict__ dinv32,
                                                 int *__restrict__ ecol, double *__restrict__ ev64,
-                                                float *__restrict__ ev32, int *__restrict__ nonsingular, lv_vbc vbc,
+                                                float *__restrict__ ev32, lv_vbc vbc,
                                                 lv_rhs_geom R, int *__restrict__ ocol, double *__restrict__ oev64,
                                                 float *__restrict__ oev32, uint8_t *__restrict__ deg8,
                                                 int16_t *__restrict__ ecol16, int16_t *__restrict__ ocol16,
-                                                int *__restrict__ wide)
+                                                int64_t nnz_cap)
 {
+    if (row_ptr[n] > nnz_cap) return;
     // The block's rows own one contiguous span of the CSR copy; it is formed in LDS and stored with
     // coalesced writes after the barrier (each thread's own entries would be 64 scattered stores an
     // edge), unless it is longer than ACSR entries.
@@ -225,8 +244,8 @@ __global__ __launch_bounds__(B) void k_assemble(lv_grid_params g, lv_fields F, l
     const bool stage = clen <= ACSR;
     if (i < n) {  // rows past n hold no slots: their lanes stay out of the group's ballots below
         assemble_row(g, F, M, n, dt, mode, i, row_ptr, stage, cbase, s_col, s_v64, s_v32, cols, val64, val32,
-                     diag64, diag32, dinv64, dinv32, ecol, ev64, ev32, nonsingular, vbc, R, ocol, oev64, oev32,
-                     deg8, ecol16, ocol16, wide);
+                     diag64, diag32, dinv64, dinv32, ecol, ev64, ev32, vbc, R, ocol, oev64, oev32,
+                     deg8, ecol16, ocol16);
     }
     if (stage) {
         __syncthreads();
@@ -1475,21 +1494,22 @@ inline int nblocks_of(int n) { return lv_nblocks(n); }
 
 // ---- host wrappers ---------------------------------------------------------------------------------
 
-hipError_t lv_launch_degree(lv_mesh_view M, int n, int *deg, hipStream_t s)
+hipError_t lv_launch_degree(lv_fields F, lv_mesh_view M, int n, double dt, int mode, int *deg, int *nonsingular,
+                            int *wide, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_degree, grid_of(n), dim3(B), 0, s, M, n, deg);
+    hipLaunchKernelGGL(k_degree, grid_of(n + 1), dim3(B), 0, s, F, M, n, dt, mode, deg, nonsingular, wide);
     return hipGetLastError();
 }
 
 hipError_t lv_launch_assemble(const lv_grid_params &g, lv_fields F, lv_mesh_view M, int n, double dt, int mode,
-                              lv_pressure_system &A, int *nonsingular, int *wide, hipStream_t s, const lv_vbc *vbc,
+                              lv_pressure_system &A, hipStream_t s, const lv_vbc *vbc,
                               const lv_rhs_geom *R)
 {
     const lv_vbc v = vbc ? *vbc : lv_vbc{};
     const lv_rhs_geom r = (R && mode == 0) ? *R : lv_rhs_geom{};
     hipLaunchKernelGGL(k_assemble, grid_of(n), dim3(B), 0, s, g, F, M, n, dt, mode, (const int *)A.row_ptr, A.cols,
-                       A.val64, A.val32, A.diag64, A.diag32, A.dinv64, A.dinv32, A.ecol, A.ev64, A.ev32, nonsingular,
-                       v, r, A.ocol, A.oev64, A.oev32, A.deg8, A.ecol16, A.ocol16, wide);
+                       A.val64, A.val32, A.diag64, A.diag32, A.dinv64, A.dinv32, A.ecol, A.ev64, A.ev32,
+                       v, r, A.ocol, A.oev64, A.oev32, A.deg8, A.ecol16, A.ocol16, A.nnz_cap);
     return hipGetLastError();
 }
 
