@@ -350,8 +350,10 @@ hipError_t lv_mph_projection(lv_mph_work *w, const lv_grid_params &g, lv_fields 
     hipLaunchKernelGGL(k_mph_init, dim3(nb), dim3(B), 0, s, m, (const double *)w->b, w->x, w->r, w->p,
                        (const double *)Prr, nb, atol, rtol, itmax, w->S);
     mph_scalars h;
-    for (int k0 = 0;; k0 += 16) {
-        for (int k = k0; k < k0 + 16; k++) {
+    // launched ahead of the host's look at the scalars: none, 2, 4, 8 and then 16 iterations.  Many steps need
+    // none or few (an iteration past the end costs four launches that do nothing, 9 us; a look 8)
+    for (int k0 = 0, batch = 0;; k0 += batch, batch = std::min(std::max(2 * batch, 2), 16)) {
+        for (int k = k0; k < k0 + batch; k++) {
             hipLaunchKernelGGL(k_mph_grad, g1(m), dim3(B), 0, s, g, F, M, n, m, (const int *)w->list,
                                (const int *)w->inv, (const double *)w->p, w->T, (const mph_scalars *)w->S);
             hipLaunchKernelGGL(k_mph_div, dim3(nb), dim3(B), 0, s, g, F, M, n, m, (const int *)w->list,
