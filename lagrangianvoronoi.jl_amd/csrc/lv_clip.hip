@@ -10,8 +10,8 @@
 //     chain, for few seeds (lv_launch_clip), and for those that outgrow the other way's slots;
 //   * one thread owns a seed, its polygon in LDS as five slot-major planes (v1x, v1y, v2x, v2y, label),
 //     so lane t of the block addresses bank-conflict-free 8-byte words.  The fewest instructions, for
-//     many seeds.  Each polygon has CAP_SMALL slots (18 KB per 64-seed block, which holds a CU at 8
-//     wavefronts); a seed whose polygon outgrows them (0.4% at a 2048^2 jittered lattice, where no
+//     many seeds.  Each polygon has CAP = 8 slots (18 KB per 64-seed block, which holds a CU at 8
+//     wavefronts), or 10 while the device holds them all at once (WIDE_MAX); a seed whose polygon outgrows them (0.4% at a 2048^2 jittered lattice, where no
 //     polygon passes 10 edges while it is clipped) is queued and clipped again from the start by a
 //     group, so the result is the same either way.
 //
@@ -34,7 +34,6 @@ static_assert(G == 16, "a group is a row of 16 lanes");
 constexpr int RETRY_BLOCKS = 1024;  // blocks over the queue (grid-stride)
 constexpr int LCAP = 64;            // candidates of a group listed in LDS at a time
 constexpr int CB = 64;              // seeds per block (one wavefront) with a thread per seed
-constexpr int CAP_SMALL = 8;        // edge capacity of its LDS polygon
 constexpr double SIGNUM_EPS = 2.0 * 2.220446049250313e-16;  // 2*eps(Float64), src/polygon.jl:2
 
 struct clip_lds {
@@ -347,21 +346,24 @@ __device__ __forceinline__ void group_clip_seed(const lv_grid_params &g, int n, 
 
 // ---- a thread per seed ----------------------------------------------------------------------------
 
+template <int CAP>
 struct lds_poly {
-    double v1x[CAP_SMALL][CB], v1y[CAP_SMALL][CB], v2x[CAP_SMALL][CB], v2y[CAP_SMALL][CB];
-    int lab[CAP_SMALL][CB];
+    double v1x[CAP][CB], v1y[CAP][CB], v2x[CAP][CB], v2y[CAP][CB];
+    int lab[CAP][CB];
 };
 
 // the slots in registers, read again whenever a cut changed them
+template <int CAP>
 struct reg_poly {
-    double v1x[CAP_SMALL], v1y[CAP_SMALL], v2x[CAP_SMALL], v2y[CAP_SMALL];
+    double v1x[CAP], v1y[CAP], v2x[CAP], v2y[CAP];
 };
 
-__device__ __forceinline__ double load_slots(reg_poly &R, const lds_poly &P, int t, int len, double x1, double x2)
+template <int CAP>
+__device__ __forceinline__ double load_slots(reg_poly<CAP> &R, const lds_poly<CAP> &P, int t, int len, double x1, double x2)
 {
     double rr = 0.0;  // influence_rr
 #pragma unroll
-    for (int k = 0; k < CAP_SMALL; k++) {
+    for (int k = 0; k < CAP; k++) {
         R.v1x[k] = P.v1x[k][t];
         R.v1y[k] = P.v1y[k][t];
         R.v2x[k] = P.v2x[k][t];
@@ -380,7 +382,8 @@ __device__ __forceinline__ double load_slots(reg_poly &R, const lds_poly &P, int
 // every candidate, so a pre-test of the corners alone costs more than it spares (1.86 ms against 1.76 at
 // 4,194,304 seeds of 0.1 dr of jitter), and lanes that each run ahead to their next cut take 3.4 to 5.6:
 // they no longer go through the path together.  A walk over the slots from LDS, edge by edge, took 2.35.
-__device__ __forceinline__ int cut(lds_poly &P, const reg_poly &R, int t, int &len, double x1, double x2, double y1,
+template <int CAP>
+__device__ __forceinline__ int cut(lds_poly<CAP> &P, const reg_poly<CAP> &R, int t, int &len, double x1, double x2, double y1,
                                    double y2, int label, bool &changed)
 {
     const double d1 = y1 - x1, d2 = y2 - x2;
@@ -388,7 +391,7 @@ __device__ __forceinline__ int cut(lds_poly &P, const reg_poly &R, int t, int &l
     const double c = d1 * m1 + d2 * m2;
     unsigned cross = 0, rem = 0;
 #pragma unroll
-    for (int k = 0; k < CAP_SMALL; k++) {
+    for (int k = 0; k < CAP; k++) {
         const double f1 = (d1 * R.v1x[k] + d2 * R.v1y[k]) - c;
         const double f2 = (d1 * R.v2x[k] + d2 * R.v2y[k]) - c;
         const bool p1 = f1 > SIGNUM_EPS, p2 = f2 > SIGNUM_EPS;
@@ -434,7 +437,7 @@ __device__ __forceinline__ int cut(lds_poly &P, const reg_poly &R, int t, int &l
         }
     } while (act != 0);
     if (!(isnan(Y1) && isnan(Y2)) && (X1 != Y1 || X2 != Y2)) {
-        if (len >= CAP_SMALL) return -1;
+        if (len >= CAP) return -1;
         const double cr = (Y1 - X1) * (x2 - X2) - (Y2 - X2) * (x1 - X1);  // cross2(Y - X, x - X)
         if (cr > 0.0) {  // invert(e), src/IO.jl:5-7
             P.v1x[len][t] = Y1; P.v1y[len][t] = Y2; P.v2x[len][t] = X1; P.v2y[len][t] = X2;
@@ -448,7 +451,8 @@ __device__ __forceinline__ int cut(lds_poly &P, const reg_poly &R, int t, int &l
     return 0;
 }
 
-__device__ __forceinline__ void swap_slots(lds_poly &P, int t, int a, int b)
+template <int CAP>
+__device__ __forceinline__ void swap_slots(lds_poly<CAP> &P, int t, int a, int b)
 {
     double tx;
     tx = P.v1x[a][t]; P.v1x[a][t] = P.v1x[b][t]; P.v1x[b][t] = tx;
@@ -472,12 +476,13 @@ __device__ __forceinline__ void path_node(const lv_grid_params &g, const int *__
 }
 
 // one seed's polygon, clipped in P's LDS slots; false when it outgrew them
+template <int CAP>
 __device__ bool clip_seed(const lv_grid_params &g, int n, int i, const double *__restrict__ x,
                           const int *__restrict__ cell_start, const int *__restrict__ cell_labels,
                           const double *__restrict__ cell_x, int m, const int *__restrict__ path_i,
                           const double *__restrict__ path_rr, int *__restrict__ ne, double *__restrict__ ev,
                           int *__restrict__ el, int ld, double *__restrict__ area, double *__restrict__ cent,
-                          int *__restrict__ err, lds_poly &P, int t)
+                          int *__restrict__ err, lds_poly<CAP> &P, int t)
 {
     const double x1 = x[i], x2 = x[n + i];
 
@@ -491,7 +496,7 @@ __device__ bool clip_seed(const lv_grid_params &g, int n, int i, const double *_
         P.v1x[3][t] = Cx; P.v1y[3][t] = Cy; P.v2x[3][t] = Bx; P.v2y[3][t] = By; P.lab[3][t] = -2;
     }
     int len = 4;
-    reg_poly R;
+    reg_poly<CAP> R;
     double prr = load_slots(R, P, t, len, x1, x2);
     int k1, k2;
     lv_findkey(g, x1, x2, k1, k2);
@@ -632,7 +637,8 @@ __device__ __forceinline__ void clip_chunk(int b, int &chunk, int &part)
     part = (b >> 3) & 3;
 }
 
-// every seed with CAP_SMALL slots; the ones that outgrow them go to the queue retry[1..retry[0]]
+// every seed with CAP slots; the ones that outgrow them go to the queue retry[1..retry[0]]
+template <int CAP>
 __global__ __launch_bounds__(CB) void k_clip(lv_grid_params g, int n, const double *__restrict__ x,
                                              const int *__restrict__ cell_start, const int *__restrict__ cell_labels,
                                              const double *__restrict__ cell_x, int m, const int *__restrict__ path_i,
@@ -641,7 +647,7 @@ __global__ __launch_bounds__(CB) void k_clip(lv_grid_params g, int n, const doub
                                              double *__restrict__ area, double *__restrict__ cent,
                                              int *__restrict__ err, int *__restrict__ retry)
 {
-    __shared__ lds_poly P;
+    __shared__ lds_poly<CAP> P;
     __shared__ unsigned char ord[CHUNK];
     const int t = threadIdx.x;
     int chunk, part;
@@ -672,12 +678,17 @@ __global__ __launch_bounds__(GB) void k_clip_group(lv_grid_params g, int n, cons
                         ev, el, ld, area, cent, err, S);
 }
 
-// Up to this many seeds, a group of lanes each.  On lattices of 0.1 dr of jitter clipping takes 35 us with
-// groups and 83 us with a thread per seed (and the queue's launch) at 1,024 seeds, 45 and 100 at 10,000,
-// 109 and 105 at 40,000, 125 and 106 at 48,400; with 0.45 dr of jitter 55 and 141, 125 and 153, 145 and
-// 154: the line lies between where the two cross.  A thread per seed takes 97 us at 65,536 (169 with groups)
-// and 168 at 262,144 (552).
-constexpr int GROUP_MAX = 49152;
+// Up to this many seeds, a group of lanes each.  On lattices of 0.1 dr of jitter clipping takes 34 us with
+// groups and 62 us with a thread per seed (and the queue's launch) at 1,024 seeds, 44 and 71 at 10,000,
+// 78 and 76 at 25,600, 109 and 79 at 40,000; with 0.45 dr of jitter 40 and 97, 54 and 131, 91 and 115, and
+// 105 and 114 at 32,400: the line lies between where the two cross.
+constexpr int GROUP_MAX = 32768;
+
+// Up to this many, a thread per seed with ten slots: a CU holds 6 of its 64-seed blocks (23 KB), all blocks are
+// resident at once and hardly a polygon goes to the queue (70 us for 96 with eight slots at 65,536 seeds,
+// 92 for 117 at 96,100; with 0.45 dr of jitter 113 for 144 and 162 for 169).  Above it the residency counts: 138
+// for 118 at 122,500 and 189 for 168 at 262,144.
+constexpr int WIDE_MAX = 6 * 256 * CB;
 
 }  // namespace
 
@@ -692,7 +703,7 @@ hipError_t lv_launch_clip(const lv_grid_params &g, int n, const double *x, const
     if (!all) {
         hipError_t e = hipMemsetAsync(retry, 0, sizeof(int), s);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_clip, dim3((n + 8 * CHUNK - 1) / (8 * CHUNK) * 32), dim3(CB), 0, s, g, n, x, cell_start, cell_labels, cell_x, m,
+        hipLaunchKernelGGL(n <= WIDE_MAX ? k_clip<10> : k_clip<8>, dim3((n + 8 * CHUNK - 1) / (8 * CHUNK) * 32), dim3(CB), 0, s, g, n, x, cell_start, cell_labels, cell_x, m,
                            path_i, path_rr, ne, ev, el, ld, area, cent, err, retry);
     }
     hipLaunchKernelGGL(k_clip_group, dim3(all ? groups : std::min(RETRY_BLOCKS, groups)), dim3(GB), 0, s, g, n, x,

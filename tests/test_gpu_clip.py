@@ -1,6 +1,6 @@
-"""The two ways clipping runs (a group of lanes per seed up to 49152 seeds and for polygons that outgrow eight
-slots, a thread per seed above): mesh bit for bit the oracle's on either side of the line, on regular,
-strongly jittered and random seeds."""
+"""The ways clipping runs (a group of lanes per seed up to 32768 seeds and for polygons that outgrow a thread's
+slots; a thread per seed above, with ten slots up to 98304 seeds and eight beyond): mesh bit for bit the oracle's on
+either side of the lines, on regular, strongly jittered and random seeds."""
 import numpy as np
 import pytest
 
@@ -58,3 +58,12 @@ def test_mesh_of_uneven_chunks_bit_exact(lv, oracle, gpu, n, seed):
     print("clip chunks %d" % n, flush=True)
     x = np.random.default_rng(seed).random(2 * n)
     _same_mesh(lv, oracle, x, 0.5 / np.sqrt(n), True, r_max=9.0 / np.sqrt(n))
+
+
+@pytest.mark.parametrize("periodic", [True, False])
+@pytest.mark.parametrize("K", [181, 182, 313, 314])
+def test_mesh_at_the_lines_between_the_ways(lv, oracle, gpu, K, periodic):
+    print("clip line %d" % K, flush=True)
+    x = lv.inputs.jittered_lattice(K, K, 1.0 / K, jitter=0.45, seed=0x5EED0B80 + K)
+    grid = _same_mesh(lv, oracle, x, 1.0 / K, periodic)
+    assert (grid.n <= 32768) == (K == 181) and (grid.n <= 98304) == (K < 314)
