@@ -2343,7 +2343,7 @@ hipError_t lv_amg_vcycle(const lv_amg *G, const lv_pressure_system &A, const flo
     return vcycle(G, fine_own(G, A), (const int *)G->agg, (const int *)G->list, r, z, Prr, S, s, false, nullptr);
 }
 
-// The test in the down pass adds 0.5 us to it at 65,536 and 265,225 rows and 1.0 at 1,000,000, for a launch of 2.6 us
+// The test in the down pass adds 0.5 us to it at 131,072 and 265,225 rows and 1.0 at 1,000,000, for a launch of 2.6 us
 // and its gap; at 4,194,304 rows 8.2 for a launch of 4.8.  The line (2 M rows) lies between, in what the workgroups
 // read together.
 static constexpr int64_t HEAD_MAX = 1ll << 21;

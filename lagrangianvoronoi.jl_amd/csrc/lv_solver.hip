@@ -1006,11 +1006,15 @@ __global__ __launch_bounds__(B) void k_correct(int n, double *__restrict__ x, co
 // Below PS_MAX_ROWS rows the two launches of an iteration are all latency (5.0 + 3.6 us at 10,000 rows, and
 // the host's turn between them: 11.8 us an iteration), so one launch runs the whole solve: a thread owns a
 // row and keeps its couplings, x, r, p and q in registers, and what an iteration exchanges, z and two
-// reductions, goes through memory between workgroups that are all resident: 5.0 us an iteration.
+// reductions, goes through memory between workgroups that are all resident: 3.7 us an iteration.
 //
 // The exchange: each workgroup publishes its partial sums with agent-scope stores, which are written
 // through to where every XCD sees them, into slots that hold a sentinel until then, and each of its threads
-// polls one workgroup's slots (ps_sum): the reduction is its own barrier.  Four sets of slots rotate; at
+// polls one workgroup's slots (ps_sum): the reduction is its own barrier.  Every set exists PS_COPIES times, and
+// a workgroup publishes in all and polls the copy of its XCD (workgroups go round the XCDs): with one set the
+// polls of all workgroups queue up at the same few lines, behind which the stores wait (4.8 us an iteration at
+// 10,000 rows, 5.5 at 32,400, 7.1 at 65,536; eight copies 3.7, 4.3 and 5.5, 4 copies 3.9, 4.6 and 5.6, 16 copies
+// 3.8, 4.5 and 6.2; one a workgroup 3.8, 7.3 and 15).  Four sets of slots rotate; at
 // sync j a workgroup puts the sentinel back into what it published at sync j - 2, which every workgroup has
 // read by then (it had to, to publish j - 1, which this one has seen); that store is complete when ps_sum
 // returns (s_waitcnt after the poll), so before this workgroup publishes j + 1, and so before anyone polls that
@@ -1031,7 +1035,10 @@ __global__ __launch_bounds__(B) void k_correct(int n, double *__restrict__ x, co
 // Rows, partial sums and their order are those of k_means, k_cg64_init, k_cg_s, k_cg_u, k_sum1, k_shift and
 // k_resid64 with one workgroup per 256 rows, so the iterates are the same bit for bit.
 constexpr int PS_MAX_ROWS = 256 * B;
-constexpr int PS_SLOTS = 4 * 3 * 256;                       // sets, values, workgroups
+constexpr int PS_COPIES = 8;
+constexpr int PS_COPY = 3 * 256;                            // values, workgroups
+constexpr int PS_SET = PS_COPIES * PS_COPY;
+constexpr int PS_SLOTS = 4 * PS_SET;
 constexpr unsigned long long PS_EMPTY = 0x7FF8A5C3DEADBEEFull;  // a NaN no arithmetic produces by itself
 constexpr unsigned long long PS_WAIT = 2000000;             // 20 ms of the 100 MHz clock
 enum { PS_OK = 0, PS_GAVE_UP = 2 };
@@ -1079,18 +1086,19 @@ __device__ __forceinline__ bool ps_sum(ps_state &Q, const double (&v)[NV], int a
     if (t == 0) late[lp] = 0;
     if (HARD) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    double *set = Q.slots + (size_t)(Q.sync & 3) * 3 * 256;
-    if (t == 0) {
-        double *old = Q.slots + (size_t)((Q.sync + 2) & 3) * 3 * 256;
+    double *set = Q.slots + (Q.sync & 3) * PS_SET;
+    if (t < PS_COPIES) {
+        double *old = Q.slots + ((Q.sync + 2) & 3) * PS_SET + t * PS_COPY;
         if (Q.sync >= 2)
             for (int q = 0; q < 3; q++) ps_store(old + q * 256 + Q.at2, __longlong_as_double((long long)PS_EMPTY));
 #pragma unroll
         for (int q = 0; q < NV; q++) {
             double s = 0.0;
             for (int k = 0; k < B / 64; k++) s += sm[q][k];
-            ps_store(set + q * 256 + at, ps_value(s));
+            ps_store(set + t * PS_COPY + q * 256 + at, ps_value(s));
         }
     }
+    set += (blockIdx.x & (PS_COPIES - 1)) * PS_COPY;
     Q.at2 = Q.at1;
     Q.at1 = at;
     Q.sync++;
@@ -1376,7 +1384,7 @@ __global__ __launch_bounds__(B) void k_normalise(int n, float *__restrict__ y, c
 
 // The Picard window's vector work (lv_find_pressure), each kernel one pass over what it reads: bound by
 // bytes at millions of rows, by launches below some 10^5.  A kernel for each combination and for each set of dots
-// took twice the launches (14 a Picard iteration, now 7) and read the temporaries again for each (a step of 65,536
+// took twice the launches (14 a Picard iteration, now 7) and read the temporaries again for each (a step of 131,072
 // particles 4.62 -> 4.40 ms, of 4,194,304 53.0 -> 52.8).
 // Q, Z: the window's directions, unused ones any valid pointer.  Sums are left as partials, k_multidot_fin's.
 struct lv_dirs8 {
