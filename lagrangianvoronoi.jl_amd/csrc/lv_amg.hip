@@ -1546,47 +1546,99 @@ __global__ __launch_bounds__(TB) void k_tail_lds(tail_lds_args T, const lv_cg_sc
 }
 
 // The matrix of level L from that of the next level (nc cells, leading dimension ldc): row j is the
-// V-visit of the unit vector of cell j = blockIdx.x, one workgroup each.  The right-hand side it leaves the
-// next level has a handful of entries, so that level's correction is a sum of as many rows of its matrix.
-// At 50 x 50 cells (level 1 of 100^2 particles) it takes 99 us once per set-up and the product 5.1 us, against
-// the 11 us of the two stencil launches, the product and the prolongation that it replaces in each cycle.
+// V-visit of the unit vector of cell j, EXT_ROWS to a workgroup, which loads each cell's couplings once
+// for all of them.  The right-hand side a unit vector leaves the next level has a handful of entries, at the parents of
+// its 3 x 3 neighbourhood, so that level's correction is a sum of as many rows of its matrix.  At 50 x 50
+// cells (level 1 of 100^2 particles) it takes 41 us once per set-up (99 with a row a workgroup and the whole down
+// pass for each) and the product 5.1 us, against the 11 us of the two stencil launches, the product and
+// the prolongation that it replaces in each cycle.
+constexpr int EXT_ROWS = 4;
 __global__ __launch_bounds__(B) void k_mat_extend(st_level L, int Kyc, int nc, const float *__restrict__ matc, int ldc,
                                                   float *__restrict__ mat, int ld)
 {
-    __shared__ float r[MAT_MAX], z[MAT_MAX], rc[TAIL_MAX], ec[TAIL_MAX];
-    __shared__ int nz[TAIL_MAX], cnt;
-    const int n = L.Kx * L.Ky;
-    for (int f = threadIdx.x; f < n; f += B) r[f] = f == (int)blockIdx.x ? 1.0f : 0.0f;
-    __syncthreads();
-    for (int base = 0; base < nc * CF2; base += B) {  // uniform trip count: every lane shuffles
-        const int tid = base + threadIdx.x;
-        const int P = tid / CF2, q = tid % CF2;
-        const float t = sum_children(st_down_lane(L, Kyc, nc, P, q, r, z));
-        if (q == 0 && P < nc) rc[P] = t;
-    }
-    __syncthreads();
-    if (threadIdx.x < 64) {  // its nonzero entries in order
-        int m = 0;
-        for (int base = 0; base < nc; base += 64) {
-            const int P = base + threadIdx.x;
-            const bool on = P < nc && rc[P] != 0.0f;
-            const unsigned long long b = __ballot(on);
-            if (on) nz[m + __popcll(b & ((1ull << threadIdx.x) - 1ull))] = P;
-            m += __popcll(b);
+    __shared__ float ec[EXT_ROWS][TAIL_MAX], cv[EXT_ROWS][9], rv[EXT_ROWS][9];
+    __shared__ int cp[EXT_ROWS][9], rp[EXT_ROWS][9], rcnt[EXT_ROWS];
+    const int n = L.Kx * L.Ky, R0 = blockIdx.x * EXT_ROWS, t = threadIdx.x;
+    static_assert(EXT_ROWS * 9 * CF2 <= B, "a lane a child");
+    {  // the parents of the unit cell's 3 x 3 neighbourhood, a lane for each of their children
+        const int k = min(t / (9 * CF2), EXT_ROWS - 1), c9 = t / CF2 % 9, q = t % CF2;
+        const int R = min(R0 + k, n - 1), cx = R / L.Ky, cy = R - cx * L.Ky;
+        bool okx, oky;
+        const int jx = wrap_near(cx + c9 / 3 - 1, L.Kx, L.xper, okx), jy = wrap_near(cy + c9 % 3 - 1, L.Ky, L.yper, oky);
+        const int P = okx && oky ? (jx / CF) * Kyc + jy / CF : nc;
+        const int Px = P / Kyc, x = CF * Px + q / CF, y = CF * (P - Px * Kyc) + q % CF;
+        float v = 0.0f;
+        if (P < nc && x < L.Kx && y < L.Ky) {  // as st_down_lane
+            const int f = x * L.Ky + y;
+            float ck[8];
+            int J[8];
+            st_nbrs(L, x, y, f, ck, J);
+            const float rf = f == R ? 1.0f : 0.0f, zf = OMEGA * L.dinv[f] * rf;
+            float acc = L.d[f] * zf;
+#pragma unroll
+            for (int m = 0; m < 8; m++) acc += ck[m] * (zf - OMEGA * L.dinv[J[m]] * (J[m] == R ? 1.0f : 0.0f));
+            v = rf - acc;
         }
-        if (threadIdx.x == 0) cnt = m;
+        v = sum_children(v);
+        if (q == 0 && t < EXT_ROWS * 9 * CF2) {
+            cp[k][c9] = P;
+            cv[k][c9] = v;
+        }
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < nc; i += B) {
-        float a = 0.0f;
-        for (int q = 0; q < cnt; q++) a += rc[nz[q]] * matc[(size_t)nz[q] * ldc + i];
-        ec[i] = a;
+    if (t < EXT_ROWS) {  // the nonzero ones in order, each once
+        int m = 0;
+        for (int last = -1;; m++) {
+            int best = nc, at = 0;
+            for (int q = 0; q < 9; q++)
+                if (cp[t][q] > last && cp[t][q] < best && cv[t][q] != 0.0f) {
+                    best = cp[t][q];
+                    at = q;
+                }
+            if (best == nc) break;
+            rp[t][m] = best;
+            rv[t][m] = cv[t][at];
+            last = best;
+        }
+        rcnt[t] = m;
     }
     __syncthreads();
-    float *row = mat + (size_t)blockIdx.x * ld;
-    for (int f = threadIdx.x; f < ld; f += B) {
-        if (f < n) st_up_cell(L, Kyc, f, r, z, ec, row);
-        else row[f] = 0.0f;
+    for (int i = t; i < nc; i += B)
+#pragma unroll
+        for (int k = 0; k < EXT_ROWS; k++) {
+            float a = 0.0f;
+            for (int q = 0; q < rcnt[k]; q++) a += rv[k][q] * matc[(size_t)rp[k][q] * ldc + i];
+            ec[k][i] = a;
+        }
+    __syncthreads();
+    float zr[EXT_ROWS];
+#pragma unroll
+    for (int k = 0; k < EXT_ROWS; k++) zr[k] = OMEGA * L.dinv[min(R0 + k, n - 1)] * 1.0f;
+    for (int f = t; f < ld; f += B) {  // as st_up_cell
+        float ck[8], d = 0.0f, di = 0.0f;
+        int J[8], PJ[8], Pf = 0;
+        if (f < n) {
+            const int cx = f / L.Ky, cy = f - cx * L.Ky;
+            st_nbrs(L, cx, cy, f, ck, J, PJ, Kyc);
+            Pf = (cx / CF) * Kyc + cy / CF;
+            d = L.d[f];
+            di = L.dinv[f];
+        }
+#pragma unroll
+        for (int k = 0; k < EXT_ROWS; k++) {
+            const int R = R0 + k;
+            if (R >= n) break;
+            float v = 0.0f;
+            if (f < n) {
+                const float z1 = (f == R ? zr[k] : 0.0f) + L.alpha * ec[k][Pf];
+                float acc = d * z1;
+#pragma unroll
+                for (int m = 0; m < 8; m++)
+                    acc += ck[m] * (z1 - ((J[m] == R ? zr[k] : 0.0f) + L.alpha * ec[k][PJ[m]]));
+                v = z1 + OMEGA * di * ((f == R ? 1.0f : 0.0f) - acc);
+            }
+            mat[(size_t)R * ld + f] = v;
+        }
     }
 }
 
@@ -2185,7 +2237,7 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
         if (G->lmat < lk) {
             const lv_amg_level &L = G->lev[G->lmat];
             AMG_CHECK(grow(&G->ext_mat, &G->cap_ext_mat, (size_t)L.n * G->mat_ld));
-            hipLaunchKernelGGL(k_mat_extend, dim3(L.n), dim3(B), 0, s,
+            hipLaunchKernelGGL(k_mat_extend, dim3((L.n + EXT_ROWS - 1) / EXT_ROWS), dim3(B), 0, s,
                                st_level{L.Kx, L.Ky, G->xper, G->yper, L.d, L.c, L.dinv, L.alpha}, G->lev[lk].Ky, nt,
                                (const float *)G->tail_mat, ldt, G->ext_mat, G->mat_ld);
             G->mat = G->ext_mat;
