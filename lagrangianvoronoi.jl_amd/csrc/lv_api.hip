@@ -1420,12 +1420,12 @@ static int ensure_picard_window(lv_ctx *ctx, int w)
 // component left enters as a zero direction, which adds nothing to later projections.
 
 // The direction in pw_t1 with its image A pw_t1 in pw_t2 made orthogonal to the set (Q, Z) of at most w, and
-// a place for it made at the set's end: it is still to be scaled into it.  pw_dots holds <q_k, pw_t2>,
+// a place for it made at the set's end: it is still to be scaled into it.  D holds <q_k, pw_t2>,
 // or |pw_t2|^2 of an empty set, and is left with |pw_t2|^2.
-static int picard_orthogonalise(lv_ctx *ctx, float **Q, float **Z, int w, int *cnt)
+static int picard_orthogonalise(lv_ctx *ctx, lv_dots &D, float **Q, float **Z, int w, int *cnt)
 {
     if (*cnt > 0)
-        LV_HIP_CHECK(lv_pw_out(ctx->n, ctx->pw_t1, ctx->pw_t2, Q, Z, *cnt, ctx->W.partials, ctx->pw_dots, ctx->s));
+        LV_HIP_CHECK(lv_pw_out(ctx->n, ctx->pw_t1, ctx->pw_t2, Q, Z, *cnt, D, ctx->s));
     if (*cnt == w) {  // drop the oldest direction
         float *q0 = Q[0], *z0 = Z[0];
         for (int k = 1; k < w; k++) {
@@ -1445,14 +1445,15 @@ static int picard_add_carried(lv_ctx *ctx, const double *z, float **Q, float **Z
 {
     const int n = ctx->n;
     hipStream_t s = ctx->s;
+    lv_dots D = lv_dots_in(ctx->W.partials, ctx->pw_dots);
     LV_HIP_CHECK(hipMemcpyAsync(ctx->pw_t1, z, sizeof(double) * n, hipMemcpyDeviceToDevice, s));
     LV_HIP_CHECK(lv_spmv64(ctx->A, n, z, ctx->pw_t2, s));
-    if (*cnt > 0) LV_HIP_CHECK(lv_dot_device(n, Q[0], ctx->pw_t2, ctx->W.partials, ctx->pw_dots, s));
-    else LV_HIP_CHECK(lv_dot_device(n, ctx->pw_t2, ctx->pw_t2, ctx->W.partials, ctx->pw_dots, s));
-    int rc = picard_orthogonalise(ctx, Q, Z, 2, cnt);
+    if (*cnt > 0) LV_HIP_CHECK(lv_dot_device(n, Q[0], ctx->pw_t2, D, s));
+    else LV_HIP_CHECK(lv_dot_device(n, ctx->pw_t2, ctx->pw_t2, D, s));
+    int rc = picard_orthogonalise(ctx, D, Q, Z, 2, cnt);
     if (rc) return rc;
-    LV_HIP_CHECK(lv_normalise(n, Q[*cnt - 1], ctx->pw_t2, ctx->pw_dots, s));
-    LV_HIP_CHECK(lv_normalise(n, Z[*cnt - 1], ctx->pw_t1, ctx->pw_dots, s));
+    LV_HIP_CHECK(lv_normalise(n, Q[*cnt - 1], ctx->pw_t2, D, s));
+    LV_HIP_CHECK(lv_normalise(n, Z[*cnt - 1], ctx->pw_t1, D, s));
     return LV_OK;
 }
 
@@ -1525,26 +1526,26 @@ int lv_find_pressure(lv_ctx *ctx, double dt, int32_t niter, const lv_solve_opts 
         // window's q's; then the same with the carried directions and what is left of r
         if (w > 0 && have >= 1) {
             const int n = ctx->n;
-            double *part = ctx->W.partials, *dots = ctx->pw_dots, *t1 = ctx->pw_t1, *t2 = ctx->pw_t2;
+            double *t1 = ctx->pw_t1, *t2 = ctx->pw_t2;
+            lv_dots D = lv_dots_in(ctx->W.partials, ctx->pw_dots);
             float *const *none = nullptr;
             const bool use_carried = ccnt > 0 && it <= 4;
             if (have >= 2) {
                 // the corrections P_2 - P_1 and P_3 - P_2, recorded for the next call
                 double *rec = carry && (it == 3 || it == 4) ? ctx->pc_new[it - 3] : nullptr;
                 LV_HIP_CHECK(lv_pw_enter(n, ctx->pw_P[0], ctx->pw_P[1], ctx->pw_AP[0], ctx->pw_AP[1], t1, rec, t2,
-                                         ctx->pw_q, cnt, part, dots, ctx->s));
-                rc = picard_orthogonalise(ctx, ctx->pw_q, ctx->pw_z, w, &cnt);
+                                         ctx->pw_q, cnt, D, ctx->s));
+                rc = picard_orthogonalise(ctx, D, ctx->pw_q, ctx->pw_z, w, &cnt);
                 if (rc) return rc;
-                LV_HIP_CHECK(lv_pw_resid(n, t1, t2, ctx->pw_q, ctx->pw_z[cnt - 1], cnt, ctx->b, ctx->pw_AP[0], part,
-                                         dots, ctx->s));
+                LV_HIP_CHECK(lv_pw_resid(n, t1, t2, ctx->pw_q, ctx->pw_z[cnt - 1], cnt, ctx->b, ctx->pw_AP[0], D, ctx->s));
                 LV_HIP_CHECK(lv_pw_guess(n, ctx->P0, t2, ctx->pw_q, ctx->pw_z, cnt, ctx->pc_q, use_carried ? ccnt : 0,
-                                         part, dots, ctx->s));
+                                         D, ctx->s));
             } else if (use_carried) {
-                LV_HIP_CHECK(lv_pw_resid(n, t1, t2, ctx->pc_q, nullptr, ccnt, ctx->b, ctx->pw_AP[0], part, dots,
+                LV_HIP_CHECK(lv_pw_resid(n, t1, t2, ctx->pc_q, nullptr, ccnt, ctx->b, ctx->pw_AP[0], D,
                                          ctx->s));
             }
             if (use_carried)
-                LV_HIP_CHECK(lv_pw_guess(n, ctx->P0, t2, ctx->pc_q, ctx->pc_o, ccnt, none, 0, part, dots, ctx->s));
+                LV_HIP_CHECK(lv_pw_guess(n, ctx->P0, t2, ctx->pc_q, ctx->pc_o, ccnt, none, 0, D, ctx->s));
         }
         rc = solve_on_device(ctx, ctx->b, ctx->P0, o, stats);
         if (rc == LV_E_NOT_CONVERGED) status = rc;

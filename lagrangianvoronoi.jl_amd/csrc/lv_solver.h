@@ -131,23 +131,30 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
 
 // Picard extrapolation helpers (vectors of length n on stream s; the window's stored directions
 // are FP32, everything else FP64; sums in FP64)
-// dots[0] = a . b, on the device
-hipError_t lv_dot_device(int n, const float *a, const double *b, double *partials, double *dots, hipStream_t s);
-hipError_t lv_dot_device(int n, const double *a, const double *b, double *partials, double *dots, hipStream_t s);
-// y = x / sqrt(*h) (0 unless *h is positive and finite)
-hipError_t lv_normalise(int n, float *y, const double *x, const double *h, hipStream_t s);
-// The Picard window (lv_find_pressure), m directions Q (images) and Z; dots: 8 device doubles.
+// Dots between the kernels below, on the device: what one leaves, the next reads, as partials of nb blocks or
+// (nb = 0) summed.  The kernel that reads some leaves its own in the other half of the work space.
+struct lv_dots {
+    const double *src;  // to be read
+    int nb;
+    double *half[2], *out, *fin;  // the halves, the one to be written, room for summed ones
+};
+lv_dots lv_dots_in(double *partials, double *fin);
+// dots[0] = a . b
+hipError_t lv_dot_device(int n, const float *a, const double *b, lv_dots &D, hipStream_t s);
+hipError_t lv_dot_device(int n, const double *a, const double *b, lv_dots &D, hipStream_t s);
+// y = x / sqrt(dots[0]) (0 unless that is positive and finite)
+hipError_t lv_normalise(int n, float *y, const double *x, const lv_dots &D, hipStream_t s);
+// The Picard window (lv_find_pressure), m directions Q (images) and Z.
 // t1 = Pc - Pp (rec, if given, a copy), t2 = APc - APp; dots[q] = Q_q . t2, or with m = 0 dots[0] = t2 . t2
 hipError_t lv_pw_enter(int n, const double *Pc, const double *Pp, const double *APc, const double *APp, double *t1,
-                       double *rec, double *t2, float *const *Q, int m, double *partials, double *dots, hipStream_t s);
+                       double *rec, double *t2, float *const *Q, int m, lv_dots &D, hipStream_t s);
 // (t2, t1) -= sum_q dots[q] (Q_q, Z_q); dots[0] = t2 . t2
-hipError_t lv_pw_out(int n, double *t1, double *t2, float *const *Q, float *const *Z, int m, double *partials,
-                     double *dots, hipStream_t s);
+hipError_t lv_pw_out(int n, double *t1, double *t2, float *const *Q, float *const *Z, int m, lv_dots &D, hipStream_t s);
 // with znew first (Q_{m-1}, znew) = (t2, t1) / sqrt(dots[0]); t2 = b - AP, dots[q] = Q_q . t2
 hipError_t lv_pw_resid(int n, const double *t1, double *t2, float *const *Q, float *znew, int m, const double *b,
-                       const double *AP, double *partials, double *dots, hipStream_t s);
+                       const double *AP, lv_dots &D, hipStream_t s);
 // P0 += sum_q dots[q] Z_q; with no > 0 (at most 2) also t2 -= sum_q dots[q] Q_q, dots[q] = O_q . t2, q < no
 hipError_t lv_pw_guess(int n, double *P0, double *t2, float *const *Q, float *const *Z, int m, float *const *O, int no,
-                       double *partials, double *dots, hipStream_t s);
+                       lv_dots &D, hipStream_t s);
 // y = A x in FP64
 hipError_t lv_spmv64(const lv_pressure_system &A, int n, const double *x, double *y, hipStream_t s);

@@ -441,9 +441,12 @@ __global__ __launch_bounds__(B) void k_write_P(lv_fields F, int n, const double 
 }
 
 // S as a solve starts from it
-__device__ __forceinline__ void init_scalars(lv_cg_scalars *S, double tol2, int itmax, int singular)
+__device__ __forceinline__ void init_scalars(lv_cg_scalars *S, double tol2, int itmax, int singular, double bmean = 0.0,
+                                             double xmean0 = 0.0)
 {
     lv_cg_scalars z = {};
+    z.bmean = bmean;
+    z.xmean0 = xmean0;
     z.tol2 = tol2;
     z.itmax = itmax;
     z.singular = singular;
@@ -518,12 +521,12 @@ __global__ __launch_bounds__(B) void k_finalize2(const double *__restrict__ Prr,
 __global__ __launch_bounds__(B) void k_means(int n, const double *__restrict__ b, const double *__restrict__ x,
                                              double *__restrict__ partials)
 {
-    double v[3] = {0.0, 0.0, 0.0};
+    double v[2] = {0.0, 0.0};
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
         v[0] += b[i];
         v[1] += x[i];
     }
-    block_partials<3>(v, partials, gridDim.x);
+    block_partials<2>(v, partials, gridDim.x);
 }
 
 // (A x)_i in the reference's difference form, from the slot-major ELL copy.  The first 8 slots are
@@ -870,16 +873,28 @@ __device__ __forceinline__ double spmv_row_shifted(int i, int n, const lv_ell_ow
 
 // true residual r = (b - bmean) - A x; partials |r|^2, |b'|^2 (FP64).  With Pxs (the partial sums
 // of x written by k_correct, singular systems) the residual is that of x - d, d = mean(x) - xmean0,
-// the x that k_shift stores at the end of the solve; block 0 records d.  Of S, bmean is read in
-// singular systems only.
+// the x that k_shift stores at the end of the solve; block 0 records d.  With Pm (the first residual of a
+// singular system; k_means' partials) block 0 also records the means of b and of the guess.  Of S, bmean
+// is read in singular systems only.
 template <bool COMPACT, class V = lv_ell_own<double>>
 __global__ __launch_bounds__(B) void k_resid64(int n, V A, const double *__restrict__ diag,
                                                const double *__restrict__ b, const double *__restrict__ x,
                                                double *__restrict__ r, double *__restrict__ partials,
-                                               const double *__restrict__ Pxs, lv_cg_scalars *S, int singular)
+                                               const double *__restrict__ Pxs, const double *__restrict__ Pm,
+                                               lv_cg_scalars *S, int singular)
 {
-    const double bmean = singular ? S->bmean : 0.0;
-    double d = 0.0;
+    double bmean = 0.0, d = 0.0;
+    if (Pm) {
+        double t[2];
+        reduce_all<2>(Pm, gridDim.x, t);
+        bmean = t[0] / n;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            S->bmean = bmean;
+            S->xmean0 = t[1] / n;
+        }
+    } else if (singular) {
+        bmean = S->bmean;
+    }
     if (Pxs) {
         double t[1];
         reduce_all<1>(Pxs, gridDim.x, t);
@@ -933,7 +948,7 @@ __device__ inline bool sweep_skipped(const lv_cg_scalars *S, int first) { return
 // multilevel cycle's pre-smoothed correction).  F.first: this is the solve's first sweep.  Then the tests
 // on the initial residual that the host makes between sweeps are made here, by every block for itself
 // from the partials of the FP64 residual (F.part), and block 0 records them with what the
-// solve starts from (in a singular system FIN_MEANS did, with the means).
+// solve starts from (in a singular system the means are in S already).
 struct first_sweep {
     const double *part;
     double tol2, floor_tol;  // floor_tol: the per-sweep floor of the inner tolerance
@@ -954,7 +969,7 @@ __global__ __launch_bounds__(B) void k_cg32_init(int n, const double *__restrict
         const double thr2 = F.tol2 * o[1];
         skip = rr <= thr2 || !(rr == rr);
         if (blockIdx.x == 0 && threadIdx.x == 0) {
-            if (!F.singular) init_scalars(S, F.tol2, F.itmax, 0);
+            init_scalars(S, F.tol2, F.itmax, F.singular, F.singular ? S->bmean : 0.0, F.singular ? S->xmean0 : 0.0);
             S->rr64 = rr;
             S->rr64_0 = rr;
             S->bb = o[1];
@@ -1349,6 +1364,37 @@ __global__ __launch_bounds__(B, 4) void k_pcg_small(int n, lv_ell_own<double> A,
 
 // ---- Picard extrapolation: the stored directions are FP32, everything is accumulated in FP64 ----------
 
+// The dots a kernel reads: summed here from the partials of nb blocks (the sums and order of reduce_all), or
+// with nb = 0 already summed (k_dots_fin)
+constexpr int FEW_BLOCKS = B;
+template <int NV>
+__device__ __forceinline__ void load_dots(const double *__restrict__ src, int nb, double (&out)[NV])
+{
+    if (nb == 0) {
+#pragma unroll
+        for (int q = 0; q < NV; q++) out[q] = src[q];
+        return;
+    }
+    __shared__ double sm[NV][B / 64];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    double p[NV];
+#pragma unroll
+    for (int q = 0; q < NV; q++) p[q] = src[(size_t)q * nb + (t < nb ? t : nb - 1)];
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        const double s = lv_wave_sum(t < nb ? 0.0 + p[q] : 0.0);
+        if (lane == 0) sm[q][w] = s;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < NV; q++) {
+        double t = 0.0;
+        for (int k = 0; k < B / 64; k++) t += sm[q][k];
+        out[q] = t;
+    }
+    __syncthreads();
+}
+
 // partials of a . b
 template <typename TA>
 __global__ __launch_bounds__(B) void k_dot(int n, const TA *__restrict__ a, const double *__restrict__ b,
@@ -1360,7 +1406,7 @@ __global__ __launch_bounds__(B) void k_dot(int n, const TA *__restrict__ a, cons
 }
 
 // a block per dot product (one block for all eight took 4.7 us)
-__global__ __launch_bounds__(B) void k_multidot_fin(const double *__restrict__ partials, int nb,
+__global__ __launch_bounds__(B) void k_dots_fin(const double *__restrict__ partials, int nb,
                                                     double *__restrict__ out)
 {
     double o[1];
@@ -1374,11 +1420,13 @@ __device__ __forceinline__ double inv_norm(double h)
     return (h > 0.0 && h <= 1.7976931348623157e308) ? 1.0 / sqrt(h) : 0.0;
 }
 
-// y = x / sqrt(*h), rounded once
+// y = x / sqrt(dots[0]), rounded once
 __global__ __launch_bounds__(B) void k_normalise(int n, float *__restrict__ y, const double *__restrict__ x,
-                                                 const double *__restrict__ h)
+                                                 const double *__restrict__ dots, int dnb)
 {
-    const double f = inv_norm(*h);
+    double h[1];
+    load_dots<1>(dots, dnb, h);
+    const double f = inv_norm(h[0]);
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) y[i] = (float)(0.0 + f * x[i]);
 }
 
@@ -1386,7 +1434,9 @@ __global__ __launch_bounds__(B) void k_normalise(int n, float *__restrict__ y, c
 // bytes at millions of rows, by launches below some 10^5.  A kernel for each combination and for each set of dots
 // took twice the launches (14 a Picard iteration, now 7) and read the temporaries again for each (a step of 131,072
 // particles 4.62 -> 4.40 ms, of 4,194,304 53.0 -> 52.8).
-// Q, Z: the window's directions, unused ones any valid pointer.  Sums are left as partials, k_multidot_fin's.
+// Q, Z: the window's directions, unused ones any valid pointer.  Sums are left as partials, which the next
+// kernel sums for itself up to FEW_BLOCKS blocks (1 us there for a launch of 2.4 and its gap; at 512 blocks no
+// gain any more) and k_dots_fin above.
 struct lv_dirs8 {
     float *v[8];
 };
@@ -1418,12 +1468,13 @@ __global__ __launch_bounds__(B) void k_pw_enter(int n, const double *__restrict_
 // t2 -= sum_q dots[q] Q_q, t1 -= sum_q dots[q] Z_q; the sum of t2 . t2
 template <int M>
 __global__ __launch_bounds__(B) void k_pw_out(int n, double *__restrict__ t1, double *__restrict__ t2, lv_dirs8 Q,
-                                              lv_dirs8 Z, const double *__restrict__ dots,
+                                              lv_dirs8 Z, const double *__restrict__ dots, int dnb,
                                               double *__restrict__ partials)
 {
     double c[M];
+    load_dots<M>(dots, dnb, c);
 #pragma unroll
-    for (int q = 0; q < M; q++) c[q] = -dots[q];
+    for (int q = 0; q < M; q++) c[q] = -c[q];
     double v[1] = {0.0};
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
         double y = t2[i], a = t1[i];
@@ -1444,11 +1495,15 @@ __global__ __launch_bounds__(B) void k_pw_out(int n, double *__restrict__ t1, do
 template <int M, bool STORE>
 __global__ __launch_bounds__(B) void k_pw_resid(int n, const double *__restrict__ t1, double *__restrict__ t2,
                                                 lv_dirs8 Q, float *__restrict__ znew, const double *__restrict__ dots,
-                                                const double *__restrict__ b, const double *__restrict__ AP,
+                                                int dnb, const double *__restrict__ b, const double *__restrict__ AP,
                                                 double *__restrict__ partials)
 {
     double f = 0.0;
-    if (STORE) f = inv_norm(dots[0]);
+    if (STORE) {
+        double h[1];
+        load_dots<1>(dots, dnb, h);
+        f = inv_norm(h[0]);
+    }
     double v[M] = {};
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
         float qn = 0.0f;
@@ -1469,12 +1524,11 @@ __global__ __launch_bounds__(B) void k_pw_resid(int n, const double *__restrict_
 template <int M, bool KEEP>
 __global__ __launch_bounds__(B) void k_pw_guess(int n, double *__restrict__ P0, double *__restrict__ t2, lv_dirs8 Q,
                                                 lv_dirs8 Z, const float *__restrict__ O0,
-                                                const float *__restrict__ O1, const double *__restrict__ dots,
+                                                const float *__restrict__ O1, const double *__restrict__ dots, int dnb,
                                                 double *__restrict__ partials)
 {
     double c[M];
-#pragma unroll
-    for (int q = 0; q < M; q++) c[q] = dots[q];
+    load_dots<M>(dots, dnb, c);
     double v[2] = {0.0, 0.0};
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
         double p = P0[i];
@@ -1666,20 +1720,21 @@ static lv_ell_own<float> own32(const lv_pressure_system &A, int n, int layout = 
 // columns when every offset fits (2 bytes a slot and 1 a row instead of 4 and 4)
 template <class V>
 static void launch_resid64_v(const V &Av, dim3 G, hipStream_t s, int n, const double *diag, const double *b,
-                             const double *x, double *r, double *p3, const double *Pxs, lv_cg_scalars *S, int singular)
+                             const double *x, double *r, double *p3, const double *Pxs, const double *Pm, lv_cg_scalars *S,
+                             int singular)
 {
     if (Av.ocap > 0)
-        hipLaunchKernelGGL((k_resid64<true, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, S, singular);
+        hipLaunchKernelGGL((k_resid64<true, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, Pm, S, singular);
     else
-        hipLaunchKernelGGL((k_resid64<false, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, S, singular);
+        hipLaunchKernelGGL((k_resid64<false, V>), G, dim3(B), 0, s, n, Av, diag, b, x, r, p3, Pxs, Pm, S, singular);
 }
 static void launch_resid64(const lv_pressure_system &A, int layout, dim3 G, hipStream_t s, int n, const double *b,
-                           const double *x, double *r, double *p3, const double *Pxs, lv_cg_scalars *S)
+                           const double *x, double *r, double *p3, const double *Pxs, const double *Pm, lv_cg_scalars *S)
 {
     if (A.narrow)
-        launch_resid64_v(own64s(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, S, (int)A.singular);
+        launch_resid64_v(own64s(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, Pm, S, (int)A.singular);
     else
-        launch_resid64_v(own64(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, S, (int)A.singular);
+        launch_resid64_v(own64(A, n, layout), G, s, n, (const double *)A.diag64, b, x, r, p3, Pxs, Pm, S, (int)A.singular);
 }
 template <class V>
 static void launch_spmv64_v(const V &Av, dim3 G, hipStream_t s, int n, const double *diag, const double *x, double *y)
@@ -1831,14 +1886,19 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
     }
     const double tol2 = opt.tol * opt.tol;
     const int itmax = opt.itmax > 0 ? opt.itmax : 1000;
-    if (A.singular || opt.method == LV_SOLVER_PCG64)
-        hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, tol2, itmax, (int)A.singular);
     hipError_t e = hipSuccess;
     // the means of b and x serve singular systems only (elsewhere bmean stays the 0 that S starts from, and xmean0
     // is read only where x's mean is restored)
-    if (A.singular) {
-        hipLaunchKernelGGL(k_means, G, dim3(B), 0, s, n, b, (const double *)x, P.p3);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_MEANS, n, W.S);
+    double *Pm = nullptr;  // their partials, which the first residual of a refinement sums
+    if (opt.method == LV_SOLVER_PCG64) {
+        hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, tol2, itmax, (int)A.singular);
+        if (A.singular) {
+            hipLaunchKernelGGL(k_means, G, dim3(B), 0, s, n, b, (const double *)x, P.p3);
+            hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_MEANS, n, W.S);
+        }
+    } else if (A.singular) {
+        Pm = P.ur;
+        hipLaunchKernelGGL(k_means, G, dim3(B), 0, s, n, b, (const double *)x, Pm);
     }
     int total = 0, nsweep = 0, skipped = 0;
     if (opt.method == LV_SOLVER_PCG64) {
@@ -1869,7 +1929,8 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
         double itol = 0.0;
         for (;;) {
             launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3,
-                           nsweep > 0 ? (const double *)Pxs : (const double *)nullptr, W.S);
+                           nsweep > 0 ? (const double *)Pxs : (const double *)nullptr,
+                           nsweep > 0 ? (const double *)nullptr : (const double *)Pm, W.S);
             if (nsweep > 0) {
                 const int seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
                 hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n,
@@ -1954,7 +2015,8 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
             hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_SUM1, n, W.S);
             hipLaunchKernelGGL(k_shift, G, dim3(B), 0, s, n, x, (const lv_cg_scalars *)W.S);
         }
-        launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3, (const double *)nullptr, W.S);
+        launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3, (const double *)nullptr,
+                       (const double *)nullptr, W.S);
         hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n, W.S);
         e = read_scalars(W.S, W.hS, &h, s);
         if (e != hipSuccess) return e;
@@ -2051,83 +2113,104 @@ static lv_dirs8 dirs_of(float *const *v, int m)
     for (int q = 0; q < 8; q++) D.v[q] = v[q < m ? q : 0];
     return D;
 }
-static hipError_t pw_fin(int m, int nb, const double *partials, double *dots, hipStream_t s)
+// the m dots a kernel has just left as partials in D.out: where the next kernel finds them
+static hipError_t pw_dots(lv_dots &D, int m, int nb, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_multidot_fin, dim3(m), dim3(B), 0, s, partials, nb, dots);
+    if (nb <= FEW_BLOCKS) {
+        D.src = D.out;
+        D.nb = nb;
+        D.out = D.out == D.half[0] ? D.half[1] : D.half[0];
+    } else {
+        hipLaunchKernelGGL(k_dots_fin, dim3(m), dim3(B), 0, s, (const double *)D.out, nb, D.fin);
+        D.src = D.fin;
+        D.nb = 0;
+    }
     return hipGetLastError();
 }
 
-hipError_t lv_dot_device(int n, const float *a, const double *b, double *partials, double *dots, hipStream_t s)
+lv_dots lv_dots_in(double *partials, double *fin)
 {
-    const int nb = nblocks_of(n);
-    hipLaunchKernelGGL(k_dot<float>, dim3(nb), dim3(B), 0, s, n, a, b, partials);
-    return pw_fin(1, nb, partials, dots, s);
-}
-hipError_t lv_dot_device(int n, const double *a, const double *b, double *partials, double *dots, hipStream_t s)
-{
-    const int nb = nblocks_of(n);
-    hipLaunchKernelGGL(k_dot<double>, dim3(nb), dim3(B), 0, s, n, a, b, partials);
-    return pw_fin(1, nb, partials, dots, s);
+    static_assert(8 * FEW_BLOCKS <= 4 * NBMAX, "eight values of few blocks fill half of the partials");
+    lv_dots D;
+    D.half[0] = partials;
+    D.half[1] = partials + 4 * NBMAX;
+    D.out = partials;
+    D.src = D.fin = fin;
+    D.nb = 0;
+    return D;
 }
 
-hipError_t lv_normalise(int n, float *y, const double *x, const double *h, hipStream_t s)
+hipError_t lv_dot_device(int n, const float *a, const double *b, lv_dots &D, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_normalise, dim3(nblocks_of(n)), dim3(B), 0, s, n, y, x, h);
+    const int nb = nblocks_of(n);
+    hipLaunchKernelGGL(k_dot<float>, dim3(nb), dim3(B), 0, s, n, a, b, D.out);
+    return pw_dots(D, 1, nb, s);
+}
+hipError_t lv_dot_device(int n, const double *a, const double *b, lv_dots &D, hipStream_t s)
+{
+    const int nb = nblocks_of(n);
+    hipLaunchKernelGGL(k_dot<double>, dim3(nb), dim3(B), 0, s, n, a, b, D.out);
+    return pw_dots(D, 1, nb, s);
+}
+
+hipError_t lv_normalise(int n, float *y, const double *x, const lv_dots &D, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_normalise, dim3(nblocks_of(n)), dim3(B), 0, s, n, y, x, (const double *)D.src, D.nb);
     return hipGetLastError();
 }
 
 hipError_t lv_pw_enter(int n, const double *Pc, const double *Pp, const double *APc, const double *APp, double *t1,
-                       double *rec, double *t2, float *const *Q, int m, double *partials, double *dots, hipStream_t s)
+                       double *rec, double *t2, float *const *Q, int m, lv_dots &D, hipStream_t s)
 {
     const int nb = nblocks_of(n);
     if (m == 0) {
         hipLaunchKernelGGL(k_pw_enter<0>, dim3(nb), dim3(B), 0, s, n, Pc, Pp, APc, APp, t1, rec, t2, lv_dirs8{},
-                           partials);
-        return pw_fin(1, nb, partials, dots, s);
+                           D.out);
+        return pw_dots(D, 1, nb, s);
     }
-    const lv_dirs8 D = dirs_of(Q, m);
-    LV_PW_BY(m, hipLaunchKernelGGL(k_pw_enter<M>, dim3(nb), dim3(B), 0, s, n, Pc, Pp, APc, APp, t1, rec, t2, D,
-                                   partials))
-    return pw_fin(m, nb, partials, dots, s);
+    const lv_dirs8 q8 = dirs_of(Q, m);
+    LV_PW_BY(m, hipLaunchKernelGGL(k_pw_enter<M>, dim3(nb), dim3(B), 0, s, n, Pc, Pp, APc, APp, t1, rec, t2, q8,
+                                   D.out))
+    return pw_dots(D, m, nb, s);
 }
 
-hipError_t lv_pw_out(int n, double *t1, double *t2, float *const *Q, float *const *Z, int m, double *partials,
-                     double *dots, hipStream_t s)
+hipError_t lv_pw_out(int n, double *t1, double *t2, float *const *Q, float *const *Z, int m, lv_dots &D,
+                     hipStream_t s)
 {
     const int nb = nblocks_of(n);
-    const lv_dirs8 D = dirs_of(Q, m), E = dirs_of(Z, m);
-    LV_PW_BY(m, hipLaunchKernelGGL(k_pw_out<M>, dim3(nb), dim3(B), 0, s, n, t1, t2, D, E, (const double *)dots,
-                                   partials))
-    return pw_fin(1, nb, partials, dots, s);
+    const lv_dirs8 q8 = dirs_of(Q, m), z8 = dirs_of(Z, m);
+    LV_PW_BY(m, hipLaunchKernelGGL(k_pw_out<M>, dim3(nb), dim3(B), 0, s, n, t1, t2, q8, z8, (const double *)D.src, D.nb,
+                                   D.out))
+    return pw_dots(D, 1, nb, s);
 }
 
 hipError_t lv_pw_resid(int n, const double *t1, double *t2, float *const *Q, float *znew, int m, const double *b,
-                       const double *AP, double *partials, double *dots, hipStream_t s)
+                       const double *AP, lv_dots &D, hipStream_t s)
 {
     const int nb = nblocks_of(n);
-    const lv_dirs8 D = dirs_of(Q, m);
+    const lv_dirs8 q8 = dirs_of(Q, m);
     if (znew) {
-        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_resid<M, true>), dim3(nb), dim3(B), 0, s, n, t1, t2, D, znew,
-                                       (const double *)dots, b, AP, partials))
+        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_resid<M, true>), dim3(nb), dim3(B), 0, s, n, t1, t2, q8, znew,
+                                       (const double *)D.src, D.nb, b, AP, D.out))
     } else {
-        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_resid<M, false>), dim3(nb), dim3(B), 0, s, n, t1, t2, D, znew,
-                                       (const double *)dots, b, AP, partials))
+        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_resid<M, false>), dim3(nb), dim3(B), 0, s, n, t1, t2, q8, znew,
+                                       (const double *)D.src, D.nb, b, AP, D.out))
     }
-    return pw_fin(m, nb, partials, dots, s);
+    return pw_dots(D, m, nb, s);
 }
 
 hipError_t lv_pw_guess(int n, double *P0, double *t2, float *const *Q, float *const *Z, int m, float *const *O, int no,
-                       double *partials, double *dots, hipStream_t s)
+                       lv_dots &D, hipStream_t s)
 {
     const int nb = nblocks_of(n);
-    const lv_dirs8 D = dirs_of(Q, m), E = dirs_of(Z, m);
+    const lv_dirs8 q8 = dirs_of(Q, m), z8 = dirs_of(Z, m);
     if (no > 0) {
-        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_guess<M, true>), dim3(nb), dim3(B), 0, s, n, P0, t2, D, E,
-                                       (const float *)O[0], (const float *)O[no > 1 ? 1 : 0], (const double *)dots,
-                                       partials))
-        return pw_fin(no, nb, partials, dots, s);
+        LV_PW_BY(m, hipLaunchKernelGGL((k_pw_guess<M, true>), dim3(nb), dim3(B), 0, s, n, P0, t2, q8, z8,
+                                       (const float *)O[0], (const float *)O[no > 1 ? 1 : 0], (const double *)D.src, D.nb,
+                                       D.out))
+        return pw_dots(D, no, nb, s);
     }
-    LV_PW_BY(m, hipLaunchKernelGGL((k_pw_guess<M, false>), dim3(nb), dim3(B), 0, s, n, P0, t2, D, E,
-                                   (const float *)nullptr, (const float *)nullptr, (const double *)dots, partials))
+    LV_PW_BY(m, hipLaunchKernelGGL((k_pw_guess<M, false>), dim3(nb), dim3(B), 0, s, n, P0, t2, q8, z8,
+                                   (const float *)nullptr, (const float *)nullptr, (const double *)D.src, D.nb, D.out))
     return hipGetLastError();
 }
