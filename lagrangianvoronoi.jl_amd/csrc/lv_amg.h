@@ -85,6 +85,18 @@ void lv_amg_free(lv_amg *G);
 // (perm_ok), else the operator's own; 1: the operator's own order.
 hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, const lv_pressure_system &A, int n,
                         const float *mval, const float *mdg, int layout, hipStream_t s);
+// A CG iteration's update left to the cycle (lv_amg_takes_update): x += alpha p, r_out = r - alpha q with
+// alpha = r.z / p.q from the partials of p.q, made by the down pass as it reads the rows; its partials of |r_out|^2 (one a
+// workgroup, G->nbfuse of them) are those of the cycle's head.
+struct lv_cycle_update {
+    const float *p, *q, *r;
+    float *x, *r_out;
+    const double *Ppq;
+    int nb, par;
+    double *Pur;
+    lv_cg_scalars *S;
+};
+bool lv_amg_takes_update(const lv_amg *G);
 // What the caller leaves to the start of a cycle instead of a launch of its own (lv_amg_takes_head): in a
 // CG iteration (k >= 0) the convergence test on the residual's partials (|r|^2); before the first
 // (k < 0) the inner solve's threshold from its init's partials (r.z, r.r).
@@ -102,7 +114,7 @@ bool lv_amg_takes_head(const lv_amg *G, int nb);
 // z = B r for the symmetric V(1,1) cycle B; writes the (r.z, r.r) partials of lv_nblocks(n) blocks
 // that the next CG kernel reduces.  Every kernel is a no-op once S->done is set.  With perm_ok, r
 // and z are in the aggregate order.  z0_ready (only when G->z0_in): G->z0 already holds
-// fine_scale D^-1 r, bit for bit as the cycle would compute it.
+// fine_scale D^-1 r, bit for bit as the cycle would compute it.  update (with head): r is its r_out.
 hipError_t lv_amg_vcycle(const lv_amg *G, const lv_pressure_system &A, const float *r, float *z, double *Prr,
                          const lv_cg_scalars *S, hipStream_t s, bool z0_ready = false,
-                         const lv_cycle_head *head = nullptr);
+                         const lv_cycle_head *head = nullptr, const lv_cycle_update *update = nullptr);

@@ -452,6 +452,31 @@ __global__ __launch_bounds__(B) void k_fine_down_j(fine_ops<V> F, const float *_
     t[i] = down_row_j(F, i, r, z0);
 }
 
+// the convergence test of lv_cycle_head (k >= 0), every workgroup for itself and block 0 for the record; true
+// when the solve has ended
+__device__ __forceinline__ bool head_stops(const lv_cycle_head &H)
+{
+    double pp[1][LV_RED_PER], o[1];
+    reduce_all_load<1>(H.part, H.nb, pp);
+    const int dn = H.S->done;
+    const double thr2 = H.S->thr2;
+    reduce_all_pin<1>(pp);
+    asm volatile("" ::"s"(dn), "s"(thr2));
+    if (dn) return true;
+    reduce_all_sum<1>(H.part, H.nb, pp, o);
+    const bool conv = o[0] <= thr2;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        if (conv) {
+            H.S->rr = o[0];
+            H.S->iters = H.k + 1;
+            H.S->done = 1;
+            if (H.prog) __hip_atomic_store(&H.prog->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+        if (H.prog) __hip_atomic_store(&H.prog->seen, H.k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    return conv;
+}
+
 // The down pass and the restriction in one kernel, for the aggregate order (the rows of level-1
 // cell I are start[I]..start[I+1]-1): block b owns the cells whose first row lies in
 // [FUSE_ROWS b, FUSE_ROWS (b+1)) (blk[b].x..blk[b+1].x-1), keeps their residuals t in LDS and sums
@@ -484,6 +509,37 @@ __device__ __forceinline__ float down_row_z0(const fine_ops<V> &F, int i, const 
         acc += F.A.value(e) * (zi - z0[F.A.column(e, i, n)]);
     }
     return r[i] - acc;
+}
+
+// the sums of a block's cells c0..c1-1 over their rows' residuals tl (first row R0); sa, sb, dv: the row-list
+// bounds and level-1 diagonals of its first FUSE_RPT trips
+__device__ __forceinline__ void fused_restrict(const float *tl, int c0, int c1, int R0, const int *__restrict__ start,
+                                               int na, const int (&sa)[FUSE_RPT], const int (&sb)[FUSE_RPT],
+                                               const float (&dv)[FUSE_RPT], float *__restrict__ rc,
+                                               const float *__restrict__ dinv1, float *__restrict__ z1)
+{
+    const int lanes = (c1 - c0) * RL;
+    // one trip of B lanes, RL per cell; the trip count is uniform, so every lane shuffles
+    auto restrict_trip = [&](int base, int a0, int s1, float di) {
+        const int idx = base + (int)threadIdx.x;
+        const int I = c0 + idx / RL, q = idx % RL;
+        float s = 0.0f;
+        if (idx < lanes)
+            for (int a = a0 + q; a < s1; a += RL) s += tl[a - R0];
+        s = sum_lanes(s);
+        if (q == 0 && idx < lanes) {
+            rc[I] = s;
+            if (z1) z1[I] = OMEGA * di * s;
+        }
+    };
+#pragma unroll
+    for (int p = 0; p < FUSE_RPT; p++)
+        if (p * B < lanes) restrict_trip(p * B, sa[p], sb[p], dv[p]);
+    for (int base = FUSE_RPT * B; base < lanes; base += B) {
+        const int I = c0 + (base + (int)threadIdx.x) / RL;
+        const int Ic = I < na ? I : na - 1;
+        restrict_trip(base, start[Ic], start[Ic + 1], dinv1[Ic]);
+    }
 }
 
 // With z1 (level 1 above the tail), each cell's pre-smoothed z1 = w D1^-1 rc is stored too, as
@@ -522,26 +578,9 @@ __global__ __launch_bounds__(B) void k_fine_down_jr(fine_ops<V> F, const float *
             }
             if (skip) return;
         } else {
-            // the bounds, the partials, the flag and the threshold in one round trip
-            double pp[1][LV_RED_PER], o[1];
-            reduce_all_load<1>(H.part, H.nb, pp);
-            const int dn = *done;
-            const double thr2 = H.S->thr2;
-            reduce_all_pin<1>(pp);
-            asm volatile("" ::"s"(p0.x), "s"(p0.y), "s"(p1.x), "s"(p1.y), "s"(dn), "s"(thr2));
-            if (dn) return;
-            reduce_all_sum<1>(H.part, H.nb, pp, o);
-            const bool conv = o[0] <= thr2;
-            if (blockIdx.x == 0 && threadIdx.x == 0) {
-                if (conv) {
-                    H.S->rr = o[0];
-                    H.S->iters = H.k + 1;
-                    H.S->done = 1;
-                    if (H.prog) __hip_atomic_store(&H.prog->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-                }
-                if (H.prog) __hip_atomic_store(&H.prog->seen, H.k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-            }
-            if (conv) return;
+            // (the bounds in the same round trip as the head's loads)
+            asm volatile("" ::"s"(p0.x), "s"(p0.y), "s"(p1.x), "s"(p1.y));
+            if (head_stops(H)) return;
         }
     } else {
         const int dn = *done;
@@ -578,28 +617,97 @@ __global__ __launch_bounds__(B) void k_fine_down_jr(fine_ops<V> F, const float *
         for (int i = R0 + (int)threadIdx.x; i < R1; i += B) tl[i - R0] = down_row_j(F, i, r, z0);
     }
     __syncthreads();
-    const int lanes = (c1 - c0) * RL;
-    // one trip of B lanes, RL per cell; the trip count is uniform, so every lane shuffles
-    auto restrict_trip = [&](int base, int a0, int s1, float di) {
-        const int idx = base + (int)threadIdx.x;
-        const int I = c0 + idx / RL, q = idx % RL;
-        float s = 0.0f;
-        if (idx < lanes)
-            for (int a = a0 + q; a < s1; a += RL) s += tl[a - R0];
-        s = sum_lanes(s);
-        if (q == 0 && idx < lanes) {
-            rc[I] = s;
-            if (z1) z1[I] = OMEGA * di * s;
-        }
-    };
+    fused_restrict(tl, c0, c1, R0, start, na, sa, sb, dv, rc, dinv1, z1);
+}
+
+// k_fine_down_jr with the CG iteration's update in front of it (lv_cycle_update): every row's r - alpha q, and its
+// neighbours' again for their z0, which k_cg_u's pass over the rows would have stored; the same values
+// bit for bit.  One launch for two where launches bound the iteration (UPDATE_MAX).
+template <class V>
+__global__ __launch_bounds__(B) void k_fine_down_u(fine_ops<V> F, lv_cycle_update U, float *__restrict__ z0,
+                                                   const int *__restrict__ start, const int2 *__restrict__ blk,
+                                                   int na, float *__restrict__ rc, const float *__restrict__ dinv1,
+                                                   float *__restrict__ z1)
+{
+    __shared__ float tl[FUSE_CAP];
+    const int b = lv_xcd_block(blockIdx.x, gridDim.x);
+    const int2 p0 = blk[b], p1 = blk[b + 1];
+    double pp[1][LV_RED_PER], pq[1];
+    reduce_all_load<1>(U.Ppq, U.nb, pp);
+    const int dn = U.S->done;
+    const double rzn = U.S->rz[U.par ^ 1];
+    reduce_all_pin<1>(pp);
+    asm volatile("" ::"s"(p0.x), "s"(p0.y), "s"(p1.x), "s"(p1.y), "s"(dn), "s"(rzn));
+    if (dn) return;
+    const int c0 = p0.x, c1 = p1.x, R0 = p0.y, R1 = p1.y;
+    int sa[FUSE_RPT], sb[FUSE_RPT];
+    float dv[FUSE_RPT];
 #pragma unroll
-    for (int p = 0; p < FUSE_RPT; p++)
-        if (p * B < lanes) restrict_trip(p * B, sa[p], sb[p], dv[p]);
-    for (int base = FUSE_RPT * B; base < lanes; base += B) {
-        const int I = c0 + (base + (int)threadIdx.x) / RL;
+    for (int p = 0; p < FUSE_RPT; p++) {
+        const int I = c0 + (p * B + (int)threadIdx.x) / RL;
         const int Ic = I < na ? I : na - 1;
-        restrict_trip(base, start[Ic], start[Ic + 1], dinv1[Ic]);
+        sa[p] = start[Ic];
+        sb[p] = start[Ic + 1];
+        dv[p] = dinv1[Ic];
     }
+    reduce_all_sum<1>(U.Ppq, U.nb, pp, pq);
+    const double alpha = rzn / pq[0];
+    const float a = (float)alpha;
+    const int n = F.n;
+    constexpr int W = 8;
+    double rr = 0.0;
+    for (int i0 = R0 + (int)threadIdx.x; i0 < R1; i0 += FUSE_RPT * B) {
+        // (all rows' loads before the sums; a clamped duplicate is computed and dropped)
+        int c[FUSE_RPT][W], d[FUSE_RPT];
+        float v[FUSE_RPT][W], rj[FUSE_RPT][W], qj[FUSE_RPT][W], dj[FUSE_RPT][W];
+        float ri[FUSE_RPT], qi[FUSE_RPT], di[FUSE_RPT], dg[FUSE_RPT], xi[FUSE_RPT], pi[FUSE_RPT];
+#pragma unroll
+        for (int h = 0; h < FUSE_RPT; h++) {
+            const int i = i0 + h * B < R1 ? i0 + h * B : R1 - 1;
+            ri[h] = U.r[i];
+            qi[h] = U.q[i];
+            di[h] = F.dinv[i];
+            dg[h] = F.diag[i];
+            xi[h] = U.x[i];
+            pi[h] = U.p[i];
+            d[h] = lv_ell_head<W>(F.A, i, n, c[h], v[h]);
+        }
+#pragma unroll
+        for (int h = 0; h < FUSE_RPT; h++)
+#pragma unroll
+            for (int k = 0; k < W; k++) {
+                rj[h][k] = U.r[c[h][k]];
+                qj[h][k] = U.q[c[h][k]];
+                dj[h][k] = F.dinv[c[h][k]];
+            }
+#pragma unroll
+        for (int h = 0; h < FUSE_RPT; h++) {
+            const int i = i0 + h * B;
+            if (i >= R1) continue;
+            const float rn = ri[h] - a * qi[h];
+            const float zi = F.scale * di[h] * rn;
+            float acc = dg[h] * zi;
+#pragma unroll
+            for (int k = 0; k < W; k++) acc += v[h][k] * (zi - F.scale * dj[h][k] * (rj[h][k] - a * qj[h][k]));
+            for (int k = W; k < d[h]; k++) {
+                const size_t e = (size_t)k * n + i;
+                const int j = F.A.column(e, i, n);
+                acc += F.A.value(e) * (zi - F.scale * F.dinv[j] * (U.r[j] - a * U.q[j]));
+            }
+            tl[i - R0] = rn - acc;
+            U.x[i] = xi[h] + a * pi[h];
+            U.r_out[i] = rn;
+            z0[i] = zi;
+            rr += (double)rn * (double)rn;
+        }
+    }
+    const double w[1] = {rr};
+    block_partials<1>(w, U.Pur, gridDim.x);  // (its barrier also stands between tl's rows and their sums)
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        U.S->pq = pq[0];
+        U.S->alpha = alpha;
+    }
+    fused_restrict(tl, c0, c1, R0, start, na, sa, sb, dv, rc, dinv1, z1);
 }
 
 // blk[b] = (the first cell I with start[I] >= FUSE_ROWS b, start[I]) for b = 0..nbf-1,
@@ -867,11 +975,17 @@ __device__ __forceinline__ void st_wsave_cell(const st_level &L, int f, float *_
 
 // down on level L: pre-smoothed z of L (given, or stored here) and the right-hand side rc of the
 // next level
-template <bool ZGIVEN>
+// (HEAD: after the down pass that made a CG update, with its convergence test)
+template <bool ZGIVEN, bool HEAD>
 __global__ __launch_bounds__(B) void k_st_down(st_level L, int Kyc, int nc, const float *__restrict__ r,
-                                               float *__restrict__ z, float *__restrict__ rc, const lv_cg_scalars *S)
+                                               float *__restrict__ z, float *__restrict__ rc, const lv_cg_scalars *S,
+                                               lv_cycle_head H)
 {
-    if (S && S->done) return;
+    if (HEAD) {
+        if (head_stops(H)) return;
+    } else if (S && S->done) {
+        return;
+    }
     // (workgroups in the XCD-aware order: the parent rows above and below a workgroup's, whose
     // children it gathers, are mostly on its own XCD)
     const int tid = lv_xcd_block(blockIdx.x, gridDim.x) * B + threadIdx.x;
@@ -1646,10 +1760,12 @@ __global__ __launch_bounds__(B) void k_mat_extend(st_level L, int Kyc, int nc, c
 // of r issued before the done flag is tested.  r is allocated to a multiple of 4; the entries past n are
 // dropped.  PROLONG (level 1 in the aggregate order): also the prolongation of each cell's correction into
 // its rows of z0, as k_prolong1 forms it.
-template <int PER, bool PROLONG>
+// (HEAD as in k_st_down)
+template <int PER, bool PROLONG, bool HEAD>
 __global__ __launch_bounds__(B) void k_mat_mv(int n, int ld, const float *__restrict__ mat, const float *__restrict__ r,
                                               float *__restrict__ t, const lv_cg_scalars *S,
-                                              const int *__restrict__ start, float alpha0, float *__restrict__ z0)
+                                              const int *__restrict__ start, float alpha0, float *__restrict__ z0,
+                                              lv_cycle_head H)
 {
     typedef float f4 __attribute__((ext_vector_type(4)));
     const int lane = threadIdx.x & 63, row = blockIdx.x * (B / 64) + (threadIdx.x >> 6);
@@ -1664,7 +1780,11 @@ __global__ __launch_bounds__(B) void k_mat_mv(int n, int ld, const float *__rest
         x[q] = r4[kk];
     }
     const int b0 = PROLONG ? start[rw] : 0, e = PROLONG ? start[rw + 1] : 0;
-    if (S && S->done) return;
+    if (HEAD) {
+        if (head_stops(H)) return;
+    } else if (S && S->done) {
+        return;
+    }
     float a = 0.0f;
 #pragma unroll
     for (int q = 0; q < PER; q++) {
@@ -2282,7 +2402,7 @@ static st_pair st_pair_of(const lv_amg *G, int l)
 template <class V>
 static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, const int *list, const float *r,
                          float *z, double *Prr, const lv_cg_scalars *S, hipStream_t s, bool z0_ready,
-                         const lv_cycle_head *head)
+                         const lv_cycle_head *head, const lv_cycle_update *update)
 {
     const int n = G->n0;
     const lv_amg_level &L1 = G->lev[1];
@@ -2305,7 +2425,10 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
                        (const int *)G->start, reinterpret_cast<const int2 *>(G->bfirst), G->na, L1.r,              \
                        (const float *)L1.dinv, z1, done, head ? *head : lv_cycle_head{})
         const bool z0_in = z0_ready && G->z0_in;
-        if (z0_in && head) LV_DOWN_JR(true, true);
+        if (update)
+            hipLaunchKernelGGL(k_fine_down_u<V>, dim3(G->nbfuse), dim3(B), 0, s, F, *update, G->z0, (const int *)G->start,
+                               reinterpret_cast<const int2 *>(G->bfirst), G->na, L1.r, (const float *)L1.dinv, z1);
+        else if (z0_in && head) LV_DOWN_JR(true, true);
         else if (z0_in) LV_DOWN_JR(true, false);
         else if (head) LV_DOWN_JR(false, true);
         else LV_DOWN_JR(false, false);
@@ -2328,12 +2451,9 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
             l++;
             continue;
         }
-        if (l == 1 && z1_given)
-            hipLaunchKernelGGL(k_st_down<true>, g1((int64_t)C.n * CF2), dim3(B), 0, s, sl, C.Ky, C.n,
-                               (const float *)L.r, L.z, C.r, S);
-        else
-            hipLaunchKernelGGL(k_st_down<false>, g1((int64_t)C.n * CF2), dim3(B), 0, s, sl, C.Ky, C.n,
-                               (const float *)L.r, L.z, C.r, S);
+        auto down = l > 1 || !z1_given ? k_st_down<false, false> : update ? k_st_down<true, true> : k_st_down<true, false>;
+        hipLaunchKernelGGL(down, g1((int64_t)C.n * CF2), dim3(B), 0, s, sl, C.Ky, C.n, (const float *)L.r, L.z, C.r, S,
+                           update ? *head : lv_cycle_head{});
     }
     // the tail: levels lt..nlev down, dense, and up, or the matrix of that; the final correction of level
     // lt in its t.  Then the coarse levels above it, up: each level's final correction in t; level 1 in the
@@ -2342,11 +2462,14 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
     const bool prolong_in_up = (lt > 1 || G->mat_ld) && !G->fine_learned && list == nullptr;
     if (G->mat_ld) {
         const bool pr = lt == 1 && prolong_in_up;
-        auto kern = LT.n <= TAIL_MAX ? (pr ? k_mat_mv<TAIL_MAX / 256, true> : k_mat_mv<TAIL_MAX / 256, false>)
-                                     : (pr ? k_mat_mv<MAT_MAX / 256, true> : k_mat_mv<MAT_MAX / 256, false>);
+        const bool hd = update && lt == 1;  // (the update comes with pr there)
+        constexpr int PT = TAIL_MAX / 256, PM = MAT_MAX / 256;
+        auto kern = LT.n <= TAIL_MAX ? (hd ? k_mat_mv<PT, true, true> : pr ? k_mat_mv<PT, true, false> : k_mat_mv<PT, false, false>)
+                                     : (hd ? k_mat_mv<PM, true, true> : pr ? k_mat_mv<PM, true, false> : k_mat_mv<PM, false, false>);
         hipLaunchKernelGGL(kern, dim3((LT.n + B / 64 - 1) / (B / 64)), dim3(B), 0, s, LT.n, G->mat_ld,
                            (const float *)G->mat, (const float *)LT.r, LT.t, S,
-                           pr ? (const int *)G->start : (const int *)nullptr, G->fine_alpha, G->z0);
+                           pr ? (const int *)G->start : (const int *)nullptr, G->fine_alpha, G->z0,
+                           hd ? *head : lv_cycle_head{});
     } else if (G->lds_ok)
         hipLaunchKernelGGL(k_tail_lds<false>, dim3(1), dim3(TB), 0, s, tail_args_of(G), S, (float *)nullptr, 0);
     else
@@ -2387,19 +2510,30 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
 }
 
 hipError_t lv_amg_vcycle(const lv_amg *G, const lv_pressure_system &A, const float *r, float *z, double *Prr,
-                         const lv_cg_scalars *S, hipStream_t s, bool z0_ready, const lv_cycle_head *head)
+                         const lv_cg_scalars *S, hipStream_t s, bool z0_ready, const lv_cycle_head *head,
+                         const lv_cycle_update *update)
 {
     if (G->perm_ok)
         return vcycle(G, fine_agg<lv_ell_agg16>(G, (const uint16_t *)G->pev16), (const int *)G->aggp,
-                      (const int *)nullptr, r, z, Prr, S, s, z0_ready, head);
-    return vcycle(G, fine_own(G, A), (const int *)G->agg, (const int *)G->list, r, z, Prr, S, s, false, nullptr);
+                      (const int *)nullptr, r, z, Prr, S, s, z0_ready, head, update);
+    return vcycle(G, fine_own(G, A), (const int *)G->agg, (const int *)G->list, r, z, Prr, S, s, false, nullptr, nullptr);
 }
 
 // The test in the down pass adds 0.5 us to it at 131,072 and 265,225 rows and 1.0 at 1,000,000, for a launch of 2.6 us
 // and its gap; at 4,194,304 rows 8.2 for a launch of 4.8.  The line (2 M rows) lies between, in what the workgroups
 // read together.
-static constexpr int64_t HEAD_MAX = 1ll << 21;
+static constexpr int64_t HEAD_MAX = 1ll << 23;
 bool lv_amg_takes_head(const lv_amg *G, int nb)
 {
     return G->perm_ok && !G->fine_learned && G->nbfuse > 0 && (int64_t)G->nbfuse * nb <= HEAD_MAX;
+}
+
+// With the update in the down pass an iteration's part up to level 1's own takes 12.1 us for 14.5 (and a gap
+// between launches less) at 10,000 rows, 11.8 for 13.7 at 131,072, 14.9 for 16.1 at 265,225, and 28.7 for 28.0 at
+// 1,000,000, where the neighbours' second and third gather count; a sweep that has converged pays for one down pass.
+static constexpr int UPDATE_MAX = 1 << 19;
+bool lv_amg_takes_update(const lv_amg *G)
+{
+    // (the kernel behind the down pass makes the convergence test: a stencil level, or the matrix as level 1)
+    return G->perm_ok && G->z0_in && G->n0 <= UPDATE_MAX && G->nbfuse <= 2 * LV_NBMAX && (G->lmat > 1 || G->mat_ld);
 }

@@ -1767,6 +1767,9 @@ hipError_t cg_iterate(int n, V A, const T *diag, const T *dinv, T *x, T *r, T *z
                       lv_timer *tm, lv_cg_scalars &h, const lv_precond *M, int *dflag)
 {
     const int nb = nblocks_of(n);
+    T *r_alt = nullptr;  // where the residual is updated out of place: the cycle's t0, which its fused down pass leaves free
+    if constexpr (std::is_same<T, float>::value)
+        if (M && M->amg) r_alt = M->amg->t0;
     // no kernel of this solve that stores progress is in flight: since the previous sweep the caller
     // has read the FP64 residual (published by k_finalize, which runs after every earlier kernel of
     // the stream has finished) or synchronised before a fallback sweep
@@ -1806,6 +1809,17 @@ hipError_t cg_iterate(int n, V A, const T *diag, const T *dinv, T *x, T *r, T *z
                                    (const double *)P.rr, P.pq, dS, dprog, par, k, k == 0 ? 1 : 0, M ? 0 : 1);
         }
         if (M) {
+            if constexpr (std::is_same<T, float>::value) {
+                if (M->amg && lv_amg_takes_update(M->amg)) {  // the whole rest of the iteration
+                    const lv_cycle_head H{P.ur, M->amg->nbfuse, dS, dprog, k, 0.0, 0};
+                    const lv_cycle_update U{p, q, r, x, r_alt, P.pq, nb, par, P.ur, dS};
+                    hipError_t e = lv_amg_vcycle(M->amg, *M->A, (const float *)r_alt, z, P.rr, (const lv_cg_scalars *)dS,
+                                                 s, true, &H, &U);
+                    if (e != hipSuccess) return e;
+                    std::swap(r, r_alt);
+                    continue;
+                }
+            }
             // the cycle's pre-smoothed z0 stored with the residual update (FP32 solves only)
             T *z0 = nullptr;
             T sc = (T)0;

@@ -481,3 +481,20 @@ def test_paired_levels_of_odd_periodic_widths_are_bit_identical(lv, oracle, gpu,
     assert np.array_equal(out[0][1], out[1][1])
     assert np.array_equal(out[0][0], out[1][0])
     assert out[0][2] == out[1][2]
+
+
+@pytest.mark.parametrize("kind,K", [("periodic", 24), ("periodic", 77), ("periodic", 150), ("xperiodic", 101),
+                                    ("walls", 40), ("walls", 110), ("walls", 210)])
+def test_cg_updates_in_the_down_pass_give_the_fp64_solution(lv, oracle, gpu, kind, K):
+    """the update made by the down pass with the test in the next kernel (a stencil level, or a singular system's matrix as
+    level 1 or as level 2) or by its own kernels (a nonsingular system small enough for one workgroup): the solution of plain
+    FP64 conjugate gradients, both to a residual of 1e-11"""
+    _flush("cg update %s %d" % (kind, K))
+    periodic = kind == "periodic"
+    grid, op, solver, x, dr, d, rp, cols, coef = _system(lv, oracle, kind, K, "tg" if periodic else "cavity", 2e-3)
+    b = np.random.default_rng(K).standard_normal(grid.n)
+    if not np.any(d > 0):
+        b -= b.mean()
+    P = {m: solver.solve(b, np.zeros(grid.n), method=m, tol=1e-11, itmax=20000) for m in ("amg", "pcg64")}
+    # |A^-1| is at most 1 / (the smallest eigenvalue): residuals of 1e-11 leave errors of 1e-11 cond(A), below 1e-5 here
+    assert rel_err(P["amg"] - P["amg"].mean(), P["pcg64"] - P["pcg64"].mean()) <= 1e-5
