@@ -167,6 +167,8 @@ int lv_set_particles(lv_ctx *ctx, int32_t n, const double *x);
 int lv_num_particles(lv_ctx *ctx, int32_t *n);
 int lv_upload(lv_ctx *ctx, int32_t field, const void *host);
 int lv_download(lv_ctx *ctx, int32_t field, void *host);
+/* a Float64 field with each particle's components side by side (D by rows), as n x 1, 2 or 4 doubles */
+int lv_download_rows(lv_ctx *ctx, int32_t field, double *host);
 /* device pointer of a field (for zero-copy interop with other device code on the same stream) */
 int lv_field_device_ptr(lv_ctx *ctx, int32_t field, void **dptr);
 

@@ -111,6 +111,7 @@ _SIGNATURES = {
     "lv_num_particles": [_P, _P],
     "lv_upload": [_P, _I, _P],
     "lv_download": [_P, _I, _P],
+    "lv_download_rows": [_P, _I, _P],
     "lv_field_device_ptr": [_P, _I, ctypes.POINTER(ctypes.c_void_p)],
     "lv_remesh": [_P],
     "lv_mesh_size": [_P, _P],
@@ -289,13 +290,10 @@ class VoronoiGrid:
     def get(self, name):
         fid, comps = FIELDS[name]
         dtype = np.int32 if name == "phase" else np.float64
-        out = np.empty(comps * self.n, dtype=dtype)
-        _check(self._ctx, lib().lv_download(self._ctx, fid, _ptr(out)))
-        if comps == 1:
-            return out
-        if comps == 2:
-            return out.reshape(2, self.n).T.copy()
-        return out.reshape(2, 2, self.n).transpose(2, 1, 0).copy()  # (n, row, col), column-major planes
+        out = np.empty((self.n,) + {1: (), 2: (2,), 4: (2, 2)}[comps], dtype=dtype)  # D: (n, row, col)
+        fetch = lib().lv_download if comps == 1 else lib().lv_download_rows
+        _check(self._ctx, fetch(self._ctx, fid, _ptr(out)))
+        return out
 
     def get_soa(self, name):
         """The raw SoA planes of a field, as the C ABI holds them."""

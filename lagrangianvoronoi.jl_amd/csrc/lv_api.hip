@@ -16,6 +16,7 @@
 
 #include "lv_spai.h"
 #include "lv_amg.h"
+#include "lv_copy.h"
 #include "lv_vtk.h"
 
 struct lv_mph_work;
@@ -62,6 +63,7 @@ struct lv_ctx {
     int *d_flags = nullptr;   // [0] error word, [1] nonsingular flag, [2] a column offset wider than 16 bits (these
                               // three zero between their uses), [3] items of the cell list, [4] couplings
     lv_mailbox mail = {};     // by which the host reads them
+    lv_ring ring = {};        // pinned buffers of the large copies
     lv_timer *timers[LV_NKTIMERS] = {nullptr, nullptr, nullptr, nullptr};
     // Picard extrapolation: orthonormal A-images q_k of past Picard corrections and their
     // preimages z_k (A z_k = q_k), the last two Picard iterates and their A-images
@@ -457,6 +459,7 @@ int lv_destroy(lv_ctx *ctx)
                     ctx->W.partials, ctx->scan_temp};
     for (void *p : ptrs) dfree(p);
     lv_mail_free(&ctx->mail);
+    lv_ring_free(&ctx->ring);
     if (ctx->W.hprog) (void)hipHostFree(ctx->W.hprog);
     if (ctx->W.hS) (void)hipHostFree(ctx->W.hS);
     if (ctx->spai_ok) lv_spai_free(&ctx->spai);
@@ -588,8 +591,9 @@ int lv_download(lv_ctx *ctx, int32_t field, void *host)
     void *p = field_ptr(ctx, field, &count, &elem, &ro);
     if (!p) return lv_fail(ctx, LV_E_INVALID, "invalid field");
     if (count == 0) return LV_OK;
-    LV_HIP_CHECK(hipMemcpyAsync(host, p, count * elem, hipMemcpyDeviceToHost, ctx->s));
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+    lv_copier C(&ctx->ring, ctx->s, count * elem);
+    LV_HIP_CHECK(C.to_host(host, p, count * elem));
+    LV_HIP_CHECK(C.finish());
     return LV_OK;
 }
 
@@ -722,8 +726,47 @@ __global__ __launch_bounds__(MB) void k_mesh_rows(lv_mesh_view M, const int *__r
     }
 }
 
-// particles a chunk of rows holds: its staging (at most LV_MAXE edges of 4 + 32 bytes each) is 18 MiB
+// particles a chunk of mesh rows holds: its staging (at most LV_MAXE edges of 4 + 32 bytes each) is 18 MiB
 constexpr int MESH_CHUNK = 32768;
+constexpr size_t STAGE_BYTES = (size_t)MESH_CHUNK * LV_MAXE * (4 + 32);
+
+// the staging of the read-outs (and of a call's scratch that fits it), kept with the context
+hipError_t make_stage(lv_ctx *ctx)
+{
+    return ctx->mesh_stage ? hipSuccess : dalloc(&ctx->mesh_stage, STAGE_BYTES / sizeof(double));
+}
+
+// particle i's C components side by side (four: the matrix of column-major planes by rows)
+template <int C>
+__global__ __launch_bounds__(MB) void k_field_rows(int n, int i0, int i1, const double *__restrict__ p,
+                                                   double *__restrict__ out)
+{
+    const int i = i0 + blockIdx.x * MB + threadIdx.x;
+    if (i >= i1) return;
+#pragma unroll
+    for (int k = 0; k < C; k++) {
+        const int plane = C == 4 ? (k & 1) * 2 + (k >> 1) : k;
+        out[(size_t)(i - i0) * C + k] = p[(size_t)plane * n + i];
+    }
+}
+
+template <int C>
+int field_rows(lv_ctx *ctx, const double *p, double *host)
+{
+    const int n = ctx->n;
+    LV_HIP_CHECK(make_stage(ctx));
+    const int chunk = (int)(STAGE_BYTES / (C * sizeof(double)));
+    lv_copier D(&ctx->ring, ctx->s, sizeof(double) * C * (size_t)n);
+    for (int i0 = 0; i0 < n; i0 += chunk) {
+        const int i1 = std::min(n, i0 + chunk);
+        hipLaunchKernelGGL(k_field_rows<C>, dim3((i1 - i0 + MB - 1) / MB), dim3(MB), 0, ctx->s, n, i0, i1, p,
+                           ctx->mesh_stage);
+        LV_HIP_CHECK(hipGetLastError());
+        LV_HIP_CHECK(D.to_host(host + (size_t)C * i0, ctx->mesh_stage, sizeof(double) * C * (size_t)(i1 - i0)));
+    }
+    LV_HIP_CHECK(D.finish());
+    return LV_OK;
+}
 
 // the edge offsets of every particle into ctx->clip_retry (work space of the next remesh, n + 1 ints) and
 // the number of edges
@@ -745,8 +788,9 @@ int mesh_rows(lv_ctx *ctx, const int *hptr, int32_t *labels, double *verts)
 {
     const int n = ctx->n;
     constexpr size_t W = PV == 4 ? 4 : 3;
-    if (!ctx->mesh_stage) LV_HIP_CHECK(dalloc(&ctx->mesh_stage, (size_t)MESH_CHUNK * LV_MAXE * 4 + MESH_CHUNK * LV_MAXE / 2));
+    LV_HIP_CHECK(make_stage(ctx));
     double *dv = ctx->mesh_stage;
+    lv_copier C(&ctx->ring, ctx->s, (size_t)hptr[n] * (W * sizeof(double) + (labels ? sizeof(int32_t) : 0)));
     int *dl = reinterpret_cast<int *>(dv + (size_t)MESH_CHUNK * LV_MAXE * 4);
     for (int i0 = 0; i0 < n; i0 += MESH_CHUNK) {
         const int i1 = std::min(n, i0 + MESH_CHUNK);
@@ -755,16 +799,29 @@ int mesh_rows(lv_ctx *ctx, const int *hptr, int32_t *labels, double *verts)
         hipLaunchKernelGGL(k_mesh_rows<PV>, dim3((i1 - i0 + MB - 1) / MB), dim3(MB), 0, ctx->s, mesh_view(ctx),
                            (const int *)ctx->clip_retry, i0, i1, labels ? dl : (int *)nullptr, dv);
         LV_HIP_CHECK(hipGetLastError());
-        if (labels) LV_HIP_CHECK(hipMemcpyAsync(labels + o, dl, sizeof(int) * m, hipMemcpyDeviceToHost, ctx->s));
-        LV_HIP_CHECK(hipMemcpyAsync(verts + W * o, dv, sizeof(double) * W * m, hipMemcpyDeviceToHost, ctx->s));
+        if (labels) LV_HIP_CHECK(C.to_host(labels + o, dl, sizeof(int) * m));
+        LV_HIP_CHECK(C.to_host(verts + W * o, dv, sizeof(double) * W * m));
     }
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+    LV_HIP_CHECK(C.finish());
     return LV_OK;
 }
 
 }  // namespace
 
 extern "C" {
+
+int lv_download_rows(lv_ctx *ctx, int32_t field, double *host)
+{
+    if (!ctx || !host) return LV_E_INVALID;
+    size_t count, elem;
+    bool ro;
+    void *p = field_ptr(ctx, field, &count, &elem, &ro);
+    if (!p || elem != sizeof(double)) return lv_fail(ctx, LV_E_INVALID, "invalid field");
+    if (count == 0) return LV_OK;
+    if (count == 2 * (size_t)ctx->n) return field_rows<2>(ctx, (const double *)p, host);
+    if (count == 4 * (size_t)ctx->n) return field_rows<4>(ctx, (const double *)p, host);
+    return lv_download(ctx, field, host);
+}
 
 int lv_mesh_size(lv_ctx *ctx, int64_t *nedges)
 {
@@ -932,14 +989,34 @@ int need_cell_list(lv_ctx *ctx)
     return LV_OK;
 }
 
-// device scratch of one call, freed on every return path
+// device scratch of one call: the context's staging when it fits, else memory freed on every return path
 struct dev_buf {
     void *p = nullptr;
+    bool own = false;
     ~dev_buf()
     {
-        if (p) (void)hipFree(p);
+        if (own) (void)hipFree(p);
+    }
+    hipError_t get(lv_ctx *ctx, size_t bytes)
+    {
+        if (bytes <= STAGE_BYTES) {
+            hipError_t e = make_stage(ctx);
+            p = ctx->mesh_stage;
+            return e;
+        }
+        hipError_t e = hipMalloc(&p, bytes);
+        own = e == hipSuccess;
+        return e;
     }
 };
+
+// whether some value is NaN (no early end, so that the loop is a vector one)
+bool any_nan(const double *v, int m)
+{
+    int bad = 0;
+    for (int t = 0; t < m; t++) bad |= v[t] != v[t];
+    return bad != 0;
+}
 
 }  // namespace
 
@@ -950,14 +1027,16 @@ int lv_nearest_polygon(lv_ctx *ctx, int32_t m, const double *q, int32_t *idx)
     if (m < 0 || (m > 0 && (!q || !idx))) return lv_fail(ctx, LV_E_INVALID, "lv_nearest_polygon");
     if ((rc = need_cell_list(ctx))) return rc;
     if (m == 0) return LV_OK;
-    dev_buf dq, di;
-    LV_HIP_CHECK(hipMalloc(&dq.p, sizeof(double) * 2 * m));
-    LV_HIP_CHECK(hipMalloc(&di.p, sizeof(int) * m));
-    LV_HIP_CHECK(hipMemcpyAsync(dq.p, q, sizeof(double) * 2 * m, hipMemcpyHostToDevice, ctx->s));
+    dev_buf d;  // the queries, then the indices
+    LV_HIP_CHECK(d.get(ctx, (sizeof(double) * 2 + sizeof(int)) * m));
+    double *dq = (double *)d.p;
+    int *di = (int *)(dq + 2 * (size_t)m);
+    LV_HIP_CHECK(hipMemcpyAsync(dq, q, sizeof(double) * 2 * m, hipMemcpyHostToDevice, ctx->s));
     LV_HIP_CHECK(lv_launch_nearest(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
-                                   ctx->max_items, ctx->path_i, ctx->path_rr, m, (const double *)dq.p, (int *)di.p, ctx->s));
-    LV_HIP_CHECK(hipMemcpyAsync(idx, di.p, sizeof(int) * m, hipMemcpyDeviceToHost, ctx->s));
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+                                   ctx->max_items, ctx->path_i, ctx->path_rr, m, (const double *)dq, di, ctx->s));
+    lv_copier C(&ctx->ring, ctx->s, sizeof(int) * m);
+    LV_HIP_CHECK(C.to_host(idx, di, sizeof(int) * m));
+    LV_HIP_CHECK(C.finish());
     for (int t = 0; t < m; t++)
         if (idx[t] < 0) return lv_fail(ctx, LV_E_INVALID, "nearest polygon beyond r_max of a query point");
     return LV_OK;
@@ -976,11 +1055,12 @@ int lv_movingls(lv_ctx *ctx, int32_t order, int32_t field, int32_t comp, double 
     const int N = order == 1 ? 2 : (order == 2 ? 5 : 9);
     const size_t bytes = sizeof(double) * (size_t)N * ctx->n;
     dev_buf d;
-    LV_HIP_CHECK(hipMalloc(&d.p, bytes));
+    LV_HIP_CHECK(d.get(ctx, bytes));
     LV_HIP_CHECK(lv_launch_movingls(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
                                     ctx->max_items, ctx->path_i, ctx->path_rr, order, f, h, (double *)d.p, ctx->s));
-    LV_HIP_CHECK(hipMemcpyAsync(coeffs, d.p, bytes, hipMemcpyDeviceToHost, ctx->s));
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
+    lv_copier C(&ctx->ring, ctx->s, bytes);
+    LV_HIP_CHECK(C.to_host(coeffs, d.p, bytes));
+    LV_HIP_CHECK(C.finish());
     return LV_OK;
 }
 
@@ -993,16 +1073,16 @@ int lv_point_values(lv_ctx *ctx, int32_t m, const double *q, int32_t field, int3
     const double *f = field_plane(ctx, field, comp);
     if (!f) return lv_fail(ctx, LV_E_INVALID, "lv_point_values: not a Float64 field component");
     if (m == 0) return LV_OK;
-    dev_buf dq, dout;
-    LV_HIP_CHECK(hipMalloc(&dq.p, sizeof(double) * 2 * m));
-    LV_HIP_CHECK(hipMalloc(&dout.p, sizeof(double) * m));
-    LV_HIP_CHECK(hipMemcpyAsync(dq.p, q, sizeof(double) * 2 * m, hipMemcpyHostToDevice, ctx->s));
+    dev_buf d;  // the queries, then the values
+    LV_HIP_CHECK(d.get(ctx, sizeof(double) * 3 * m));
+    double *dq = (double *)d.p, *dout = dq + 2 * (size_t)m;
+    LV_HIP_CHECK(hipMemcpyAsync(dq, q, sizeof(double) * 2 * m, hipMemcpyHostToDevice, ctx->s));
     LV_HIP_CHECK(lv_launch_point_value(ctx->g, ctx->F.x, ctx->n, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
-                                       ctx->max_items, ctx->path_i, ctx->path_rr, m, (const double *)dq.p, f, ctx->g.h, (double *)dout.p, ctx->s));
-    LV_HIP_CHECK(hipMemcpyAsync(out, dout.p, sizeof(double) * m, hipMemcpyDeviceToHost, ctx->s));
-    LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
-    for (int t = 0; t < m; t++)
-        if (out[t] != out[t]) return lv_fail(ctx, LV_E_INVALID, "nearest polygon beyond r_max of a query point");
+                                       ctx->max_items, ctx->path_i, ctx->path_rr, m, (const double *)dq, f, ctx->g.h, dout, ctx->s));
+    lv_copier C(&ctx->ring, ctx->s, sizeof(double) * m);
+    LV_HIP_CHECK(C.to_host(out, dout, sizeof(double) * m));
+    LV_HIP_CHECK(C.finish());
+    if (any_nan(out, m)) return lv_fail(ctx, LV_E_INVALID, "nearest polygon beyond r_max of a query point");
     return LV_OK;
 }
 
