@@ -15,7 +15,7 @@
 
 constexpr int LV_RING = 8;
 constexpr size_t LV_PIECE = (size_t)2 << 20;
-constexpr int LV_COPIERS = 6;                       // threads at most, one for each MiB
+constexpr int LV_COPIERS = 4;                       // threads at most, one for each MiB (6 and more are no faster)
 constexpr size_t LV_STAGED_MIN = (size_t)3 << 20;
 
 // the pinned ring of a context (16 MiB, made by its first large copy)
