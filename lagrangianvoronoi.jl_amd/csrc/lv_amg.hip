@@ -2008,7 +2008,6 @@ hipError_t lv_amg_init(lv_amg *G)
     AMG_CHECK(hipMalloc(&G->desc, sizeof(int) * (LV_AMG_MAXLEV + 1) * LV_DESC));
     AMG_CHECK(hipMalloc(&G->pflag, 2 * sizeof(int)));
     AMG_CHECK(hipMemset(G->pflag, 0, 2 * sizeof(int)));
-    AMG_CHECK(lv_mail_init(&G->mail));
     return hipSuccess;
 }
 
@@ -2222,6 +2221,7 @@ static tail_lds_args tail_args_of(const lv_amg *G)
 hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, const lv_pressure_system &A, int n,
                         const float *mval, const float *mdg, int layout, hipStream_t s)
 {
+    if (!G->mail.host) AMG_CHECK(lv_mail_init(&G->mail));
     G->n0 = n;
     G->xper = g.xperiodic;
     G->yper = g.yperiodic;

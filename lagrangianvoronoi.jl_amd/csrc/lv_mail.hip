@@ -28,10 +28,15 @@ hipError_t lv_mail_init(lv_mailbox *mb)
 {
     const size_t bytes = sizeof(int) * (1 + LV_MAIL_MAX);
     hipError_t e = hipHostMalloc((void **)&mb->host, bytes, hipHostMallocCoherent | hipHostMallocMapped);
-    if (e != hipSuccess) return e;
+    if (e != hipSuccess) {
+        mb->host = nullptr;
+        return e;
+    }
     memset(mb->host, 0, bytes);
     mb->seq = 0;
-    return hipHostGetDevicePointer((void **)&mb->dev, mb->host, 0);
+    e = hipHostGetDevicePointer((void **)&mb->dev, mb->host, 0);
+    if (e != hipSuccess) lv_mail_free(mb);
+    return e;
 }
 
 void lv_mail_free(lv_mailbox *mb)
