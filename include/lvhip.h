@@ -296,7 +296,7 @@ int lv_spai_outputs(lv_ctx *ctx, float *o_edge, float *o_node, float *w, float *
  * the context stream and accumulates their device time: every launch for on == 1, every on-th
  * launch for on > 1 (each event pair adds a few microseconds between the launches it brackets);
  * launches counts the bracketed ones. kernel ids: 0 = FP32 SpMV, 1 = FP64 SpMV, 2 = clipping,
- * 3 = cell-list scatter.  The algorithmic bytes of kernel 0 follow the layout of the
+ * 3 = the cell list.  The algorithmic bytes of kernel 0 follow the layout of the
  * last solve (the operator's own ELL, or the aggregate order's 8-bit degrees and 16-bit offsets). */
 int lv_timing_enable(lv_ctx *ctx, int32_t kernel_id, int32_t on);
 int lv_timing_read(lv_ctx *ctx, int32_t kernel_id, double *total_ms, int64_t *launches, double *bytes_per_launch);

@@ -86,8 +86,8 @@ void lv_amg_free(lv_amg *G);
 hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, const lv_pressure_system &A, int n,
                         const float *mval, const float *mdg, int layout, hipStream_t s);
 // A CG iteration's update left to the cycle (lv_amg_takes_update): x += alpha p, r_out = r - alpha q with
-// alpha = r.z / p.q from the partials of p.q, made by the down pass as it reads the rows; its partials of |r_out|^2 (one a
-// workgroup, G->nbfuse of them) are those of the cycle's head.
+// alpha = r.z / p.q from the partials of p.q, made by the down pass as it reads the rows; its partials of
+// |r_out|^2 (one a workgroup, G->nbfuse of them) are those of the cycle's head.
 struct lv_cycle_update {
     const float *p, *q, *r;
     float *x, *r_out;

@@ -19,8 +19,10 @@
 //            for the V-cycle: on the 2048^2 benchmark system PCG needs ~60 iterations with them,
 //            ~40 with 2 x 2);
 //   the coarsest level (<= LV_AMG_DENSE_MAX cells) is inverted densely once per assembly.
-// The levels of at most TAIL_MAX cells run inside one single-workgroup kernel per cycle (k_tail):
-// they are too small to fill the device, and one launch replaces two per level.  Above them, levels
+// The small levels (from the first of at most LDS_MAX cells, or TAIL_MAX in a singular system) run inside
+// one single-workgroup kernel per cycle (k_tail_lds; k_tail where its LDS does not hold them): they are
+// too small to fill the device, and one launch replaces two per level.  A singular system's cycle multiplies by
+// the matrix of that kernel's W-visit instead (k_mat_mv).  Above them, levels
 // 2 and up run in pairs, each pair as one down and one up kernel (k_st_down2, k_st_up2) that
 // recompute a halo around each workgroup's tile instead of waiting for a second launch.
 // Every sum is a gather in a fixed order (per-aggregate row lists are sorted), so the hierarchy
@@ -1041,10 +1043,11 @@ __global__ __launch_bounds__(B) void k_st_up(st_level L, int Kyc, const float *_
 // coordinates; the last cell of an odd periodic axis is its parent's only child, so that beyond the
 // wrap children and parents lie one cell nearer than twice and half (child_near, parent_near; ODD: a
 // periodic axis of level l or l+1 is odd.  The arithmetic costs a pair 1 us, so even ones go without).  Level
-// l is at least PAIR_MIN_K cells wide on both axes, so the unwrapped coordinates of every region stay within one width of the level and
-// one conditional add or subtract wraps them.  The down tile is small (PD = 4: 4 lanes of work per
-// cell of level l+2) so that the small levels spread over many workgroups; 8 x 8 tiles left one
-// wavefront per SIMD working through six halo cells a lane, no faster than two one-level kernels.
+// l is at least PAIR_MIN_K cells wide on both axes, so the unwrapped coordinates of every region stay
+// within one width of the level and one conditional add or subtract wraps them.  The down tile is small
+// (PD = 4: 4 lanes of work per cell of level l+2) so that the small levels spread over many workgroups;
+// 8 x 8 tiles left one wavefront per SIMD working through six halo cells a lane, no faster than two
+// one-level kernels.
 
 constexpr int PD = 4;   // down: a block owns PD x PD cells of level l+2
 constexpr int PU = 16;  // up: a block owns PU x PU cells of level l, one a lane
@@ -1591,9 +1594,9 @@ __device__ __forceinline__ void tail_step(int op, const tail_lev &L, const tail_
 // leading dimension ld: the operator is symmetric), and each cycle multiplies by the matrix (k_mat_mv).  The
 // W-visit is a serial chain of about 30 operations on one CU, 25-29 us a cycle whatever the rest of the device
 // does; the product reads at most 4 MB spread over the device in one round trip, 2.7-4.7 us, and the columns
-// take 60 us once per set-up (25 x 25 cells, 3 turns of the device).  A nonsingular system keeps the program: its V-visit takes 7-11 us, and its
-// solves keep their iterates bit for bit (velocities near rest are small differences of pressures, and
-// would show another rounding of the cycle magnified).
+// take 60 us once per set-up (25 x 25 cells, 3 turns of the device).  A nonsingular system keeps the
+// program: its V-visit takes 7-11 us, and its solves keep their iterates bit for bit (velocities near rest
+// are small differences of pressures, and would show another rounding of the cycle magnified).
 struct tail_lds_args {
     const int *desc, *prog;  // the levels' descriptors (LV_DESC ints each), the operations
     int nprog;
@@ -2446,7 +2449,8 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
         if (pairs && G->pair[l]) {
             const lv_amg_level &C2 = G->lev[l + 2];
             const st_pair q = st_pair_of(G, l);
-            hipLaunchKernelGGL(G->pair[l] == 2 ? k_st_down2<true> : k_st_down2<false>, dim3((C2.Kx + PD - 1) / PD, (C2.Ky + PD - 1) / PD), dim3(B), 0, s, q,
+            hipLaunchKernelGGL(G->pair[l] == 2 ? k_st_down2<true> : k_st_down2<false>,
+                               dim3((C2.Kx + PD - 1) / PD, (C2.Ky + PD - 1) / PD), dim3(B), 0, s, q,
                                (const float *)L.r, L.z, C.r, C.z, C2.r, S);
             l++;
             continue;
@@ -2464,8 +2468,12 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
         const bool pr = lt == 1 && prolong_in_up;
         const bool hd = update && lt == 1;  // (the update comes with pr there)
         constexpr int PT = TAIL_MAX / 256, PM = MAT_MAX / 256;
-        auto kern = LT.n <= TAIL_MAX ? (hd ? k_mat_mv<PT, true, true> : pr ? k_mat_mv<PT, true, false> : k_mat_mv<PT, false, false>)
-                                     : (hd ? k_mat_mv<PM, true, true> : pr ? k_mat_mv<PM, true, false> : k_mat_mv<PM, false, false>);
+        auto kern = LT.n <= TAIL_MAX ? (hd   ? k_mat_mv<PT, true, true>
+                                        : pr ? k_mat_mv<PT, true, false>
+                                             : k_mat_mv<PT, false, false>)
+                                     : (hd   ? k_mat_mv<PM, true, true>
+                                        : pr ? k_mat_mv<PM, true, false>
+                                             : k_mat_mv<PM, false, false>);
         hipLaunchKernelGGL(kern, dim3((LT.n + B / 64 - 1) / (B / 64)), dim3(B), 0, s, LT.n, G->mat_ld,
                            (const float *)G->mat, (const float *)LT.r, LT.t, S,
                            pr ? (const int *)G->start : (const int *)nullptr, G->fine_alpha, G->z0,
@@ -2478,7 +2486,8 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
     for (int l = lt - 1; l >= 1; l--) {
         if (pairs && l >= 3 && G->pair[l - 1]) {
             const lv_amg_level &L = G->lev[l - 1], &C = G->lev[l], &C2 = G->lev[l + 1];
-            hipLaunchKernelGGL(G->pair[l - 1] == 2 ? k_st_up2<true> : k_st_up2<false>, dim3((L.Kx + PU - 1) / PU, (L.Ky + PU - 1) / PU), dim3(B), 0, s,
+            hipLaunchKernelGGL(G->pair[l - 1] == 2 ? k_st_up2<true> : k_st_up2<false>,
+                               dim3((L.Kx + PU - 1) / PU, (L.Ky + PU - 1) / PU), dim3(B), 0, s,
                                st_pair_of(G, l - 1), (const float *)L.r, (const float *)L.z, (const float *)C.r,
                                (const float *)C.z, (const float *)C2.t, L.t, S);
             l--;

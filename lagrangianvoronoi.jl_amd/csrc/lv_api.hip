@@ -635,10 +635,6 @@ int grow_cell_list(lv_ctx *ctx, int64_t want)
 
 }  // namespace
 
-extern "C" {
-
-}  // extern "C"
-
 // remesh!; after a move whose error, if any, is in the flags
 static int remesh(lv_ctx *ctx)
 {

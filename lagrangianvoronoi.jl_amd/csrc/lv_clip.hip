@@ -9,11 +9,12 @@
 //     evaluates every edge at once, and 16 candidates are loaded and tested at once.  The shortest
 //     chain, for few seeds (lv_launch_clip), and for those that outgrow the other way's slots;
 //   * one thread owns a seed, its polygon in LDS as five slot-major planes (v1x, v1y, v2x, v2y, label),
-//     so lane t of the block addresses bank-conflict-free 8-byte words.  The fewest instructions, for
-//     many seeds.  Each polygon has CAP = 8 slots (18 KB per 64-seed block, which holds a CU at 8
-//     wavefronts), or 10 while the device holds them all at once (WIDE_MAX); a seed whose polygon outgrows them (0.4% at a 2048^2 jittered lattice, where no
-//     polygon passes 10 edges while it is clipped) is queued and clipped again from the start by a
-//     group, so the result is the same either way.
+//     so lane t of the block addresses bank-conflict-free 8-byte words, and mirrored in registers for the
+//     tests.  The fewest instructions, for many seeds.  Each polygon has CAP = 8 slots (18 KB per 64-seed
+//     block, which holds a CU at 8 wavefronts), or 10 while the device holds them all at once (WIDE_MAX);
+//     a seed whose polygon outgrows them (0.4% at a 2048^2 jittered lattice with eight, where no polygon
+//     passes 10 edges while it is clipped) is queued and clipped again from the start by a group, so the
+//     result is the same either way.
 //
 // The edge list keeps the reference's storage semantics exactly: cut edges are rewritten in place,
 // deleted edges are replaced by the last edge (FastVector deleteat!, src/fastvector.jl:44-50) and
@@ -622,11 +623,11 @@ __device__ __forceinline__ int clip_seed_of(const lv_grid_params &g, int n, int 
 }
 
 // The chunk a workgroup works on and its part of it.  Workgroups are dispatched round-robin over the 8
-// XCDs, so workgroup b runs on XCD b mod 8: 32 workgroups take 8 chunks, the four parts of a chunk on one XCD,
-// whose L2 joins their stores.  The clipping work per seed varies across the domain, and mapped straight each XCD would get
-// every 8th chunk, on a lattice whose rows span a multiple of 8 chunks the same few column strips of
-// the domain in every row: XCDs with the costly strips ran up to 28% longer while the others idled for
-// the last third of the launch.  Rotating each group by a hash of its index (the top 3 bits of a
+// XCDs, so workgroup b runs on XCD b mod 8: 32 workgroups take 8 chunks, the four parts of a chunk on one
+// XCD, whose L2 joins their stores.  The clipping work per seed varies across the domain, and mapped
+// straight each XCD would get every 8th chunk, on a lattice whose rows span a multiple of 8 chunks the same
+// few column strips of the domain in every row: XCDs with the costly strips ran up to 28% longer while the
+// others idled for the last third of the launch.  Rotating each group by a hash of its index (the top 3 bits of a
 // multiplicative hash, so that no period of the domain lines up with it) gives every XCD an even share
 // of every column.
 __device__ __forceinline__ void clip_chunk(int b, int &chunk, int &part)
@@ -703,7 +704,8 @@ hipError_t lv_launch_clip(const lv_grid_params &g, int n, const double *x, const
     if (!all) {
         hipError_t e = hipMemsetAsync(retry, 0, sizeof(int), s);
         if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(n <= WIDE_MAX ? k_clip<10> : k_clip<8>, dim3((n + 8 * CHUNK - 1) / (8 * CHUNK) * 32), dim3(CB), 0, s, g, n, x, cell_start, cell_labels, cell_x, m,
+        hipLaunchKernelGGL(n <= WIDE_MAX ? k_clip<10> : k_clip<8>, dim3((n + 8 * CHUNK - 1) / (8 * CHUNK) * 32),
+                           dim3(CB), 0, s, g, n, x, cell_start, cell_labels, cell_x, m,
                            path_i, path_rr, ne, ev, el, ld, area, cent, err, retry);
     }
     hipLaunchKernelGGL(k_clip_group, dim3(all ? groups : std::min(RETRY_BLOCKS, groups)), dim3(GB), 0, s, g, n, x,

@@ -939,8 +939,9 @@ __global__ __launch_bounds__(B) void k_shift(int n, double *__restrict__ x, cons
 
 // ---- FP32 inner PCG of the refinement --------------------------------------------------------
 
-// A first sweep that k_cg32_init flagged skip (initial residual within tol, zero, or NaN) must leave x as it is: its FP32 vectors are zeros and its correction scale is 0, so neither
-// 1/sqrt(0) nor a NaN residual reaches x.
+// A first sweep that k_cg32_init flagged skip (initial residual within tol, zero, or NaN) must leave x as
+// it is: its FP32 vectors are zeros and its correction scale is 0, so neither 1/sqrt(0) nor a NaN residual
+// reaches x.
 __device__ inline bool sweep_skipped(const lv_cg_scalars *S, int first) { return first && S->skip; }
 
 // r32 = r64 / |r64|, e = 0, z = dinv r, p = z; partials r.z, r.r.  With perm, the FP32 vectors
@@ -1937,8 +1938,8 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
         double *Pxs = A.singular ? P.ur : nullptr;
         // the iterations of a sweep are still in S at the next sweep's read of the FP64 residual
         // (k_resid64 and k_finalize leave them), so a sweep ends without a synchronising read.
-        // Nor does the first sweep wait for one: k_cg32_init makes the tests below on the device, and a first sweep with nothing to solve starts done and changes nothing
-        // (its correction is zero).
+        // Nor does the first sweep wait for one: k_cg32_init makes the tests below on the device, and a first
+        // sweep with nothing to solve starts done and changes nothing (its correction is zero).
         bool pending = false;
         double itol = 0.0;
         for (;;) {
