@@ -36,6 +36,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "lv_amg.h"
 #include "lv_ell.h"
@@ -2513,6 +2514,15 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
         if (!prolong_in_up)
             hipLaunchKernelGGL(k_prolong1, g1((n + PROLONG_RPT - 1) / PROLONG_RPT), dim3(B), 0, s, n, agg,
                                (const float *)L1.t, G->fine_alpha, G->z0, S);
+        if constexpr (std::is_same<V, lv_ell_agg16>::value) {
+            if (n > LV_NT_ROWS) {
+                typedef decltype(lv_ell_streamed(F.A)) VS;
+                const fine_ops<VS> FS{F.n, lv_ell_streamed(F.A), F.diag, F.dinv, F.mval, F.mdg, F.scale, F.alpha};
+                hipLaunchKernelGGL(k_fine_up_j<VS>, dim3(lv_nblocks(n)), dim3(B), 0, s, FS, r, (const float *)G->z0, z,
+                                   Prr, S);
+                return hipGetLastError();
+            }
+        }
         hipLaunchKernelGGL(k_fine_up_j<V>, dim3(lv_nblocks(n)), dim3(B), 0, s, F, r, (const float *)G->z0, z, Prr, S);
     }
     return hipGetLastError();

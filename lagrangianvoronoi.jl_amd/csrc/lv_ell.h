@@ -54,7 +54,15 @@ __host__ __device__ __forceinline__ uint16_t lv_bf16_bits(float f)
 #define LV_OVF_BASE 6
 #define LV_OVF_CAP 64
 
-template <typename DEG, typename COL, typename VAL>
+// NT: the slots' columns and values are loaded non-temporally.  A V-cycle-preconditioned iteration of more than
+// LV_NT_ROWS rows streams the Krylov operator's and the up pass's matrices and its solution vector this way: they
+// would otherwise push the vectors that the next kernel reads again out of the 256 MB last-level cache.  A step of
+// 2048 x 2048 particles 53.3 -> 52.1 ms (k_cg_s 58.6 -> 57.3 us, the up pass 47.2 -> 46.3, k_cg_u 24.1 -> 21.7 by the
+// matrices alone), of 4096 x 4096 151.0 -> 149.7 by the matrices alone.  Smaller systems find part of the matrices still
+// cached: with streaming, 1732 x 1732 goes 39.9 -> 40.1 and 1448 x 1448 27.9 -> 29.3, so the line lies between 3.0
+// and 4.2 million rows.  The down pass is not streamed (47.6 -> 51.7 us at 2048 x 2048).
+#define LV_NT_ROWS (7 << 19)
+template <typename DEG, typename COL, typename VAL, bool NT = false>
 struct lv_ell_view {
     const DEG *deg;
     const COL *col;
@@ -63,9 +71,30 @@ struct lv_ell_view {
     const VAL *oval = nullptr;
     int ocap = 0;               // groups with at most this many overflow slots use it (0: none)
     __device__ __forceinline__ int degree(int i) const { return lv_ell_deg(deg, i); }
-    __device__ __forceinline__ int column(size_t e, int i, int n) const { return lv_ell_col(col, e, i, n); }
-    __device__ __forceinline__ auto value(size_t e) const { return lv_ell_val(val, e); }
+    __device__ __forceinline__ int column(size_t e, int i, int n) const
+    {
+        if constexpr (NT) {
+            const COL c = __builtin_nontemporal_load(col + e);
+            return lv_ell_col(&c, 0, i, n);
+        }
+        return lv_ell_col(col, e, i, n);
+    }
+    __device__ __forceinline__ auto value(size_t e) const
+    {
+        if constexpr (NT) {
+            const VAL v = __builtin_nontemporal_load(val + e);
+            return lv_ell_val(&v, 0);
+        }
+        return lv_ell_val(val, e);
+    }
 };
+
+// the same view, streamed
+template <typename DEG, typename COL, typename VAL>
+lv_ell_view<DEG, COL, VAL, true> lv_ell_streamed(const lv_ell_view<DEG, COL, VAL> &A)
+{
+    return {A.deg, A.col, A.val, A.ocol, A.oval, A.ocap};
+}
 
 // Where row i's overflow slots start in its group, and the group's total: the exclusive prefix and
 // the sum of max(d - LV_OVF_BASE, 0) over the wavefront's lanes, by one ballot per overflow depth.
@@ -190,8 +219,8 @@ template <class V>
 struct lv_ell_compact {
     static constexpr bool value = false;
 };
-template <typename DEG, typename COL, typename VAL>
-struct lv_ell_compact<lv_ell_view<DEG, COL, VAL>> {
+template <typename DEG, typename COL, typename VAL, bool NT>
+struct lv_ell_compact<lv_ell_view<DEG, COL, VAL, NT>> {
     static constexpr bool value = true;
 };
 

@@ -718,7 +718,8 @@ __global__ __launch_bounds__(B, (cg_waves<T, COMPACT>::value)) void k_cg_s(int n
 // x += alpha p, r -= alpha q.  With Jacobi (JACOBI) also z = D^-1 r and the partials of r.z, r.r
 // for the next k_cg_s; otherwise the partials of r.r alone (Pur), which k_conv_check tests before
 // the preconditioner is applied, and with z0 the multilevel cycle's pre-smoothed z0 = sc D^-1 r.
-template <typename T, bool JACOBI>
+// NT: x, which nothing else in the iteration reads, is streamed past the caches (LV_NT_ROWS).
+template <typename T, bool JACOBI, bool NT = false>
 __global__ __launch_bounds__(B) void k_cg_u(int n, T *__restrict__ x, T *__restrict__ r, T *__restrict__ z,
                                             const T *__restrict__ p, const T *__restrict__ q,
                                             const T *__restrict__ dinv, const double *__restrict__ Ppq,
@@ -739,7 +740,10 @@ __global__ __launch_bounds__(B) void k_cg_u(int n, T *__restrict__ x, T *__restr
     const T a = (T)alpha;
     double v[2] = {0.0, 0.0};
     for (int i = blockIdx.x * B + threadIdx.x; i < n; i += gridDim.x * B) {
-        x[i] += a * p[i];
+        if constexpr (NT)
+            __builtin_nontemporal_store(__builtin_nontemporal_load(x + i) + a * p[i], x + i);
+        else
+            x[i] += a * p[i];
         const T ri = r[i] - a * q[i];
         r[i] = ri;
         if (!JACOBI && z0) z0[i] = sc * dinv[i] * ri;
@@ -1829,8 +1833,8 @@ hipError_t cg_iterate(int n, V A, const T *diag, const T *dinv, T *x, T *r, T *z
                     z0 = M->amg->z0;
                     sc = M->amg->fine_scale;
                 }
-            hipLaunchKernelGGL((k_cg_u<T, false>), dim3(nb), dim3(B), 0, s, n, x, r, z, (const T *)p,
-                               (const T *)q, dinv, (const double *)P.pq, P.rr, P.ur, dS, par, z0, sc);
+            hipLaunchKernelGGL((n > LV_NT_ROWS ? k_cg_u<T, false, true> : k_cg_u<T, false>), dim3(nb), dim3(B), 0, s, n,
+                               x, r, z, (const T *)p, (const T *)q, dinv, (const double *)P.pq, P.rr, P.ur, dS, par, z0, sc);
             const bool head = M->amg && lv_amg_takes_head(M->amg, nb);
             if (!head)
                 hipLaunchKernelGGL(k_conv_check, dim3(1), dim3(B), 0, s, (const double *)P.ur, nb, dS, dprog, k);
@@ -1996,12 +2000,14 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
                                        (const lv_cg_scalars *)W.S);
                 }
                 int done = 0;
-                if (Gp)
-                    e = cg_iterate<float>(n, lv_ell_agg32{Gp->pdeg, Gp->poff, Gp->pev32, Gp->ooff, Gp->oev32, Gp->ovf_cap},
-                                          (const float *)Gp->pdiag32,
-                                          dinv32, W.e32, W.r32, W.z32, W.p32, W.q32, P, W.S, W.hprog, W.dprog,
-                                          W.hS, s, t32, h, Mi, &done);
-                else
+                if (Gp) {
+                    const lv_ell_agg32 V{Gp->pdeg, Gp->poff, Gp->pev32, Gp->ooff, Gp->oev32, Gp->ovf_cap};
+                    auto iterate = [&](const auto &Av) {
+                        return cg_iterate<float>(n, Av, (const float *)Gp->pdiag32, dinv32, W.e32, W.r32, W.z32, W.p32,
+                                                 W.q32, P, W.S, W.hprog, W.dprog, W.hS, s, t32, h, Mi, &done);
+                    };
+                    e = n > LV_NT_ROWS ? iterate(lv_ell_streamed(V)) : iterate(V);
+                } else
                     e = cg_iterate<float>(n, own32(A, n, opt.amg_layout), (const float *)A.diag32,
                                           dinv32, W.e32, W.r32, W.z32, W.p32, W.q32, P, W.S, W.hprog, W.dprog,
                                           W.hS, s, t32, h, Mi, &done);
