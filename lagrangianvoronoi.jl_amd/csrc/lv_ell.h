@@ -57,8 +57,8 @@ __host__ __device__ __forceinline__ uint16_t lv_bf16_bits(float f)
 // NT: the slots' columns and values are loaded non-temporally.  A V-cycle-preconditioned iteration of more than
 // LV_NT_ROWS rows streams the Krylov operator's and the up pass's matrices and its solution vector this way: they
 // would otherwise push the vectors that the next kernel reads again out of the 256 MB last-level cache.  A step of
-// 2048 x 2048 particles 53.3 -> 52.1 ms (k_cg_s 58.6 -> 57.3 us, the up pass 47.2 -> 46.3, k_cg_u 24.1 -> 21.7 by the
-// matrices alone), of 4096 x 4096 151.0 -> 149.7 by the matrices alone.  Smaller systems find part of the matrices still
+// 2048 x 2048 particles 53.3 -> 52.1 ms (k_cg_s 59.3 -> 57.9 us, the up pass 47.0 -> 43.8, k_cg_u 24.0 -> 22.8, level
+// 1's passes 34.2 -> 30.8), of 4096 x 4096 151.0 -> 148.5.  Smaller systems find part of the matrices still
 // cached: with streaming, 1732 x 1732 goes 39.9 -> 40.1 and 1448 x 1448 27.9 -> 29.3, so the line lies between 3.0
 // and 4.2 million rows.  The down pass is not streamed (47.6 -> 51.7 us at 2048 x 2048).
 #define LV_NT_ROWS (7 << 19)
