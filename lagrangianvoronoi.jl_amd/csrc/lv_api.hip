@@ -245,6 +245,14 @@ double *field_ptr(lv_ctx *c, int f, size_t *count, size_t *elem, bool *readonly)
 lv_mesh_view mesh_view(lv_ctx *c) { return lv_mesh_view{c->ne, c->ev, c->el, c->n}; }
 
 constexpr int NFLAGS = 5;
+// device memory to the host behind everything queued on the context's stream (which the null stream of a plain
+// hipMemcpy does not wait for), complete on return
+hipError_t fetch(lv_ctx *ctx, void *dst, const void *src, size_t bytes)
+{
+    hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->s);
+    return e == hipSuccess ? hipStreamSynchronize(ctx->s) : e;
+}
+
 hipError_t post_flags(lv_ctx *ctx) { return lv_mail_post(&ctx->mail, ctx->d_flags, NFLAGS, 3, ctx->s); }
 hipError_t await_flags(lv_ctx *ctx, int *flags) { return lv_mail_await(&ctx->mail, flags, NFLAGS, ctx->s); }
 
@@ -885,13 +893,13 @@ int export_columns(lv_ctx *ctx, const int32_t *fields, int32_t nfields, std::vec
         std::vector<double> &c = cols[a];
         if (ef->id == LV_FIELD_PHASE) {
             std::vector<int> h(n);
-            if (n) LV_HIP_CHECK(hipMemcpy(h.data(), p, sizeof(int) * n, hipMemcpyDeviceToHost));
+            if (n) LV_HIP_CHECK(fetch(ctx, h.data(), p, sizeof(int) * n));
             c.assign(h.begin(), h.end());
             arr[a] = lv_vtk_array{ef->name, 1, c.data()};
             continue;
         }
         std::vector<double> h(count);
-        if (count) LV_HIP_CHECK(hipMemcpy(h.data(), p, sizeof(double) * count, hipMemcpyDeviceToHost));
+        if (count) LV_HIP_CHECK(fetch(ctx, h.data(), p, sizeof(double) * count));
         if (count == (size_t)n) {
             c = std::move(h);
             arr[a] = lv_vtk_array{ef->name, 1, c.data()};
@@ -920,7 +928,7 @@ int lv_export_grid(lv_ctx *ctx, const char *filename, const int32_t *fields, int
     int64_t o = 0;
     if ((rc = mesh_offsets(ctx, &o))) return rc;
     std::vector<int> ptr((size_t)n + 1);
-    LV_HIP_CHECK(hipMemcpy(ptr.data(), ctx->clip_retry, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToHost));
+    LV_HIP_CHECK(fetch(ctx, ptr.data(), ctx->clip_retry, sizeof(int) * ((size_t)n + 1)));
     std::vector<double> pts((size_t)3 * o);
     if ((rc = mesh_rows<2>(ctx, ptr.data(), nullptr, pts.data()))) return rc;
     std::vector<int64_t> conn(o), offs(ptr.begin() + 1, ptr.end());
@@ -943,7 +951,7 @@ int lv_export_points(lv_ctx *ctx, const char *filename, const int32_t *fields, i
     if (!filename || nfields < 0 || (nfields > 0 && !fields)) return lv_fail(ctx, LV_E_INVALID, "lv_export_points");
     const int n = ctx->n;
     std::vector<double> x((size_t)2 * n), pts((size_t)3 * n);
-    if (n) LV_HIP_CHECK(hipMemcpy(x.data(), ctx->F.x, sizeof(double) * 2 * n, hipMemcpyDeviceToHost));
+    if (n) LV_HIP_CHECK(fetch(ctx, x.data(), ctx->F.x, sizeof(double) * 2 * n));
     std::vector<int64_t> conn(n), offs(n);
     for (int i = 0; i < n; i++) {
         pts[3 * (size_t)i] = x[i];
@@ -1138,8 +1146,8 @@ int lv_get_cell_list(lv_ctx *ctx, int32_t *cell_start, int32_t *cell_labels)
     int rc = check_ctx(ctx, true);
     if (rc) return rc;
     const int64_t ncells = (int64_t)ctx->g.n1 * ctx->g.n2;
-    LV_HIP_CHECK(hipMemcpy(cell_start, ctx->cell_start, sizeof(int) * (ncells + 1), hipMemcpyDeviceToHost));
-    LV_HIP_CHECK(hipMemcpy(cell_labels, ctx->cell_labels, sizeof(int) * ctx->nitems, hipMemcpyDeviceToHost));
+    LV_HIP_CHECK(fetch(ctx, cell_start, ctx->cell_start, sizeof(int) * (ncells + 1)));
+    LV_HIP_CHECK(fetch(ctx, cell_labels, ctx->cell_labels, sizeof(int) * ctx->nitems));
     return LV_OK;
 }
 
@@ -1253,10 +1261,10 @@ int lv_get_pressure_operator(lv_ctx *ctx, double *diag, int32_t *row_ptr, int32_
     rc = need_pressure_operator(ctx);
     if (rc) return rc;
     const int n = ctx->n;
-    LV_HIP_CHECK(hipMemcpy(diag, ctx->A.diag64, sizeof(double) * n, hipMemcpyDeviceToHost));
-    LV_HIP_CHECK(hipMemcpy(row_ptr, ctx->A.row_ptr, sizeof(int) * (n + 1), hipMemcpyDeviceToHost));
-    if (cols) LV_HIP_CHECK(hipMemcpy(cols, ctx->A.cols, sizeof(int) * ctx->A.nnz, hipMemcpyDeviceToHost));
-    if (coef) LV_HIP_CHECK(hipMemcpy(coef, ctx->A.val64, sizeof(double) * ctx->A.nnz, hipMemcpyDeviceToHost));
+    LV_HIP_CHECK(fetch(ctx, diag, ctx->A.diag64, sizeof(double) * n));
+    LV_HIP_CHECK(fetch(ctx, row_ptr, ctx->A.row_ptr, sizeof(int) * (n + 1)));
+    if (cols) LV_HIP_CHECK(fetch(ctx, cols, ctx->A.cols, sizeof(int) * ctx->A.nnz));
+    if (coef) LV_HIP_CHECK(fetch(ctx, coef, ctx->A.val64, sizeof(double) * ctx->A.nnz));
     return LV_OK;
 }
 
