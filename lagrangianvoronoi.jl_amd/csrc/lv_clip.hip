@@ -43,6 +43,10 @@ struct clip_lds {
     double term[GB / G][3][G];        // area and centroid terms by edge position
 };
 
+// The move in front of this remesh was refused (a NaN velocity), which the host learns with the remesh's own
+// flags: the polygons, areas and centroids stay those of the last remesh.  err: as the kernel found it.
+__device__ __forceinline__ bool move_refused(int err) { return err == LV_E_NAN_VELOCITY; }
+
 __device__ __forceinline__ int signum(double v)
 {
     if (v < -SIGNUM_EPS) return -1;
@@ -651,11 +655,12 @@ __global__ __launch_bounds__(CB) void k_clip(lv_grid_params g, int n, const doub
     __shared__ lds_poly<CAP> P;
     __shared__ unsigned char ord[CHUNK];
     const int t = threadIdx.x;
+    const int before = *err;
     int chunk, part;
     clip_chunk(blockIdx.x, chunk, part);
     if (chunk * CHUNK >= n) return;
     const int i = clip_seed_of<2>(g, n, chunk, part, x, ord);
-    if (i >= n) return;  // no block-wide barriers below
+    if (i >= n || move_refused(before)) return;  // no block-wide barriers below
     if (!clip_seed(g, n, i, x, cell_start, cell_labels, cell_x, m, path_i, path_rr, ne, ev, el, ld, area, cent, err, P, t))
         retry[1 + atomicAdd(&retry[0], 1)] = i;
 }
@@ -673,7 +678,9 @@ __global__ __launch_bounds__(GB) void k_clip_group(lv_grid_params g, int n, cons
 {
     __shared__ clip_lds S;
     const int l = threadIdx.x & (G - 1), gi = threadIdx.x / G;
+    const int before = *err;
     const int cnt = queue ? queue[0] : n;
+    if (move_refused(before)) return;
     for (int q = blockIdx.x * (GB / G) + gi; q < cnt; q += gridDim.x * (GB / G))
         group_clip_seed(g, n, queue ? queue[1 + q] : q, l, gi, x, cell_start, cell_labels, cell_x, m, path_i, path_rr, ne,
                         ev, el, ld, area, cent, err, S);

@@ -79,3 +79,19 @@ def test_more_seeds_than_the_first_list(lv, gpu):
         assert np.array_equal(a, b)
     for a, b in zip(grid.cell_list(), fresh.cell_list()):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("K", [20, 190, 320])
+def test_a_refused_move_leaves_the_polygons_of_the_last_remesh(lv, gpu, tmp_path, K):
+    print("refused move %d" % K, flush=True)
+    grid = lv.VoronoiGrid(lv.UnitRectangle(), 1.0 / K, xperiodic=True, yperiodic=True, positions=_lattice(lv, K, 0.45))
+    lv.remesh(grid)
+    area = grid.get("area")
+    polygons = open(lv.export_grid(grid, str(tmp_path / "before")), "rb").read()
+    v = np.full(2 * grid.n, 0.25)
+    v[5] = np.nan
+    grid.set("v", v)
+    with pytest.raises(lv.LVError, match="Velocity field invalidated"):
+        lv.move(grid, 0.5 / K)
+    assert np.array_equal(grid.get("area"), area)
+    assert open(lv.export_grid(grid, str(tmp_path / "after")), "rb").read() == polygons
