@@ -235,12 +235,12 @@ __device__ __forceinline__ void group_clip_seed(const lv_grid_params &g, int n, 
         bool stop = false;
         for (int c0 = 0; c0 < total && !stop; c0 += LCAP) {
             lds_visible();
-            for (int s = s0; s < s1; s++) {
-                const int o = pre + (s - s0) - c0;
-                if (o >= 0 && o < LCAP) {
-                    S.s[gi][o] = s;
-                    S.q[gi][o] = (unsigned char)l;
-                }
+            // (of each node only what falls into these LCAP: going through all of it for every LCAP made a seed's work
+            // quadratic in its candidates: 8,000 seeds in one cell 46 ms, 0.76 this way)
+            const int first = max(0, c0 - pre), end = min(s1 - s0, c0 + LCAP - pre);
+            for (int t = first; t < end; t++) {
+                S.s[gi][pre + t - c0] = s0 + t;
+                S.q[gi][pre + t - c0] = (unsigned char)l;
             }
             lds_visible();
             const int cnt = min(LCAP, total - c0);

@@ -67,3 +67,35 @@ def test_mesh_at_the_lines_between_the_ways(lv, oracle, gpu, K, periodic):
     x = lv.inputs.jittered_lattice(K, K, 1.0 / K, jitter=0.45, seed=0x5EED0B80 + K)
     grid = _same_mesh(lv, oracle, x, 1.0 / K, periodic)
     assert (grid.n <= 32768) == (K == 181) and (grid.n <= 98304) == (K < 314)
+
+
+def _clip_ms(lv, n, h):
+    import ctypes
+
+    grid = lv.VoronoiGrid(lv.UnitRectangle(), 1.0 / np.sqrt(n), h=h, r_max=3.0,
+                          positions=np.random.default_rng(n).random(2 * n))
+    lv.remesh(grid)
+    assert lv.lib().lv_timing_enable(grid.ctx, 2, 1) == 0
+    lv.remesh(grid)
+    ms, count = ctypes.c_double(), ctypes.c_int64()
+    assert lv.lib().lv_timing_read(grid.ctx, 2, ctypes.byref(ms), ctypes.byref(count), None) == 0
+    assert count.value == 1
+    return ms.value
+
+
+def test_crowded_cells_are_read_once_by_a_group(lv, oracle, gpu):
+    """Every seed in one cell, 2,000 and then 8,000 of them.  Four times the candidates for a seed, and its groups' 2,000
+    wavefronts share the 1,024 SIMDs, two to each, where 500 had one to themselves: at most eight times as long, if a
+    group lists each candidate once.  (Reading the cell anew for every 64 of its candidates makes it 16 times the
+    reads a seed.)"""
+    print("clip crowded", flush=True)
+    few, many = (min(_clip_ms(lv, n, 1.0) for _ in range(3)) for n in (2000, 8000))
+    print("clip crowded: %.2f ms, %.2f ms" % (few, many), flush=True)
+    assert many <= 8.0 * few
+    x = np.random.default_rng(5).random(2 * 3000)
+    grid = lv.VoronoiGrid(lv.UnitRectangle(), 1.0 / np.sqrt(3000), h=0.5, r_max=3.0, positions=x)
+    lv.remesh(grid)
+    op = oracle.Particles(oracle.Grid((0.0, 0.0), (1.0, 1.0), 1.0 / np.sqrt(3000), h=0.5, r_max=3.0), x)
+    op.remesh()
+    for a, b in zip(grid.mesh(), op.mesh()):
+        assert np.array_equal(a, b)
