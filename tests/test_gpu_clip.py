@@ -102,7 +102,7 @@ def test_crowded_cells_are_read_once_by_a_group(lv, oracle, gpu):
 
 
 @pytest.mark.parametrize("n,h,periodic", [(32768, 2.0, False), (32769, 2.0, False), (98304, 2.0, False), (98305, 2.0, False),
-                                          (98304 + 255, 0.5, True), (131073, 0.5, True)])
+                                          (98304 + 255, 1.0, True), (131073, 1.0, True)])
 def test_mesh_of_random_seeds_at_the_lines_between_the_ways(lv, oracle, gpu, n, h, periodic):
     """random seeds, whose polygons outgrow a thread's slots far more often than a lattice's: on either side of both lines,
     and with eight slots a last chunk and a last group of chunks that are not full"""
