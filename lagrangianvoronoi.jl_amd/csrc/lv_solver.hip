@@ -1862,6 +1862,66 @@ hipError_t cg_iterate(int n, V A, const T *diag, const T *dinv, T *x, T *r, T *z
 
 }  // namespace
 
+// One run of the FP64 Jacobi-PCG from x, at most itmax iterations: h holds the sums and iterations of the run, with
+// the true residual of the returned x (which is also left in W.r) and, in rr64_0, of the guess.
+static hipError_t run_pcg64(const lv_pressure_system &A, lv_solver_work &W, int n, const double *b, double *x,
+                            const lv_solve_opts &opt, int itmax, hipStream_t s, lv_timer *t64, lv_cg_scalars &h)
+{
+    const int nb = nblocks_of(n);
+    const dim3 G(nb);
+    const parts P = parts_of(W.partials);
+    const double tol2 = opt.tol * opt.tol;
+    memset(&h, 0, sizeof(h));
+    // a small system in one launch (not while its launches are being timed)
+    if (n <= PS_MAX_ROWS && !(t64 && t64->on)) {
+        double *slots = W.partials + (size_t)8 * NBMAX;
+        const int seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
+        const ps_ring Z{{W.z, W.p, W.q}};
+        hipLaunchKernelGGL(k_ps_init, G, dim3(B), 0, s, W.S, tol2, itmax, (int)A.singular, slots, n, Z);
+        hipLaunchKernelGGL(k_pcg_small, G, dim3(B), 0, s, n, own64(A, n), (const double *)A.diag64,
+                           (const double *)A.dinv64, b, x, W.r, Z, tol2, itmax, (int)A.singular, slots, W.S, W.dprog,
+                           seq);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+        e = await_published(W.hprog, seq, W.S, W.hS, &h, s);
+        if (e != hipSuccess) return e;
+        if (h.skip == PS_OK) return hipSuccess;
+        // some workgroup was not scheduled in time: launch by launch, after the last of them has ended
+        e = hipStreamSynchronize(s);
+        if (e != hipSuccess) return e;
+        memset(&h, 0, sizeof(h));
+    }
+    hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, tol2, itmax, (int)A.singular);
+    // (the means of b and x serve singular systems only: elsewhere bmean stays 0, and xmean0 is read only where
+    // x's mean is restored)
+    if (A.singular) {
+        hipLaunchKernelGGL(k_means, G, dim3(B), 0, s, n, b, (const double *)x, P.p3);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_MEANS, n, W.S);
+    }
+    const lv_ell_own<double> V = own64(A, n, opt.amg_layout);
+    LV_LAUNCH_BY_OCAP(k_cg64_init, V, G, dim3(B), 0, s, n, V, (const double *)A.diag64, (const double *)A.dinv64, b,
+                      (const double *)x, W.r, W.z, P.rr, P.p3, (const lv_cg_scalars *)W.S);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_INIT64, n, W.S);
+    int done = 0;
+    hipError_t e = cg_iterate<double>(n, V, (const double *)A.diag64, (const double *)A.dinv64, x, W.r, W.z, W.p, W.q, P,
+                                      W.S, W.hprog, W.dprog, W.hS, s, t64, h, (const lv_precond *)nullptr, &done);
+    if (e != hipSuccess) return e;
+    // the FP64 residual of the returned x
+    if (A.singular) {
+        hipLaunchKernelGGL(k_sum1, G, dim3(B), 0, s, n, (const double *)x, P.p3);
+        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_SUM1, n, W.S);
+        hipLaunchKernelGGL(k_shift, G, dim3(B), 0, s, n, x, (const lv_cg_scalars *)W.S);
+    }
+    launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3, (const double *)nullptr,
+                   (const double *)nullptr, W.S);
+    hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n, W.S);
+    e = read_scalars(W.S, W.hS, &h, s);
+    h.rr64_0 = h.rr0;
+    return e;
+}
+
+static double relative(double rr, double bb) { return bb > 0.0 ? sqrt(rr / bb) : sqrt(rr); }
+
 // Solves A x = b (device vectors; x holds the initial guess and is iterated in place).  Writes
 // iterations, sweeps and the final FP64 relative residual.  *converged tells whether tol was met.
 hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n, const double *b, double *x,
@@ -1876,175 +1936,135 @@ hipError_t lv_solve_device(const lv_pressure_system &A, lv_solver_work &W, int n
     const parts P = parts_of(W.partials);
     lv_cg_scalars h;
     memset(&h, 0, sizeof(h));
-    // a small FP64 solve in one launch (not while its launches are being timed)
-    if (opt.method == LV_SOLVER_PCG64 && n <= PS_MAX_ROWS && !(t64 && t64->on)) {
-        double *slots = W.partials + (size_t)8 * NBMAX;
-        const double tol2 = opt.tol * opt.tol;
-        const int itmax = opt.itmax > 0 ? opt.itmax : 1000, seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
-        const ps_ring Z{{W.z, W.p, W.q}};
-        hipLaunchKernelGGL(k_ps_init, G, dim3(B), 0, s, W.S, tol2, itmax, (int)A.singular, slots, n, Z);
-        hipLaunchKernelGGL(k_pcg_small, G, dim3(B), 0, s, n, own64(A, n), (const double *)A.diag64,
-                           (const double *)A.dinv64, b, x, W.r, Z, tol2, itmax, (int)A.singular, slots, W.S, W.dprog,
-                           seq);
-        hipError_t e1 = hipGetLastError();
-        if (e1 != hipSuccess) return e1;
-        e1 = await_published(W.hprog, seq, W.S, W.hS, &h, s);
-        if (e1 != hipSuccess) return e1;
-        if (h.skip == PS_OK) {
-            *iters = h.iters;
-            *sweeps = 0;
-            *relres0 = (h.bb > 0.0) ? sqrt(h.rr64_0 / h.bb) : sqrt(h.rr64_0);
-            *relres = (h.bb > 0.0) ? sqrt(h.rr64 / h.bb) : sqrt(h.rr64);
-            *converged = (h.rr64 <= h.thr2);
-            return hipSuccess;
-        }
-        // some workgroup was not scheduled in time: launch by launch, after the last of them has ended
-        e1 = hipStreamSynchronize(s);
-        if (e1 != hipSuccess) return e1;
-        memset(&h, 0, sizeof(h));
-    }
     const double tol2 = opt.tol * opt.tol;
     const int itmax = opt.itmax > 0 ? opt.itmax : 1000;
     hipError_t e = hipSuccess;
-    // the means of b and x serve singular systems only (elsewhere bmean stays the 0 that S starts from, and xmean0
-    // is read only where x's mean is restored)
-    double *Pm = nullptr;  // their partials, which the first residual of a refinement sums
+    int total = 0;
     if (opt.method == LV_SOLVER_PCG64) {
-        hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, tol2, itmax, (int)A.singular);
-        if (A.singular) {
-            hipLaunchKernelGGL(k_means, G, dim3(B), 0, s, n, b, (const double *)x, P.p3);
-            hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_MEANS, n, W.S);
+        // A run ends on its recurrence's residual, from which the true one drifts: little at 1e-10, by a tenth of it and
+        // more at 1e-13.  Where the true one misses the tolerance the next run starts from it, once, and again
+        // while that at least halves it.
+        double last = 0.0;
+        for (int run = 0;; run++) {
+            e = run_pcg64(A, W, n, b, x, opt, itmax - total, s, t64, h);
+            if (e != hipSuccess) return e;
+            total += h.iters;
+            if (run == 0) *relres0 = relative(h.rr64_0, h.bb);
+            if (h.rr64 <= h.thr2 || !(h.rr64 == h.rr64) || total >= itmax || h.iters == 0) break;
+            if (run > 0 && !(4.0 * h.rr64 <= last)) break;
+            last = h.rr64;
         }
-    } else if (A.singular) {
+        *iters = total;
+        *sweeps = 0;
+        *relres = relative(h.rr64, h.bb);
+        *converged = (h.rr64 <= h.thr2);
+        return hipSuccess;
+    }
+    // the partials of the means of b and x, which the first residual sums (a singular system; elsewhere bmean stays the
+    // 0 that S starts from, and xmean0 is read only where x's mean is restored)
+    double *Pm = nullptr;
+    if (A.singular) {
         Pm = P.ur;
         hipLaunchKernelGGL(k_means, G, dim3(B), 0, s, n, b, (const double *)x, Pm);
     }
-    int total = 0, nsweep = 0, skipped = 0;
-    if (opt.method == LV_SOLVER_PCG64) {
-        LV_LAUNCH_BY_OCAP(k_cg64_init, own64(A, n, opt.amg_layout), G, dim3(B), 0, s, n, own64(A, n, opt.amg_layout), (const double *)A.diag64, (const double *)A.dinv64, b,
-                           (const double *)x, W.r, W.z, P.rr, P.p3, (const lv_cg_scalars *)W.S);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_INIT64, n, W.S);
-        int done = 0;
-        e = cg_iterate<double>(n, own64(A, n, opt.amg_layout), (const double *)A.diag64,
-                               (const double *)A.dinv64, x, W.r, W.z, W.p, W.q, P, W.S, W.hprog,
-                               W.dprog, W.hS, s, t64, h, (const lv_precond *)nullptr, &done);
-        if (e != hipSuccess) return e;
-        e = read_scalars(W.S, W.hS, &h, s);
-        if (e != hipSuccess) return e;
-        total = h.iters;
-        *relres0 = (h.bb > 0.0) ? sqrt(h.rr0 / h.bb) : sqrt(h.rr0);
-    } else {
-        const int outer_max = opt.outer_max > 0 ? opt.outer_max : 20;
-        const double floor_tol = opt.inner_tol > 0.0 ? opt.inner_tol : 1e-4;
-        // singular systems: the residual after a correction is that of x shifted back to the initial
-        // guess's mean (k_correct writes the sums of x, k_resid64 shifts what it reads); k_shift
-        // stores that x when the sweeps end, so the last residual is the returned x's
-        double *Pxs = A.singular ? P.ur : nullptr;
-        // the iterations of a sweep are still in S at the next sweep's read of the FP64 residual
-        // (k_resid64 and k_finalize leave them), so a sweep ends without a synchronising read.
-        // Nor does the first sweep wait for one: k_cg32_init makes the tests below on the device, and a first
-        // sweep with nothing to solve starts done and changes nothing (its correction is zero).
-        bool pending = false;
-        double itol = 0.0;
-        for (;;) {
-            launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3,
-                           nsweep > 0 ? (const double *)Pxs : (const double *)nullptr,
-                           nsweep > 0 ? (const double *)nullptr : (const double *)Pm, W.S);
-            if (nsweep > 0) {
-                const int seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
-                hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n,
-                                   W.S, W.dprog, seq);
-                e = await_published(W.hprog, seq, W.S, W.hS, &h, s);
-                if (e != hipSuccess) return e;
-                if (pending) total += h.iters;
-                pending = false;
-                if (nsweep == 1) {
-                    *relres0 = (h.bb > 0.0) ? sqrt(h.rr64_0 / h.bb) : sqrt(h.rr64_0);
-                    skipped = h.skip;  // the first sweep had nothing to solve (not reported as a sweep)
-                }
-                if (h.rr64 <= h.thr2 || nsweep >= outer_max || !(h.rr64 == h.rr64)) break;
-                // ask the FP32 sweep for just the reduction still missing, with a margin of 0.8 for
-                // the FP32 residual's drift from the FP64 one (a few per cent at these reductions: at
-                // margins up to 0.9 no 2048^2 benchmark solve needed an extra sweep), but not below
-                // what FP32 arithmetic can deliver in one sweep (the first sweep's is the same rule,
-                // evaluated by k_cg32_init)
-                const double need = 0.8 * sqrt(h.thr2 / h.rr64);
-                itol = need > floor_tol ? need : floor_tol;
-                if (itol > 0.8) itol = 0.8;
+    int nsweep = 0, skipped = 0;
+    const int outer_max = opt.outer_max > 0 ? opt.outer_max : 20;
+    const double floor_tol = opt.inner_tol > 0.0 ? opt.inner_tol : 1e-4;
+    // singular systems: the residual after a correction is that of x shifted back to the initial
+    // guess's mean (k_correct writes the sums of x, k_resid64 shifts what it reads); k_shift
+    // stores that x when the sweeps end, so the last residual is the returned x's
+    double *Pxs = A.singular ? P.ur : nullptr;
+    // the iterations of a sweep are still in S at the next sweep's read of the FP64 residual
+    // (k_resid64 and k_finalize leave them), so a sweep ends without a synchronising read.
+    // Nor does the first sweep wait for one: k_cg32_init makes the tests below on the device, and a first
+    // sweep with nothing to solve starts done and changes nothing (its correction is zero).
+    bool pending = false;
+    double itol = 0.0;
+    for (;;) {
+        launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3,
+                       nsweep > 0 ? (const double *)Pxs : (const double *)nullptr,
+                       nsweep > 0 ? (const double *)nullptr : (const double *)Pm, W.S);
+        if (nsweep > 0) {
+            const int seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
+            hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n,
+                               W.S, W.dprog, seq);
+            e = await_published(W.hprog, seq, W.S, W.hS, &h, s);
+            if (e != hipSuccess) return e;
+            if (pending) total += h.iters;
+            pending = false;
+            if (nsweep == 1) {
+                *relres0 = relative(h.rr64_0, h.bb);
+                skipped = h.skip;  // the first sweep had nothing to solve (not reported as a sweep)
             }
-            const lv_precond *Mi = (opt.method == LV_SOLVER_SPAI || opt.method == LV_SOLVER_AMG) ? M : nullptr;
-            // with the multilevel preconditioner in the aggregate order, the whole FP32 sweep runs in
-            // that order (the FP64 residual and correction stay in the particles' order)
-            const lv_amg *Gp = (Mi && Mi->amg && Mi->amg->perm_ok) ? Mi->amg : nullptr;
-            const float *dinv32 = Gp ? (const float *)Gp->pdinv32 : (const float *)A.dinv32;
-            for (int attempt = 0; attempt < 2; attempt++) {
-                float *z0 = (Mi && Mi->amg && Mi->amg->z0_in) ? Mi->amg->z0 : nullptr;
-                hipLaunchKernelGGL(k_cg32_init, G, dim3(B), 0, s, n, (const double *)W.r,
-                                   Gp ? (const int *)Gp->list : (const int *)nullptr, dinv32, W.e32, W.r32, W.z32,
-                                   P.rr, W.S, z0, z0 ? Mi->amg->fine_scale : 0.0f,
-                                   first_sweep{P.p3, tol2, floor_tol, itmax, (int)A.singular, nsweep == 0 ? 1 : 0});
-                // the threshold, and the done flag of the previous sweep cleared: before the first
-                // application of the preconditioner (which is skipped while done is set), or at its start
-                const bool head = Mi && Mi->amg && lv_amg_takes_head(Mi->amg, nb);
-                if (!head)
-                    hipLaunchKernelGGL(k_finalize2, dim3(1), dim3(B), 0, s, (const double *)P.rr, nb, itol * itol,
-                                       W.S, nsweep == 0 ? 1 : 0);
-                if (Mi && Mi->amg) {
-                    const lv_cycle_head H{P.rr, nb, W.S, W.dprog, -1, itol * itol, nsweep == 0 ? 1 : 0};
-                    e = lv_amg_vcycle(Mi->amg, A, (const float *)W.r32, W.z32, P.rr, (const lv_cg_scalars *)W.S, s,
-                                      z0 != nullptr, head ? &H : nullptr);
-                    if (e != hipSuccess) return e;
-                } else if (Mi) {
-                    hipLaunchKernelGGL(k_apply_m32, G, dim3(B), 0, s, n, (const int *)A.deg, (const int *)A.ecol,
-                                       Mi->mval, Mi->mdg, (const float *)W.r32, W.z32, P.rr,
-                                       (const lv_cg_scalars *)W.S);
-                }
-                int done = 0;
-                if (Gp) {
-                    const lv_ell_agg32 V{Gp->pdeg, Gp->poff, Gp->pev32, Gp->ooff, Gp->oev32, Gp->ovf_cap};
-                    auto iterate = [&](const auto &Av) {
-                        return cg_iterate<float>(n, Av, (const float *)Gp->pdiag32, dinv32, W.e32, W.r32, W.z32, W.p32,
-                                                 W.q32, P, W.S, W.hprog, W.dprog, W.hS, s, t32, h, Mi, &done);
-                    };
-                    e = n > LV_NT_ROWS ? iterate(lv_ell_streamed(V)) : iterate(V);
-                } else
-                    e = cg_iterate<float>(n, own32(A, n, opt.amg_layout), (const float *)A.diag32,
-                                          dinv32, W.e32, W.r32, W.z32, W.p32, W.q32, P, W.S, W.hprog, W.dprog,
-                                          W.hS, s, t32, h, Mi, &done);
+            if (h.rr64 <= h.thr2 || nsweep >= outer_max || !(h.rr64 == h.rr64)) break;
+            // ask the FP32 sweep for just the reduction still missing, with a margin of 0.8 for
+            // the FP32 residual's drift from the FP64 one (a few per cent at these reductions: at
+            // margins up to 0.9 no 2048^2 benchmark solve needed an extra sweep), but not below
+            // what FP32 arithmetic can deliver in one sweep (the first sweep's is the same rule,
+            // evaluated by k_cg32_init)
+            const double need = 0.8 * sqrt(h.thr2 / h.rr64);
+            itol = need > floor_tol ? need : floor_tol;
+            if (itol > 0.8) itol = 0.8;
+        }
+        const lv_precond *Mi = (opt.method == LV_SOLVER_SPAI || opt.method == LV_SOLVER_AMG) ? M : nullptr;
+        // with the multilevel preconditioner in the aggregate order, the whole FP32 sweep runs in
+        // that order (the FP64 residual and correction stay in the particles' order)
+        const lv_amg *Gp = (Mi && Mi->amg && Mi->amg->perm_ok) ? Mi->amg : nullptr;
+        const float *dinv32 = Gp ? (const float *)Gp->pdinv32 : (const float *)A.dinv32;
+        for (int attempt = 0; attempt < 2; attempt++) {
+            float *z0 = (Mi && Mi->amg && Mi->amg->z0_in) ? Mi->amg->z0 : nullptr;
+            hipLaunchKernelGGL(k_cg32_init, G, dim3(B), 0, s, n, (const double *)W.r,
+                               Gp ? (const int *)Gp->list : (const int *)nullptr, dinv32, W.e32, W.r32, W.z32,
+                               P.rr, W.S, z0, z0 ? Mi->amg->fine_scale : 0.0f,
+                               first_sweep{P.p3, tol2, floor_tol, itmax, (int)A.singular, nsweep == 0 ? 1 : 0});
+            // the threshold, and the done flag of the previous sweep cleared: before the first
+            // application of the preconditioner (which is skipped while done is set), or at its start
+            const bool head = Mi && Mi->amg && lv_amg_takes_head(Mi->amg, nb);
+            if (!head)
+                hipLaunchKernelGGL(k_finalize2, dim3(1), dim3(B), 0, s, (const double *)P.rr, nb, itol * itol,
+                                   W.S, nsweep == 0 ? 1 : 0);
+            if (Mi && Mi->amg) {
+                const lv_cycle_head H{P.rr, nb, W.S, W.dprog, -1, itol * itol, nsweep == 0 ? 1 : 0};
+                e = lv_amg_vcycle(Mi->amg, A, (const float *)W.r32, W.z32, P.rr, (const lv_cg_scalars *)W.S, s,
+                                  z0 != nullptr, head ? &H : nullptr);
                 if (e != hipSuccess) return e;
-                // Jacobi-PCG is the fallback: a sweep of the learned preconditioner that stalls or breaks
-                // down is redone with Jacobi (after a synchronising read, which also counts its iterations)
-                if (!Mi || done == 1) break;
-                e = read_scalars(W.S, W.hS, &h, s);
-                if (e != hipSuccess) return e;
-                total += h.iters;
-                (*fallbacks)++;
-                Mi = nullptr;
+            } else if (Mi) {
+                hipLaunchKernelGGL(k_apply_m32, G, dim3(B), 0, s, n, (const int *)A.deg, (const int *)A.ecol,
+                                   Mi->mval, Mi->mdg, (const float *)W.r32, W.z32, P.rr,
+                                   (const lv_cg_scalars *)W.S);
             }
-            pending = true;
-            hipLaunchKernelGGL(k_correct, G, dim3(B), 0, s, n, x, (const float *)W.e32,
-                               Gp ? (const int *)Gp->iperm : (const int *)nullptr, Pxs, (const lv_cg_scalars *)W.S,
-                               nsweep == 0 ? 1 : 0);
-            nsweep++;
+            int done = 0;
+            if (Gp) {
+                const lv_ell_agg32 V{Gp->pdeg, Gp->poff, Gp->pev32, Gp->ooff, Gp->oev32, Gp->ovf_cap};
+                auto iterate = [&](const auto &Av) {
+                    return cg_iterate<float>(n, Av, (const float *)Gp->pdiag32, dinv32, W.e32, W.r32, W.z32, W.p32,
+                                             W.q32, P, W.S, W.hprog, W.dprog, W.hS, s, t32, h, Mi, &done);
+                };
+                e = n > LV_NT_ROWS ? iterate(lv_ell_streamed(V)) : iterate(V);
+            } else
+                e = cg_iterate<float>(n, own32(A, n, opt.amg_layout), (const float *)A.diag32,
+                                      dinv32, W.e32, W.r32, W.z32, W.p32, W.q32, P, W.S, W.hprog, W.dprog,
+                                      W.hS, s, t32, h, Mi, &done);
+            if (e != hipSuccess) return e;
+            // Jacobi-PCG is the fallback: a sweep of the learned preconditioner that stalls or breaks
+            // down is redone with Jacobi (after a synchronising read, which also counts its iterations)
+            if (!Mi || done == 1) break;
+            e = read_scalars(W.S, W.hS, &h, s);
+            if (e != hipSuccess) return e;
+            total += h.iters;
+            (*fallbacks)++;
+            Mi = nullptr;
         }
-        if (Pxs && nsweep > 0) hipLaunchKernelGGL(k_shift, G, dim3(B), 0, s, n, x, (const lv_cg_scalars *)W.S);
+        pending = true;
+        hipLaunchKernelGGL(k_correct, G, dim3(B), 0, s, n, x, (const float *)W.e32,
+                           Gp ? (const int *)Gp->iperm : (const int *)nullptr, Pxs, (const lv_cg_scalars *)W.S,
+                           nsweep == 0 ? 1 : 0);
+        nsweep++;
     }
-    if (opt.method == LV_SOLVER_PCG64) {
-        // final FP64 residual of the returned x
-        if (A.singular) {
-            hipLaunchKernelGGL(k_sum1, G, dim3(B), 0, s, n, (const double *)x, P.p3);
-            hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_SUM1, n, W.S);
-            hipLaunchKernelGGL(k_shift, G, dim3(B), 0, s, n, x, (const lv_cg_scalars *)W.S);
-        }
-        launch_resid64(A, opt.amg_layout, G, s, n, b, (const double *)x, W.r, P.p3, (const double *)nullptr,
-                       (const double *)nullptr, W.S);
-        hipLaunchKernelGGL(k_finalize, dim3(1), dim3(B), 0, s, (const double *)P.p3, nb, (int)FIN_RESID, n, W.S);
-        e = read_scalars(W.S, W.hS, &h, s);
-        if (e != hipSuccess) return e;
-    }
+    if (Pxs && nsweep > 0) hipLaunchKernelGGL(k_shift, G, dim3(B), 0, s, n, x, (const lv_cg_scalars *)W.S);
     *iters = total;
     *sweeps = nsweep - skipped;
-    *relres = (h.bb > 0.0) ? sqrt(h.rr64 / h.bb) : sqrt(h.rr64);
+    *relres = relative(h.rr64, h.bb);
     *converged = (h.rr64 <= h.thr2);
     return hipSuccess;
 }

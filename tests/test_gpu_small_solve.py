@@ -77,3 +77,23 @@ def test_steps_equal_launch_by_launch(lv, gpu):
         st = [lv.step_fused(g, d) for _ in range(2)]
         out.append((g.get_soa("x"), g.get_soa("P"), g.get_soa("v"), [k["iters"] for k in st]))
     assert all(np.array_equal(p, q) for p, q in zip(out[0][:3], out[1][:3])) and out[0][3] == out[1][3]
+
+
+@pytest.mark.parametrize("tol", [1e-12, 1e-13])
+@pytest.mark.parametrize("singular,periodic", [(True, False), (False, True)])
+def test_the_true_residual_meets_the_tolerance(lv, gpu, tol, singular, periodic):
+    """near what FP64 reaches the recurrence's residual falls below the tolerance before the true one does: the
+    solve goes on from where it is until the true one has, on either route"""
+    print("true residual %g" % tol, flush=True)
+    g, dt = _grid(lv, 100, 100, singular, periodic)
+    s = lv.PressureSolver(g, method="pcg64", tol=tol, itmax=20000)
+    s.assemble(dt)
+    for seed in range(6):
+        b = np.random.default_rng(seed).standard_normal(g.n)
+        got = []
+        for on in (1, 0):
+            _by_launches(lv, g, on)
+            x = s.solve(b, np.zeros(g.n))
+            assert s.last_stats["relres"][0] <= tol
+            got.append((x, s.last_stats["iters"]))
+        assert np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
