@@ -9,6 +9,7 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <limits.h>
 #include <algorithm>
 #include <mutex>
 #include <string>
@@ -416,6 +417,7 @@ int lv_create(const lv_grid_desc *d, lv_ctx **out)
         e = hipHostMalloc((void **)&ctx->W.hprog, sizeof(lv_progress), hipHostMallocCoherent | hipHostMallocMapped);
     if (e == hipSuccess) {
         memset(ctx->W.hprog, 0, sizeof(lv_progress));
+        ctx->W.ps_looks = INT_MAX;
         e = hipHostGetDevicePointer((void **)&ctx->W.dprog, ctx->W.hprog, 0);
     }
     if (e == hipSuccess) e = lv_mail_init(&ctx->mail);
@@ -1951,6 +1953,14 @@ int lv_timing_seen(lv_ctx *ctx, int32_t kernel_id, int64_t *seen)
 {
     if (!ctx || kernel_id < 0 || kernel_id >= LV_NKTIMERS || !seen) return LV_E_INVALID;
     *seen = ctx->timers[kernel_id]->seen;
+    return LV_OK;
+}
+
+int lv_test_small_solve(lv_ctx *ctx, int32_t looks, int64_t *gave_up)
+{
+    if (!ctx) return LV_E_INVALID;
+    ctx->W.ps_looks = looks < 0 ? INT_MAX : looks;
+    if (gave_up) *gave_up = ctx->W.ps_gave_up;
     return LV_OK;
 }
 

@@ -60,6 +60,9 @@ struct lv_solver_work {
     lv_cg_scalars *S;
     lv_progress *hprog, *dprog;  // the same pinned record: host and device addresses
     lv_cg_scalars *hS;           // pinned host copy of S for the synchronising reads
+    // small FP64 solves in one launch: looks after which a wait ends, and how many solves gave up
+    int ps_looks;
+    int64_t ps_gave_up;
 };
 
 #define LV_TPOOL 1024

@@ -1048,8 +1048,9 @@ __global__ __launch_bounds__(B) void k_correct(int n, double *__restrict__ x, co
 // published, and gathered after they had been seen, an iteration took 5.8 us).
 //
 // A wait ends after 20 ms at the latest: a workgroup that has not been scheduled by then (other work
-// fills the device) makes the launch give up, x untouched or at a valid iterate, and the host runs
-// the solve launch by launch.  256 workgroups of 256 threads at 4 wavefronts per SIMD and more leave room
+// fills the device) makes the launch give up, and the host runs the solve launch by launch.  Some workgroups may
+// have stored their rows of x by then and some not, so k_ps_init keeps the guess, which the host puts back
+// first (a singular system's solution has the guess's mean).  256 workgroups of 256 threads at 4 wavefronts per SIMD and more leave room
 // for the four hardware queues of a process to run one each.
 //
 // Rows, partial sums and their order are those of k_means, k_cg64_init, k_cg_s, k_cg_u, k_sum1, k_shift and
@@ -1084,7 +1085,8 @@ __device__ __forceinline__ double ps_value(double v) { return ps_empty(v) ? __bu
 
 struct ps_state {
     double *slots;
-    int nb, sync;    // workgroups; syncs so far
+    int nb, looks;   // workgroups; a wait also ends after this many looks (tests shorten it)
+    int sync;        // syncs so far
     int at1, at2;    // the slots this workgroup published in at the last two syncs
 };
 
@@ -1135,7 +1137,7 @@ __device__ __forceinline__ bool ps_sum(ps_state &Q, const double (&v)[NV], int a
 #pragma unroll
             for (int q = 0; q < NV; q++) got = got && !ps_empty(p[q]);
             if (got) break;
-            if (expired) {
+            if (expired || spin >= Q.looks) {
                 late[lp] = 1;
                 break;
             }
@@ -1169,10 +1171,12 @@ __device__ __forceinline__ bool ps_sum(ps_state &Q, const double (&v)[NV], int a
 // long)
 template <bool POLL>
 __device__ __forceinline__ double ps_row(const lv_ell_own<double> &A, int i, int n, int deg, const unsigned (&c)[8],
-                                         const double (&v)[8], double di, double yi, const double *y, bool &ok)
+                                         const double (&v)[8], double di, double yi, const double *y, bool &ok,
+                                         int looks = 0)
 {
     unsigned long long t0 = 0;
     auto wait = [&](int spin) {  // false: too long, and looked once more since
+        if (spin >= looks) return false;
         if (spin & 63) return true;
         const unsigned long long now = wall_clock64();
         if (spin == 0) t0 = now;
@@ -1218,13 +1222,17 @@ struct ps_ring {
 };
 
 __global__ __launch_bounds__(B) void k_ps_init(lv_cg_scalars *S, double tol2, int itmax, int singular,
-                                               double *__restrict__ slots, int n, ps_ring Z)
+                                               double *__restrict__ slots, int n, ps_ring Z,
+                                               const double *__restrict__ x, int *__restrict__ lo, int *__restrict__ hi)
 {
     const double empty = __longlong_as_double((long long)PS_EMPTY);
     const int t = blockIdx.x * B + threadIdx.x;
     for (int k = t; k < PS_SLOTS; k += gridDim.x * B) slots[k] = empty;
-    if (t < n)
+    if (t < n) {
         for (int q = 0; q < 3; q++) Z.z[q][t] = empty;
+        lo[t] = __double2loint(x[t]);
+        hi[t] = __double2hiint(x[t]);
+    }
     if (t != 0) return;
     lv_cg_scalars z = {};
     z.tol2 = tol2;
@@ -1233,19 +1241,27 @@ __global__ __launch_bounds__(B) void k_ps_init(lv_cg_scalars *S, double tol2, in
     *S = z;
 }
 
+// the guess that k_ps_init kept
+__global__ __launch_bounds__(B) void k_ps_restore(int n, double *__restrict__ x, const int *__restrict__ lo,
+                                                  const int *__restrict__ hi)
+{
+    const int i = blockIdx.x * B + threadIdx.x;
+    if (i < n) x[i] = __hiloint2double(hi[i], lo[i]);
+}
+
 // x (in/out), r (out: the FP64 residual of the returned x), Z (work); the scalars the host reads in S and
 // published in pub under seq
 __global__ __launch_bounds__(B, 4) void k_pcg_small(int n, lv_ell_own<double> A, const double *__restrict__ diag,
                                                     const double *__restrict__ dinv, const double *__restrict__ b,
                                                     double *x, double *__restrict__ r_out, ps_ring Z, double tol2,
                                                     int itmax, int singular, double *slots, lv_cg_scalars *S,
-                                                    lv_progress *pub, int seq)
+                                                    lv_progress *pub, int seq, int looks)
 {
     const int blk = lv_xcd_block(blockIdx.x, gridDim.x);  // the 256 rows this workgroup owns
     const int i = blk * B + threadIdx.x;
     const bool on = i < n;
     const int row = on ? i : n - 1;
-    ps_state Q{slots, (int)gridDim.x, 0, 0, 0};
+    ps_state Q{slots, (int)gridDim.x, looks, 0, 0, 0};
     unsigned c[8];  // byte offsets
     double v[8];
     int deg;
@@ -1292,7 +1308,7 @@ __global__ __launch_bounds__(B, 4) void k_pcg_small(int n, lv_ell_own<double> A,
                 break;
             }
             const double beta = k == 0 ? 0.0 : rz / rzp;
-            const double w = ps_row<true>(A, row, n, deg, c, v, di, zi, za, ok);
+            const double w = ps_row<true>(A, row, n, deg, c, v, di, zi, za, ok, looks);
             qi = k == 0 ? w : w + beta * qi;
             pi = k == 0 ? zi : zi + beta * pi;
             const double m1[1] = {on ? pi * qi : 0.0};
@@ -1358,7 +1374,10 @@ __global__ __launch_bounds__(B, 4) void k_pcg_small(int n, lv_ell_own<double> A,
         pub->bb = bb;
         pub->thr2 = tol2 * bb;
         pub->iters = k;
+        __threadfence_system();
     }
+    // (after a workgroup that gave up at the last sum of a solve that the others ended, either is right: the host
+    // takes PS_OK only with the values above)
     S->skip = status;
     pub->skip = status;
     __threadfence_system();
@@ -1657,12 +1676,12 @@ hipError_t await_published(lv_progress *hprog, int seq, lv_cg_scalars *dS, lv_cg
     const auto t0 = std::chrono::steady_clock::now();
     for (int spin = 1;; spin++) {
         if (__atomic_load_n(&hprog->fseq, __ATOMIC_ACQUIRE) == seq) {
+            h->skip = __atomic_load_n(&hprog->skip, __ATOMIC_ACQUIRE);
             h->rr64 = hprog->rr64;
             h->rr64_0 = hprog->rr64_0;
             h->bb = hprog->bb;
             h->thr2 = hprog->thr2;
             h->iters = hprog->iters;
-            h->skip = hprog->skip;
             return hipSuccess;
         }
         if ((spin & 255) == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(20))
@@ -1873,22 +1892,26 @@ static hipError_t run_pcg64(const lv_pressure_system &A, lv_solver_work &W, int 
     const double tol2 = opt.tol * opt.tol;
     memset(&h, 0, sizeof(h));
     // a small system in one launch (not while its launches are being timed)
-    if (n <= PS_MAX_ROWS && !(t64 && t64->on)) {
+    const bool small = n <= PS_MAX_ROWS && !(t64 && t64->on);
+    if (small) {
         double *slots = W.partials + (size_t)8 * NBMAX;
         const int seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
         const ps_ring Z{{W.z, W.p, W.q}};
-        hipLaunchKernelGGL(k_ps_init, G, dim3(B), 0, s, W.S, tol2, itmax, (int)A.singular, slots, n, Z);
+        hipLaunchKernelGGL(k_ps_init, G, dim3(B), 0, s, W.S, tol2, itmax, (int)A.singular, slots, n, Z,
+                           (const double *)x, (int *)W.e32, (int *)W.r32);
         hipLaunchKernelGGL(k_pcg_small, G, dim3(B), 0, s, n, own64(A, n), (const double *)A.diag64,
                            (const double *)A.dinv64, b, x, W.r, Z, tol2, itmax, (int)A.singular, slots, W.S, W.dprog,
-                           seq);
+                           seq, W.ps_looks);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         e = await_published(W.hprog, seq, W.S, W.hS, &h, s);
         if (e != hipSuccess) return e;
         if (h.skip == PS_OK) return hipSuccess;
-        // some workgroup was not scheduled in time: launch by launch, after the last of them has ended
+        // some workgroup was not scheduled in time: launch by launch from the guess, after the last of them has ended
         e = hipStreamSynchronize(s);
         if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_ps_restore, grid_of(n), dim3(B), 0, s, n, x, (const int *)W.e32, (const int *)W.r32);
+        W.ps_gave_up++;
         memset(&h, 0, sizeof(h));
     }
     hipLaunchKernelGGL(k_init_scalars, dim3(1), dim3(1), 0, s, W.S, tol2, itmax, (int)A.singular);

@@ -97,3 +97,39 @@ def test_the_true_residual_meets_the_tolerance(lv, gpu, tol, singular, periodic)
             assert s.last_stats["relres"][0] <= tol
             got.append((x, s.last_stats["iters"]))
         assert np.array_equal(got[0][0], got[1][0]) and got[0][1] == got[1][1]
+
+
+def _looks(lv, grid, looks):
+    """waits of at most so many looks from now on; how many solves gave up so far"""
+    c = ctypes.c_int64()
+    assert lv.lib().lv_test_small_solve(grid.ctx, looks, ctypes.byref(c)) == 0
+    return c.value
+
+
+# two workgroups, which often pass a sum that they wait a few looks for; and the most there are
+@pytest.mark.parametrize("nx,ny,tries", [(32, 16, 400), (256, 256, 40)])
+@pytest.mark.parametrize("singular", [True, False])
+def test_a_solve_that_gives_up_starts_again_from_the_guess(lv, gpu, nx, ny, tries, singular):
+    """whatever sum of it a workgroup gave up at, the last ones before and after the workgroups store their rows among them
+    (one iteration, so that every sum has its turn): the launch-by-launch solve of the guess, its mean too, bit for bit"""
+    print("small solve gives up %dx%d" % (nx, ny), flush=True)
+    g, dt = _grid(lv, nx, ny, singular, False)
+    s = lv.PressureSolver(g, method="pcg64", tol=1e-10)
+    s.assemble(dt)
+    rng = np.random.default_rng(nx)
+    b, x0 = rng.standard_normal(g.n), rng.standard_normal(g.n)
+    for itmax in (1, 2):
+        _by_launches(lv, g, 1)
+        want = s.solve(b, x0, raise_on_fail=False, itmax=itmax)
+        _by_launches(lv, g, 0)
+        before = _looks(lv, g, 0)
+        for k in range(tries):
+            _looks(lv, g, k // 10)
+            x = s.solve(b, x0, raise_on_fail=False, itmax=itmax)
+            assert np.array_equal(x, want), "looks %d" % (k // 10)
+            assert s.last_stats["iters"][0] == itmax
+        gave_up = _looks(lv, g, -1) - before
+        print("small solve gave up %d of %d" % (gave_up, tries), flush=True)
+        assert gave_up > 0
+    if singular:
+        assert abs(want.mean() - x0.mean()) < 1e-12
