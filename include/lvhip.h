@@ -304,7 +304,8 @@ int lv_timing_read(lv_ctx *ctx, int32_t kernel_id, double *total_ms, int64_t *la
 int lv_timing_seen(lv_ctx *ctx, int32_t kernel_id, int64_t *seen);
 
 /* For tests of the way out of a small FP64 solve in one launch: from now on its waits end after `looks` looks at
- * what they wait for (negative: not before their 20 ms), and *gave_up (may be null) receives how many gave up so far. */
+ * what they wait for (negative: not before their 20 ms), the rest that follows a solve that gave up is over, and
+ * *gave_up (may be null) receives how many gave up so far. */
 int lv_test_small_solve(lv_ctx *ctx, int32_t looks, int64_t *gave_up);
 
 #ifdef __cplusplus

@@ -1960,6 +1960,7 @@ int lv_test_small_solve(lv_ctx *ctx, int32_t looks, int64_t *gave_up)
 {
     if (!ctx) return LV_E_INVALID;
     ctx->W.ps_looks = looks < 0 ? INT_MAX : looks;
+    ctx->W.ps_rest = 0;
     if (gave_up) *gave_up = ctx->W.ps_gave_up;
     return LV_OK;
 }

@@ -60,8 +60,9 @@ struct lv_solver_work {
     lv_cg_scalars *S;
     lv_progress *hprog, *dprog;  // the same pinned record: host and device addresses
     lv_cg_scalars *hS;           // pinned host copy of S for the synchronising reads
-    // small FP64 solves in one launch: looks after which a wait ends, and how many solves gave up
-    int ps_looks;
+    // small FP64 solves in one launch: looks after which a wait ends, solves still to go launch by launch after one
+    // gave up, and how many did
+    int ps_looks, ps_rest;
     int64_t ps_gave_up;
 };
 

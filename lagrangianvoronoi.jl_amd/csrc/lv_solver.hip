@@ -1050,7 +1050,8 @@ __global__ __launch_bounds__(B) void k_correct(int n, double *__restrict__ x, co
 // A wait ends after 20 ms at the latest: a workgroup that has not been scheduled by then (other work
 // fills the device) makes the launch give up, and the host runs the solve launch by launch.  Some workgroups may
 // have stored their rows of x by then and some not, so k_ps_init keeps the guess, which the host puts back
-// first (a singular system's solution has the guess's mean).  256 workgroups of 256 threads at 4 wavefronts per SIMD and more leave room
+// first (a singular system's solution has the guess's mean).  The next PS_REST solves go launch by launch
+// at once: what filled the device may still be there.  256 workgroups of 256 threads at 4 wavefronts per SIMD and more leave room
 // for the four hardware queues of a process to run one each.
 //
 // Rows, partial sums and their order are those of k_means, k_cg64_init, k_cg_s, k_cg_u, k_sum1, k_shift and
@@ -1062,6 +1063,7 @@ constexpr int PS_SET = PS_COPIES * PS_COPY;
 constexpr int PS_SLOTS = 4 * PS_SET;
 constexpr unsigned long long PS_EMPTY = 0x7FF8A5C3DEADBEEFull;  // a NaN no arithmetic produces by itself
 constexpr unsigned long long PS_WAIT = 2000000;             // 20 ms of the 100 MHz clock
+constexpr int PS_REST = 32;
 enum { PS_OK = 0, PS_GAVE_UP = 2 };
 
 __device__ __forceinline__ void ps_store(double *p, double v)
@@ -1893,7 +1895,9 @@ static hipError_t run_pcg64(const lv_pressure_system &A, lv_solver_work &W, int 
     memset(&h, 0, sizeof(h));
     // a small system in one launch (not while its launches are being timed)
     const bool small = n <= PS_MAX_ROWS && !(t64 && t64->on);
-    if (small) {
+    if (small && W.ps_rest > 0) {
+        W.ps_rest--;
+    } else if (small) {
         double *slots = W.partials + (size_t)8 * NBMAX;
         const int seq = __atomic_load_n(&W.hprog->fseq, __ATOMIC_ACQUIRE) + 1;
         const ps_ring Z{{W.z, W.p, W.q}};
@@ -1911,6 +1915,7 @@ static hipError_t run_pcg64(const lv_pressure_system &A, lv_solver_work &W, int 
         e = hipStreamSynchronize(s);
         if (e != hipSuccess) return e;
         hipLaunchKernelGGL(k_ps_restore, grid_of(n), dim3(B), 0, s, n, x, (const int *)W.e32, (const int *)W.r32);
+        W.ps_rest = PS_REST;
         W.ps_gave_up++;
         memset(&h, 0, sizeof(h));
     }

@@ -133,3 +133,16 @@ def test_a_solve_that_gives_up_starts_again_from_the_guess(lv, gpu, nx, ny, trie
         assert gave_up > 0
     if singular:
         assert abs(want.mean() - x0.mean()) < 1e-12
+
+
+def test_solves_after_one_that_gave_up_do_not_wait_again(lv, gpu):
+    print("small solve rests", flush=True)
+    g, dt = _grid(lv, 100, 100, True, False)
+    s = lv.PressureSolver(g, method="pcg64", tol=1e-10, itmax=4000)
+    s.assemble(dt)
+    b = np.random.default_rng(3).standard_normal(g.n)
+    want = s.solve(b, np.zeros(g.n))
+    before = _looks(lv, g, 0)
+    for _ in range(30):
+        assert np.array_equal(s.solve(b, np.zeros(g.n)), want)
+    assert _looks(lv, g, -1) == before + 1
