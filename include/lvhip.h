@@ -303,6 +303,17 @@ int lv_timing_read(lv_ctx *ctx, int32_t kernel_id, double *total_ms, int64_t *la
 /* launches of the kernel since lv_timing_enable, bracketed or not */
 int lv_timing_seen(lv_ctx *ctx, int32_t kernel_id, int64_t *seen);
 
+/* For tests of the error paths: the next time the context comes to this point it fails there as an allocation does
+ * (0: none). */
+enum {
+    LV_FAIL_CELL_LIST_ROOM = 1, /* room for a larger cell list */
+    LV_FAIL_CELL_LIST = 2,      /* a remesh, between the counts of the cells and their filling */
+    LV_FAIL_ASSEMBLY = 3,       /* an assembly, once its flags may be set */
+    LV_FAIL_AMG_COUNTS = 4,     /* a multilevel set-up, between the counts of the aggregates and their filling */
+    LV_FAIL_AMG_LEVELS = 5      /* the same, at its coarse levels */
+};
+int lv_test_fail(lv_ctx *ctx, int32_t point);
+
 /* For tests of the way out of a small FP64 solve in one launch: from now on its waits end after `looks` looks at
  * what they wait for (negative: not before their 20 ms), the rest that follows a solve that gave up is over, and
  * *gave_up (may be null) receives how many gave up so far. */

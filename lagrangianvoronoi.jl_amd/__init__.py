@@ -156,6 +156,7 @@ _SIGNATURES = {
     "lv_timing_enable": [_P, _I, _I],
     "lv_timing_read": [_P, _I, _P, _P, _P],
     "lv_timing_seen": [_P, _I, _P],
+    "lv_test_fail": [_P, _I],
     "lv_test_small_solve": [_P, _I, _P],
 }
 

@@ -23,7 +23,9 @@ struct lv_amg {
     int nlev;       // coarse levels; level nlev is the dense one
     int n0, na;     // fine rows, level-1 cells
     int xper, yper;
-    int *agg, *cnt, *start, *list;
+    int *agg, *cnt, *start, *list;  // cnt and pflag: zero between set-ups
+    int midway;      // a set-up has not come to its end
+    int fail_at;     // lv_test_fail
     void *scan_tmp;
     size_t cap_agg, cap_list, cap_t0, cap_z0, cap_cnt, cap_start, cap_scan;
     float *t0, *z0; // fine residual and pre-smoothed correction

@@ -2239,12 +2239,15 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
     AMG_CHECK(grow(&G->z0, &G->cap_z0, (size_t)n));
     const size_t cap_cnt = G->cap_cnt;
     AMG_CHECK(grow(&G->cnt, &G->cap_cnt, (size_t)na + 1));
-    if (G->cap_cnt != cap_cnt) AMG_CHECK(hipMemsetAsync(G->cnt, 0, sizeof(int) * (na + 1), s));
+    if (G->cap_cnt != cap_cnt || G->midway) AMG_CHECK(hipMemsetAsync(G->cnt, 0, sizeof(int) * G->cap_cnt, s));
+    if (G->midway) AMG_CHECK(hipMemsetAsync(G->pflag, 0, 2 * sizeof(int), s));
+    G->midway = 1;
     AMG_CHECK(grow(&G->start, &G->cap_start, (size_t)na + 1));
     AMG_CHECK(grow((char **)&G->scan_tmp, &G->cap_scan, lv_scan_temp_bytes((int64_t)na + 1)));
     hipLaunchKernelGGL(k_agg_key, g1(n), dim3(B), 0, s, n, x, g.bxmin0, g.bxmin1, Lx / Kx, Ly / Ky, Kx, Ky, G->agg,
                        G->cnt);
     AMG_CHECK(lv_exclusive_scan_i32(G->cnt, G->start, (int64_t)na + 1, nullptr, G->scan_tmp, s));
+    AMG_CHECK(lv_fail_here(&G->fail_at, LV_FAIL_AMG_COUNTS));
     hipLaunchKernelGGL(k_agg_fill, g1(n), dim3(B), 0, s, n, (const int *)G->agg, (const int *)G->start, G->cnt,
                        G->list);
     AMG_CHECK(level_alloc(G->lev[1], Kx, Ky));
@@ -2290,6 +2293,7 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
         AMG_CHECK(grow(&G->bfirst, &G->cap_bfirst, 2 * ((size_t)nbf + 2)));
         hipLaunchKernelGGL(k_fuse_blocks, g1((int64_t)na + 1), dim3(B), 0, s, na, nbf, (const int *)G->start,
                            reinterpret_cast<int2 *>(G->bfirst), G->pflag);
+        AMG_CHECK(lv_fail_here(&G->fail_at, LV_FAIL_AMG_LEVELS));
         AMG_CHECK(lv_mail_post(&G->mail, G->pflag, 2, 2, s));  // read when the coarse levels are launched
     }
     hipLaunchKernelGGL(k_coarse1, g1((int64_t)na * RL), dim3(B), 0, s, na, Kx, Ky, G->xper, G->yper,
@@ -2390,7 +2394,9 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
             G->fine_scale = OMEGA;
         }
     }
-    return hipGetLastError();
+    AMG_CHECK(hipGetLastError());
+    G->midway = 0;
+    return hipSuccess;
 }
 
 // levels l and l+1 for the pair kernels

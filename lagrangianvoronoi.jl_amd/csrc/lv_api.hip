@@ -63,6 +63,8 @@ struct lv_ctx {
     void *scan_temp = nullptr;
     int *d_flags = nullptr;   // [0] error word, [1] nonsingular flag, [2] a column offset wider than 16 bits (these
                               // three zero between their uses), [3] items of the cell list, [4] couplings
+    bool midway = false;      // a call that uses them (or the cells' counters) has not come to its end
+    int fail_at = 0;          // lv_test_fail: the point that fails next (LV_FAIL_*)
     lv_mailbox mail = {};     // by which the host reads them
     lv_ring ring = {};        // pinned buffers of the large copies
     lv_timer *timers[LV_NKTIMERS] = {nullptr, nullptr, nullptr, nullptr};
@@ -444,6 +446,8 @@ int lv_create(const lv_grid_desc *d, lv_ctx **out)
         memset(ctx->timers[k], 0, sizeof(lv_timer));
         for (int q = 0; q < 2 * LV_TPOOL && e == hipSuccess; q++) e = hipEventCreate(&ctx->timers[k]->ev[q]);
     }
+    // what was cleared and copied above on the null stream, which the context's own does not wait for
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         int code = lv_fail_hip(ctx, e, "lv_create", __FILE__, __LINE__);
         lv_destroy(ctx);
@@ -624,6 +628,17 @@ int lv_field_device_ptr(lv_ctx *ctx, int32_t field, void **dptr)
 
 namespace {
 
+// What calls keep at zero between them (d_flags[0..2], the counters of the cells) cleared, where the last one ended
+// midway: for want of memory, or at a launch that failed.
+int clear_midway(lv_ctx *ctx)
+{
+    if (!ctx->midway) return LV_OK;
+    LV_HIP_CHECK(hipMemsetAsync(ctx->d_flags, 0, 3 * sizeof(int), ctx->s));
+    if (ctx->cl_temp) LV_HIP_CHECK(lv_celllist_temp_init(ctx->cl_temp, (int64_t)ctx->g.n1 * ctx->g.n2, ctx->s));
+    ctx->midway = false;
+    return LV_OK;
+}
+
 // room for `want` items in the cell list (whatever the lists held is dropped)
 int grow_cell_list(lv_ctx *ctx, int64_t want)
 {
@@ -636,6 +651,7 @@ int grow_cell_list(lv_ctx *ctx, int64_t want)
     ctx->cl_temp = nullptr;
     ctx->max_items = 0;
     LV_HIP_CHECK(dalloc(&ctx->cell_labels, want));
+    LV_HIP_CHECK(lv_fail_here(&ctx->fail_at, LV_FAIL_CELL_LIST_ROOM));
     LV_HIP_CHECK(dalloc(&ctx->cell_x, 2 * want + 1));
     LV_HIP_CHECK(hipMalloc(&ctx->cl_temp, lv_celllist_temp_bytes(want, ncells)));
     LV_HIP_CHECK(lv_celllist_temp_init(ctx->cl_temp, ncells, ctx->s));
@@ -660,19 +676,24 @@ static int remesh(lv_ctx *ctx)
     int flags[NFLAGS];
     for (int attempt = 0; attempt < 2; attempt++) {
         if (tc && tc->used == LV_TPOOL) lv_timer_flush(tc);
-        LV_HIP_CHECK(lv_build_cell_list(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x,
-                                        ctx->max_items, ctx->d_flags + 3, ctx->cl_temp, ctx->s,
-                                        tc ? tc->ev[2 * tc->used] : nullptr, tc ? tc->ev[2 * tc->used + 1] : nullptr,
-                                        tc != nullptr));
+        ctx->midway = true;
+        ctx->mesh_valid = false;
+        if (tc) hipEventRecord(tc->ev[2 * tc->used], ctx->s);
+        LV_HIP_CHECK(lv_count_cells(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->max_items, ctx->d_flags + 3,
+                                    ctx->cl_temp, ctx->s));
+        LV_HIP_CHECK(lv_fail_here(&ctx->fail_at, LV_FAIL_CELL_LIST));
+        LV_HIP_CHECK(lv_fill_cells(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x, ctx->max_items,
+                                   ctx->d_flags + 3, ctx->cl_temp, ctx->s));
+        if (tc) hipEventRecord(tc->ev[2 * tc->used + 1], ctx->s);
         if (tc) tc->used++;
         if (tk) lv_timer_begin(tk, ctx->s);
         LV_HIP_CHECK(lv_launch_clip(ctx->g, n, ctx->F.x, ctx->cell_start, ctx->cell_labels, ctx->cell_x, ctx->path_i,
                                     ctx->path_rr, ctx->ne, ctx->ev, ctx->el, n, ctx->F.area, ctx->F.cent, ctx->d_flags,
                                     ctx->clip_retry, ctx->s, (int)ctx->max_items));
         if (tk) lv_timer_end(tk, ctx->s);
-        ctx->mesh_valid = false;
         LV_HIP_CHECK(post_flags(ctx));
         LV_HIP_CHECK(await_flags(ctx, flags));
+        ctx->midway = false;
         if (flags[0] == LV_E_NAN_VELOCITY) break;  // the move's
         ctx->A.valid = 0;
         ctx->nitems = flags[3];
@@ -695,6 +716,8 @@ extern "C" {
 int lv_remesh(lv_ctx *ctx)
 {
     int rc = check_ctx(ctx, false);
+    if (rc) return rc;
+    rc = clear_midway(ctx);
     return rc ? rc : remesh(ctx);
 }
 
@@ -1159,6 +1182,8 @@ int lv_move(lv_ctx *ctx, double dt)
 {
     int rc = check_ctx(ctx, false);
     if (rc) return rc;
+    if ((rc = clear_midway(ctx))) return rc;
+    ctx->midway = true;
     LV_HIP_CHECK(lv_launch_move(ctx->g, ctx->F, mesh_view(ctx), ctx->n, dt, ctx->d_flags, ctx->s));
     ctx->mesh_valid = false;
     return remesh(ctx);
@@ -1204,10 +1229,13 @@ static int assemble_system(lv_ctx *ctx, double dt, int mode, int64_t *nnz, const
     if (rc) return rc;
     const int n = ctx->n;
     lv_mesh_view M = mesh_view(ctx);
+    if ((rc = clear_midway(ctx))) return rc;
+    ctx->midway = true;
     // the degrees, with what the host has to know of the operator; it reads that while the operator is formed
     LV_HIP_CHECK(lv_launch_degree(ctx->F, M, n, dt, mode, ctx->deg, ctx->d_flags + 1, ctx->d_flags + 2, ctx->s));
     // row_ptr[0..n] = exclusive scan of the n degrees followed by one extra slot: deg[n] is 0
     LV_HIP_CHECK(lv_exclusive_scan_i32(ctx->deg, ctx->A.row_ptr, n + 1, ctx->d_flags + 4, ctx->scan_temp, ctx->s));
+    LV_HIP_CHECK(lv_fail_here(&ctx->fail_at, LV_FAIL_ASSEMBLY));
     LV_HIP_CHECK(post_flags(ctx));
     auto assemble = [&]() {  // (does nothing where the couplings have no room)
         return lv_launch_assemble(ctx->g, ctx->F, M, n, dt, mode, ctx->A, ctx->s, rhs_vbc, rhs_vbc ? &ctx->rg : nullptr);
@@ -1215,6 +1243,7 @@ static int assemble_system(lv_ctx *ctx, double dt, int mode, int64_t *nnz, const
     if (ctx->A.nnz_cap > 0) LV_HIP_CHECK(assemble());
     int flags[NFLAGS];
     LV_HIP_CHECK(await_flags(ctx, flags));
+    ctx->midway = false;
     const int total = flags[4];
     if (total > ctx->A.nnz_cap || ctx->A.nnz_cap == 0) {
         LV_HIP_CHECK(hipStreamSynchronize(ctx->s));
@@ -1953,6 +1982,14 @@ int lv_timing_seen(lv_ctx *ctx, int32_t kernel_id, int64_t *seen)
 {
     if (!ctx || kernel_id < 0 || kernel_id >= LV_NKTIMERS || !seen) return LV_E_INVALID;
     *seen = ctx->timers[kernel_id]->seen;
+    return LV_OK;
+}
+
+int lv_test_fail(lv_ctx *ctx, int32_t point)
+{
+    if (!ctx || point < 0) return LV_E_INVALID;
+    ctx->fail_at = point;
+    ctx->amg.fail_at = point;
     return LV_OK;
 }
 

@@ -146,30 +146,32 @@ hipError_t lv_celllist_temp_init(void *temp, int64_t ncells, hipStream_t s)
     return hipGetLastError();
 }
 
-// Builds the cell list of n seeds without waiting for it.  d_nitems receives the item count.  If that
-// exceeds max_items the list is cut off there (cell_start never points beyond it): the caller, who reads
-// the count with its next flags, throws it away and builds again with more room.
-hipError_t lv_build_cell_list(const lv_grid_params &g, int n, const double *x, int *cell_start, int *cell_labels,
-                              double *cell_x, int64_t max_items, int *d_nitems, void *temp, hipStream_t s,
-                              hipEvent_t ev0, hipEvent_t ev1, bool timed)
+// The cell list of n seeds, built in two parts without waiting for either.  The first counts: cell_start, and in
+// d_nitems the item count.  If that exceeds max_items the list is cut off there (cell_start never points beyond
+// it): the caller, who reads the count with its next flags, throws it away and builds again with more room.
+hipError_t lv_count_cells(const lv_grid_params &g, int n, const double *x, int *cell_start, int64_t max_items,
+                          int *d_nitems, void *temp, hipStream_t s)
 {
     const int64_t ncells = (int64_t)g.n1 * g.n2;
     int *cnt = (int *)temp;
     void *scan_tmp = (char *)temp + cell_cnt_bytes(ncells);
-    int2 *items = (int2 *)((char *)scan_tmp + cell_scan_bytes(ncells));
-
-    if (timed) hipEventRecord(ev0, s);
     if (n > 0) hipLaunchKernelGGL(k_img_count, dim3((n + B - 1) / B), dim3(B), 0, s, g, n, x, cnt);
-    hipError_t e = lv_exclusive_scan_i32(cnt, cell_start, ncells + 1, d_nitems, scan_tmp, s,
-                                         (int)(max_items < INT_MAX ? max_items : INT_MAX));
-    if (e != hipSuccess) return e;
+    return lv_exclusive_scan_i32(cnt, cell_start, ncells + 1, d_nitems, scan_tmp, s,
+                                 (int)(max_items < INT_MAX ? max_items : INT_MAX));
+}
+
+// The second fills, and leaves the counters at zero.
+hipError_t lv_fill_cells(const lv_grid_params &g, int n, const double *x, const int *cell_start, int *cell_labels,
+                         double *cell_x, int64_t max_items, const int *d_nitems, void *temp, hipStream_t s)
+{
+    const int64_t ncells = (int64_t)g.n1 * g.n2;
+    int *cnt = (int *)temp;
+    int2 *items = (int2 *)((char *)temp + cell_cnt_bytes(ncells) + cell_scan_bytes(ncells));
     if (n > 0) {
-        hipLaunchKernelGGL(k_img_fill, dim3((n + B - 1) / B), dim3(B), 0, s, g, n, x, cnt, (const int *)cell_start,
+        hipLaunchKernelGGL(k_img_fill, dim3((n + B - 1) / B), dim3(B), 0, s, g, n, x, cnt, cell_start,
                            items, max_items);
         hipLaunchKernelGGL(k_cell_rank, dim3((unsigned)((max_items + B - 1) / B)), dim3(B), 0, s,
-                           (const int *)d_nitems, (const int2 *)items, (const int *)cell_start, cell_labels, cell_x,
-                           x, n, max_items);
+                           d_nitems, (const int2 *)items, cell_start, cell_labels, cell_x, x, n, max_items);
     }
-    if (timed) hipEventRecord(ev1, s);
     return hipGetLastError();
 }

@@ -188,6 +188,14 @@ void lv_mail_free(lv_mailbox *mb);
 hipError_t lv_mail_post(lv_mailbox *mb, int *src, int cnt, int nclear, hipStream_t s);
 hipError_t lv_mail_await(lv_mailbox *mb, int *out, int cnt, hipStream_t s);
 
+// Tests of the error paths (lv_test_fail): the armed point fails, once, as an allocation does.
+static inline hipError_t lv_fail_here(int *armed, int point)
+{
+    if (*armed != point) return hipSuccess;
+    *armed = 0;
+    return hipErrorOutOfMemory;
+}
+
 // lv_scan.hip
 size_t lv_scan_temp_bytes(int64_t n);
 hipError_t lv_exclusive_scan_i32(const int *in, int *out, int64_t n, int *d_total, void *temp, hipStream_t s,
@@ -195,9 +203,10 @@ hipError_t lv_exclusive_scan_i32(const int *in, int *out, int64_t n, int *d_tota
 
 // lv_celllist.hip
 size_t lv_celllist_temp_bytes(int64_t max_items, int64_t ncells);
-hipError_t lv_build_cell_list(const lv_grid_params &g, int n, const double *x, int *cell_start, int *cell_labels,
-                              double *cell_x, int64_t max_items, int *d_nitems, void *temp, hipStream_t s,
-                              hipEvent_t ev0, hipEvent_t ev1, bool timed);
+hipError_t lv_count_cells(const lv_grid_params &g, int n, const double *x, int *cell_start, int64_t max_items,
+                          int *d_nitems, void *temp, hipStream_t s);
+hipError_t lv_fill_cells(const lv_grid_params &g, int n, const double *x, const int *cell_start, int *cell_labels,
+                         double *cell_x, int64_t max_items, const int *d_nitems, void *temp, hipStream_t s);
 hipError_t lv_celllist_temp_init(void *temp, int64_t ncells, hipStream_t s);
 
 // lv_clip.hip.  retry: n + 1 ints of work space (the seeds whose polygon needs the full capacity).

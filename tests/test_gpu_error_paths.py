@@ -1,0 +1,101 @@
+"""Calls that end in the middle (no memory: lv_test_fail makes a point fail as an allocation does) leave nothing behind:
+the next call gives what a context gives that never failed."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+CELL_LIST_ROOM, CELL_LIST, ASSEMBLY, AMG_COUNTS, AMG_LEVELS = 1, 2, 3, 4, 5
+
+
+def _fail(lv, grid, point):
+    assert lv.lib().lv_test_fail(grid.ctx, point) == 0
+
+
+def _grid(lv, K=48, c2=2500.0, remesh=True):
+    x = lv.inputs.jittered_lattice(K, K, 1.0 / K, jitter=0.2, seed=0x5EED1100)
+    grid = lv.VoronoiGrid(lv.UnitRectangle(), 1.0 / K, positions=x)
+    if remesh:
+        lv.remesh(grid)
+        _set(lv, grid, c2)
+    return grid
+
+
+def _set(lv, grid, c2):
+    for name, v in (("rho", 1.0), ("mass", 1.0 / grid.n), ("c2", c2), ("mu", 1e-3)):
+        grid.set(name, np.full(grid.n, v))
+
+
+def _same(a, b):
+    return len(a) == len(b) and all(np.array_equal(p, q) for p, q in zip(a, b))
+
+
+def test_a_refused_move_without_room_for_its_list(lv, gpu):
+    """the move's error is not the next remesh's"""
+    print("fails: room of the list behind a refused move", flush=True)
+    grid = _grid(lv, remesh=False)
+    v = np.zeros(2 * grid.n)
+    v[3] = np.nan
+    grid.set("v", v)
+    _fail(lv, grid, CELL_LIST_ROOM)
+    with pytest.raises(lv.LVError):
+        lv.move(grid, 1e-3)
+    lv.remesh(grid)
+    assert _same(grid.mesh(), _grid(lv).mesh())
+
+
+@pytest.mark.parametrize("point", [CELL_LIST_ROOM, CELL_LIST])
+def test_a_remesh_that_ends_in_the_middle(lv, gpu, point):
+    print("fails: remesh at %d" % point, flush=True)
+    grid = _grid(lv, remesh=False)
+    for again in range(2):  # (the second time there is a list already)
+        if point == CELL_LIST or again == 0:
+            _fail(lv, grid, point)
+            with pytest.raises(lv.LVError):
+                lv.remesh(grid)
+            with pytest.raises(lv.LVError):
+                grid.mesh()
+        lv.remesh(grid)
+        fresh = _grid(lv)
+        assert _same(grid.mesh(), fresh.mesh()) and _same(grid.cell_list(), fresh.cell_list())
+
+
+def test_an_assembly_that_ends_in_the_middle(lv, gpu):
+    """a compressible one, then an incompressible system: singular, its solution with the guess's mean"""
+    print("fails: assembly", flush=True)
+    out = []
+    for failed in (True, False):
+        grid = _grid(lv)
+        s = lv.PressureSolver(grid, method="pcg64", tol=1e-10, itmax=2000)
+        if failed:
+            _fail(lv, grid, ASSEMBLY)
+            with pytest.raises(lv.LVError):
+                s.assemble(1e-3)
+        grid.set("c2", np.inf)
+        s.assemble(1e-3)
+        b = np.random.default_rng(1).standard_normal(grid.n)
+        out.append((s.solve(b, np.full(grid.n, 0.5)),) + tuple(s.operator()))
+    assert _same(*out)
+    assert abs(out[0][0].mean() - 0.5) < 1e-12
+
+
+@pytest.mark.parametrize("point", [AMG_COUNTS, AMG_LEVELS])
+@pytest.mark.parametrize("c2", [2500.0, np.inf])
+def test_a_multilevel_set_up_that_ends_in_the_middle(lv, gpu, point, c2):
+    print("fails: multilevel set-up at %d" % point, flush=True)
+    out = []
+    for failed in (True, False):
+        grid = _grid(lv, c2=c2)
+        s = lv.PressureSolver(grid, method="amg", tol=1e-8)
+        s.assemble(1e-3)
+        b = np.random.default_rng(2).standard_normal(grid.n)
+        for again in range(2):  # (the second time the work space is there)
+            if failed:
+                _fail(lv, grid, point)
+                with pytest.raises(lv.LVError):
+                    s.solve(b, np.zeros(grid.n))
+            x = s.solve(b, np.zeros(grid.n))
+            lv.remesh(grid)
+            s.assemble(1e-3)
+        out.append((x, np.array(s.last_stats["iters"])))
+    assert _same(*out)
