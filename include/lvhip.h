@@ -310,7 +310,8 @@ enum {
     LV_FAIL_CELL_LIST = 2,      /* a remesh, between the counts of the cells and their filling */
     LV_FAIL_ASSEMBLY = 3,       /* an assembly, once its flags may be set */
     LV_FAIL_AMG_COUNTS = 4,     /* a multilevel set-up, between the counts of the aggregates and their filling */
-    LV_FAIL_AMG_LEVELS = 5      /* the same, at its coarse levels */
+    LV_FAIL_AMG_LEVELS = 5,     /* the same, at its coarse levels */
+    LV_FAIL_OPERATOR_ROOM = 6   /* an assembly, room for more couplings */
 };
 int lv_test_fail(lv_ctx *ctx, int32_t point);
 

@@ -1997,6 +1997,7 @@ static hipError_t grow(T **p, size_t *cap, size_t want)
     if (*cap >= want && *p) return hipSuccess;
     if (*p) AMG_CHECK(hipFree(*p));
     *p = nullptr;
+    *cap = 0;
     AMG_CHECK(hipMalloc((void **)p, sizeof(T) * (want ? want : 1)));
     *cap = want;
     return hipSuccess;
@@ -2037,15 +2038,17 @@ static hipError_t level_alloc(lv_amg_level &L, int Kx, int Ky)
     L.Kx = Kx;
     L.Ky = Ky;
     L.n = Kx * Ky;
-    if (L.cap < (size_t)L.n || !L.d) {
+    if (L.cap < (size_t)L.n) {
         void *q[] = {L.d, L.c, L.dinv, L.r, L.z, L.t, L.acc};
+        L.d = L.c = L.dinv = L.r = L.z = L.t = L.acc = nullptr;
+        L.cap = 0;
         for (void *p : q)
             if (p) AMG_CHECK(hipFree(p));
         const size_t m = (size_t)L.n;
         AMG_CHECK(hipMalloc(&L.d, sizeof(float) * m));
         AMG_CHECK(hipMalloc(&L.c, sizeof(float) * 8 * m));
         AMG_CHECK(hipMalloc(&L.dinv, sizeof(float) * m));
-        AMG_CHECK(hipMalloc(&L.r, sizeof(float) * ((m + 3) & ~(size_t)3)));  // read as float4 by k_tail_mv
+        AMG_CHECK(hipMalloc(&L.r, sizeof(float) * ((m + 3) & ~(size_t)3)));  // read as float4 by k_mat_mv
         AMG_CHECK(hipMalloc(&L.z, sizeof(float) * m));
         AMG_CHECK(hipMalloc(&L.t, sizeof(float) * m));
         AMG_CHECK(hipMalloc(&L.acc, sizeof(float) * m));

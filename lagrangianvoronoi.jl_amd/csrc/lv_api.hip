@@ -1231,6 +1231,7 @@ static int assemble_system(lv_ctx *ctx, double dt, int mode, int64_t *nnz, const
     lv_mesh_view M = mesh_view(ctx);
     if ((rc = clear_midway(ctx))) return rc;
     ctx->midway = true;
+    ctx->A.valid = 0;
     // the degrees, with what the host has to know of the operator; it reads that while the operator is formed
     LV_HIP_CHECK(lv_launch_degree(ctx->F, M, n, dt, mode, ctx->deg, ctx->d_flags + 1, ctx->d_flags + 2, ctx->s));
     // row_ptr[0..n] = exclusive scan of the n degrees followed by one extra slot: deg[n] is 0
@@ -1250,7 +1251,12 @@ static int assemble_system(lv_ctx *ctx, double dt, int mode, int64_t *nnz, const
         dfree(ctx->A.cols);
         dfree(ctx->A.val64);
         dfree(ctx->A.val32);
+        ctx->A.cols = nullptr;
+        ctx->A.val64 = nullptr;
+        ctx->A.val32 = nullptr;
+        ctx->A.nnz_cap = 0;
         int64_t want = (int64_t)total + total / 8 + 1024;
+        LV_HIP_CHECK(lv_fail_here(&ctx->fail_at, LV_FAIL_OPERATOR_ROOM));
         LV_HIP_CHECK(dalloc(&ctx->A.cols, want));
         LV_HIP_CHECK(dalloc(&ctx->A.val64, want));
         LV_HIP_CHECK(dalloc(&ctx->A.val32, want));
@@ -1373,6 +1379,7 @@ static int spai_prepare(lv_ctx *ctx, const lv_solve_opts &opt, lv_precond *M, bo
     if (!ctx->amg_ok) return lv_fail(ctx, LV_E_INVALID, "multilevel preconditioner unavailable");
     if (ctx->amg_built_for != ctx->assembly_id || ctx->amg_learned != (int)learned ||
         ctx->amg_layout != opt.amg_layout) {
+        ctx->amg_built_for = -1;  // (none, if this one fails)
         LV_HIP_CHECK(lv_amg_setup(&ctx->amg, ctx->g, ctx->F.x, ctx->A, ctx->n, learned ? ctx->spai.mval : nullptr,
                                   learned ? ctx->spai.mdg : nullptr, opt.amg_layout, ctx->s));
         ctx->amg_built_for = ctx->assembly_id;

@@ -950,6 +950,7 @@ static hipError_t grow(T **p, size_t *cap, size_t want)
     if (*cap >= want && *p) return hipSuccess;
     if (*p) SP_CHECK(hipFree(*p));
     *p = nullptr;
+    *cap = 0;
     SP_CHECK(hipMalloc((void **)p, sizeof(T) * (want ? want : 1)));
     *cap = want;
     return hipSuccess;

@@ -5,7 +5,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-CELL_LIST_ROOM, CELL_LIST, ASSEMBLY, AMG_COUNTS, AMG_LEVELS = 1, 2, 3, 4, 5
+CELL_LIST_ROOM, CELL_LIST, ASSEMBLY, AMG_COUNTS, AMG_LEVELS, OPERATOR_ROOM = 1, 2, 3, 4, 5, 6
 
 
 def _fail(lv, grid, point):
@@ -99,3 +99,39 @@ def test_a_multilevel_set_up_that_ends_in_the_middle(lv, gpu, point, c2):
             s.assemble(1e-3)
         out.append((x, np.array(s.last_stats["iters"])))
     assert _same(*out)
+
+
+def test_an_operator_without_room(lv, gpu):
+    """the couplings' old room is gone and there is no new: no operator, until an assembly finds room (one of as many
+    couplings as the old room held, which is no longer there)"""
+    print("fails: room of the operator", flush=True)
+    K = 48
+    few = lv.inputs.jittered_lattice(K, K, 1.0 / K, jitter=0.0, seed=1)  # four couplings a row
+    grid = _grid(lv, K)
+    s = lv.PressureSolver(grid, method="amg", tol=1e-8)
+    b = np.random.default_rng(3).standard_normal(grid.n)
+    grid.set_positions(few)
+    lv.remesh(grid)
+    _set(lv, grid, 2500.0)
+    s.assemble(1e-3)
+    many = lv.inputs.jittered_lattice(K, K, 1.0 / K, jitter=0.4, seed=2)
+    grid.set_positions(many)
+    lv.remesh(grid)
+    _set(lv, grid, 2500.0)
+    _fail(lv, grid, OPERATOR_ROOM)
+    with pytest.raises(lv.LVError):
+        s.assemble(1e-3)
+    with pytest.raises(lv.LVError, match="not assembled"):
+        s.solve(b, np.zeros(grid.n))
+    with pytest.raises(lv.LVError, match="not assembled"):
+        s.operator()
+    for x in (few, many):
+        out = []
+        for g in (grid, _grid(lv, K)):
+            g.set_positions(x)
+            lv.remesh(g)
+            _set(lv, g, 2500.0)
+            t = lv.PressureSolver(g, method="amg", tol=1e-8)
+            t.assemble(1e-3)
+            out.append((t.solve(b, np.zeros(g.n)),) + tuple(t.operator()))
+        assert _same(*out)
