@@ -311,7 +311,9 @@ enum {
     LV_FAIL_ASSEMBLY = 3,       /* an assembly, once its flags may be set */
     LV_FAIL_AMG_COUNTS = 4,     /* a multilevel set-up, between the counts of the aggregates and their filling */
     LV_FAIL_AMG_LEVELS = 5,     /* the same, at its coarse levels */
-    LV_FAIL_OPERATOR_ROOM = 6   /* an assembly, room for more couplings */
+    LV_FAIL_OPERATOR_ROOM = 6,  /* an assembly, room for more couplings */
+    LV_FAIL_WHOLE_STAGE = 7,    /* the staging of the read-outs, at its full size */
+    LV_FAIL_STAGE = 8           /* the same at every size, until another point is set */
 };
 int lv_test_fail(lv_ctx *ctx, int32_t point);
 

@@ -93,7 +93,8 @@ struct lv_ctx {
     int amg_layout = -1;   // the fine-level layout it was asked for (lv_solve_opts.amg_layout)
     int spmv32_agg = 0;    // the last FP32 inner solve ran in the aggregate order
     int A_kind = 0;        // what A holds: 0 the pressure operator, 1 the implicit viscous operator
-    double *mesh_stage = nullptr;  // staging of the mesh's rows on their way to the host (first use)
+    double *stage = nullptr;       // staging of rows on their way to the host (first use), and its size
+    size_t stage_bytes = 0;
     // multiphase projection work space (allocated on first use)
     lv_mph_work *mph = nullptr;
     // solve timing: event pairs recorded around each solve and read when the API call returns its
@@ -487,7 +488,7 @@ int lv_destroy(lv_ctx *ctx)
         dfree(ctx->pw_P[k]);
         dfree(ctx->pw_AP[k]);
     }
-    dfree(ctx->mesh_stage);
+    dfree(ctx->stage);
     dfree(ctx->pw_t1);
     dfree(ctx->pw_t2);
     dfree(ctx->pw_dots);
@@ -755,14 +756,35 @@ __global__ __launch_bounds__(MB) void k_mesh_rows(lv_mesh_view M, const int *__r
     }
 }
 
-// particles a chunk of mesh rows holds: its staging (at most LV_MAXE edges of 4 + 32 bytes each) is 18 MiB
-constexpr int MESH_CHUNK = 32768;
-constexpr size_t STAGE_BYTES = (size_t)MESH_CHUNK * LV_MAXE * (4 + 32);
+// a particle's mesh rows in the staging: at most LV_MAXE edges of 4 + 32 bytes.  32768 particles at a time: 18 MiB
+constexpr size_t MESH_ROW_BYTES = LV_MAXE * (4 + 32);
+constexpr size_t STAGE_BYTES = 32768 * MESH_ROW_BYTES;
+constexpr size_t STAGE_MIN = STAGE_BYTES / 64;
 
-// the staging of the read-outs (and of a call's scratch that fits it), kept with the context
-hipError_t make_stage(lv_ctx *ctx)
+// The staging of the read-outs (and of a call's scratch that fits it), kept with the context.  A context that fills
+// the device's memory reads out all the same: through what there is, and else through the work space of
+// the pressure gradient, which holds nothing between calls.
+struct stage_view {
+    double *p;
+    size_t bytes;
+};
+bool make_stage(lv_ctx *ctx, size_t bytes)
 {
-    return ctx->mesh_stage ? hipSuccess : dalloc(&ctx->mesh_stage, STAGE_BYTES / sizeof(double));
+    if (ctx->stage) return true;
+    if (ctx->fail_at == LV_FAIL_STAGE || lv_fail_here(&ctx->fail_at, LV_FAIL_WHOLE_STAGE) != hipSuccess ||
+        dalloc(&ctx->stage, bytes / sizeof(double)) != hipSuccess) {
+        (void)hipGetLastError();
+        ctx->stage = nullptr;
+        return false;
+    }
+    ctx->stage_bytes = bytes;
+    return true;
+}
+stage_view stage_of(lv_ctx *ctx)
+{
+    for (size_t bytes = STAGE_BYTES; bytes >= STAGE_MIN; bytes /= 2)
+        if (make_stage(ctx, bytes)) return stage_view{ctx->stage, ctx->stage_bytes};
+    return stage_view{ctx->GP, sizeof(double) * 2 * (size_t)ctx->cap};
 }
 
 // particle i's C components side by side (four: the matrix of column-major planes by rows)
@@ -783,15 +805,16 @@ template <int C>
 int field_rows(lv_ctx *ctx, const double *p, double *host)
 {
     const int n = ctx->n;
-    LV_HIP_CHECK(make_stage(ctx));
-    const int chunk = (int)(STAGE_BYTES / (C * sizeof(double)));
+    const stage_view S = stage_of(ctx);
+    const int chunk = (int)(S.bytes / (C * sizeof(double)));
+    if (chunk < 1) return lv_fail(ctx, LV_E_HIP, "no device memory for a read-out");
     lv_copier D(&ctx->ring, ctx->s, sizeof(double) * C * (size_t)n);
     for (int i0 = 0; i0 < n; i0 += chunk) {
         const int i1 = std::min(n, i0 + chunk);
         hipLaunchKernelGGL(k_field_rows<C>, dim3((i1 - i0 + MB - 1) / MB), dim3(MB), 0, ctx->s, n, i0, i1, p,
-                           ctx->mesh_stage);
+                           S.p);
         LV_HIP_CHECK(hipGetLastError());
-        LV_HIP_CHECK(D.to_host(host + (size_t)C * i0, ctx->mesh_stage, sizeof(double) * C * (size_t)(i1 - i0)));
+        LV_HIP_CHECK(D.to_host(host + (size_t)C * i0, S.p, sizeof(double) * C * (size_t)(i1 - i0)));
     }
     LV_HIP_CHECK(D.finish());
     return LV_OK;
@@ -817,12 +840,14 @@ int mesh_rows(lv_ctx *ctx, const int *hptr, int32_t *labels, double *verts)
 {
     const int n = ctx->n;
     constexpr size_t W = PV == 4 ? 4 : 3;
-    LV_HIP_CHECK(make_stage(ctx));
-    double *dv = ctx->mesh_stage;
+    const stage_view S = stage_of(ctx);
+    const int chunk = (int)(S.bytes / MESH_ROW_BYTES);
+    if (chunk < 1) return lv_fail(ctx, LV_E_HIP, "no device memory for a read-out");
+    double *dv = S.p;
     lv_copier C(&ctx->ring, ctx->s, (size_t)hptr[n] * (W * sizeof(double) + (labels ? sizeof(int32_t) : 0)));
-    int *dl = reinterpret_cast<int *>(dv + (size_t)MESH_CHUNK * LV_MAXE * 4);
-    for (int i0 = 0; i0 < n; i0 += MESH_CHUNK) {
-        const int i1 = std::min(n, i0 + MESH_CHUNK);
+    int *dl = reinterpret_cast<int *>(dv + (size_t)chunk * LV_MAXE * 4);
+    for (int i0 = 0; i0 < n; i0 += chunk) {
+        const int i1 = std::min(n, i0 + chunk);
         const size_t o = (size_t)hptr[i0], m = (size_t)hptr[i1] - o;
         if (m == 0) continue;
         hipLaunchKernelGGL(k_mesh_rows<PV>, dim3((i1 - i0 + MB - 1) / MB), dim3(MB), 0, ctx->s, mesh_view(ctx),
@@ -1028,12 +1053,18 @@ struct dev_buf {
     }
     hipError_t get(lv_ctx *ctx, size_t bytes)
     {
-        if (bytes <= STAGE_BYTES) {
-            hipError_t e = make_stage(ctx);
-            p = ctx->mesh_stage;
-            return e;
+        if (bytes <= STAGE_BYTES && make_stage(ctx, STAGE_BYTES) && bytes <= ctx->stage_bytes) {
+            p = ctx->stage;
+            return hipSuccess;
         }
         hipError_t e = hipMalloc(&p, bytes);
+        if (e != hipSuccess && ctx->stage) {  // (the call's own memory may fit where the staging is)
+            e = hipStreamSynchronize(ctx->s);
+            dfree(ctx->stage);
+            ctx->stage = nullptr;
+            (void)hipGetLastError();
+            if (e == hipSuccess) e = hipMalloc(&p, bytes);
+        }
         own = e == hipSuccess;
         return e;
     }

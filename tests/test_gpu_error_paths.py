@@ -5,7 +5,7 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-CELL_LIST_ROOM, CELL_LIST, ASSEMBLY, AMG_COUNTS, AMG_LEVELS, OPERATOR_ROOM = 1, 2, 3, 4, 5, 6
+CELL_LIST_ROOM, CELL_LIST, ASSEMBLY, AMG_COUNTS, AMG_LEVELS, OPERATOR_ROOM, WHOLE_STAGE, STAGE = range(1, 9)
 
 
 def _fail(lv, grid, point):
@@ -135,3 +135,26 @@ def test_an_operator_without_room(lv, gpu):
             t.assemble(1e-3)
             out.append((t.solve(b, np.zeros(g.n)),) + tuple(t.operator()))
         assert _same(*out)
+
+
+@pytest.mark.parametrize("point", [WHOLE_STAGE, STAGE])
+def test_read_outs_without_room_for_their_staging(lv, gpu, tmp_path, point):
+    """in smaller pieces, or through the context's own work space; a call's scratch in memory of its own"""
+    print("fails: staging %d" % point, flush=True)
+    K = 300
+    q = np.random.default_rng(4).random((5000, 2))
+
+    def grid_of():
+        grid = _grid(lv, K)
+        grid.set_soa("D", np.random.default_rng(5).standard_normal(4 * grid.n))
+        grid.set_soa("v", np.random.default_rng(6).standard_normal(2 * grid.n))
+        return grid
+
+    reads = [lambda g: g.mesh(), lambda g: (g.get("v"), g.get("D")), lambda g: (lv.point_value(g, q, "v[1]"),),
+             lambda g: (lv.nearest_polygon(g, q),), lambda g: (lv.movingls(lv.QuadraticExpansion, g, "v[2]"),),
+             lambda g: (np.frombuffer(open(lv.export_grid(g, str(tmp_path / "f"), "v"), "rb").read(), np.uint8),)]
+    whole = grid_of()
+    for k, read in enumerate(reads):
+        grid = grid_of()
+        _fail(lv, grid, point)
+        assert _same(read(grid), read(whole)), k
