@@ -61,7 +61,8 @@ void lv_copier::work()
 {
     for (;;) {
         unsigned k = claimed.load(std::memory_order_relaxed);
-        if (k == published.load(std::memory_order_acquire)) {
+        // (not == : a claim of another thread may be seen before the piece it claimed is)
+        if ((int)(published.load(std::memory_order_acquire) - k) <= 0) {
             if (stop.load(std::memory_order_acquire)) return;
             std::this_thread::yield();
             continue;
