@@ -32,15 +32,16 @@ struct lv_amg {
     lv_amg_level lev[LV_AMG_MAXLEV + 1];
     float *dense_inv;    // nc * nc, column-major
     float *tail_img;     // the tail levels' constant arrays in their LDS layout (packed per set-up)
-    float *tail_mat, *ext_mat;  // a singular system's W-visit of the tail as a matrix on its first level, and of
-    size_t cap_tail_mat, cap_ext_mat;  // the level above it when that is small enough
+    float *tail_mat, *ext_mat;  // a singular system's W-visit of the tail as a matrix on its first level, and of the
+                                // level above it when that is small enough
+    float *tail_work;           // work space of the former where the LDS does not hold the tail
+    size_t cap_tail_mat, cap_ext_mat, cap_tail_work;
     const float *mat;    // the one the cycle multiplies by, on level lmat, leading dimension mat_ld (0: none, the
     int lmat, mat_ld;    // visit runs its program)
     double *pw;          // power-iteration partials and norms
     float *pv, *pu;      // power-iteration vectors (n0)
     size_t cap_pv, cap_pu;
     int lk;              // first level of the single-workgroup kernel's program (levels lk..nlev)
-    int lds_ok;          // 1: their arrays fit its LDS
     int *desc;           // their descriptors (device) and the host copy
     int tail_coef, tail_inv, tail_total;  // the LDS image's size, its dense inverse, and the LDS in use
     int pair[LV_AMG_MAXLEV + 1];  // pair[l]: levels l and l+1 (both above that kernel's) run as one down and

@@ -20,7 +20,7 @@
 //            ~40 with 2 x 2);
 //   the coarsest level (<= LV_AMG_DENSE_MAX cells) is inverted densely once per assembly.
 // The small levels (from the first of at most LDS_MAX cells, or TAIL_MAX in a singular system) run inside
-// one single-workgroup kernel per cycle (k_tail_lds; k_tail where its LDS does not hold them): they are
+// one single-workgroup kernel per cycle (k_tail_lds): they are
 // too small to fill the device, and one launch replaces two per level.  A singular system's cycle multiplies by
 // the matrix of that kernel's W-visit instead (k_mat_mv).  Above them, levels
 // 2 and up run in pairs, each pair as one down and one up kernel (k_st_down2, k_st_up2) that
@@ -1394,12 +1394,23 @@ struct tail_layout {
     int inv, coef, total;  // [0, coef): the constants, then the work vectors
 };
 
-// the program on the levels' own arrays in global memory, each operation followed by a barrier that makes its
-// writes visible to the workgroup
-__global__ __launch_bounds__(TB) void k_tail(tail_levels T, const int *__restrict__ prog, int nprog,
-                                             const float *__restrict__ inv, const lv_cg_scalars *S)
+// Columns of the W-visited tail's matrix (k_tail_lds<true>) where the levels do not fit the LDS: strips one cell
+// wide, with halos three times their cells.  The program on arrays in global memory, a copy of them (stride floats)
+// for each column, each operation followed by a barrier that makes its writes visible to the workgroup.  (Run
+// in every cycle on the levels' own arrays it made a singular solve on 4000 x 4 particles 4.15 ms, with the matrix
+// from here 0.74.)
+__global__ __launch_bounds__(TB) void k_tail_columns(tail_levels T, const int *__restrict__ prog, int nprog,
+                                                     const float *__restrict__ inv, int stride, float *__restrict__ mat,
+                                                     int ld)
 {
-    if (S && S->done) return;
+    const size_t at = (size_t)blockIdx.x * stride;
+    auto R = [&](int l) { return T.r[l] + at; };
+    auto Z = [&](int l) { return T.z[l] + at; };
+    auto E = [&](int l) { return T.t[l] + at; };
+    auto A = [&](int l) { return T.acc[l] + at; };
+    const int n0 = T.Kx[T.first] * T.Ky[T.first];
+    for (int f = threadIdx.x; f < n0; f += TB) R(T.first)[f] = f == (int)blockIdx.x ? 1.0f : 0.0f;
+    __syncthreads();
     for (int pc = 0; pc < nprog; pc++) {
         const int code = prog[pc];
         const int op = code >> OP_SHIFT, l = code & ((1 << OP_SHIFT) - 1);
@@ -1410,29 +1421,31 @@ __global__ __launch_bounds__(TB) void k_tail(tail_levels T, const int *__restric
             for (int base = 0; base < nc * CF2; base += TB) {  // uniform trip count: every lane shuffles
                 const int tid = base + threadIdx.x;
                 const int P = tid / CF2, q = tid % CF2;
-                const float t = sum_children(st_down_lane(L, Kyc, nc, P, q, T.r[l], T.z[l]));
-                if (q == 0 && P < nc) T.r[l + 1][P] = t;
+                const float t = sum_children(st_down_lane(L, Kyc, nc, P, q, R(l), Z(l)));
+                if (q == 0 && P < nc) R(l + 1)[P] = t;
             }
         } else if (op == OP_DENSE) {
             // t = inv r: 16 lanes per row (LV_AMG_DENSE_MAX * 16 == TB)
             const int i = threadIdx.x >> 4, q = threadIdx.x & 15;
             float acc = 0.0f;
             if (i < n)
-                for (int j = q; j < n; j += 16) acc += inv[j * n + i] * T.r[l][j];
+                for (int j = q; j < n; j += 16) acc += inv[j * n + i] * R(l)[j];
             acc += __shfl_xor(acc, 1);
             acc += __shfl_xor(acc, 2);
             acc += __shfl_xor(acc, 4);
             acc += __shfl_xor(acc, 8);
-            if (q == 0 && i < n) T.t[l][i] = acc;
+            if (q == 0 && i < n) E(l)[i] = acc;
         } else if (op == OP_UP) {
-            for (int f = threadIdx.x; f < n; f += TB) st_up_cell(L, T.Ky[l + 1], f, T.r[l], T.z[l], T.t[l + 1], T.t[l]);
+            for (int f = threadIdx.x; f < n; f += TB) st_up_cell(L, T.Ky[l + 1], f, R(l), Z(l), E(l + 1), E(l));
         } else if (op == OP_WSAVE) {
-            for (int f = threadIdx.x; f < n; f += TB) st_wsave_cell(L, f, T.r[l], T.t[l], T.acc[l]);
+            for (int f = threadIdx.x; f < n; f += TB) st_wsave_cell(L, f, R(l), E(l), A(l));
         } else {  // OP_WADD
-            for (int f = threadIdx.x; f < n; f += TB) T.t[l][f] += T.acc[l][f];
+            for (int f = threadIdx.x; f < n; f += TB) E(l)[f] += A(l)[f];
         }
         __syncthreads();
     }
+    float *row = mat + (size_t)blockIdx.x * ld;
+    for (int f = threadIdx.x; f < ld; f += TB) row[f] = f < n0 ? E(T.first)[f] : 0.0f;
 }
 
 // a / K with rK = 1 / K in FP32, for 0 <= a < 8192: (a + 1/2) / K is at least 1 / (2 K) from an integer, a
@@ -2018,7 +2031,7 @@ hipError_t lv_amg_init(lv_amg *G)
 
 void lv_amg_free(lv_amg *G)
 {
-    void *ptrs[] = {G->agg, G->cnt, G->start, G->list, G->scan_tmp, G->t0, G->z0, G->dense_inv, G->tail_img, G->tail_mat, G->ext_mat,
+    void *ptrs[] = {G->agg, G->cnt, G->start, G->list, G->scan_tmp, G->t0, G->z0, G->dense_inv, G->tail_img, G->tail_mat, G->ext_mat, G->tail_work,
                     G->pw, G->pv, G->pu, G->prog, G->desc, G->iperm, G->aggp, G->pdeg, G->poff, G->pev32, G->pev16,
                     G->pdiag32, G->pdinv32, G->pmval, G->pmdg, G->pflag, G->bfirst, G->ooff, G->oev32};
     for (void *p : ptrs)
@@ -2323,19 +2336,20 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
     while (lt > 1 && G->lev[lt - 1].n <= TAIL_MAX) lt--;
     G->wcycle = A.singular ? 1 : 0;
     // the first level of the single-workgroup kernel: a singular system W-visits the levels of at most TAIL_MAX
-    // cells, a nonsingular one may start a level earlier
+    // cells, a nonsingular one may start a level earlier, or where its levels first fit (strips one cell wide)
     G->lk = lt;
-    if (!G->wcycle)
+    if (!G->wcycle) {
         while (G->lk > 1 && G->lev[G->lk - 1].n <= LDS_MAX) G->lk--;
+        while (G->lk < G->nlev && tail_layout_of(G).total > TAIL_LDS) G->lk++;
+    }
     const int lk = G->lk;
     G->nprog = tail_program(lk, G->nlev, G->wcycle != 0, G->hprog);
     const tail_layout Y = tail_layout_of(G);
-    G->lds_ok = Y.total <= TAIL_LDS && G->nprog <= LV_AMG_MAXPROG ? 1 : 0;  // else its arrays stay in global memory
     G->tail_coef = Y.coef;
     G->tail_inv = Y.inv;
     G->tail_total = Y.total;
-    // a singular system's tail as a matrix (k_tail_lds<true>), and the level above it when it is small
-    const bool mat = G->lds_ok && G->wcycle;
+    // a singular system's tail as a matrix, and the level above it when it is small
+    const bool mat = G->wcycle;
     G->lmat = mat && lk > 1 && G->lev[lk - 1].n <= MAT_MAX ? lk - 1 : lk;
     G->mat_ld = mat ? (G->lev[G->lmat].n + 3) & ~3 : 0;
     // pairs of levels above the tail that run as one kernel each way, from the tail upwards (the
@@ -2355,15 +2369,30 @@ hipError_t lv_amg_setup(lv_amg *G, const lv_grid_params &g, const double *x, con
     const lv_amg_level &D = G->lev[l];
     hipLaunchKernelGGL(k_dense_inverse, dim3(1), dim3(DTB), 0, s, D.Kx, D.Ky, G->xper, G->yper, (const float *)D.d,
                        (const float *)D.c, A.singular, G->dense_inv);
-    if (G->lds_ok) {
+    const bool lds = Y.total <= TAIL_LDS;
+    if (lds)
         hipLaunchKernelGGL(k_tail_pack, dim3(64), dim3(B), 0, s, tail_levels_of(G), Y, (const float *)G->dense_inv,
                            G->tail_img);
-    }
     if (mat) {
         const int nt = G->lev[lk].n, ldt = (nt + 3) & ~3;
         AMG_CHECK(grow(&G->tail_mat, &G->cap_tail_mat, (size_t)nt * ldt));
-        hipLaunchKernelGGL(k_tail_lds<true>, dim3(nt), dim3(TB), 0, s, tail_args_of(G), (const lv_cg_scalars *)nullptr,
-                           G->tail_mat, ldt);
+        if (lds) {
+            hipLaunchKernelGGL(k_tail_lds<true>, dim3(nt), dim3(TB), 0, s, tail_args_of(G),
+                               (const lv_cg_scalars *)nullptr, G->tail_mat, ldt);
+        } else {
+            tail_levels T = tail_levels_of(G);
+            size_t stride = 0;
+            for (int k = lk; k <= G->nlev; k++) stride += 4 * (size_t)G->lev[k].n;
+            AMG_CHECK(grow(&G->tail_work, &G->cap_tail_work, stride * nt));
+            float *w = G->tail_work;
+            for (int k = lk; k <= G->nlev; k++)
+                for (float **p : {&T.r[k], &T.z[k], &T.t[k], &T.acc[k]}) {
+                    *p = w;
+                    w += G->lev[k].n;
+                }
+            hipLaunchKernelGGL(k_tail_columns, dim3(nt), dim3(TB), 0, s, T, (const int *)G->prog, G->nprog,
+                               (const float *)G->dense_inv, (int)stride, G->tail_mat, ldt);
+        }
         G->mat = G->tail_mat;
         if (G->lmat < lk) {
             const lv_amg_level &L = G->lev[G->lmat];
@@ -2488,11 +2517,8 @@ static hipError_t vcycle(const lv_amg *G, const fine_ops<V> &F, const int *agg, 
                            (const float *)G->mat, (const float *)LT.r, LT.t, S,
                            pr ? (const int *)G->start : (const int *)nullptr, G->fine_alpha, G->z0,
                            hd ? *head : lv_cycle_head{});
-    } else if (G->lds_ok)
+    } else
         hipLaunchKernelGGL(k_tail_lds<false>, dim3(1), dim3(TB), 0, s, tail_args_of(G), S, (float *)nullptr, 0);
-    else
-        hipLaunchKernelGGL(k_tail, dim3(1), dim3(TB), 0, s, tail_levels_of(G), (const int *)G->prog, G->nprog,
-                           (const float *)G->dense_inv, S);
     for (int l = lt - 1; l >= 1; l--) {
         if (pairs && l >= 3 && G->pair[l - 1]) {
             const lv_amg_level &L = G->lev[l - 1], &C = G->lev[l], &C2 = G->lev[l + 1];

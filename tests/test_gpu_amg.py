@@ -498,3 +498,48 @@ def test_cg_updates_in_the_down_pass_give_the_fp64_solution(lv, oracle, gpu, kin
     P = {m: solver.solve(b, np.zeros(grid.n), method=m, tol=1e-11, itmax=20000) for m in ("amg", "pcg64")}
     # |A^-1| is at most 1 / (the smallest eigenvalue): residuals of 1e-11 leave errors of 1e-11 cond(A), below 1e-5 here
     assert rel_err(P["amg"] - P["amg"].mean(), P["pcg64"] - P["pcg64"].mean()) <= 1e-5
+
+
+def _strip(lv, nx, ny, c2, periodic=False):
+    dr = 1.0 / nx
+    x = lv.inputs.jittered_lattice(nx, ny, dr, seed=0x5EED0560 + nx)
+    grid = lv.VoronoiGrid(lv.Rectangle((0.0, 0.0), (1.0, ny * dr)), dr, xperiodic=periodic, positions=x)
+    lv.remesh(grid)
+    for k, v in (("rho", np.ones(grid.n)), ("mass", grid.get("area")), ("c2", np.full(grid.n, c2))):
+        grid.set(k, v)
+    solver = lv.PressureSolver(grid, method="amg", tol=1e-8)
+    solver.assemble(0.1 * dr)
+    return grid, solver, x, dr
+
+
+# levels one cell wide whose halos are three times their cells: the tail fits the LDS up to 865 cells long in a W-visit and
+# 904 in a V-visit (each cell's 12 constants, the haloed z and t, r, and a W-visit's accumulator, on levels of n, n/2,
+# ... cells); 4096 x 4 particles have one of 1024, 4400 x 4 one of 1100, 2000 x 2 a first level of 1000
+@pytest.mark.parametrize("nx,ny", [(3000, 4), (4096, 4), (4400, 4), (2000, 2), (8000, 8)])
+@pytest.mark.parametrize("c2,periodic", [(np.inf, False), (2500.0, False), (2500.0, True)])
+def test_strips_match_the_oracle(lv, oracle, gpu, nx, ny, c2, periodic):
+    _flush("amg strip %dx%d" % (nx, ny))
+    grid, solver, x, dr = _strip(lv, nx, ny, c2, periodic)
+    d, rp, cols, coef = solver.operator()
+    H = amg_ref.Hierarchy(x, d, rp, cols, coef, (0.0, 0.0), (1.0, ny * dr), dr, periodic, False, np.isinf(c2))
+    r = np.random.default_rng(11).standard_normal(grid.n)
+    z, zr = solver.apply_preconditioner(r, "amg"), H.apply(r)
+    assert np.linalg.norm(z - zr) <= 1e-4 * np.linalg.norm(zr), np.linalg.norm(z - zr) / np.linalg.norm(zr)
+
+
+def test_a_longer_strip_takes_no_more_than_its_rows(lv, gpu):
+    """singular strips of 3000 x 4 and 4000 x 4 particles, whose tail does and does not fit the LDS: a third more rows and
+    cells, so at most half as long again for an iteration"""
+    _flush("amg strips timed")
+    ms = []
+    for nx in (3000, 4000):
+        grid, solver, x, dr = _strip(lv, nx, 4, np.inf)
+        b = np.random.default_rng(1).standard_normal(grid.n)
+        b = (b - b.mean()) * grid.get("area")
+        best = np.inf
+        for _ in range(6):
+            solver.solve(b, np.zeros(grid.n))
+            best = min(best, solver.last_stats["solve_ms"][0] / solver.last_stats["iters"][0])
+        ms.append(best)
+    print("amg strips: %.1f and %.1f us an iteration" % (1e3 * ms[0], 1e3 * ms[1]), flush=True)
+    assert ms[1] <= 1.5 * ms[0]
