@@ -1360,12 +1360,16 @@ __global__ __launch_bounds__(B) void k_st_up2(st_pair Q, const float *__restrict
 constexpr int TB = 1024;
 constexpr int TAIL_MAX = 1024;  // levels of at most this many cells run in the tail
 // A singular system's cycle multiplies by the matrix of its first level of at most MAT_MAX cells: 26 MB, what
-// the eight L2s hold, so that a small system's cycles find it there (above that the two stencil launches
-// that the level saves cost less than the bytes).
+// the eight L2s hold, so that a small system's cycles find it there.  An iteration with the matrix and with the level's two
+// stencil launches and the next level's matrix: 22.4 and 25.5 us at 33 x 33 cells, 22.1 and 25.7 at 45 x 45, 23.6
+// and 25.7 at 50 x 50, 23.8 and 25.8 at 53 x 53, 26.6 and 25.5 at 56 x 56, 30.2 and 25.4 at 64 x 64, and the set-up
+// 20 to 60 us more: the two cross just above the line.
 constexpr int MAT_MAX = 2560;
 // A nonsingular system, whose tail is visited once a cycle, starts it at its first level of at most LDS_MAX
-// cells (33 x 33 cells: 11.0 us with them, 9.0 and two launches of 3.3 without; the level above, 65 x 65 cells with
-// its couplings in registers, cost it 17 us more, so that level keeps its launches)
+// cells (33 x 33 cells: 11.0 us with them, 9.0 and two launches of 3.3 without).  An iteration at 132^2 to 144^2
+// particles, 33 x 33 to 36 x 36 cells on level 2, takes 34.2 to 35.1 us with them and 37.1 to 38 without; as level 1 (66^2
+// to 70^2 particles) 31 to 32 either way, since the down pass then makes no CG update.  The LDS would hold 38 x 38
+// cells; the level above, 65 x 65 with its couplings in registers, cost 17 us more, so that one keeps its launches.
 constexpr int LDS_MAX = 1280;
 constexpr int LV_DESC = 16;  // ints of a level's descriptor (tail_descriptors)
 constexpr int LV_CELL = 12;  // floats of a cell's constants in the LDS image: c[8], d, 1 / (d + sum c), two unused

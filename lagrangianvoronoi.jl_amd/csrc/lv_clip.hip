@@ -687,9 +687,9 @@ __global__ __launch_bounds__(GB) void k_clip_group(lv_grid_params g, int n, cons
 }
 
 // Up to this many seeds, a group of lanes each.  On lattices of 0.1 dr of jitter clipping takes 34 us with
-// groups and 62 us with a thread per seed (and the queue's launch) at 1,024 seeds, 44 and 71 at 10,000,
-// 78 and 76 at 25,600, 109 and 79 at 40,000; with 0.45 dr of jitter 40 and 97, 54 and 131, 91 and 115, and
-// 105 and 114 at 32,400: the line lies between where the two cross.
+// groups and 62 us with a thread per seed (and the queue's launch) at 1,024 seeds, 43 and 71 at 10,000,
+// 77 and 76 at 25,600, 107 and 79 at 40,000; with 0.45 dr of jitter 40 and 97, 52 and 131, 89 and 114, 103 and 113 at
+// 32,400, and 123 and 152 at 40,000: the line lies between where the two cross.
 constexpr int GROUP_MAX = 32768;
 
 // Up to this many, a thread per seed with ten slots: a CU holds 6 of its 64-seed blocks (23 KB), all blocks are

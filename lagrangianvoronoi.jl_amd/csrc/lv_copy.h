@@ -4,7 +4,8 @@
 // read-out into fresh arrays is that thread's page faults (54 MB: 5.3 ms of a transfer of 1.0).  Here the pieces
 // go through a ring of pinned buffers and a few threads, which live as long as the copy, move them on.  Pieces
 // end at multiples of 2 MiB of the caller's addresses, so that no two threads fault the same huge page.  A mesh of
-// 250,000 particles (54 MB) takes 2.4 ms for 5.3, 10 MB 0.47 for 0.69; 2 MB 0.13 for 0.11, so smaller copies
+// 250,000 particles (54 MB) takes 2.4 ms for 5.3.  Of one field, into memory already touched: 16 MB 0.57 ms for 0.93, 8 MB
+// 0.35 for 0.47, 5 MB 0.26 for 0.29, 3 MB 0.18 for 0.19, 2.5 MB 0.16 for 0.15, 2 MB 0.14 for 0.12: copies below 3 MiB
 // stay the runtime's, and so do copies to the device (3.2 MB 0.15 ms longer this way).
 #pragma once
 

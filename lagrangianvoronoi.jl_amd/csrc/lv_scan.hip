@@ -135,7 +135,8 @@ size_t lv_scan_temp_bytes(int64_t n)
     return (size_t)(nb + 1) * sizeof(int);
 }
 
-// out[j] = min(cap, sum_{k<j} in[j]); *d_total (device, may be null) = sum of all.  in and out may alias.
+// out[j] = min(cap, sum_{k<j} in[j]); *d_total (device, may be null) = sum of all.  in and out are
+// different arrays.
 hipError_t lv_exclusive_scan_i32(const int *in, int *out, int64_t n, int *d_total, void *temp, hipStream_t s, int cap)
 {
     if (n <= 0) return hipSuccess;
